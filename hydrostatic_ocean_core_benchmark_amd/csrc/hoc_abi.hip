@@ -2151,8 +2151,7 @@ static int step_impl(hoc_stepper* h, const hoc_state* in, hoc_state* out, void* 
   { ProfScope _ps(h, "k_momentum_explicit", s);
   launch_momentum_explicit_tiled((h->fp32_parts & HOC_FP32_MOMENTUM_FLUX) != 0, s, d, p, geo,
                                  in->u, in->v, in->b, h->phi,
-                                 h->w, h->Km, h->pgx, h->pgy, nullptr, nullptr, h->dzu, h->dzv,
-                                 h->stu, h->stv); }
+                                 h->w, h->Km, h->pgx, h->pgy, h->dzu, h->dzv, h->stu, h->stv); }
   LAUNCH_CHECK("explicit momentum");
   if (theta) k_div2<<<blocks(d.n2), TPB, 0, s>>>(d, p, geo, h->U0, h->V0, in->eta, h->div0);
   const double* u_it = in->u;

@@ -86,6 +86,12 @@ __device__ __forceinline__ double cg_zc(const double* zs, double dzr, int nw, do
   if (k < nw) return zs[k] + 0.5 * cg_dz(dzr, nw, hb, k);
   return nw > 0 ? zs[nw - 1] + hb : 0.0;
 }
+// The same from zs[k] itself and the depth of the column's bottom (`bottom`,
+// what cg_zc gives at k >= nw).
+__device__ __forceinline__ double cg_zc_at(double zs_k, double dzr, int nw, double hb,
+                                           double bottom, int k) {
+  return k < nw ? zs_k + 0.5 * cg_dz(dzr, nw, hb, k) : bottom;
+}
 // Centre spacing on interface k = 0..nz (libs/core/vertical_var.py:21-32).
 __device__ __forceinline__ double cg_dzi(double dzr, int nw, double hb, int k, int nz) {
   if (k == 0) return cg_dz(dzr, nw, hb, 0);
@@ -177,12 +183,89 @@ __device__ __forceinline__ void xcd_tile(int& bx, int& by) {
   by = L / gx;
 }
 
-// Superbee limiter phi(r) = max(0, max(min(2r, 1), min(r, 2))).
-// F is the arithmetic type (double: the reference's; float: the mixed
-// step's advective fluxes).
+// The same for a 1D grid of gx x gy tiles by `parts` workgroups per tile and
+// range of levels: part fastest (a tile's parts read the same fields, so they
+// run side by side on one XCD), then x, y and the range of levels z.
+struct BlockTile {
+  int part, x, y, z;
+};
+__device__ __forceinline__ BlockTile xcd_block(int gx, int gy, int parts) {
+  const int nb = (int)gridDim.x, id = (int)blockIdx.x;
+  const int x = id % 8, q = nb / 8, r = nb % 8;
+  int L = x * q + (x < r ? x : r) + id / 8;
+  BlockTile t;
+  t.part = L % parts;
+  L /= parts;
+  t.x = L % gx;
+  L /= gx;
+  t.y = L % gy;
+  t.z = L / gy;
+  return t;
+}
+
+// Half the Superbee limiter, phi(r) / 2 = max(0, max(min(r, 1/2), min(r / 2, 1))), with
+// phi(r) = max(0, max(min(2r, 1), min(r, 2))): halving every operand is exact, so
+// half_superbee(r) * d has the bits of (0.5 * phi(r)) * d. The hardware minimum and maximum
+// drop a NaN that NumPy's keep, so a NaN ratio is put back at the end: 8 instructions against
+// 17 for four compare-and-select pairs. F is the arithmetic type (double: the reference's;
+// float: the mixed step's advective fluxes).
+__device__ __forceinline__ double hw_max(double a, double b) { return __builtin_fmax(a, b); }
+__device__ __forceinline__ double hw_min(double a, double b) { return __builtin_fmin(a, b); }
+__device__ __forceinline__ float hw_max(float a, float b) { return __builtin_fmaxf(a, b); }
+__device__ __forceinline__ float hw_min(float a, float b) { return __builtin_fminf(a, b); }
 template <class F>
-__device__ __forceinline__ F superbee(F r) {
-  return nmax(F(0), nmax(nmin(F(2) * r, F(1)), nmin(r, F(2))));
+__device__ __forceinline__ F half_superbee(F r) {
+  const F t = hw_max(hw_max(hw_min(r, F(0.5)), hw_min(F(0.5) * r, F(1))), F(0));
+  return r != r ? r : t;
+}
+
+// Division by a number used many times (a grid spacing, a pivot of several right-hand
+// sides). The compiler's fp64 division is v_rcp, two Newton steps, quotient, remainder and
+// correction, with the operands scaled when they are near the ends of the exponent range;
+// here the reciprocal's part is done once and the quotient's for each numerator, the same
+// operations in the same order (Newton-Raphson with a final remainder correction, Markstein
+// 1990), so the quotient has the same bits: 4 instructions against 11 with a quarter-rate
+// reciprocal. Without the scaling that holds for a normal divisor of moderate exponent
+// (every spacing, thickness and pivot here) and numerators that are 0, non-finite or of
+// magnitude 2^-969 and above; below that the last bit may differ.
+template <class F>
+struct Divisor;
+template <>
+struct Divisor<double> {
+  double d, y;
+  __device__ __forceinline__ explicit Divisor(double d_) : d(d_) {
+    const double y0 = __builtin_amdgcn_rcp(d);
+    const double y1 = __builtin_fma(y0, __builtin_fma(-d, y0, 1.0), y0);
+    y = __builtin_fma(y1, __builtin_fma(-d, y1, 1.0), y1);
+  }
+  __device__ __forceinline__ double operator()(double a) const {
+    const double q = a * y;
+    const double r = __builtin_fma(-d, q, a);
+    return __builtin_amdgcn_div_fixup(__builtin_fma(r, y, q), d, a);
+  }
+};
+// float: the double product with 1/d rounded once more. A quotient of two floats is never
+// within 2^-49 of the middle between two floats unless it is exact, and the product is within
+// 2^-52 of it, so this is the correctly rounded quotient.
+template <>
+struct Divisor<float> {
+  double y;
+  __device__ __forceinline__ explicit Divisor(double d) : y(1.0 / (double)(float)d) {}
+  __device__ __forceinline__ float operator()(float a) const { return (float)((double)a * y); }
+};
+// The same for a divisor that is the same in every lane: its two words are kept in scalar
+// registers.
+__device__ __forceinline__ double uniform_value(double x) {
+  const unsigned long long b = __double_as_longlong(x);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+template <class F>
+__device__ __forceinline__ Divisor<F> uniform_divisor(double d) {
+  Divisor<F> v(d);
+  v.y = uniform_value(v.y);
+  return v;
 }
 
 constexpr double KAPPA = 1.0 / 3.0;
@@ -206,11 +289,11 @@ __device__ __forceinline__ F kappa_face(F cm, F c0, F c1, F c2, F vel, bool wm, 
   F t;
   if (limited) {
     const F r = dc == F(0) ? F(0) : num / dc;
-    t = F(0.5) * superbee(r) * dc;
+    t = half_superbee(r) * dc;
   } else {
     t = F(0.25) * (F(K1M) * num + F(K1P) * dc);
   }
-  const F f = up ? base + t : base - t;
+  const F f = base + (up ? t : -t);
   return (up ? wm : w2) ? f : base;
 }
 
@@ -228,39 +311,59 @@ __device__ __forceinline__ F kappa_face_z(F far_up, F above, F below, F far_dn, 
   F t;
   if (limited) {
     const F r = d == F(0) ? F(0) : num / d;
-    t = F(0.5) * superbee(r) * d;
+    t = half_superbee(r) * d;
   } else {
     t = F(0.25) * (F(K1M) * num + F(K1P) * d);
   }
-  const F f = up ? base + t : base - t;
+  const F f = base + (up ? t : -t);
   return (up ? has_dn : has_up) ? f : base;
 }
 
+// Inverse thicknesses of a column whose levels are all `full` thick down to its
+// last wet one (level n - 1, `last` thick; 0 below): 1/thickness at level k
+// and 1/spacing on interface k (1 <= k < nz, libs/core/vertical_var.py:21-32),
+// formed once per column instead of one division per level. `full` is the same in
+// every lane.
+struct InvCol {
+  int n;
+  double i_full, i_last, z_full, z_step, z_last;
+  __device__ __forceinline__ double inv(int k) const {
+    return k < n - 1 ? i_full : (k == n - 1 ? i_last : 0.0);
+  }
+  __device__ __forceinline__ double idzi(int k) const {
+    return k < n - 1 ? z_full : (k == n - 1 ? z_step : (k == n ? z_last : 0.0));
+  }
+};
+__device__ __forceinline__ InvCol inv_col(int n, double full, double last) {
+  return InvCol{n, uniform_value(safe_inv(full)), safe_inv(last),
+                uniform_value(safe_inv(0.5 * (full + full))),
+                safe_inv(0.5 * (full + last)), safe_inv(0.5 * (last + 0.0))};
+}
+
 // Explicit vertical diffusion of a velocity at level k from its column
-// values f0..f2 (levels k-1..k+1), thicknesses dz0..dz2 and cell masks
-// m0..m2 (libs/core/vertical_var.py:80-106, mask3 branch).
-__device__ __forceinline__ double explicit_diffusion_w(int k, int nz, double f0, double f1,
-                                                       double f2, double dz0, double dz1,
-                                                       double dz2, bool m0, bool m1, bool m2,
-                                                       double nu_k, double nu_k1, double sflux,
-                                                       double drag) {
+// values f0..f2 (levels k-1..k+1), the inverse spacings of interfaces k and
+// k+1, the inverse thickness of level k and the cell masks m0..m2
+// (libs/core/vertical_var.py:80-106, mask3 branch).
+__device__ __forceinline__ double explicit_diffusion_inv(int k, int nz, double f0, double f1,
+                                                         double f2, double idzi_t,
+                                                         double idzi_b, double inv, bool m0,
+                                                         bool m1, bool m2, double nu_k,
+                                                         double nu_k1, double sflux,
+                                                         double drag) {
   const bool bot_km1 = k >= 1 && m0 && !m1;
   const bool bot_k = m1 && !((k + 1 < nz) && m2);
   double ft;
   if (k == 0) {
     ft = sflux;
   } else {
-    const double dzi = (k == nz) ? dz0 : 0.5 * (dz0 + dz1);
-    ft = nu_k * (f0 - f1) * safe_inv(dzi);
+    ft = nu_k * (f0 - f1) * idzi_t;
     if (bot_km1) ft = 0.0;
   }
   double fb = 0.0;
   if (k + 1 < nz) {
-    const double dzi = 0.5 * (dz1 + dz2);
-    fb = nu_k1 * (f1 - f2) * safe_inv(dzi);
+    fb = nu_k1 * (f1 - f2) * idzi_b;
     if (bot_k) fb = 0.0;
   }
-  const double inv = safe_inv(dz1);
   const double out = (ft - fb) * inv;
   const double dr = drag * f1 * (bot_k ? 1.0 : 0.0);
   return (out - dr * inv) * (m1 ? 1.0 : 0.0);

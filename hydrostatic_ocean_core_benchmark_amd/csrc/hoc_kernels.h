@@ -137,8 +137,8 @@ void launch_tracers_tiled(bool mixed, hipStream_t s, Dims d, StepParams p, Geo g
 void launch_momentum_explicit_tiled(bool mixed, hipStream_t s, Dims d, StepParams p, Geo geo,
                                     const double* u, const double* v, const double* b,
                                     const double* phi, const double* w, const double* Km,
-                                    double* pgx, double* pgy, double* avu, double* avv,
-                                    double* dzu, double* dzv, double* stu, double* stv);
+                                    double* pgx, double* pgy, double* dzu, double* dzv,
+                                    double* stu, double* stv);
 
 // hoc_adjoint.hip
 __global__ void k_thomas_adjoint(long long ncol, int n, const double* sub, const double* diag,

@@ -757,522 +757,476 @@ __attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 1))) void k_tracers_col(
 
 namespace hoc {
 
-// Staged tile of one level: the advected velocities and w in the flux type
-// R, the pressure-gradient inputs in fp64.
+// ------------------------------------------------- explicit momentum terms
+// Staged tile of one level for one velocity component A (u or v): A with a
+// 2-cell halo and the other component on the face points around the tile
+// (two buffers: level k + 1 lands while level k is read). Row and column 0 of
+// the other component are the tile's own first row and column for v's faces
+// (A = v) shifted one column west, for u's (A = u) one row south.
 template <class R>
 struct MomLds {
-  R u[SY][SX], v[SY][SX];               // velocities, 2-cell halo
-  uint8_t mu[SY][SX], mv[SY][SX];       // mask3u, mask3v, 2-cell halo
+  R a[SY][SX];
+  R o[TY + 1][TX + 1];
 };
 
-// What only the cell pass reads (one buffer: level k + 1 is stored after the
-// barrier that ends level k and before the face pass of level k + 1, whose
-// closing barrier orders it before the cell pass).
-template <class R>
-struct MomPLds {
-  double phi[TY + 1][TX + 1];           // potential, +1 east / north
-  double b[TY + 1][TX + 1];
-  double zc[TY + 1][TX + 1];
-  R w[TY + 1][TX + 1];                  // w at interface k + 1
+// The level's face masks, for geometry read from the arrays: A's with the
+// halo, the other component's on the own points and one row / column before.
+struct MomMaskLds {
+  uint8_t ma[SY][SX];
+  uint8_t mo[TY + 1][TX + 1];
 };
 
-// Momentum face fluxes of one level, each computed once: advective fluxes
-// (advecting velocity times the face value) and the A_h gradients, on the
-// x-faces (index q: between tile columns q-1 and q) and y-faces (between
-// rows q-1 and q) of the u and v points.
+// Face fluxes of one component on one level, each computed once: the
+// advective flux (advecting velocity times the face value) and the A_h
+// gradient, on the x-faces (index q: between tile columns q-1 and q) and the
+// y-faces (between rows q-1 and q).
 template <class R>
 struct MomFaces {
-  R fux[TY][TX + 1], fvx[TY][TX + 1], gux[TY][TX + 1], gvx[TY][TX + 1];
-  R fuy[TY + 1][TX], fvy[TY + 1][TX], guy[TY + 1][TX], gvy[TY + 1][TX];
+  R fx[TY][TX + 1], gx[TY][TX + 1];
+  R fy[TY + 1][TX], gy[TY + 1][TX];
 };
 
 constexpr int MS_H = (SX * SY + TILE_THREADS - 1) / TILE_THREADS;              // halo slots
-constexpr int MS_P = ((TY + 1) * (TX + 1) + TILE_THREADS - 1) / TILE_THREADS;  // +1 slots
+constexpr int MS_O = ((TY + 1) * (TX + 1) + TILE_THREADS - 1) / TILE_THREADS;  // +1 slots
 
+// Level-k staging held in registers between its global loads and its LDS
+// stores or its use, and this thread's plane offsets.
 template <class R>
 struct MomRegs {
-  R u[MS_H], v[MS_H];
-  uint8_t mu[MS_H], mv[MS_H];
-  double phi[MS_P], b[MS_P], zc[MS_P];
-  R w[MS_P];
+  R a[MS_H], o[MS_O];
+  double phi[2], b[2];  // at the own point and the next one along the component's direction
+  R w[2];               // on interface k + 1
 };
-
+struct MomGeoRegs {  // geometry read from the arrays
+  uint8_t ma[MS_H], mo[MS_O];
+  double zc[2];
+};
 struct MomOffs {
-  int h[MS_H], p[MS_P];
+  unsigned h[MS_H];  // A with its halo
+  unsigned o[MS_O];  // the other component's points
 };
 
+// Value of a plane at a byte offset. The plane's address is the same in every
+// lane and is kept in scalar registers, so that one vector register holds the
+// offset for every array (a plane is below 2^32 bytes). Without the empty asm
+// the compiler keeps a 64-bit vector address per array across the march, 30
+// registers here.
+template <class T>
+__device__ __forceinline__ T at_byte(const T* plane, unsigned off) {
+  unsigned long long a = (unsigned long long)plane;
+  __asm__("" : "+s"(a));
+  using G = const __attribute__((address_space(1))) char;
+  return *(const __attribute__((address_space(1))) T*)((G*)a + off);
+}
+__device__ __forceinline__ void put_byte(double* plane, unsigned off, double v) {
+  unsigned long long a = (unsigned long long)plane;
+  __asm__("" : "+s"(a));
+  using G = __attribute__((address_space(1))) char;
+  *(__attribute__((address_space(1))) double*)((G*)a + off) = v;
+}
+
+// Slots beyond the tile read the own point (the value is not stored).
+template <int COMP>
 __device__ __forceinline__ MomOffs mom_offsets(int tid, int i0, int j0, int nx, int ny) {
   MomOffs F;
 #pragma unroll
   for (int q = 0; q < MS_H; ++q) {
     const int t = tid + q * TILE_THREADS;
-    F.h[q] = t < SX * SY ? pmod(j0 + t / SX - HALO, ny) * nx + pmod(i0 + t % SX - HALO, nx) : -1;
+    const int tt = t < SX * SY ? t : tid;
+    F.h[q] = (unsigned)(pmod(j0 + tt / SX - HALO, ny) * nx + pmod(i0 + tt % SX - HALO, nx));
   }
 #pragma unroll
-  for (int q = 0; q < MS_P; ++q) {
+  for (int q = 0; q < MS_O; ++q) {
     const int t = tid + q * TILE_THREADS;
-    F.p[q] = t < (TY + 1) * (TX + 1)
-                 ? pmod(j0 + t / (TX + 1), ny) * nx + pmod(i0 + t % (TX + 1), nx)
-                 : -1;
+    const int tt = t < (TY + 1) * (TX + 1) ? t : tid;
+    const int lx = tt % (TX + 1), ly = tt / (TX + 1);
+    F.o[q] = (unsigned)(pmod(j0 + ly - (COMP == 0 ? 1 : 0), ny) * nx +
+                        pmod(i0 + lx - (COMP == 0 ? 0 : 1), nx));
   }
   return F;
 }
 
-template <class RT>
-__device__ __forceinline__ void mom_load(MomRegs<RT>& R, const MomOffs& F, long long o, long long n2,
-                                         const double* u, const double* v, const double* phi,
-                                         const double* b, const double* w, const Geo& geo) {
-#pragma unroll
-  for (int q = 0; q < MS_H; ++q) {
-    if (F.h[q] >= 0) {
-      const long long g = o + F.h[q];
-      R.u[q] = (RT)u[g];
-      R.v[q] = (RT)v[g];
-      R.mu[q] = geo.m3u[g];
-      R.mv[q] = geo.m3v[g];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < MS_P; ++q) {
-    if (F.p[q] >= 0) {
-      const long long g = o + F.p[q];
-      R.phi[q] = phi[g];
-      R.b[q] = b[g];
-      R.zc[q] = geo.zc[g];
-      R.w[q] = (RT)w[g + n2];
-    }
-  }
-}
-
-template <class RT>
-__device__ __forceinline__ void mom_store(MomLds<RT>& L, const MomRegs<RT>& R, int tid) {
-#pragma unroll
-  for (int q = 0; q < MS_H; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    if (t < SX * SY) {
-      const int lx = t % SX, ly = t / SX;
-      L.u[ly][lx] = R.u[q];
-      L.v[ly][lx] = R.v[q];
-      L.mu[ly][lx] = R.mu[q];
-      L.mv[ly][lx] = R.mv[q];
-    }
-  }
-}
-
-template <class RT>
-__device__ __forceinline__ void mom_store_p(MomPLds<RT>& P, const MomRegs<RT>& R, int tid) {
-#pragma unroll
-  for (int q = 0; q < MS_P; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    if (t < (TY + 1) * (TX + 1)) {
-      const int lx = t % (TX + 1), ly = t / (TX + 1);
-      P.phi[ly][lx] = R.phi[q];
-      P.b[ly][lx] = R.b[q];
-      P.zc[ly][lx] = R.zc[q];
-      P.w[ly][lx] = R.w[q];
-    }
-  }
-}
-
-// Column-form staging: the velocities with halo and the pressure-gradient
-// inputs are loaded; the level's face masks (with halo) and centre depths
-// are formed from the tile's column geometry into the same LDS layout the
-// field form loads them into.
-template <class R>
-struct MomRegsC {
-  R u[MS_H], v[MS_H];
-  double phi[MS_P], b[MS_P];
-  R w[MS_P];
-};
-
-template <class RT>
-__device__ __forceinline__ void mom_load_c(MomRegsC<RT>& R, const MomOffs& F, long long o,
-                                           long long n2, const double* u, const double* v,
-                                           const double* phi, const double* b, const double* w) {
-#pragma unroll
-  for (int q = 0; q < MS_H; ++q) {
-    if (F.h[q] >= 0) {
-      const long long g = o + F.h[q];
-      R.u[q] = (RT)u[g];
-      R.v[q] = (RT)v[g];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < MS_P; ++q) {
-    if (F.p[q] >= 0) {
-      const long long g = o + F.p[q];
-      R.phi[q] = phi[g];
-      R.b[q] = b[g];
-      R.w[q] = (RT)w[g + n2];
-    }
-  }
-}
-
-template <class RT>
-__device__ __forceinline__ void mom_store_c(MomLds<RT>& L, const MomRegsC<RT>& R,
-                                            const ColTile& CG, int kk, int tid) {
-#pragma unroll
-  for (int q = 0; q < MS_H; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    if (t < SX * SY) {
-      const int lx = t % SX, ly = t / SX;
-      L.u[ly][lx] = R.u[q];
-      L.v[ly][lx] = R.v[q];
-      L.mu[ly][lx] = col_wet_u(CG, ly, lx, kk);
-      L.mv[ly][lx] = col_wet_v(CG, ly, lx, kk);
-    }
-  }
-}
-
-template <class RT>
-__device__ __forceinline__ void mom_store_p_c(MomPLds<RT>& P, const MomRegsC<RT>& R,
-                                              const ColTile& CG, const double* zs, double dzr,
-                                              int kk, int tid) {
-#pragma unroll
-  for (int q = 0; q < MS_P; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    if (t < (TY + 1) * (TX + 1)) {
-      const int lx = t % (TX + 1), ly = t / (TX + 1);
-      P.phi[ly][lx] = R.phi[q];
-      P.b[ly][lx] = R.b[q];
-      P.zc[ly][lx] = cg_zc(zs, dzr, CG.nw[ly + HALO][lx + HALO], CG.hb[ly + HALO][lx + HALO], kk);
-      P.w[ly][lx] = R.w[q];
-    }
-  }
-}
-
 struct NoTile {};
+
+// First threads that form the tile's west column of faces (TY of them) and
+// its south row (TX).
+constexpr int EDGE_X = 64, EDGE_Y = 0;
+static_assert(EDGE_X + TY <= TILE_THREADS && EDGE_Y + TX <= TILE_THREADS, "edge threads");
 
 // Vertical momentum flux on interface kk of the column: wb times the
 // interface value of the advected velocity (advection_v06.py:95-99,
 // advection.py:75-79); f* hold the velocity at kk-2..kk+1, m* the wet flags
 // of kk-2 and kk+1.
-template <class R>
+template <class R, bool TVD>
 __device__ __forceinline__ R mom_flux_z(int adv, int kk, int nz, R wb, R far_up, R above, R below,
                                         R far_dn, bool mup, bool mdn) {
-  if (kk <= 0 || kk >= nz) return R(0);
-  if (adv == ADV_CENTRED2) return wb * R(0.5) * (above + below);
-  const bool hu = kk >= 2 && mup;
-  const bool hd = kk <= nz - 2 && mdn;
-  return wb * kappa_face_z<R>(kk >= 2 ? far_up : R(0), above, below, kk <= nz - 2 ? far_dn : R(0),
-                              wb, hu, hd, adv == ADV_UP3_TVD);
+  R f;
+  if (!TVD && adv == ADV_CENTRED2) {
+    f = wb * R(0.5) * (above + below);
+  } else {
+    const bool hu = kk >= 2 && mup;
+    const bool hd = kk <= nz - 2 && mdn;
+    f = wb * kappa_face_z<R>(kk >= 2 ? far_up : R(0), above, below,
+                             kk <= nz - 2 ? far_dn : R(0), wb, hu, hd,
+                             TVD || adv == ADV_UP3_TVD);
+  }
+  return kk <= 0 || kk >= nz ? R(0) : f;
 }
 
-// The step's explicit momentum terms (libs/core/model3d_v05.py:352-370),
-// tile by tile and level by level; same outputs as k_momentum_explicit.
-// Staging is double-buffered (level k + 1 loads in flight while level k is
-// computed) and every horizontal face flux is formed once. R is the type of
-// the advective fluxes and the A_h gradients (double: bitwise the
-// reference; float: the mixed step); the pressure gradient, the Coriolis
-// partners, the vertical diffusion and the tendencies stay fp64. ZC: the
-// static z-level geometry in column form (masks, face thicknesses and
-// centre depths formed from the tile's column geometry, the same bits).
-template <class R, bool ZC>
-__global__ __launch_bounds__(TILE_THREADS)
-__attribute__((amdgpu_waves_per_eu(ZC ? 3 : 1))) void k_momentum_explicit_tiled(
-    Dims d, StepParams p, Geo geo, const double* __restrict__ u, const double* __restrict__ v,
-    const double* __restrict__ b, const double* __restrict__ phi, const double* __restrict__ w,
-    const double* __restrict__ Km, double* __restrict__ pgx, double* __restrict__ pgy,
-    double* __restrict__ avu, double* __restrict__ avv, double* __restrict__ dzu,
-    double* __restrict__ dzv, double* __restrict__ stu, double* __restrict__ stv) {
-  __shared__ MomLds<R> LB[2];
-  __shared__ MomPLds<R> P;
-  __shared__ MomFaces<R> F;
-  __shared__ std::conditional_t<ZC, ColTile, NoTile> CG;
+// Levels at which the east (axis 0) or north (axis 1) face of column (j, i)
+// is wet, for a static z-level geometry.
+__device__ __forceinline__ int face_levels(const Geo& geo, int axis, int j, int i, int ny,
+                                           int nx) {
+  const int c0 = j * nx + i;
+  const int c1 = axis == 0 ? j * nx + pmod(i + 1, nx) : pmod(j + 1, ny) * nx + i;
+  const int a = geo.nw[c0], b = geo.nw[c1];
+  return (axis == 0 ? geo.mu2[c0] : geo.mv2[c0]) ? (a < b ? a : b) : 0;
+}
+
+// Wet flags that the values of component COMP on the x-face (axis 0) or
+// y-face (axis 1) after column (j, i) need: A's points before and beyond the
+// face's two, and the face's own gradient mask. Each is k < a number of
+// levels, kept in a register for the whole march (bytes: before, beyond, own;
+// a count is at most 255).
+template <int COMP>
+__device__ __forceinline__ unsigned mom_face_wet(const Geo& geo, int axis, int j, int i, int ny,
+                                                 int nx) {
+  const int j0 = pmod(j, ny), i0 = pmod(i, nx);
+  const int jm = axis ? pmod(j - 1, ny) : j0, j2 = axis ? pmod(j + 2, ny) : j0;
+  const int im = axis ? i0 : pmod(i - 1, nx), i2 = axis ? i0 : pmod(i + 2, nx);
+  return (unsigned)face_levels(geo, COMP, jm, im, ny, nx) |
+         (unsigned)face_levels(geo, COMP, j2, i2, ny, nx) << 8 |
+         (unsigned)face_levels(geo, axis, j0, i0, ny, nx) << 16;
+}
+
+// The explicit terms of one velocity component (COMP 0: u, 1: v) of the tile
+// with origin (i0, j0) on the levels [k0, k1).
+template <class R, bool ZC, bool TVD, int COMP, class Mask>
+__device__ __forceinline__ void momentum_component(
+    const Dims& d, const StepParams& p, const Geo& geo, int i0, int j0, int k0, int k1,
+    MomLds<R>* LB, Mask* MB, MomFaces<R>& F, const double* __restrict__ A,
+    const double* __restrict__ O, const double* __restrict__ b, const double* __restrict__ phi,
+    const double* __restrict__ w, const double* __restrict__ Km, const double* __restrict__ zs,
+    double* __restrict__ pg, double* __restrict__ dzo, double* __restrict__ st) {
   const int nx = d.nx, ny = d.ny, nz = d.nz;
   const long long n2 = d.n2;
   const int tid = threadIdx.x;
   const int tx = tid % TX, ty = tid / TX;
-  int bx, by;
-  xcd_tile(bx, by);
-  const int i0 = bx * TX, j0 = by * TY;
   const int i = i0 + tx, j = j0 + ty;
   const bool active = i < nx && j < ny;
-  const long long c = active ? (long long)j * nx + i : 0;
-  int adv = p.advection;
-  if (adv == ADV_UPWIND1) adv = ADV_CENTRED2;  // momentum keeps the centred form
+  // momentum keeps the centred form for upwind1; TVD: the scheme is known at
+  // compile time, so that a level's face values are one straight line
+  const int adv = TVD ? (int)ADV_UP3_TVD
+                      : (p.advection == ADV_UPWIND1 ? (int)ADV_CENTRED2 : p.advection);
   const bool lim = adv == ADV_UP3_TVD;
+  // the tile's west faces and south faces are formed by two different waves
+  const int xe = tid - EDGE_X, ye = tid - EDGE_Y;
+  const Divisor<R> by_dx = uniform_divisor<R>(p.dx), by_dy = uniform_divisor<R>(p.dy),
+                   by_dz = uniform_divisor<R>(p.dz_nom);
+  const Divisor<double> by_ds = uniform_divisor<double>(COMP == 0 ? p.dx : p.dy);
+  const uint8_t* mA = COMP == 0 ? geo.m3u : geo.m3v;
+  const uint8_t* mO = COMP == 0 ? geo.m3v : geo.m3u;
+  const double* dzf = COMP == 0 ? geo.dz3u : geo.dz3v;
+  const double* tau = COMP == 0 ? geo.tau_u : geo.tau_v;
 
-  double km_k = active ? Km[c] : 0.0;
-  R fzu_top = R(0), fzv_top = R(0);
-  const int cx = tx + HALO, cy = ty + HALO;
+  // plane indexes of the own point and of the next one along the component's
+  // direction (clamped into the grid for the lanes beyond it)
+  const int jc = pmod(j, ny), ic = pmod(i, nx);
+  const int cc = jc * nx + ic;
+  const int c1 = COMP == 0 ? jc * nx + pmod(i + 1, nx) : pmod(j + 1, ny) * nx + ic;
+  const unsigned b0 = 8u * (unsigned)cc, b1 = 8u * (unsigned)c1;
 
-  std::conditional_t<ZC, MomRegsC<R>, MomRegs<R>> RG;
-  const MomOffs MO = mom_offsets(tid, i0, j0, nx, ny);
+  MomRegs<R> RG;
+  MomGeoRegs GG;
+  const MomOffs MO = mom_offsets<COMP>(tid, i0, j0, nx, ny);
+  auto load = [&](long long o) {
+#pragma unroll
+    for (int q = 0; q < MS_H; ++q) {
+      RG.a[q] = (R)at_byte(A + o, 8u * MO.h[q]);
+      if constexpr (!ZC) GG.ma[q] = at_byte(mA + o, MO.h[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < MS_O; ++q) {
+      RG.o[q] = (R)at_byte(O + o, 8u * MO.o[q]);
+      if constexpr (!ZC) GG.mo[q] = at_byte(mO + o, MO.o[q]);
+    }
+    RG.phi[0] = at_byte(phi + o, b0);
+    RG.phi[1] = at_byte(phi + o, b1);
+    RG.b[0] = at_byte(b + o, b0);
+    RG.b[1] = at_byte(b + o, b1);
+    RG.w[0] = (R)at_byte(w + o + n2, b0);
+    RG.w[1] = (R)at_byte(w + o + n2, b1);
+    if constexpr (!ZC) {
+      GG.zc[0] = at_byte(geo.zc + o, b0);
+      GG.zc[1] = at_byte(geo.zc + o, b1);
+    }
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < MS_H; ++q) {
+      const int t = tid + q * TILE_THREADS;
+      if (t < SX * SY) {
+        LB[buf].a[t / SX][t % SX] = RG.a[q];
+        if constexpr (!ZC) MB[buf].ma[t / SX][t % SX] = GG.ma[q];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < MS_O; ++q) {
+      const int t = tid + q * TILE_THREADS;
+      if (t < (TY + 1) * (TX + 1)) {
+        LB[buf].o[t / (TX + 1)][t % (TX + 1)] = RG.o[q];
+        if constexpr (!ZC) MB[buf].mo[t / (TX + 1)][t % (TX + 1)] = GG.mo[q];
+      }
+    }
+  };
+  load((long long)k0 * n2);
+
+  // the column form, in registers: wet levels of the east, north and edge
+  // faces' points, the own A point's column, and the cell's and its neighbour's
+  unsigned xw = 0, yw = 0, exw = 0, eyw = 0;
+  InvCol ca{};
+  int nw0 = 0, nw1 = 0, na = 0;
+  double hb0 = 0.0, hb1 = 0.0, bot0 = 0.0, bot1 = 0.0;
   if constexpr (ZC) {
-    mom_load_c(RG, MO, 0, n2, u, v, phi, b, w);
-    col_tile_load(CG, geo, tid, i0, j0, nx, ny);
-    __syncthreads();
-    mom_store_c(LB[0], RG, CG, 0, tid);
-  } else {
-    mom_load(RG, MO, 0, n2, u, v, phi, b, w, geo);
-    mom_store(LB[0], RG, tid);
+    xw = mom_face_wet<COMP>(geo, 0, j, i, ny, nx);
+    yw = mom_face_wet<COMP>(geo, 1, j, i, ny, nx);
+    if (xe >= 0 && xe < TY) exw = mom_face_wet<COMP>(geo, 0, j0 + xe, i0 - 1, ny, nx);
+    if (ye >= 0 && ye < TX) eyw = mom_face_wet<COMP>(geo, 1, j0 - 1, i0 + ye, ny, nx);
+    na = (int)((COMP == 0 ? xw : yw) >> 16);
+    nw0 = geo.nw[cc];
+    nw1 = geo.nw[c1];
+    hb0 = geo.hb[cc];
+    hb1 = geo.hb[c1];
+    bot0 = nw0 > 0 ? zs[nw0 - 1] + hb0 : 0.0;
+    bot1 = nw1 > 0 ? zs[nw1 - 1] + hb1 : 0.0;
+    const double full = uniform_value(face_value(p.face_rule, p.dzr, p.dzr));
+    const double last = na > 0 ? face_value(p.face_rule, cg_dz(p.dzr, nw0, hb0, na - 1),
+                                            cg_dz(p.dzr, nw1, hb1, na - 1))
+                               : 0.0;
+    ca = inv_col(na, full, last);
+  }
+  auto own_wet = [&](int kk) -> bool {  // the own A point
+    if constexpr (ZC) return kk < na;
+    else return at_byte(mA + kk * n2, (unsigned)cc) != 0;
+  };
+  auto cell_wet = [&](int kk) -> bool {
+    if constexpr (ZC) return kk < nw0;
+    else return at_byte(geo.m3 + kk * n2, (unsigned)cc) != 0;
+  };
+  auto idz = [&](int kk) -> double {  // 1 / A's spacing on interface kk, 1 <= kk < nz
+    if constexpr (ZC) return ca.idzi(kk);
+    else return safe_inv(0.5 * (at_byte(dzf + (kk - 1) * n2, b0) + at_byte(dzf + kk * n2, b0)));
+  };
+  auto inv = [&](int kk) -> double {  // 1 / A's thickness
+    if constexpr (ZC) return ca.inv(kk);
+    else return safe_inv(at_byte(dzf + kk * n2, b0));
+  };
+
+  store(0);
+  // own-column window of A at k-2..k+2; its wet flags follow from the level
+  // count, or are bits of one register (bit q: level k-2+q)
+  double a5[5];
+  unsigned m5 = 0;
+  bool cw0 = k0 >= 1 && cell_wet(k0 - 1), cw1 = cell_wet(k0);  // cells k-1, k
+#pragma unroll
+  for (int q = 0; q < 5; ++q) {
+    const int kk = k0 + q - 2;
+    const bool in = kk >= 0 && kk < nz;
+    a5[q] = in ? at_byte(A + kk * n2, b0) : 0.0;
+    if constexpr (!ZC)
+      if (in && own_wet(kk)) m5 |= 1u << q;
+  }
+  auto wet_at = [&](int k, int q) -> bool {  // A's point at level k-2+q
+    if constexpr (ZC) return k + q - 2 >= 0 && k + q - 2 < na;
+    else return (m5 >> q & 1u) != 0;
+  };
+  double km_k = at_byte(Km + k0 * n2, b0);  // K_m and 1 / spacing on interface k
+  double idz_k = k0 > 0 ? idz(k0) : 0.0;
+  R fz_top = R(0);
+  if (k0 > 0 && adv != ADV_NONE) {
+    // the flux through this range's top interface, which the range above
+    // forms as its bottom one: the same operands, the same bits
+    const double* wk = w + (long long)k0 * n2;
+    fz_top = mom_flux_z<R, TVD>(adv, k0, nz, R(0.5) * ((R)at_byte(wk, b0) + (R)at_byte(wk, b1)),
+                           R(a5[0]), R(a5[1]), R(a5[2]), R(a5[3]), wet_at(k0, 0),
+                           wet_at(k0, 3));
   }
   __syncthreads();
-  // own-column windows at k-2..k+2: u, v, mask3u, mask3v; and k-1..k+1 of
-  // dz3u, dz3v, mask3
-  double uw5[5], vw5[5];
-  bool muw[5], mvw[5];
-  double duw[3], dvw[3];
-  bool m3w[3];
-  // own-column geometry at level kk (0 <= kk < nz)
-  auto own_mu = [&](int kk) -> bool {
-    if constexpr (ZC) return col_wet_u(CG, ty + HALO, tx + HALO, kk);
-    else return geo.m3u[kk * n2 + c] != 0;
-  };
-  auto own_mv = [&](int kk) -> bool {
-    if constexpr (ZC) return col_wet_v(CG, ty + HALO, tx + HALO, kk);
-    else return geo.m3v[kk * n2 + c] != 0;
-  };
-  auto own_m3 = [&](int kk) -> bool {
-    if constexpr (ZC) return kk < CG.nw[ty + HALO][tx + HALO];
-    else return geo.m3[kk * n2 + c] != 0;
-  };
-  auto own_du = [&](int kk) -> double {
-    if constexpr (ZC) {
-      const int yy = ty + HALO, xx = tx + HALO;
-      return cg_face(p.face_rule, p.dzr, CG.mu[yy][xx] != 0, CG.nw[yy][xx], CG.hb[yy][xx],
-                     CG.nw[yy][xx + 1], CG.hb[yy][xx + 1], kk);
-    } else {
-      return geo.dz3u[kk * n2 + c];
-    }
-  };
-  auto own_dv = [&](int kk) -> double {
-    if constexpr (ZC) {
-      const int yy = ty + HALO, xx = tx + HALO;
-      return cg_face(p.face_rule, p.dzr, CG.mv[yy][xx] != 0, CG.nw[yy][xx], CG.hb[yy][xx],
-                     CG.nw[yy + 1][xx], CG.hb[yy + 1][xx], kk);
-    } else {
-      return geo.dz3v[kk * n2 + c];
-    }
-  };
-  for (int q = 0; q < 5; ++q) {
-    uw5[q] = vw5[q] = 0.0;
-    muw[q] = mvw[q] = false;
-  }
-  for (int q = 0; q < 3; ++q) {
-    duw[q] = dvw[q] = 0.0;
-    m3w[q] = false;
-  }
-  if (active) {
-    for (int q = 2; q < 5; ++q) {
-      const int kk = q - 2;
-      if (kk < nz) {
-        uw5[q] = u[kk * n2 + c];
-        vw5[q] = v[kk * n2 + c];
-        muw[q] = own_mu(kk);
-        mvw[q] = own_mv(kk);
-      }
-    }
-    for (int q = 1; q < 3; ++q) {
-      const int kk = q - 1;
-      if (kk < nz) {
-        duw[q] = own_du(kk);
-        dvw[q] = own_dv(kk);
-        m3w[q] = own_m3(kk);
-      }
-    }
-  }
-  for (int k = 0; k < nz; ++k) {
+  for (int k = k0; k < k1; ++k) {
     const long long o = (long long)k * n2;
-    const MomLds<R>& L = LB[k & 1];
-    // level k's cell-pass inputs, loaded during level k - 1 (before the
-    // loads of level k + 1 reuse the registers)
-    if constexpr (ZC) mom_store_p_c(P, RG, CG, geo.zs, p.dzr, k, tid);
-    else mom_store_p(P, RG, tid);
-    if (k + 1 < nz) {
-      if constexpr (ZC) mom_load_c(RG, MO, o + n2, n2, u, v, phi, b, w);
-      else mom_load(RG, MO, o + n2, n2, u, v, phi, b, w, geo);
+    const MomLds<R>& L = LB[(k - k0) & 1];
+    // level k's cell-pass inputs, loaded during level k - 1, before the loads
+    // of level k + 1 reuse the registers
+    const double phi0 = RG.phi[0], phi1 = RG.phi[1], bb0 = RG.b[0], bb1 = RG.b[1];
+    const R wb = R(0.5) * (RG.w[0] + RG.w[1]);
+    double zc0, zc1;
+    if constexpr (ZC) {
+      zc0 = cg_zc_at(zs[k], p.dzr, nw0, hb0, bot0, k);
+      zc1 = cg_zc_at(zs[k], p.dzr, nw1, hb1, bot1, k);
+    } else {
+      zc0 = GG.zc[0];
+      zc1 = GG.zc[1];
     }
-    // level-k wet flags of the east (u) and north (v) faces of tile column
-    // (ly, lx), and the centre depth of tile point (ly, lx) of the +1 tile
-    auto MUf = [&](int ly, int lx) -> bool { return L.mu[ly][lx] != 0; };
-    auto MVf = [&](int ly, int lx) -> bool { return L.mv[ly][lx] != 0; };
-    auto ZCf = [&](int ly, int lx) -> double { return P.zc[ly][lx]; };
     // the own column's viscosity below level k, issued before the face pass
-    const double km_k1 = active ? Km[o + n2 + c] : 0.0;
+    const double km_k1 = at_byte(Km + o + n2, b0);
+    if (k + 1 < k1) load(o + n2);
+    const double a_k3 = k + 3 < nz ? at_byte(A + o + 3 * n2, b0) : 0.0;  // the window's next
+    // ---- faces
     {
-      const R(*U)[SX] = L.u;
-      const R(*V)[SX] = L.v;
-      // x-face q of row fy_ (between columns q-1 and q)
-      auto xface = [&](int fy_, int q) {
-        const int yy = fy_ + HALO, x0 = q - 1 + HALO;  // x0: the column west of the face
-        if (adv != ADV_NONE) {
-          const R ub = R(0.5) * (U[yy][x0] + U[yy][x0 + 1]);
-          const R uu = R(0.5) * (U[yy][x0] + U[yy + 1][x0]);
-          if (adv == ADV_CENTRED2) {
-            F.fux[fy_][q] = ub * ub;
-            F.fvx[fy_][q] = uu * (R(0.5) * (V[yy][x0] + V[yy][x0 + 1]));
-          } else {
-            F.fux[fy_][q] = ub * kappa_face<R>(U[yy][x0 - 1], U[yy][x0], U[yy][x0 + 1],
-                                               U[yy][x0 + 2], ub, MUf(yy, x0 - 1),
-                                               MUf(yy, x0 + 2), lim);
-            F.fvx[fy_][q] = uu * kappa_face<R>(V[yy][x0 - 1], V[yy][x0], V[yy][x0 + 1],
-                                               V[yy][x0 + 2], uu, MVf(yy, x0 - 1),
-                                               MVf(yy, x0 + 2), lim);
-          }
+      // the face's wet flags from its packed level counts or the mask tile:
+      // (ym, xm), (y2, x2) the far points, (yy, xx) the point before the face
+      auto flags = [&](unsigned f, int axis, int yy, int xx, bool* m) {
+        if constexpr (ZC) {
+          m[0] = k < (int)(f & 255u);
+          m[1] = k < (int)(f >> 8 & 255u);
+          m[2] = k < (int)(f >> 16);
+        } else {
+          const MomMaskLds& M = MB[(k - k0) & 1];
+          m[0] = (axis ? M.ma[yy - 1][xx] : M.ma[yy][xx - 1]) != 0;
+          m[1] = (axis ? M.ma[yy + 2][xx] : M.ma[yy][xx + 2]) != 0;
+          // the gradient mask: A's own for the face along A, the other's across
+          m[2] = axis == COMP ? M.ma[yy][xx] != 0
+                 : COMP == 0  ? M.mo[yy - HALO + 1][xx - HALO] != 0
+                              : M.mo[yy - HALO][xx - HALO + 1] != 0;
         }
-        const R m = MUf(yy, x0) ? R(1) : R(0);
-        F.gux[fy_][q] = m * (U[yy][x0 + 1] - U[yy][x0]) / R(p.dx);
-        F.gvx[fy_][q] = m * (V[yy][x0 + 1] - V[yy][x0]) / R(p.dx);
       };
-      // y-face q of column fx_ (between rows q-1 and q)
-      auto yface = [&](int q, int fx_) {
-        const int xx = fx_ + HALO, y0 = q - 1 + HALO;  // y0: the row south of the face
+      // x-face q of row r (between columns q-1 and q)
+      auto xface = [&](int r, int q, unsigned f) {
+        const int yy = r + HALO, x0 = q - 1 + HALO;  // x0: the column west of the face
+        bool m[3];
+        flags(f, 0, yy, x0, m);
+        const R a0 = L.a[yy][x0], a1 = L.a[yy][x0 + 1];
         if (adv != ADV_NONE) {
-          const R vb = R(0.5) * (V[y0][xx] + V[y0][xx + 1]);
-          const R vv = R(0.5) * (V[y0][xx] + V[y0 + 1][xx]);
-          if (adv == ADV_CENTRED2) {
-            F.fuy[q][fx_] = vb * (R(0.5) * (U[y0][xx] + U[y0 + 1][xx]));
-            F.fvy[q][fx_] = vv * vv;
-          } else {
-            F.fuy[q][fx_] = vb * kappa_face<R>(U[y0 - 1][xx], U[y0][xx], U[y0 + 1][xx],
-                                               U[y0 + 2][xx], vb, MUf(y0 - 1, xx),
-                                               MUf(y0 + 2, xx), lim);
-            F.fvy[q][fx_] = vv * kappa_face<R>(V[y0 - 1][xx], V[y0][xx], V[y0 + 1][xx],
-                                               V[y0 + 2][xx], vv, MVf(y0 - 1, xx),
-                                               MVf(y0 + 2, xx), lim);
-          }
+          const R vel = COMP == 0 ? R(0.5) * (a0 + a1) : R(0.5) * (L.o[r][q] + L.o[r + 1][q]);
+          if (adv == ADV_CENTRED2)
+            F.fx[r][q] = COMP == 0 ? vel * vel : vel * (R(0.5) * (a0 + a1));
+          else
+            F.fx[r][q] = vel * kappa_face<R>(L.a[yy][x0 - 1], a0, a1, L.a[yy][x0 + 2], vel, m[0],
+                                             m[1], lim);
         }
-        const R m = MVf(y0, xx) ? R(1) : R(0);
-        F.guy[q][fx_] = m * (U[y0 + 1][xx] - U[y0][xx]) / R(p.dy);
-        F.gvy[q][fx_] = m * (V[y0 + 1][xx] - V[y0][xx]) / R(p.dy);
+        F.gx[r][q] = by_dx((m[2] ? R(1) : R(0)) * (a1 - a0));
       };
-      xface(ty, tx + 1);
-      yface(ty + 1, tx);
-      if (tid < TY) xface(tid, 0);
-      else if (tid < TY + TX) yface(0, tid - TY);
+      // y-face q of column r (between rows q-1 and q)
+      auto yface = [&](int q, int r, unsigned f) {
+        const int xx = r + HALO, y0 = q - 1 + HALO;  // y0: the row south of the face
+        bool m[3];
+        flags(f, 1, y0, xx, m);
+        const R a0 = L.a[y0][xx], a1 = L.a[y0 + 1][xx];
+        if (adv != ADV_NONE) {
+          const R vel = COMP == 0 ? R(0.5) * (L.o[q][r] + L.o[q][r + 1]) : R(0.5) * (a0 + a1);
+          if (adv == ADV_CENTRED2)
+            F.fy[q][r] = COMP == 0 ? vel * (R(0.5) * (a0 + a1)) : vel * vel;
+          else
+            F.fy[q][r] = vel * kappa_face<R>(L.a[y0 - 1][xx], a0, a1, L.a[y0 + 2][xx], vel, m[0],
+                                             m[1], lim);
+        }
+        F.gy[q][r] = by_dy((m[2] ? R(1) : R(0)) * (a1 - a0));
+      };
+      xface(ty, tx + 1, xw);
+      yface(ty + 1, tx, yw);
+      if (xe >= 0 && xe < TY) xface(xe, 0, exw);
+      if (ye >= 0 && ye < TX) yface(0, ye, eyw);
     }
     __syncthreads();
-    if (active) {
-      const long long t = o + c;
-      const double mu_c = MUf(cy, cx) ? 1.0 : 0.0, mv_c = MVf(cy, cx) ? 1.0 : 0.0;
+    {
+      const double m_c = wet_at(k, 2) ? 1.0 : 0.0;
       // pressure gradient at the face depth (model3d_v05.py:195-230)
-      double gx, gy;
+      double pg_k;
       if (p.pgf_correction) {
-        const double zc = ZCf(ty, tx);
-        {
-          const double zr = ZCf(ty, tx + 1);
-          const double zf = 0.5 * (zc + zr);
-          const double left = P.phi[ty][tx] + P.b[ty][tx] * (zf - zc);
-          const double right = P.phi[ty][tx + 1] + P.b[ty][tx + 1] * (zf - zr);
-          gx = mu_c * (right - left) / p.dx;
-        }
-        {
-          const double zr = ZCf(ty + 1, tx);
-          const double zf = 0.5 * (zc + zr);
-          const double left = P.phi[ty][tx] + P.b[ty][tx] * (zf - zc);
-          const double right = P.phi[ty + 1][tx] + P.b[ty + 1][tx] * (zf - zr);
-          gy = mv_c * (right - left) / p.dy;
-        }
+        const double zf = 0.5 * (zc0 + zc1);
+        const double left = phi0 + bb0 * (zf - zc0);
+        const double right = phi1 + bb1 * (zf - zc1);
+        pg_k = by_ds(m_c * (right - left));
       } else {
-        gx = mu_c * (P.phi[ty][tx + 1] - P.phi[ty][tx]) / p.dx * mu_c;
-        gy = mv_c * (P.phi[ty + 1][tx] - P.phi[ty][tx]) / p.dy * mv_c;
+        pg_k = by_ds(m_c * (phi1 - phi0)) * m_c;
       }
-      pgx[t] = gx;
-      pgy[t] = gy;
-      // Coriolis partners (operators_masked.py:45-61), fp64: from the tile
-      // in the plain step, from the fp64 fields (neighbours in cache) when
-      // the tile holds fp32 velocities
-      double vc0, vs, ve, vse, uc0, uw, un, unw;
-      if constexpr (sizeof(R) == sizeof(double)) {
-        vc0 = L.v[cy][cx], vs = L.v[cy - 1][cx], ve = L.v[cy][cx + 1], vse = L.v[cy - 1][cx + 1];
-        uc0 = L.u[cy][cx], uw = L.u[cy][cx - 1], un = L.u[cy + 1][cx], unw = L.u[cy + 1][cx - 1];
-      } else {
-        const long long rj = (long long)j * nx, rs = (long long)pmod(j - 1, ny) * nx,
-                        rn = (long long)pmod(j + 1, ny) * nx;
-        const int ie = pmod(i + 1, nx), iw = pmod(i - 1, nx);
-        vc0 = vw5[2], vs = v[o + rs + i], ve = v[o + rj + ie], vse = v[o + rs + ie];
-        uc0 = uw5[2], uw = u[o + rj + iw], un = u[o + rn + i], unw = u[o + rn + iw];
-      }
-      if (avv) {  // the Coriolis partners, for callers that ask for them
-        const double w0 = mv_c, w1 = MVf(cy - 1, cx) ? 1.0 : 0.0,
-                     w2 = MVf(cy, cx + 1) ? 1.0 : 0.0, w3 = MVf(cy - 1, cx + 1) ? 1.0 : 0.0;
-        const double num = 0.0 + w0 * vc0 + w1 * vs + w2 * ve + w3 * vse;
-        const double den = 0.0 + w0 + w1 + w2 + w3;
-        avv[t] = (den > 0.0 ? num / den : 0.0) * mu_c;
-      }
-      if (avu) {
-        const double w0 = mu_c, w1 = MUf(cy, cx - 1) ? 1.0 : 0.0,
-                     w2 = MUf(cy + 1, cx) ? 1.0 : 0.0, w3 = MUf(cy + 1, cx - 1) ? 1.0 : 0.0;
-        const double num = 0.0 + w0 * uc0 + w1 * uw + w2 * un + w3 * unw;
-        const double den = 0.0 + w0 + w1 + w2 + w3;
-        avu[t] = (den > 0.0 ? num / den : 0.0) * mv_c;
-      }
-      // explicit vertical diffusion with surface stress and bottom drag (for
-      // callers that ask for it: the column-form predictor forms it itself)
-      if (dzu)
-        dzu[t] = explicit_diffusion_w(k, nz, uw5[1], uw5[2], uw5[3], duw[0], duw[1], duw[2],
-                                      m3w[0], m3w[1], m3w[2], km_k, km_k1,
-                                      k == 0 ? geo.tau_u[c] : 0.0, p.bottom_drag);
-      if (dzv)
-        dzv[t] = explicit_diffusion_w(k, nz, vw5[1], vw5[2], vw5[3], dvw[0], dvw[1], dvw[2],
-                                      m3w[0], m3w[1], m3w[2], km_k, km_k1,
-                                      k == 0 ? geo.tau_v[c] : 0.0, p.bottom_drag);
+      // explicit vertical diffusion with surface stress and bottom drag
+      const bool lower = k + 1 < nz;
+      const bool cw2 = lower && cell_wet(k + 1);
+      const double idz_k1 = lower ? idz(k + 1) : 0.0;
+      const double iv = inv(k);
+      const double tau_k = k == 0 ? at_byte(tau, b0) : 0.0;
+      const double dz_k = explicit_diffusion_inv(k, nz, a5[1], a5[2], a5[3], idz_k, idz_k1, iv,
+                                                 cw0, cw1, cw2, km_k, km_k1, tau_k,
+                                                 p.bottom_drag);
       // advection and horizontal viscosity
-      double exu = 0.0, exv = 0.0;
+      double ex = 0.0;
       if (adv != ADV_NONE) {
-        const R ax = (F.fux[ty][tx + 1] - F.fux[ty][tx]) / R(p.dx);
-        const R ay = (F.fuy[ty + 1][tx] - F.fuy[ty][tx]) / R(p.dy);
-        const R by_ = (F.fvy[ty + 1][tx] - F.fvy[ty][tx]) / R(p.dy);
-        const R bx_ = (F.fvx[ty][tx + 1] - F.fvx[ty][tx]) / R(p.dx);
+        const R ax = by_dx(F.fx[ty][tx + 1] - F.fx[ty][tx]);
+        const R ay = by_dy(F.fy[ty + 1][tx] - F.fy[ty][tx]);
         // vertical fluxes: the top one is the bottom one of the level above
-        const R wbu = R(0.5) * (P.w[ty][tx] + P.w[ty][tx + 1]);
-        const R wbv = R(0.5) * (P.w[ty][tx] + P.w[ty + 1][tx]);
-        const R fzu_bot = mom_flux_z<R>(adv, k + 1, nz, wbu, R(uw5[1]), R(uw5[2]), R(uw5[3]),
-                                        R(uw5[4]), muw[1], muw[4]);
-        const R fzv_bot = mom_flux_z<R>(adv, k + 1, nz, wbv, R(vw5[1]), R(vw5[2]), R(vw5[3]),
-                                        R(vw5[4]), mvw[1], mvw[4]);
-        const R az = (fzu_top - fzu_bot) / R(p.dz_nom);
-        const R bz = (fzv_top - fzv_bot) / R(p.dz_nom);
-        fzu_top = fzu_bot;
-        fzv_top = fzv_bot;
-        exu = exu - (double)((ax + ay + az) * R(mu_c));
-        exv = exv - (double)((bx_ + by_ + bz) * R(mv_c));
+        const R fz_bot = mom_flux_z<R, TVD>(adv, k + 1, nz, wb, R(a5[1]), R(a5[2]), R(a5[3]),
+                                       R(a5[4]), wet_at(k, 1), wet_at(k, 4));
+        const R az = by_dz(fz_top - fz_bot);
+        fz_top = fz_bot;
+        ex = ex - (double)((ax + ay + az) * R(m_c));
       }
-      if (p.has_A_h) {
-        exu = exu + p.A_h * (double)(R(mu_c) * ((F.gux[ty][tx + 1] - F.gux[ty][tx]) / R(p.dx) +
-                                                (F.guy[ty + 1][tx] - F.guy[ty][tx]) / R(p.dy)));
-        exv = exv + p.A_h * (double)(R(mv_c) * ((F.gvx[ty][tx + 1] - F.gvx[ty][tx]) / R(p.dx) +
-                                                (F.gvy[ty + 1][tx] - F.gvy[ty][tx]) / R(p.dy)));
+      if (p.has_A_h)
+        ex = ex + p.A_h * (double)(R(m_c) * (by_dx(F.gx[ty][tx + 1] - F.gx[ty][tx]) +
+                                             by_dy(F.gy[ty + 1][tx] - F.gy[ty][tx])));
+      double s0 = 0.0;
+      if (k == 0) s0 = p.thv_dt * tau_k * iv;
+      if (active) {
+        put_byte(pg + o, b0, pg_k);
+        put_byte(dzo + o, b0, dz_k);
+        put_byte(st + o, b0, s0 + p.dt * ex);
       }
-      double s0u = 0.0, s0v = 0.0;
-      if (k == 0) {
-        s0u = p.thv_dt * geo.tau_u[c] * safe_inv(duw[1]);
-        s0v = p.thv_dt * geo.tau_v[c] * safe_inv(dvw[1]);
-      }
-      stu[t] = s0u + p.dt * exu;
-      stv[t] = s0v + p.dt * exv;
+      // advance the windows
       km_k = km_k1;
+      idz_k = idz_k1;
+      cw0 = cw1;
+      cw1 = cw2;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) a5[q] = a5[q + 1];
+      a5[4] = a_k3;
+      if constexpr (!ZC) m5 = m5 >> 1 | (k + 3 < nz && own_wet(k + 3) ? 16u : 0u);
     }
-    // advance the windows
-    for (int q = 0; q < 4; ++q) {
-      uw5[q] = uw5[q + 1];
-      vw5[q] = vw5[q + 1];
-      muw[q] = muw[q + 1];
-      mvw[q] = mvw[q + 1];
-    }
-    for (int q = 0; q < 2; ++q) {
-      duw[q] = duw[q + 1];
-      dvw[q] = dvw[q + 1];
-      m3w[q] = m3w[q + 1];
-    }
-    if (active) {
-      const int k3 = k + 3, k2 = k + 2;
-      uw5[4] = k3 < nz ? u[(long long)k3 * n2 + c] : 0.0;
-      vw5[4] = k3 < nz ? v[(long long)k3 * n2 + c] : 0.0;
-      muw[4] = k3 < nz && own_mu(k3);
-      mvw[4] = k3 < nz && own_mv(k3);
-      duw[2] = k2 < nz ? own_du(k2) : 0.0;
-      dvw[2] = k2 < nz ? own_dv(k2) : 0.0;
-      m3w[2] = k2 < nz && own_m3(k2);
-    }
-    if (k + 1 < nz) {
-      if constexpr (ZC) mom_store_c(LB[(k + 1) & 1], RG, CG, k + 1, tid);
-      else mom_store(LB[(k + 1) & 1], RG, tid);
-    }
+    if (k + 1 < k1) store((k + 1 - k0) & 1);
     __syncthreads();
   }
+}
+
+// The step's explicit momentum terms (libs/core/model3d_v05.py:352-370): the
+// pressure gradient, the explicit vertical diffusion, and the stress,
+// advection and viscosity of u and v; same outputs as k_momentum_explicit.
+// One workgroup marches one component of one tile down the levels [k0, k0 +
+// nk). Staging is double-buffered (level k + 1 loads in flight while level k
+// is computed) and every horizontal face flux is formed once. R is the type
+// of the advective fluxes and the A_h gradients (double: bitwise the
+// reference; float: the mixed step); the rest stays fp64. ZC: the static
+// z-level geometry in column form (masks, inverse thicknesses and centre
+// depths from the columns' wet-level counts and deepest thicknesses, in
+// registers; the same bits).
+// Bound by the latency of its fp64 chains (about 600 VALU instructions per
+// cell for both components, five divisions in a row on a face), so what counts
+// is waves in flight without spills and straight-line code: u and v in
+// workgroups of their own (159 registers against 230 for both: 3 waves per
+// SIMD), the scheme a template argument (the face values of a level
+// interleave), the levels cut into ranges (1024 tiles of 512 x 512 on 768
+// resident workgroups left a third of the second round idle, and 64 tiles of
+// 128 x 128 three quarters of the chip). Measured per launch, before -> now:
+// 128 x 4 x 20 132 -> 11 us, 128 x 128 x 30 204 -> 37, 512 x 512 x 40 600 ->
+// 364, 1000 x 1000 x 30 1487 -> 1069. At 4 waves per SIMD it spills 30
+// registers and takes 478 us at 512 x 512 x 40.
+template <class R, bool ZC, bool TVD>
+__global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(3))) void k_momentum_explicit_tiled(
+    Dims d, StepParams p, Geo geo, int nk, const double* __restrict__ u,
+    const double* __restrict__ v, const double* __restrict__ b, const double* __restrict__ phi,
+    const double* __restrict__ w, const double* __restrict__ Km, const double* __restrict__ zs,
+    double* __restrict__ pgx, double* __restrict__ pgy, double* __restrict__ dzu,
+    double* __restrict__ dzv, double* __restrict__ stu, double* __restrict__ stv) {
+  __shared__ MomLds<R> LB[2];
+  __shared__ MomFaces<R> F;
+  __shared__ std::conditional_t<ZC, NoTile, MomMaskLds> MB[2];
+  const BlockTile T = xcd_block((d.nx + TX - 1) / TX, (d.ny + TY - 1) / TY, 2);
+  const int k0 = T.z * nk;
+  const int k1 = k0 + nk < d.nz ? k0 + nk : d.nz;
+  if (T.part == 0)
+    momentum_component<R, ZC, TVD, 0>(d, p, geo, T.x * TX, T.y * TY, k0, k1, LB, MB, F, u, v, b,
+                                 phi, w, Km, zs, pgx, dzu, stu);
+  else
+    momentum_component<R, ZC, TVD, 1>(d, p, geo, T.x * TX, T.y * TY, k0, k1, LB, MB, F, v, u, b,
+                                 phi, w, Km, zs, pgy, dzv, stv);
 }
 
 void launch_tracers_tiled(bool mixed, hipStream_t s, Dims d, StepParams p, Geo geo,
@@ -1296,25 +1250,41 @@ void launch_tracers_tiled(bool mixed, hipStream_t s, Dims d, StepParams p, Geo g
   }
 }
 
+// Levels per workgroup of a tiled march: all of them where the tiles alone give `target`
+// workgroups, else as few as make up that number (each range of levels reads the two levels
+// above and below it again and forms its top interface's fluxes a second time).
+int levels_per_block(long long tiles, int nz, long long target) {
+  const long long parts = tiles >= target ? 1 : (target + tiles - 1) / tiles;
+  const int n = (int)((nz + parts - 1) / parts);
+  return n < 1 ? 1 : n;
+}
+
 void launch_momentum_explicit_tiled(bool mixed, hipStream_t s, Dims d, StepParams p, Geo geo,
                                     const double* u, const double* v, const double* b,
                                     const double* phi, const double* w, const double* Km,
-                                    double* pgx, double* pgy, double* avu, double* avv,
-                                    double* dzu, double* dzv, double* stu, double* stv) {
-  const dim3 grid((d.nx + TX - 1) / TX, (d.ny + TY - 1) / TY);
+                                    double* pgx, double* pgy, double* dzu, double* dzv,
+                                    double* stu, double* stv) {
+  const int gx = (d.nx + TX - 1) / TX, gy = (d.ny + TY - 1) / TY;
+  // 2048 workgroups: 768 are resident at a time (3 per CU). Measured with 2048 / 4096 / 8192:
+  // 128 x 128 x 30 37 / 47 / 47 us, 512 x 512 x 40 364 / 366 / 384, 1000 x 1000 x 30 1069 /
+  // 1083 / 1116; 128 x 4 x 20 (one level each) 11 us in all three.
+  const int nk = levels_per_block(2LL * gx * gy, d.nz, 2048);
+  const unsigned grid = 2u * gx * gy * ((d.nz + nk - 1) / nk);
+  const bool tvd = p.advection == ADV_UP3_TVD;
+  auto go = [&](auto kernel) {
+    kernel<<<grid, TILE_THREADS, 0, s>>>(d, p, geo, nk, u, v, b, phi, w, Km, geo.zs, pgx, pgy,
+                                         dzu, dzv, stu, stv);
+  };
   if (p.zcol) {
-    if (mixed)
-      k_momentum_explicit_tiled<float, true><<<grid, TILE_THREADS, 0, s>>>(
-          d, p, geo, u, v, b, phi, w, Km, pgx, pgy, avu, avv, dzu, dzv, stu, stv);
-    else
-      k_momentum_explicit_tiled<double, true><<<grid, TILE_THREADS, 0, s>>>(
-          d, p, geo, u, v, b, phi, w, Km, pgx, pgy, avu, avv, dzu, dzv, stu, stv);
+    if (mixed) go(tvd ? k_momentum_explicit_tiled<float, true, true>
+                      : k_momentum_explicit_tiled<float, true, false>);
+    else go(tvd ? k_momentum_explicit_tiled<double, true, true>
+                : k_momentum_explicit_tiled<double, true, false>);
   } else if (mixed) {
-    k_momentum_explicit_tiled<float, false><<<grid, TILE_THREADS, 0, s>>>(
-        d, p, geo, u, v, b, phi, w, Km, pgx, pgy, avu, avv, dzu, dzv, stu, stv);
+    go(k_momentum_explicit_tiled<float, false, false>);
   } else {
-    k_momentum_explicit_tiled<double, false><<<grid, TILE_THREADS, 0, s>>>(
-        d, p, geo, u, v, b, phi, w, Km, pgx, pgy, avu, avv, dzu, dzv, stu, stv);
+    go(tvd ? k_momentum_explicit_tiled<double, false, true>
+           : k_momentum_explicit_tiled<double, false, false>);
   }
 }
 
