@@ -2227,7 +2227,7 @@ static int step_impl(hoc_stepper* h, const hoc_state* in, hoc_state* out, void* 
     k_w_diag<<<blocks(d.n2), TPB, 0, s>>>(d, p, geo, out->u, out->v, h->w);
   }
   { ProfScope _ps(h, "k_tracers", s);
-  launch_tracers_tiled((h->fp32_parts & HOC_FP32_TRACER_FLUX) != 0, s, d, p, geo, in->T, in->S,
+  launch_tracers((h->fp32_parts & HOC_FP32_TRACER_FLUX) != 0, s, d, p, geo, in->T, in->S,
                        in->b, out->u, out->v,
                        h->w, h->Kh, h->cst_b, out->T, out->S, out->b); }
   LAUNCH_CHECK("k_tracers");

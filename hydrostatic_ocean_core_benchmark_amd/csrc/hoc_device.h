@@ -370,14 +370,13 @@ __device__ __forceinline__ double explicit_diffusion_inv(int k, int nz, double f
 }
 
 // Row k of one implicit vertical-diffusion matrix (I - theta_v dt D[nu]) of
-// a column, factored for the Thomas sweep: sub, den = diag - sub c*_{k-1}
-// and c* = sup / den (libs/core/vertical_var.py:35-77). inv_dz, idzi_t and
-// idzi_b are 1/dz3 and 1/dzi above and below the cell.
-__device__ __forceinline__ void factor_row(const StepParams& p, int k, double inv_dz,
-                                           double nu_t, double nu_b, double idzi_t,
-                                           double idzi_b, bool wet, bool below,
-                                           double drag_term, double c_prev, double& sub_o,
-                                           double& den_o, double& cst_o) {
+// a column and its pivot in the Thomas sweep: sub, sup and den = diag - sub
+// c*_{k-1} (libs/core/vertical_var.py:35-77). inv_dz, idzi_t and idzi_b are
+// 1/dz3 and 1/dzi above and below the cell.
+__device__ __forceinline__ void matrix_row(const StepParams& p, int k, double inv_dz, double nu_t,
+                                           double nu_b, double idzi_t, double idzi_b, bool wet,
+                                           bool below, double drag_term, double c_prev,
+                                           double& sub_o, double& sup_o, double& den_o) {
   const double fac = p.thv_dt * inv_dz;
   const double a_top = fac * nu_t * idzi_t;
   const double a_bot = fac * nu_b * idzi_b;
@@ -397,8 +396,19 @@ __device__ __forceinline__ void factor_row(const StepParams& p, int k, double in
     sup = 0.0;
   }
   den_o = (k == 0) ? diag : diag - sub * c_prev;
-  cst_o = sup / den_o;
   sub_o = sub;
+  sup_o = sup;
+}
+// The same factored: sub, den and c* = sup / den.
+__device__ __forceinline__ void factor_row(const StepParams& p, int k, double inv_dz,
+                                           double nu_t, double nu_b, double idzi_t,
+                                           double idzi_b, bool wet, bool below,
+                                           double drag_term, double c_prev, double& sub_o,
+                                           double& den_o, double& cst_o) {
+  double sup;
+  matrix_row(p, k, inv_dz, nu_t, nu_b, idzi_t, idzi_b, wet, below, drag_term, c_prev, sub_o, sup,
+             den_o);
+  cst_o = sup / den_o;
 }
 
 // ------------------------------------------------------------------ EOS

@@ -130,10 +130,10 @@ __global__ void k_momentum_advection(Dims d, StepParams p, Geo geo, const double
 
 // hoc_tiled.hip: the LDS-tiled tracer and explicit-momentum passes; mixed
 // selects the fp32 advective fluxes (and EOS), else the fp64 plain step
-void launch_tracers_tiled(bool mixed, hipStream_t s, Dims d, StepParams p, Geo geo,
-                          const double* T, const double* S, const double* b, const double* u,
-                          const double* v, const double* w, const double* Kh, double* cst,
-                          double* T_out, double* S_out, double* b_out);
+void launch_tracers(bool mixed, hipStream_t s, Dims d, StepParams p, Geo geo, const double* T,
+                    const double* S, const double* b, const double* u, const double* v,
+                    const double* w, const double* Kh, double* cst, double* T_out,
+                    double* S_out, double* b_out);
 void launch_momentum_explicit_tiled(bool mixed, hipStream_t s, Dims d, StepParams p, Geo geo,
                                     const double* u, const double* v, const double* b,
                                     const double* phi, const double* w, const double* Km,

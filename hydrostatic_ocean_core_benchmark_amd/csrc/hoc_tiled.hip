@@ -1,5 +1,5 @@
 // LDS-tiled column kernels ("2.5D"): a workgroup owns a TX x TY tile of
-// columns and marches down the levels. At each level the fields that enter
+// columns and marches down a range of levels. At each level the fields that enter
 // horizontal stencils are staged once in LDS with a 2-cell periodic halo,
 // so every value is read from HBM about once instead of once per stencil
 // point; the column's own vertical neighbours stay in a register window.
@@ -54,708 +54,500 @@ __device__ __forceinline__ R tracer_face_z(int adv, int kk, int nz, R far_up, R 
                          hu, hd, adv == ADV_UP3_TVD);
 }
 
-// Staged tile of one level in the flux type R: what the face pass and the
-// cell pass both read (double-buffered, so level k + 1 lands while level k
-// is still read) ...
-template <class R>
-struct TileLds {
-  R c[2][SY][SX];           // the tracers (T, S) or b, with halo
-  uint8_t m[SY][SX];        // mask3 with halo
-  uint8_t mu[TY][TX + 1];   // mask3u
-  uint8_t mv[TY + 1][TX];   // mask3v
-};
-
-// ... and what only the face pass reads (one buffer: the barrier after the
-// face pass ends its reads before level k + 1 is stored).
-template <class R>
-struct VelLds {
-  R u[TY][TX + 1];          // u at i-1 .. i
-  R v[TY + 1][TX];          // v at j-1 .. j
-  R du[TY][TX + 1];         // dz3u
-  R dv[TY + 1][TX];         // dz3v
-};
-
-// Advective face fluxes dz_f u_f c_f of one level, each computed once, on
-// the x-faces (index q: between tile columns q-1 and q) and y-faces
-// (between rows q-1 and q), for both tracers. The K_h face gradients are
-// formed by the cell that uses them, from the staged tile (each interior
-// gradient twice, from the same operands): with the single velocity buffer
-// this holds a workgroup to 33 KB of LDS, so four fit on a CU.
-template <class R>
-struct FaceLds {
-  R fx[2][TY][TX + 1];
-  R fy[2][TY + 1][TX];
-};
-
-// K_h gradient mask_f (c_1 - c_0) / d across one face of the staged tile.
-template <class R>
-__device__ __forceinline__ R face_grad(uint8_t mf, R c0, R c1, double d) {
-  return R(mk(mf)) * (c1 - c0) / R(d);
+// Value of a plane at a byte offset. The plane's address is the same in every
+// lane and is kept in scalar registers, so that one vector register holds the
+// offset for every array (a plane is below 2^32 bytes). Without the empty asm
+// the compiler keeps a 64-bit vector address per array across the march, 30
+// registers in the momentum kernel.
+template <class T>
+__device__ __forceinline__ T at_byte(const T* plane, unsigned off) {
+  unsigned long long a = (unsigned long long)plane;
+  __asm__("" : "+s"(a));
+  using G = const __attribute__((address_space(1))) char;
+  return *(const __attribute__((address_space(1))) T*)((G*)a + off);
+}
+__device__ __forceinline__ void put_byte(double* plane, unsigned off, double v) {
+  unsigned long long a = (unsigned long long)plane;
+  __asm__("" : "+s"(a));
+  using G = __attribute__((address_space(1))) char;
+  *(__attribute__((address_space(1))) double*)((G*)a + off) = v;
 }
 
-// Level-k staging of one tile held in registers between its global loads
-// and its LDS stores, so the loads of level k + 1 are in flight while
-// level k is computed (two LDS buffers, one barrier per level).
-constexpr int ST_C = (SX * SY + TILE_THREADS - 1) / TILE_THREADS;        // tracer + mask slots
-constexpr int ST_U = (TY * (TX + 1) + TILE_THREADS - 1) / TILE_THREADS;  // u-face slots
-constexpr int ST_V = ((TY + 1) * TX + TILE_THREADS - 1) / TILE_THREADS;  // v-face slots
+struct NoTile {};
 
+// First threads that form the tile's west column of faces (TY of them) and
+// its south row (TX): two different waves.
+constexpr int EDGE_X = TX > 64 ? TX : 64, EDGE_Y = 0;
+static_assert(EDGE_X + TY <= TILE_THREADS && EDGE_Y + TX <= EDGE_X, "edge threads");
+
+// Levels at which the east (axis 0) or north (axis 1) face of column (j, i)
+// is wet, for a static z-level geometry, and the face's thickness at the last
+// of them (its other levels are the face rule of two full cells).
+__device__ __forceinline__ int face_levels(const Geo& geo, int axis, int j, int i, int ny,
+                                           int nx) {
+  const int c0 = j * nx + i;
+  const int c1 = axis == 0 ? j * nx + pmod(i + 1, nx) : pmod(j + 1, ny) * nx + i;
+  const int a = geo.nw[c0], b = geo.nw[c1];
+  return (axis == 0 ? geo.mu2[c0] : geo.mv2[c0]) ? (a < b ? a : b) : 0;
+}
+__device__ __forceinline__ double face_last(const StepParams& p, const Geo& geo, int axis, int n,
+                                            int j, int i, int ny, int nx) {
+  if (n <= 0) return 0.0;
+  const int c0 = j * nx + i;
+  const int c1 = axis == 0 ? j * nx + pmod(i + 1, nx) : pmod(j + 1, ny) * nx + i;
+  return face_value(p.face_rule, cg_dz(p.dzr, geo.nw[c0], geo.hb[c0], n - 1),
+                    cg_dz(p.dzr, geo.nw[c1], geo.hb[c1], n - 1));
+}
+
+// ------------------------------------------------------------- tracers
+// Staged tile of one tracer on one level (two buffers: level k + 1 lands
+// while level k is read), with the cell masks for geometry read from the
+// arrays.
 template <class R>
-struct TileRegs {
-  R c0[ST_C], c1[ST_C];
-  uint8_t m[ST_C];
-  R u[ST_U], du[ST_U];
-  uint8_t mu[ST_U];
-  R v[ST_V], dv[ST_V];
-  uint8_t mv[ST_V];
+struct TracerLds {
+  R c[SY][SX];
+};
+struct TracerMaskLds {
+  uint8_t m[SY][SX];
 };
 
-// Plane offsets of this thread's staging slots (independent of k; -1: no slot).
-struct TileOffs {
-  int c[ST_C], u[ST_U], v[ST_V];
+// Face fluxes of one field on one level, each computed once: the advective
+// flux and the horizontal-diffusion gradient, on the x-faces (index q:
+// between tile columns q-1 and q) and the y-faces (between rows q-1 and q).
+template <class R>
+struct FaceLds {
+  R fx[TY][TX + 1], gx[TY][TX + 1];
+  R fy[TY + 1][TX], gy[TY + 1][TX];
 };
 
-__device__ __forceinline__ TileOffs tile_offsets(int tid, int i0, int j0, int nx, int ny) {
-  TileOffs F;
+constexpr int ST_H = (SX * SY + TILE_THREADS - 1) / TILE_THREADS;  // halo slots per thread
+
+// Plane indexes of this thread's slots of the tile with its halo (slots
+// beyond the tile read its first ones again; the value is not stored).
+struct HaloOffs {
+  unsigned h[ST_H];
+};
+__device__ __forceinline__ HaloOffs halo_offsets(int tid, int i0, int j0, int nx, int ny) {
+  HaloOffs F;
 #pragma unroll
-  for (int q = 0; q < ST_C; ++q) {
+  for (int q = 0; q < ST_H; ++q) {
     const int t = tid + q * TILE_THREADS;
-    F.c[q] = t < SX * SY ? pmod(j0 + t / SX - HALO, ny) * nx + pmod(i0 + t % SX - HALO, nx) : -1;
-  }
-#pragma unroll
-  for (int q = 0; q < ST_U; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    F.u[q] = t < TY * (TX + 1) ? pmod(j0 + t / (TX + 1), ny) * nx + pmod(i0 + t % (TX + 1) - 1, nx)
-                               : -1;
-  }
-#pragma unroll
-  for (int q = 0; q < ST_V; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    F.v[q] = t < (TY + 1) * TX ? pmod(j0 + t / TX - 1, ny) * nx + pmod(i0 + t % TX, nx) : -1;
+    const int tt = t < SX * SY ? t : tid;
+    F.h[q] = (unsigned)(pmod(j0 + tt / SX - HALO, ny) * nx + pmod(i0 + tt % SX - HALO, nx));
   }
   return F;
 }
 
-template <class RT>
-__device__ __forceinline__ void tile_load(TileRegs<RT>& R, const TileOffs& F, long long o, bool ts,
-                                          const double* A, const double* S, const double* u,
-                                          const double* v, const Geo& geo) {
-#pragma unroll
-  for (int q = 0; q < ST_C; ++q) {
-    if (F.c[q] >= 0) {
-      const long long g = o + F.c[q];
-      R.c0[q] = (RT)A[g];
-      R.c1[q] = ts ? (RT)S[g] : RT(0);
-      R.m[q] = geo.m3[g];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < ST_U; ++q) {
-    if (F.u[q] >= 0) {
-      const long long g = o + F.u[q];
-      R.u[q] = (RT)u[g];
-      R.du[q] = (RT)geo.dz3u[g];
-      R.mu[q] = geo.m3u[g];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < ST_V; ++q) {
-    if (F.v[q] >= 0) {
-      const long long g = o + F.v[q];
-      R.v[q] = (RT)v[g];
-      R.dv[q] = (RT)geo.dz3v[g];
-      R.mv[q] = geo.m3v[g];
-    }
-  }
-}
+// Operands of the own east face, the own north face and, for the edge
+// threads, the edge face at one level: velocity and, for geometry read from
+// the arrays, thickness and mask.
+struct TracerFaceRegs {
+  double vel[3];
+  double dz[3];
+  uint8_t m[3];
+};
 
-template <class RT>
-__device__ __forceinline__ void tile_store(TileLds<RT>& L, VelLds<RT>& V, const TileRegs<RT>& R,
-                                           int tid) {
-#pragma unroll
-  for (int q = 0; q < ST_C; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    if (t < SX * SY) {
-      const int lx = t % SX, ly = t / SX;
-      L.c[0][ly][lx] = R.c0[q];
-      L.c[1][ly][lx] = R.c1[q];
-      L.m[ly][lx] = R.m[q];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < ST_U; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    if (t < TY * (TX + 1)) {
-      const int lx = t % (TX + 1), ly = t / (TX + 1);
-      V.u[ly][lx] = R.u[q];
-      V.du[ly][lx] = R.du[q];
-      L.mu[ly][lx] = R.mu[q];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < ST_V; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    if (t < (TY + 1) * TX) {
-      const int lx = t % TX, ly = t / TX;
-      V.v[ly][lx] = R.v[q];
-      V.dv[ly][lx] = R.dv[q];
-      L.mv[ly][lx] = R.mv[q];
-    }
-  }
-}
-
-// Both tracers of the tile's columns: advection + K_h Laplacian + explicit
-// part of the vertical diffusion + surface flux, the forward sweep on tri_b
-// (d* parked in the outputs), then the back-substitution and the EOS
-// (libs/core/model3d_v05.py:466-533). R is the type of the horizontal and
-// vertical advective fluxes, the K_h gradients and the EOS: double for the
-// plain step (bitwise the reference), float for the mixed step; the column
-// update, the vertical diffusion and the tridiagonal solve stay fp64.
-// The fp32-flux instantiation runs at 4 waves per SIMD (128 VGPRs): measured
-// at 1024 x 1024 x 60, 3.65 ms per step against 4.19 ms at the compiler's
-// default of 3 waves.
-template <class R>
-__global__ __launch_bounds__(TILE_THREADS)
-__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 1))) void k_tracers_tiled(
-    Dims d, StepParams p, Geo geo, const double* __restrict__ T, const double* __restrict__ S,
-    const double* __restrict__ b, const double* __restrict__ u, const double* __restrict__ v,
-    const double* __restrict__ w, const double* __restrict__ Kh, double* __restrict__ cst,
+// Right-hand sides of the tracers' implicit vertical diffusion: one tracer of
+// one tile on the levels [k0, k0 + nk) per workgroup: advection + K_h
+// Laplacian + explicit part of the vertical diffusion + surface flux
+// (libs/core/model3d_v05.py:466-512), which k_tracer_solve then solves in
+// place. R is the type of the advective fluxes and the K_h gradients: double
+// for the plain step (bitwise the reference), float for the mixed step. ZC:
+// the static z-level geometry in column form (thicknesses, their inverses and
+// masks from the columns' wet-level counts and deepest thicknesses, in
+// registers; the same bits).
+// Bound by the latency of its fp64 chains, like the momentum kernel: one
+// tracer per workgroup (128 registers, 4 waves per SIMD), the column solve in
+// a kernel of its own so that the levels can be cut into ranges, and the own
+// faces' velocities straight from their arrays. Two more fields pass through
+// memory than with the solve in the same march (67 us of traffic at 512 x 512
+// x 40), which marched 64 tiles at 128 x 128 with the recurrence in every
+// level. Both kernels per step, before -> now: 128 x 4 x 20 135 -> 24 us,
+// 128 x 128 x 30 224 -> 63, 512 x 512 x 40 689 -> 424, 1000 x 1000 x 30 1690 ->
+// 1175; fp32 fluxes at 640 x 512 x 48 1244 -> 625.
+template <class R, bool ZC, bool TVD>
+__global__ __launch_bounds__(TILE_THREADS) void k_tracer_rhs(
+    Dims d, StepParams p, Geo geo, int nk, const double* __restrict__ T,
+    const double* __restrict__ S, const double* __restrict__ b, const double* __restrict__ u,
+    const double* __restrict__ v, const double* __restrict__ w, const double* __restrict__ Kh,
     double* __restrict__ T_out, double* __restrict__ S_out, double* __restrict__ b_out) {
-  __shared__ TileLds<R> LB[2];
-  __shared__ VelLds<R> VL;
+  __shared__ TracerLds<R> LB[2];
   __shared__ FaceLds<R> F;
+  __shared__ std::conditional_t<ZC, NoTile, TracerMaskLds> MB[2];
   const int nx = d.nx, ny = d.ny, nz = d.nz;
   const long long n2 = d.n2;
+  const bool ts = p.tracers_ts != 0;
+  const BlockTile B = xcd_block((nx + TX - 1) / TX, (ny + TY - 1) / TY, ts ? 2 : 1);
+  const double* C = B.part == 1 ? S : (ts ? T : b);
+  double* out = B.part == 1 ? S_out : (ts ? T_out : b_out);
+  const double flux = B.part == 1 ? p.flux_S : (ts ? p.flux_T : 0.0);
   const int tid = threadIdx.x;
   const int tx = tid % TX, ty = tid / TX;
-  int bx, by;
-  xcd_tile(bx, by);
-  const int i0 = bx * TX, j0 = by * TY;
+  const int i0 = B.x * TX, j0 = B.y * TY;
   const int i = i0 + tx, j = j0 + ty;
   const bool active = i < nx && j < ny;
-  const long long c = active ? (long long)j * nx + i : 0;
-  const bool ts = p.tracers_ts != 0;
-  const int ntr = ts ? 2 : 1;
-  const double* A = ts ? T : b;
-  double* Ao = ts ? T_out : b_out;
-  const double flux[2] = {ts ? p.flux_T : 0.0, p.flux_S};
-  const int adv = p.advection;
+  const int k0 = B.z * nk;
+  const int k1 = k0 + nk < nz ? k0 + nk : nz;
+  const int adv = TVD ? (int)ADV_UP3_TVD : p.advection;
+  const bool has_adv = adv != ADV_NONE;
+  const Divisor<R> by_dx = uniform_divisor<R>(p.dx), by_dy = uniform_divisor<R>(p.dy);
+  // plane indexes of the own point (clamped into the grid for the lanes
+  // beyond it) and of the point before this thread's edge face
+  const int jc = pmod(j, ny), ic = pmod(i, nx);
+  const int cc = jc * nx + ic;
+  const int xe = tid - EDGE_X, ye = tid - EDGE_Y;
+  const bool is_x = xe >= 0 && xe < TY, is_y = ye >= 0 && ye < TX;
+  const int je = is_x ? pmod(j0 + xe, ny) : (is_y ? pmod(j0 - 1, ny) : jc);
+  const int ie = is_x ? pmod(i0 - 1, nx) : (is_y ? pmod(i0 + ye, nx) : ic);
+  const int ce = je * nx + ie;
+  const unsigned b0 = 8u * (unsigned)cc, be = 8u * (unsigned)ce;
+  const double* ve = is_x ? u : v;  // the edge face's velocity, thickness and mask arrays
+  const double* dze = is_x ? geo.dz3u : geo.dz3v;
+  const uint8_t* me = is_x ? geo.m3u : geo.m3v;
 
-  // own-column windows: tracer at k-2..k+2, mask3 at k-2..k+2
-  double win[2][5];
-  bool mw[5];
+  R rc[ST_H];
+  uint8_t rm[ST_H];
+  TracerFaceRegs rf;
+  const HaloOffs HO = halo_offsets(tid, i0, j0, nx, ny);
+  auto load = [&](long long o) {
+#pragma unroll
+    for (int q = 0; q < ST_H; ++q) {
+      rc[q] = (R)at_byte(C + o, 8u * HO.h[q]);
+      if constexpr (!ZC) rm[q] = at_byte(geo.m3 + o, HO.h[q]);
+    }
+    rf.vel[0] = at_byte(u + o, b0);
+    rf.vel[1] = at_byte(v + o, b0);
+    rf.vel[2] = ve[o + ce];
+    if constexpr (!ZC) {
+      rf.dz[0] = at_byte(geo.dz3u + o, b0);
+      rf.dz[1] = at_byte(geo.dz3v + o, b0);
+      rf.dz[2] = dze[o + ce];
+      rf.m[0] = at_byte(geo.m3u + o, (unsigned)cc);
+      rf.m[1] = at_byte(geo.m3v + o, (unsigned)cc);
+      rf.m[2] = me[o + ce];
+    }
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < ST_H; ++q) {
+      const int t = tid + q * TILE_THREADS;
+      if (t < SX * SY) {
+        LB[buf].c[t / SX][t % SX] = rc[q];
+        if constexpr (!ZC) MB[buf].m[t / SX][t % SX] = rm[q];
+      }
+    }
+  };
+  load((long long)k0 * n2);
+
+  // the column form: wet levels of the far cells and of the face itself
+  // (bytes: before, beyond, own; a count is at most 255) and the thickness at
+  // the last one, for the east, north and edge face; the own column
+  unsigned fw[3] = {0, 0, 0};
+  double fl[3] = {0.0, 0.0, 0.0};
+  double full = 0.0;
+  InvCol ca{};
+  int nwc = 0;
+  if constexpr (ZC) {
+    auto face = [&](int axis, int jj, int ii, unsigned& wet, double& last) {
+      const int jm = axis ? pmod(jj - 1, ny) : jj, j2 = axis ? pmod(jj + 2, ny) : jj;
+      const int im = axis ? ii : pmod(ii - 1, nx), i2 = axis ? ii : pmod(ii + 2, nx);
+      const int n = face_levels(geo, axis, jj, ii, ny, nx);
+      wet = (unsigned)geo.nw[jm * nx + im] | (unsigned)geo.nw[j2 * nx + i2] << 8 |
+            (unsigned)n << 16;
+      last = face_last(p, geo, axis, n, jj, ii, ny, nx);
+    };
+    face(0, jc, ic, fw[0], fl[0]);
+    face(1, jc, ic, fw[1], fl[1]);
+    if (is_x || is_y) face(is_x ? 0 : 1, je, ie, fw[2], fl[2]);
+    full = uniform_value(face_value(p.face_rule, p.dzr, p.dzr));
+    nwc = geo.nw[cc];
+    ca = inv_col(nwc, uniform_value(p.dzr), nwc > 0 ? geo.hb[cc] : 0.0);
+  }
+  auto cell_wet = [&](int kk) -> bool {  // the own column, 0 <= kk < nz
+    if constexpr (ZC) return kk < nwc;
+    else return at_byte(geo.m3 + kk * n2, (unsigned)cc) != 0;
+  };
+  auto idz = [&](int kk) -> double {  // 1 / spacing on interface kk, 1 <= kk < nz
+    if constexpr (ZC) return ca.idzi(kk);
+    else return safe_inv(at_byte(geo.dzi + kk * n2, b0));
+  };
+  auto inv = [&](int kk) -> double {
+    if constexpr (ZC) return ca.inv(kk);
+    else return safe_inv(at_byte(geo.dz3 + kk * n2, b0));
+  };
+
+  store(0);
+  // own-column window of the tracer at k-2..k+2, with its wet flags (bits of
+  // one register, or from the level count)
+  double c5[5];
+  unsigned m5 = 0;
+#pragma unroll
   for (int q = 0; q < 5; ++q) {
-    win[0][q] = 0.0;
-    win[1][q] = 0.0;
-    mw[q] = false;
+    const int kk = k0 + q - 2;
+    const bool in = kk >= 0 && kk < nz;
+    c5[q] = in ? at_byte(C + kk * n2, b0) : 0.0;
+    if constexpr (!ZC)
+      if (in && cell_wet(kk)) m5 |= 1u << q;
   }
-  if (active) {
-    for (int q = 2; q < 5; ++q) {
-      const int kk = q - 2;
-      if (kk < nz) {
-        win[0][q] = A[kk * n2 + c];
-        if (ts) win[1][q] = S[kk * n2 + c];
-        mw[q] = geo.m3[kk * n2 + c] != 0;
-      }
-    }
-  }
-  double w_k = active ? w[c] : 0.0;
-  double kh_k = active ? Kh[c] : 0.0;
-  double dzi_k = active ? geo.dzi[c] : 0.0;
-  R cf_top[2] = {R(0), R(0)};  // interface value at the top of level k
-  double dprev[2] = {0.0, 0.0};
-  double cb_prev = 0.0;  // c* of tri_b at the level above
-
-  TileRegs<R> RG;
-  const TileOffs TO = tile_offsets(tid, i0, j0, nx, ny);
-  tile_load(RG, TO, 0, ts, A, S, u, v, geo);
-  tile_store(LB[0], VL, RG, tid);
+  auto wet_at = [&](int k, int q) -> bool {  // cell k-2+q
+    if constexpr (ZC) return k + q - 2 >= 0 && k + q - 2 < nwc;
+    else return (m5 >> q & 1u) != 0;
+  };
+  double w_k = at_byte(w + k0 * n2, b0);
+  double kh_k = at_byte(Kh + k0 * n2, b0);  // K_h and 1 / spacing on interface k
+  double idz_k = k0 > 0 ? idz(k0) : 0.0;
+  // interface value at the top of level k: of the first level the surface
+  // cell's, else what the range above forms as its bottom one
+  R cf_top = k0 == 0 ? R(c5[2])
+                     : tracer_face_z<R>(adv, k0, nz, R(c5[0]), R(c5[1]), R(c5[2]), R(c5[3]),
+                                        wet_at(k0, 0), wet_at(k0, 3), R(w_k));
   __syncthreads();
-  const bool has_adv = adv != ADV_NONE;
-  for (int k = 0; k < nz; ++k) {
+  for (int k = k0; k < k1; ++k) {
     const long long o = (long long)k * n2;
-    const TileLds<R>& L = LB[k & 1];
-    if (k + 1 < nz) tile_load(RG, TO, o + n2, ts, A, S, u, v, geo);
-    // the own column's operands of level k, issued before the face pass so
-    // their latency hides behind it
-    double w_k1 = 0.0, kh_k1 = 0.0, dzi_k1 = 0.0, dz = 0.0;
-    if (active) {
-      w_k1 = w[o + n2 + c];
-      kh_k1 = Kh[o + n2 + c];
-      dzi_k1 = geo.dzi[o + n2 + c];
-      dz = geo.dz3[o + c];
-    }
-    // ---- faces: the east and north face of every cell, plus the tile's
-    // west column (8) and south row (32) of faces by threads 0..39
+    const TracerLds<R>& L = LB[(k - k0) & 1];
+    const TracerFaceRegs f = rf;
+    if (k + 1 < k1) load(o + n2);
+    // the own column's operands below level k, issued before the face pass
+    const double w_k1 = at_byte(w + o + n2, b0);
+    const double kh_k1 = at_byte(Kh + o + n2, b0);
+    const double c_k3 = k + 3 < nz ? at_byte(C + o + 3 * n2, b0) : 0.0;
+    // ---- faces: the own east and north ones, and the tile's west and south
+    // edge ones by the edge threads
     {
-      auto xface = [&](int fy_, int q) {
-        const int cy = fy_ + HALO, c0x = q - 1 + HALO;
-        const R vel = VL.u[fy_][q];
-        const R ddu = VL.du[fy_][q];
-        const bool wm = L.m[cy][c0x - 1] != 0, w2 = L.m[cy][c0x + 2] != 0;
-        for (int r = 0; r < ntr; ++r) {
-          const R(*C)[SX] = L.c[r];
-          F.fx[r][fy_][q] = ddu * vel * tracer_face<R>(adv, C[cy][c0x - 1], C[cy][c0x],
-                                                       C[cy][c0x + 1], C[cy][c0x + 2], vel, wm,
-                                                       w2);
+      // thickness, far wet flags and own mask of face q whose point before it
+      // is (yy, xx) of the tile
+      auto geometry = [&](int q, int axis, int yy, int xx, R& dz, bool* m) {
+        if constexpr (ZC) {
+          const int n = (int)(fw[q] >> 16);
+          dz = R(k < n - 1 ? full : (k == n - 1 ? fl[q] : 0.0));
+          m[0] = k < (int)(fw[q] & 255u);
+          m[1] = k < (int)(fw[q] >> 8 & 255u);
+          m[2] = k < n;
+        } else {
+          const TracerMaskLds& M = MB[(k - k0) & 1];
+          dz = R(f.dz[q]);
+          m[0] = (axis ? M.m[yy - 1][xx] : M.m[yy][xx - 1]) != 0;
+          m[1] = (axis ? M.m[yy + 2][xx] : M.m[yy][xx + 2]) != 0;
+          m[2] = f.m[q] != 0;
         }
       };
-      auto yface = [&](int q, int fx_) {
-        const int cx = fx_ + HALO, c0y = q - 1 + HALO;
-        const R vel = VL.v[q][fx_];
-        const R ddv = VL.dv[q][fx_];
-        const bool wm = L.m[c0y - 1][cx] != 0, w2 = L.m[c0y + 2][cx] != 0;
-        for (int r = 0; r < ntr; ++r) {
-          const R(*C)[SX] = L.c[r];
-          F.fy[r][q][fx_] = ddv * vel * tracer_face<R>(adv, C[c0y - 1][cx], C[c0y][cx],
-                                                       C[c0y + 1][cx], C[c0y + 2][cx], vel, wm,
-                                                       w2);
-        }
+      // x-face q of row r (between columns q-1 and q), operands s
+      auto xface = [&](int r, int q, int s) {
+        const int yy = r + HALO, x0 = q - 1 + HALO;
+        R dz;
+        bool m[3];
+        geometry(s, 0, yy, x0, dz, m);
+        const R a0 = L.c[yy][x0], a1 = L.c[yy][x0 + 1], vel = R(f.vel[s]);
+        if (TVD || has_adv)
+          F.fx[r][q] = dz * vel * tracer_face<R>(adv, L.c[yy][x0 - 1], a0, a1, L.c[yy][x0 + 2],
+                                                 vel, m[0], m[1]);
+        F.gx[r][q] = by_dx((m[2] ? R(1) : R(0)) * (a1 - a0));
       };
-      if (has_adv) {
-        xface(ty, tx + 1);
-        yface(ty + 1, tx);
-        if (tid < TY) xface(tid, 0);
-        else if (tid < TY + TX) yface(0, tid - TY);
-      }
+      // y-face q of column r (between rows q-1 and q)
+      auto yface = [&](int q, int r, int s) {
+        const int xx = r + HALO, y0 = q - 1 + HALO;
+        R dz;
+        bool m[3];
+        geometry(s, 1, y0, xx, dz, m);
+        const R a0 = L.c[y0][xx], a1 = L.c[y0 + 1][xx], vel = R(f.vel[s]);
+        if (TVD || has_adv)
+          F.fy[q][r] = dz * vel * tracer_face<R>(adv, L.c[y0 - 1][xx], a0, a1, L.c[y0 + 2][xx],
+                                                 vel, m[0], m[1]);
+        F.gy[q][r] = by_dy((m[2] ? R(1) : R(0)) * (a1 - a0));
+      };
+      xface(ty, tx + 1, 0);
+      yface(ty + 1, tx, 1);
+      if (is_x) xface(xe, 0, 2);
+      if (is_y) yface(0, ye, 2);
     }
     __syncthreads();
-    if (active) {
-      // ---- own-column values for level k
-      const double inv = safe_inv(dz);
-      const bool m_k = mw[2];
-      const bool bot_km1 = k >= 1 && mw[1] && !mw[2];          // cell k-1 is a bottom cell
-      const bool bot_k = m_k && !((k + 1 < nz) && mw[3]);      // cell k is a bottom cell
-      const int cx = tx + HALO, cy = ty + HALO;
-      // row k of tri_b (K_h, no drag), factored here from the operands the
-      // diffusion terms read anyway; c* parked in `cst` for the back-substitution
-      double sub_k, den_k, cst_k;
-      factor_row(p, k, inv, kh_k, kh_k1, safe_inv(dzi_k), safe_inv(dzi_k1), m_k,
-                 (k + 1 < nz) && mw[3], p.thv_dt * 0.0, cb_prev, sub_k, den_k, cst_k);
-      cst[o + c] = cst_k;
-      cb_prev = cst_k;
-
-      for (int r = 0; r < ntr; ++r) {
-        const double cc = win[r][2];  // the tile's own cell, in fp64
-        double tend = 0.0;
-        if (!ts) tend = p.neg_N2 * (0.5 * (w_k + w_k1));
-        if (has_adv) {
-          const R hdiv = ((F.fx[r][ty][tx + 1] - F.fx[r][ty][tx]) / R(p.dx) +
-                          (F.fy[r][ty + 1][tx] - F.fy[r][ty][tx]) / R(p.dy)) * R(inv);
-          const R cft = (k == 0) ? R(win[r][2]) : cf_top[r];
-          const R cfb = tracer_face_z<R>(adv, k + 1, nz, R(win[r][1]), R(win[r][2]),
-                                         R(win[r][3]), R(win[r][4]), mw[1], mw[4], R(w_k1));
-          cf_top[r] = cfb;
-          const R vdiv = (R(w_k) * cft - R(w_k1) * cfb) * R(inv);
-          tend = tend - (double)((hdiv + vdiv) * (m_k ? R(1) : R(0)));
-        }
-        if (p.has_K_h) {
-          const R(*C)[SX] = L.c[r];
-          const R ge = face_grad<R>(L.mu[ty][tx + 1], C[cy][cx], C[cy][cx + 1], p.dx);
-          const R gw = face_grad<R>(L.mu[ty][tx], C[cy][cx - 1], C[cy][cx], p.dx);
-          const R gn = face_grad<R>(L.mv[ty + 1][tx], C[cy][cx], C[cy + 1][cx], p.dy);
-          const R gs = face_grad<R>(L.mv[ty][tx], C[cy - 1][cx], C[cy][cx], p.dy);
-          tend = tend + p.K_h * (double)((m_k ? R(1) : R(0)) *
-                                         ((ge - gw) / R(p.dx) + (gn - gs) / R(p.dy)));
-        }
-        // explicit vertical diffusion with the surface flux (vertical_var.py:80-106)
-        double ft;
-        if (k == 0) {
-          ft = flux[r];
-        } else {
-          ft = kh_k * (win[r][1] - win[r][2]) * safe_inv(dzi_k);
-          if (bot_km1) ft = 0.0;
-        }
-        double fb = 0.0;
-        if (k + 1 < nz) {
-          fb = kh_k1 * (win[r][2] - win[r][3]) * safe_inv(dzi_k1);
-          if (bot_k) fb = 0.0;
-        }
-        const double out = (ft - fb) * inv;
-        const double dr = 0.0 * win[r][2] * (bot_k ? 1.0 : 0.0);
-        const double dzd = (out - dr * inv) * (m_k ? 1.0 : 0.0);
-        double rhs = cc + p.dt * tend + p.c_dzd * dzd;
-        if (k == 0) rhs = rhs + p.thv_dt * flux[r] * safe_inv(dz);
-        const long long t = o + c;
-        const double dd = (k == 0) ? rhs / den_k : (rhs - sub_k * dprev[r]) / den_k;
-        dprev[r] = dd;
-        (r == 0 ? Ao : S_out)[t] = dd;
+    // ---- the own cell
+    {
+      const bool m_k = wet_at(k, 2);
+      const double iv = inv(k);
+      const bool lower = k + 1 < nz;
+      const double idz_k1 = lower ? idz(k + 1) : 0.0;
+      double tend = 0.0;
+      if (!ts) tend = p.neg_N2 * (0.5 * (w_k + w_k1));
+      if (TVD || has_adv) {
+        const R hdiv = (by_dx(F.fx[ty][tx + 1] - F.fx[ty][tx]) +
+                        by_dy(F.fy[ty + 1][tx] - F.fy[ty][tx])) * R(iv);
+        const R cfb = tracer_face_z<R>(adv, k + 1, nz, R(c5[1]), R(c5[2]), R(c5[3]), R(c5[4]),
+                                       wet_at(k, 1), wet_at(k, 4), R(w_k1));
+        const R vdiv = (R(w_k) * cf_top - R(w_k1) * cfb) * R(iv);
+        cf_top = cfb;
+        tend = tend - (double)((hdiv + vdiv) * (m_k ? R(1) : R(0)));
       }
-      // ---- advance the windows
-      for (int r = 0; r < 2; ++r)
-        for (int q = 0; q < 4; ++q) win[r][q] = win[r][q + 1];
-      for (int q = 0; q < 4; ++q) mw[q] = mw[q + 1];
-      const int kn = k + 3;
-      if (kn < nz) {
-        win[0][4] = A[(long long)kn * n2 + c];
-        if (ts) win[1][4] = S[(long long)kn * n2 + c];
-        mw[4] = geo.m3[(long long)kn * n2 + c] != 0;
-      } else {
-        win[0][4] = 0.0;
-        win[1][4] = 0.0;
-        mw[4] = false;
-      }
+      if (p.has_K_h)
+        tend = tend + p.K_h * (double)((m_k ? R(1) : R(0)) *
+                                       (by_dx(F.gx[ty][tx + 1] - F.gx[ty][tx]) +
+                                        by_dy(F.gy[ty + 1][tx] - F.gy[ty][tx])));
+      // explicit vertical diffusion with the surface flux (vertical_var.py:80-106)
+      const double dzd = explicit_diffusion_inv(k, nz, c5[1], c5[2], c5[3], idz_k, idz_k1, iv,
+                                                wet_at(k, 1), m_k, lower && wet_at(k, 3), kh_k,
+                                                kh_k1, flux, 0.0);
+      double rhs = c5[2] + p.dt * tend + p.c_dzd * dzd;
+      if (k == 0) rhs = rhs + p.thv_dt * flux * iv;
+      if (active) put_byte(out + o, b0, rhs);
+      // advance the windows
+#pragma unroll
+      for (int q = 0; q < 4; ++q) c5[q] = c5[q + 1];
+      c5[4] = c_k3;
+      if constexpr (!ZC) m5 = m5 >> 1 | (k + 3 < nz && cell_wet(k + 3) ? 16u : 0u);
       w_k = w_k1;
       kh_k = kh_k1;
-      dzi_k = dzi_k1;
+      idz_k = idz_k1;
     }
-    if (k + 1 < nz) tile_store(LB[(k + 1) & 1], VL, RG, tid);
+    if (k + 1 < k1) store((k + 1 - k0) & 1);
     __syncthreads();
   }
-  if (!active) return;
-  // back-substitution with the next level's operands loaded one level ahead
-  double xa = 0.0, xb = 0.0;
-  long long t = (long long)(nz - 1) * n2 + c;
-  double a_n = Ao[t], s_n = ts ? S_out[t] : 0.0, c_n = cst[t], z_n = ts ? geo.zc[t] : 0.0;
-  uint8_t m_n = geo.m3[t];
-  for (int k = nz - 1; k >= 0; --k) {
-    const double a_k = a_n, s_k = s_n, c_k = c_n, z_k = z_n;
-    const double mm = mk(m_n);
-    const long long tk = t;
-    if (k > 0) {
-      t -= n2;
-      a_n = Ao[t];
-      if (ts) s_n = S_out[t];
-      c_n = cst[t];
-      if (ts) z_n = geo.zc[t];
-      m_n = geo.m3[t];
-    }
-    xa = (k == nz - 1) ? a_k : a_k - c_k * xa;
-    Ao[tk] = xa * mm;
-    if (ts) {
-      xb = (k == nz - 1) ? s_k : s_k - c_k * xb;
-      S_out[tk] = xb * mm;
-      if (p.eos_mixed)
-        b_out[tk] = buoyancy_mixed(p, xa * mm, xb * mm, z_k) * mm;
-      else
-        b_out[tk] = buoyancy(p, xa * mm, xb * mm, z_k) * mm;
-    }
-  }
 }
 
-}  // namespace hoc
-
-namespace hoc {
-
-// ------------------------------------------------ column-form geometry
-// Column geometry of a tile and its 2-cell halo, staged once per launch:
-// wet levels nw and deepest wet thickness hb per column, and the 2D face
-// masks. Every thickness, face thickness and 3D mask of the tile at any
-// level follows from these (cg_dz, cg_face in hoc_device.h).
-struct ColTile {  // [SY + 1][SX + 1]: the face flags of the last halo row and column
-  double hb[SY + 1][SX + 1];  // need the column beyond them
-  uint8_t nw[SY + 1][SX + 1];
-  uint8_t mu[SY + 1][SX + 1];  // mask_u: the east face of the column is open
-  uint8_t mv[SY + 1][SX + 1];  // mask_v: the north face of the column is open
-};
-
-__device__ __forceinline__ void col_tile_load(ColTile& CG, const Geo& geo, int tid, int i0,
-                                              int j0, int nx, int ny) {
-  for (int t = tid; t < (SX + 1) * (SY + 1); t += TILE_THREADS) {
-    const int lx = t % (SX + 1), ly = t / (SX + 1);
-    const long long g = (long long)pmod(j0 + ly - HALO, ny) * nx + pmod(i0 + lx - HALO, nx);
-    CG.hb[ly][lx] = geo.hb[g];
-    CG.nw[ly][lx] = geo.nw[g];
-    CG.mu[ly][lx] = geo.mu2[g];
-    CG.mv[ly][lx] = geo.mv2[g];
-  }
-}
-
-// Level-k wet flags of the east face of tile column (ly, lx) and of its
-// north face (mask3u, mask3v).
-__device__ __forceinline__ bool col_wet_u(const ColTile& CG, int ly, int lx, int k) {
-  return CG.mu[ly][lx] && k < CG.nw[ly][lx] && k < CG.nw[ly][lx + 1];
-}
-__device__ __forceinline__ bool col_wet_v(const ColTile& CG, int ly, int lx, int k) {
-  return CG.mv[ly][lx] && k < CG.nw[ly][lx] && k < CG.nw[ly + 1][lx];
-}
-
-// Per-level staging of the column-form tracer tile: the tracers with halo
-// and the face velocities; no geometry.
-template <class R>
-struct TracerLdsC {
-  R c[2][SY][SX];
-};
-template <class R>
-struct VelLdsC {
-  R u[TY][TX + 1];  // u at i-1 .. i
-  R v[TY + 1][TX];  // v at j-1 .. j
-};
-template <class R>
-struct TracerRegsC {
-  R c0[ST_C], c1[ST_C];
-  R u[ST_U];
-  R v[ST_V];
-};
-
-template <class RT>
-__device__ __forceinline__ void tracer_load_c(TracerRegsC<RT>& R, const TileOffs& F, long long o,
-                                              bool ts, const double* A, const double* S,
-                                              const double* u, const double* v) {
-#pragma unroll
-  for (int q = 0; q < ST_C; ++q) {
-    if (F.c[q] >= 0) {
-      const long long g = o + F.c[q];
-      R.c0[q] = (RT)A[g];
-      R.c1[q] = ts ? (RT)S[g] : RT(0);
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < ST_U; ++q)
-    if (F.u[q] >= 0) R.u[q] = (RT)u[o + F.u[q]];
-#pragma unroll
-  for (int q = 0; q < ST_V; ++q)
-    if (F.v[q] >= 0) R.v[q] = (RT)v[o + F.v[q]];
-}
-
-template <class RT>
-__device__ __forceinline__ void tracer_store_c(TracerLdsC<RT>& L, VelLdsC<RT>& V,
-                                               const TracerRegsC<RT>& R, int tid) {
-#pragma unroll
-  for (int q = 0; q < ST_C; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    if (t < SX * SY) {
-      const int lx = t % SX, ly = t / SX;
-      L.c[0][ly][lx] = R.c0[q];
-      L.c[1][ly][lx] = R.c1[q];
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < ST_U; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    if (t < TY * (TX + 1)) V.u[t / (TX + 1)][t % (TX + 1)] = R.u[q];
-  }
-#pragma unroll
-  for (int q = 0; q < ST_V; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    if (t < (TY + 1) * TX) V.v[t / TX][t % TX] = R.v[q];
-  }
-}
-
-// k_tracers_tiled for a static z-level geometry in column form: the same
-// operations on the same operands in the same order (so the same bits),
-// with every thickness, face thickness, centre depth and 3D mask formed from
-// the tile's column geometry instead of read per cell, and tri_b factored
-// in the forward sweep. Per layer cell it reads T, S, u, v, w and K_h, and
-// writes T, S, b, with d* (in the outputs) and c* (in `cst`) parked between
-// the sweeps.
-template <class R>
-__global__ __launch_bounds__(TILE_THREADS)
-__attribute__((amdgpu_waves_per_eu(sizeof(R) == 4 ? 4 : 1))) void k_tracers_col(
-    Dims d, StepParams p, Geo geo, const double* __restrict__ T, const double* __restrict__ S,
-    const double* __restrict__ b, const double* __restrict__ u, const double* __restrict__ v,
-    const double* __restrict__ w, const double* __restrict__ Kh, double* __restrict__ cst,
-    double* __restrict__ T_out, double* __restrict__ S_out, double* __restrict__ b_out) {
-  __shared__ TracerLdsC<R> LB[2];
-  __shared__ VelLdsC<R> VL;
-  __shared__ FaceLds<R> F;
-  __shared__ ColTile CG;
-  const int nx = d.nx, ny = d.ny, nz = d.nz;
+// The tracers' implicit vertical diffusion, in place on the right-hand sides
+// k_tracer_rhs left in the outputs: tri_b (K_h, no drag) factored and the
+// forward sweep in one march down the column (c* parked in `cst`, d* in the
+// outputs), then the back-substitution, the mask and the EOS
+// (libs/core/model3d_v05.py:476-533). One pivot serves c* and both tracers:
+// its reciprocal is formed once. Bound by HBM where the columns fill the chip
+// (12 fields of 8 bytes per cell: 165 us at 512 x 512 x 40, 6.1 TB/s) and by the
+// recurrence's latency below that, so operands are loaded SOLVE_AHEAD levels
+// at a time ahead of it (2 / 4 / 8 levels: 436 / 425 / 454 us for both tracer
+// kernels at 512 x 512 x 40, equal at 128 x 128 x 30) and a workgroup is one
+// wave, which spreads few columns over the most compute units.
+constexpr int SOLVE_AHEAD = 4, SOLVE_THREADS = 64;
+template <bool ZC>
+__global__ __launch_bounds__(SOLVE_THREADS) void k_tracer_solve(
+    Dims d, StepParams p, Geo geo, const double* __restrict__ zs, const double* __restrict__ Kh,
+    double* __restrict__ cst, double* __restrict__ T_out, double* __restrict__ S_out,
+    double* __restrict__ b_out) {
+  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= d.n2) return;
+  const int nz = d.nz;
   const long long n2 = d.n2;
-  const int tid = threadIdx.x;
-  const int tx = tid % TX, ty = tid / TX;
-  int bx, by;
-  xcd_tile(bx, by);
-  const int i0 = bx * TX, j0 = by * TY;
-  const int i = i0 + tx, j = j0 + ty;
-  const bool active = i < nx && j < ny;
-  const long long c = active ? (long long)j * nx + i : 0;
   const bool ts = p.tracers_ts != 0;
-  const int ntr = ts ? 2 : 1;
-  const double* A = ts ? T : b;
-  double* Ao = ts ? T_out : b_out;
-  const double flux[2] = {ts ? p.flux_T : 0.0, p.flux_S};
-  const int adv = p.advection;
-  const double dzr = p.dzr;
-  const int rule = p.face_rule;
-  const int cx = tx + HALO, cy = ty + HALO;
-
-  TracerRegsC<R> RG;
-  const TileOffs TO = tile_offsets(tid, i0, j0, nx, ny);
-  tracer_load_c(RG, TO, 0, ts, A, S, u, v);
-  col_tile_load(CG, geo, tid, i0, j0, nx, ny);
-  tracer_store_c(LB[0], VL, RG, tid);
-  __syncthreads();
-  const int nwc = CG.nw[cy][cx];
-  const double hbc = CG.hb[cy][cx];
-  auto wet = [&](int kk) { return kk >= 0 && kk < nwc; };
-
-  // own-column window: tracer at k-2..k+2
-  double win[2][5];
-  for (int q = 0; q < 5; ++q) win[0][q] = win[1][q] = 0.0;
-  if (active) {
-    for (int q = 2; q < 5; ++q) {
-      const int kk = q - 2;
-      if (kk < nz) {
-        win[0][q] = A[kk * n2 + c];
-        if (ts) win[1][q] = S[kk * n2 + c];
-      }
-    }
+  double* A = ts ? T_out : b_out;
+  constexpr int W = SOLVE_AHEAD;
+  InvCol ca{};
+  int nwc = 0;
+  double hbc = 0.0, bot = 0.0;
+  if constexpr (ZC) {
+    nwc = geo.nw[c];
+    hbc = geo.hb[c];
+    ca = inv_col(nwc, p.dzr, nwc > 0 ? hbc : 0.0);
+    bot = nwc > 0 ? zs[nwc - 1] + hbc : 0.0;
   }
-  double w_k = active ? w[c] : 0.0;
-  double kh_k = active ? Kh[c] : 0.0;
-  double dzi_k = cg_dzi(dzr, nwc, hbc, 0, nz);
-  R cf_top[2] = {R(0), R(0)};  // interface value at the top of level k
-  double dprev[2] = {0.0, 0.0};
-  double cb_prev = 0.0;  // c* of tri_b at the level above
-
-  const bool has_adv = adv != ADV_NONE;
-  for (int k = 0; k < nz; ++k) {
-    const long long o = (long long)k * n2;
-    const TracerLdsC<R>& L = LB[k & 1];
-    if (k + 1 < nz) tracer_load_c(RG, TO, o + n2, ts, A, S, u, v);
-    double w_k1 = 0.0, kh_k1 = 0.0;
-    if (active) {
-      w_k1 = w[o + n2 + c];
-      kh_k1 = Kh[o + n2 + c];
-    }
-    const double dzi_k1 = cg_dzi(dzr, nwc, hbc, k + 1, nz);
-    const double dz = cg_dz(dzr, nwc, hbc, k);
-    // ---- faces: the east and north face of every cell, plus the tile's
-    // west column (8) and south row (32) of faces by threads 0..39
-    if (has_adv) {
-      auto xface = [&](int fy_, int q) {
-        const int yy = fy_ + HALO, c0x = q - 1 + HALO;
-        const R vel = VL.u[fy_][q];
-        const R ddu = R(cg_face(rule, dzr, CG.mu[yy][c0x] != 0, CG.nw[yy][c0x], CG.hb[yy][c0x],
-                                CG.nw[yy][c0x + 1], CG.hb[yy][c0x + 1], k));
-        const bool wm = k < CG.nw[yy][c0x - 1], w2 = k < CG.nw[yy][c0x + 2];
-        for (int r = 0; r < ntr; ++r) {
-          const R(*C)[SX] = L.c[r];
-          F.fx[r][fy_][q] = ddu * vel * tracer_face<R>(adv, C[yy][c0x - 1], C[yy][c0x],
-                                                       C[yy][c0x + 1], C[yy][c0x + 2], vel, wm,
-                                                       w2);
-        }
-      };
-      auto yface = [&](int q, int fx_) {
-        const int xx = fx_ + HALO, c0y = q - 1 + HALO;
-        const R vel = VL.v[q][fx_];
-        const R ddv = R(cg_face(rule, dzr, CG.mv[c0y][xx] != 0, CG.nw[c0y][xx], CG.hb[c0y][xx],
-                                CG.nw[c0y + 1][xx], CG.hb[c0y + 1][xx], k));
-        const bool wm = k < CG.nw[c0y - 1][xx], w2 = k < CG.nw[c0y + 2][xx];
-        for (int r = 0; r < ntr; ++r) {
-          const R(*C)[SX] = L.c[r];
-          F.fy[r][q][fx_] = ddv * vel * tracer_face<R>(adv, C[c0y - 1][xx], C[c0y][xx],
-                                                       C[c0y + 1][xx], C[c0y + 2][xx], vel, wm,
-                                                       w2);
-        }
-      };
-      xface(ty, tx + 1);
-      yface(ty + 1, tx);
-      if (tid < TY) xface(tid, 0);
-      else if (tid < TY + TX) yface(0, tid - TY);
-    }
-    __syncthreads();
-    if (active) {
-      const double inv = safe_inv(dz);
-      const bool m_k = wet(k);
-      const bool m_k1 = wet(k + 1);
-      const bool bot_km1 = k >= 1 && wet(k - 1) && !m_k;  // cell k-1 is a bottom cell
-      const bool bot_k = m_k && !((k + 1 < nz) && m_k1);   // cell k is a bottom cell
-      double sub_k, den_k, cst_k;
-      factor_row(p, k, inv, kh_k, kh_k1, safe_inv(dzi_k), safe_inv(dzi_k1), m_k,
-                 (k + 1 < nz) && m_k1, p.thv_dt * 0.0, cb_prev, sub_k, den_k, cst_k);
-      cst[o + c] = cst_k;
-      cb_prev = cst_k;
-      const uint8_t mue = col_wet_u(CG, cy, cx, k), muw = col_wet_u(CG, cy, cx - 1, k);
-      const uint8_t mvn = col_wet_v(CG, cy, cx, k), mvs = col_wet_v(CG, cy - 1, cx, k);
-
-      for (int r = 0; r < ntr; ++r) {
-        const double cc = win[r][2];  // the tile's own cell, in fp64
-        double tend = 0.0;
-        if (!ts) tend = p.neg_N2 * (0.5 * (w_k + w_k1));
-        if (has_adv) {
-          const R hdiv = ((F.fx[r][ty][tx + 1] - F.fx[r][ty][tx]) / R(p.dx) +
-                          (F.fy[r][ty + 1][tx] - F.fy[r][ty][tx]) / R(p.dy)) * R(inv);
-          const R cft = (k == 0) ? R(win[r][2]) : cf_top[r];
-          const R cfb = tracer_face_z<R>(adv, k + 1, nz, R(win[r][1]), R(win[r][2]),
-                                         R(win[r][3]), R(win[r][4]), wet(k - 1), wet(k + 2),
-                                         R(w_k1));
-          cf_top[r] = cfb;
-          const R vdiv = (R(w_k) * cft - R(w_k1) * cfb) * R(inv);
-          tend = tend - (double)((hdiv + vdiv) * (m_k ? R(1) : R(0)));
-        }
-        if (p.has_K_h) {
-          const R(*C)[SX] = L.c[r];
-          const R ge = face_grad<R>(mue, C[cy][cx], C[cy][cx + 1], p.dx);
-          const R gw = face_grad<R>(muw, C[cy][cx - 1], C[cy][cx], p.dx);
-          const R gn = face_grad<R>(mvn, C[cy][cx], C[cy + 1][cx], p.dy);
-          const R gs = face_grad<R>(mvs, C[cy - 1][cx], C[cy][cx], p.dy);
-          tend = tend + p.K_h * (double)((m_k ? R(1) : R(0)) *
-                                         ((ge - gw) / R(p.dx) + (gn - gs) / R(p.dy)));
-        }
-        // explicit vertical diffusion with the surface flux (vertical_var.py:80-106)
-        double ft;
-        if (k == 0) {
-          ft = flux[r];
-        } else {
-          ft = kh_k * (win[r][1] - win[r][2]) * safe_inv(dzi_k);
-          if (bot_km1) ft = 0.0;
-        }
-        double fb = 0.0;
-        if (k + 1 < nz) {
-          fb = kh_k1 * (win[r][2] - win[r][3]) * safe_inv(dzi_k1);
-          if (bot_k) fb = 0.0;
-        }
-        const double out = (ft - fb) * inv;
-        const double dr = 0.0 * win[r][2] * (bot_k ? 1.0 : 0.0);
-        const double dzd = (out - dr * inv) * (m_k ? 1.0 : 0.0);
-        double rhs = cc + p.dt * tend + p.c_dzd * dzd;
-        if (k == 0) rhs = rhs + p.thv_dt * flux[r] * safe_inv(dz);
-        const double dd = (k == 0) ? rhs / den_k : (rhs - sub_k * dprev[r]) / den_k;
-        dprev[r] = dd;
-        (r == 0 ? Ao : S_out)[o + c] = dd;
+  // operands of W levels: right-hand sides, K_h below, and the geometry read
+  // from the arrays
+  struct Ahead {
+    double a[W], s[W], kh[W], dz[W], dzi[W];
+    bool wet[W];
+  };
+  auto load = [&](int kb, Ahead& g) {
+#pragma unroll
+    for (int q = 0; q < W; ++q) {
+      const long long k = kb + q < nz ? kb + q : nz - 1;
+      g.a[q] = A[k * n2 + c];
+      g.s[q] = ts ? S_out[k * n2 + c] : 0.0;
+      g.kh[q] = Kh[(k + 1) * n2 + c];
+      if constexpr (!ZC) {
+        g.dz[q] = geo.dz3[k * n2 + c];
+        g.dzi[q] = geo.dzi[(k + 1) * n2 + c];
+        g.wet[q] = kb + q + 1 < nz && geo.m3[(k + 1 < nz ? k + 1 : k) * n2 + c] != 0;
       }
-      // ---- advance the window
-      for (int r = 0; r < 2; ++r)
-        for (int q = 0; q < 4; ++q) win[r][q] = win[r][q + 1];
-      const int kn = k + 3;
-      if (kn < nz) {
-        win[0][4] = A[(long long)kn * n2 + c];
-        if (ts) win[1][4] = S[(long long)kn * n2 + c];
+    }
+  };
+  Ahead cur, nxt;
+  load(0, cur);
+  double kh_t = Kh[c], c_prev = 0.0, da = 0.0, ds = 0.0;
+  double idzi_t;
+  bool wet;
+  if constexpr (ZC) {
+    idzi_t = ca.inv(0);
+    wet = nwc > 0;
+  } else {
+    idzi_t = safe_inv(geo.dzi[c]);
+    wet = geo.m3[c] != 0;
+  }
+  for (int kb = 0; kb < nz; kb += W) {
+    if (kb + W < nz) load(kb + W, nxt);
+#pragma unroll
+    for (int q = 0; q < W; ++q) {
+      const int k = kb + q;
+      if (k >= nz) break;
+      double inv, idzi_b;
+      bool below;
+      if constexpr (ZC) {
+        inv = ca.inv(k);
+        idzi_b = k + 1 == nz ? inv : ca.idzi(k + 1);
+        below = k + 1 < nwc;
       } else {
-        win[0][4] = 0.0;
-        win[1][4] = 0.0;
+        inv = safe_inv(cur.dz[q]);
+        idzi_b = safe_inv(cur.dzi[q]);
+        below = cur.wet[q];
       }
-      w_k = w_k1;
-      kh_k = kh_k1;
+      double sub, sup, den;
+      matrix_row(p, k, inv, kh_t, cur.kh[q], idzi_t, idzi_b, wet, below, p.thv_dt * 0.0, c_prev,
+                 sub, sup, den);
+      const Divisor<double> by_den(den);
+      const double cs = by_den(sup);
+      da = k == 0 ? by_den(cur.a[q]) : by_den(cur.a[q] - sub * da);
+      ds = k == 0 ? by_den(cur.s[q]) : by_den(cur.s[q] - sub * ds);
+      const long long t = k * n2 + c;
+      cst[t] = cs;
+      A[t] = da;
+      if (ts) S_out[t] = ds;
+      c_prev = cs;
+      kh_t = cur.kh[q];
+      idzi_t = idzi_b;
+      wet = below;
     }
-    dzi_k = dzi_k1;
-    if (k + 1 < nz) tracer_store_c(LB[(k + 1) & 1], VL, RG, tid);
-    __syncthreads();
+    cur = nxt;
   }
-  if (!active) return;
-  // back-substitution with the next level's operands loaded one level ahead
-  double xa = 0.0, xb = 0.0;
-  long long t = (long long)(nz - 1) * n2 + c;
-  double a_n = Ao[t], s_n = ts ? S_out[t] : 0.0, c_n = cst[t];
-  for (int k = nz - 1; k >= 0; --k) {
-    const double a_k = a_n, s_k = s_n, c_k = c_n;
-    const double mm = wet(k) ? 1.0 : 0.0;
-    const long long tk = t;
-    if (k > 0) {
-      t -= n2;
-      a_n = Ao[t];
-      if (ts) s_n = S_out[t];
-      c_n = cst[t];
+  // back-substitution, W levels loaded ahead
+  struct Back {
+    double a[W], s[W], cs[W], z[W];
+    bool wet[W];
+  };
+  auto load_back = [&](int kt, Back& g) {  // levels kt, kt - 1, ...
+#pragma unroll
+    for (int q = 0; q < W; ++q) {
+      const long long k = kt - q > 0 ? kt - q : 0;
+      g.a[q] = A[k * n2 + c];
+      g.s[q] = ts ? S_out[k * n2 + c] : 0.0;
+      g.cs[q] = cst[k * n2 + c];
+      if constexpr (ZC) {
+        g.z[q] = cg_zc_at(zs[k], p.dzr, nwc, hbc, bot, (int)k);
+        g.wet[q] = k < nwc;
+      } else {
+        g.z[q] = ts ? geo.zc[k * n2 + c] : 0.0;
+        g.wet[q] = geo.m3[k * n2 + c] != 0;
+      }
     }
-    xa = (k == nz - 1) ? a_k : a_k - c_k * xa;
-    Ao[tk] = xa * mm;
-    if (ts) {
-      xb = (k == nz - 1) ? s_k : s_k - c_k * xb;
-      S_out[tk] = xb * mm;
-      const double z_k = cg_zc(geo.zs, dzr, nwc, hbc, k);
-      if (p.eos_mixed)
-        b_out[tk] = buoyancy_mixed(p, xa * mm, xb * mm, z_k) * mm;
-      else
-        b_out[tk] = buoyancy(p, xa * mm, xb * mm, z_k) * mm;
+  };
+  Back bc, bn;
+  load_back(nz - 1, bc);
+  double xa = 0.0, xs = 0.0;
+  for (int kt = nz - 1; kt >= 0; kt -= W) {
+    if (kt - W >= 0) load_back(kt - W, bn);
+#pragma unroll
+    for (int q = 0; q < W; ++q) {
+      const int k = kt - q;
+      if (k < 0) break;
+      const long long t = k * n2 + c;
+      const double mm = bc.wet[q] ? 1.0 : 0.0;
+      xa = k == nz - 1 ? bc.a[q] : bc.a[q] - bc.cs[q] * xa;
+      A[t] = xa * mm;
+      if (ts) {
+        xs = k == nz - 1 ? bc.s[q] : bc.s[q] - bc.cs[q] * xs;
+        S_out[t] = xs * mm;
+        const double bb = p.eos_mixed ? buoyancy_mixed(p, xa * mm, xs * mm, bc.z[q])
+                                      : buoyancy(p, xa * mm, xs * mm, bc.z[q]);
+        b_out[t] = bb * mm;
+      }
     }
+    bc = bn;
   }
 }
-
-}  // namespace hoc
-
-namespace hoc {
 
 // ------------------------------------------------- explicit momentum terms
 // Staged tile of one level for one velocity component A (u or v): A with a
@@ -776,65 +568,28 @@ struct MomMaskLds {
   uint8_t mo[TY + 1][TX + 1];
 };
 
-// Face fluxes of one component on one level, each computed once: the
-// advective flux (advecting velocity times the face value) and the A_h
-// gradient, on the x-faces (index q: between tile columns q-1 and q) and the
-// y-faces (between rows q-1 and q).
-template <class R>
-struct MomFaces {
-  R fx[TY][TX + 1], gx[TY][TX + 1];
-  R fy[TY + 1][TX], gy[TY + 1][TX];
-};
-
-constexpr int MS_H = (SX * SY + TILE_THREADS - 1) / TILE_THREADS;              // halo slots
 constexpr int MS_O = ((TY + 1) * (TX + 1) + TILE_THREADS - 1) / TILE_THREADS;  // +1 slots
 
 // Level-k staging held in registers between its global loads and its LDS
 // stores or its use, and this thread's plane offsets.
 template <class R>
 struct MomRegs {
-  R a[MS_H], o[MS_O];
+  R a[ST_H], o[MS_O];
   double phi[2], b[2];  // at the own point and the next one along the component's direction
   R w[2];               // on interface k + 1
 };
 struct MomGeoRegs {  // geometry read from the arrays
-  uint8_t ma[MS_H], mo[MS_O];
+  uint8_t ma[ST_H], mo[MS_O];
   double zc[2];
 };
+
+// Plane indexes of this thread's slots of the other component's points.
 struct MomOffs {
-  unsigned h[MS_H];  // A with its halo
-  unsigned o[MS_O];  // the other component's points
+  unsigned o[MS_O];
 };
-
-// Value of a plane at a byte offset. The plane's address is the same in every
-// lane and is kept in scalar registers, so that one vector register holds the
-// offset for every array (a plane is below 2^32 bytes). Without the empty asm
-// the compiler keeps a 64-bit vector address per array across the march, 30
-// registers here.
-template <class T>
-__device__ __forceinline__ T at_byte(const T* plane, unsigned off) {
-  unsigned long long a = (unsigned long long)plane;
-  __asm__("" : "+s"(a));
-  using G = const __attribute__((address_space(1))) char;
-  return *(const __attribute__((address_space(1))) T*)((G*)a + off);
-}
-__device__ __forceinline__ void put_byte(double* plane, unsigned off, double v) {
-  unsigned long long a = (unsigned long long)plane;
-  __asm__("" : "+s"(a));
-  using G = __attribute__((address_space(1))) char;
-  *(__attribute__((address_space(1))) double*)((G*)a + off) = v;
-}
-
-// Slots beyond the tile read the own point (the value is not stored).
 template <int COMP>
 __device__ __forceinline__ MomOffs mom_offsets(int tid, int i0, int j0, int nx, int ny) {
   MomOffs F;
-#pragma unroll
-  for (int q = 0; q < MS_H; ++q) {
-    const int t = tid + q * TILE_THREADS;
-    const int tt = t < SX * SY ? t : tid;
-    F.h[q] = (unsigned)(pmod(j0 + tt / SX - HALO, ny) * nx + pmod(i0 + tt % SX - HALO, nx));
-  }
 #pragma unroll
   for (int q = 0; q < MS_O; ++q) {
     const int t = tid + q * TILE_THREADS;
@@ -845,13 +600,6 @@ __device__ __forceinline__ MomOffs mom_offsets(int tid, int i0, int j0, int nx, 
   }
   return F;
 }
-
-struct NoTile {};
-
-// First threads that form the tile's west column of faces (TY of them) and
-// its south row (TX).
-constexpr int EDGE_X = 64, EDGE_Y = 0;
-static_assert(EDGE_X + TY <= TILE_THREADS && EDGE_Y + TX <= TILE_THREADS, "edge threads");
 
 // Vertical momentum flux on interface kk of the column: wb times the
 // interface value of the advected velocity (advection_v06.py:95-99,
@@ -871,16 +619,6 @@ __device__ __forceinline__ R mom_flux_z(int adv, int kk, int nz, R wb, R far_up,
                              TVD || adv == ADV_UP3_TVD);
   }
   return kk <= 0 || kk >= nz ? R(0) : f;
-}
-
-// Levels at which the east (axis 0) or north (axis 1) face of column (j, i)
-// is wet, for a static z-level geometry.
-__device__ __forceinline__ int face_levels(const Geo& geo, int axis, int j, int i, int ny,
-                                           int nx) {
-  const int c0 = j * nx + i;
-  const int c1 = axis == 0 ? j * nx + pmod(i + 1, nx) : pmod(j + 1, ny) * nx + i;
-  const int a = geo.nw[c0], b = geo.nw[c1];
-  return (axis == 0 ? geo.mu2[c0] : geo.mv2[c0]) ? (a < b ? a : b) : 0;
 }
 
 // Wet flags that the values of component COMP on the x-face (axis 0) or
@@ -904,7 +642,7 @@ __device__ __forceinline__ unsigned mom_face_wet(const Geo& geo, int axis, int j
 template <class R, bool ZC, bool TVD, int COMP, class Mask>
 __device__ __forceinline__ void momentum_component(
     const Dims& d, const StepParams& p, const Geo& geo, int i0, int j0, int k0, int k1,
-    MomLds<R>* LB, Mask* MB, MomFaces<R>& F, const double* __restrict__ A,
+    MomLds<R>* LB, Mask* MB, FaceLds<R>& F, const double* __restrict__ A,
     const double* __restrict__ O, const double* __restrict__ b, const double* __restrict__ phi,
     const double* __restrict__ w, const double* __restrict__ Km, const double* __restrict__ zs,
     double* __restrict__ pg, double* __restrict__ dzo, double* __restrict__ st) {
@@ -938,12 +676,13 @@ __device__ __forceinline__ void momentum_component(
 
   MomRegs<R> RG;
   MomGeoRegs GG;
+  const HaloOffs HO = halo_offsets(tid, i0, j0, nx, ny);
   const MomOffs MO = mom_offsets<COMP>(tid, i0, j0, nx, ny);
   auto load = [&](long long o) {
 #pragma unroll
-    for (int q = 0; q < MS_H; ++q) {
-      RG.a[q] = (R)at_byte(A + o, 8u * MO.h[q]);
-      if constexpr (!ZC) GG.ma[q] = at_byte(mA + o, MO.h[q]);
+    for (int q = 0; q < ST_H; ++q) {
+      RG.a[q] = (R)at_byte(A + o, 8u * HO.h[q]);
+      if constexpr (!ZC) GG.ma[q] = at_byte(mA + o, HO.h[q]);
     }
 #pragma unroll
     for (int q = 0; q < MS_O; ++q) {
@@ -963,7 +702,7 @@ __device__ __forceinline__ void momentum_component(
   };
   auto store = [&](int buf) {
 #pragma unroll
-    for (int q = 0; q < MS_H; ++q) {
+    for (int q = 0; q < ST_H; ++q) {
       const int t = tid + q * TILE_THREADS;
       if (t < SX * SY) {
         LB[buf].a[t / SX][t % SX] = RG.a[q];
@@ -1216,7 +955,7 @@ __global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(3)
     double* __restrict__ pgx, double* __restrict__ pgy, double* __restrict__ dzu,
     double* __restrict__ dzv, double* __restrict__ stu, double* __restrict__ stv) {
   __shared__ MomLds<R> LB[2];
-  __shared__ MomFaces<R> F;
+  __shared__ FaceLds<R> F;
   __shared__ std::conditional_t<ZC, NoTile, MomMaskLds> MB[2];
   const BlockTile T = xcd_block((d.nx + TX - 1) / TX, (d.ny + TY - 1) / TY, 2);
   const int k0 = T.z * nk;
@@ -1229,27 +968,6 @@ __global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(3)
                                  phi, w, Km, zs, pgy, dzv, stv);
 }
 
-void launch_tracers_tiled(bool mixed, hipStream_t s, Dims d, StepParams p, Geo geo,
-                          const double* T, const double* S, const double* b, const double* u,
-                          const double* v, const double* w, const double* Kh, double* cst,
-                          double* T_out, double* S_out, double* b_out) {
-  const dim3 grid((d.nx + TX - 1) / TX, (d.ny + TY - 1) / TY);
-  if (p.zcol) {
-    if (mixed)
-      k_tracers_col<float><<<grid, TILE_THREADS, 0, s>>>(d, p, geo, T, S, b, u, v, w, Kh, cst,
-                                                         T_out, S_out, b_out);
-    else
-      k_tracers_col<double><<<grid, TILE_THREADS, 0, s>>>(d, p, geo, T, S, b, u, v, w, Kh, cst,
-                                                          T_out, S_out, b_out);
-  } else if (mixed) {
-    k_tracers_tiled<float><<<grid, TILE_THREADS, 0, s>>>(d, p, geo, T, S, b, u, v, w, Kh, cst,
-                                                         T_out, S_out, b_out);
-  } else {
-    k_tracers_tiled<double><<<grid, TILE_THREADS, 0, s>>>(d, p, geo, T, S, b, u, v, w, Kh, cst,
-                                                          T_out, S_out, b_out);
-  }
-}
-
 // Levels per workgroup of a tiled march: all of them where the tiles alone give `target`
 // workgroups, else as few as make up that number (each range of levels reads the two levels
 // above and below it again and forms its top interface's fluxes a second time).
@@ -1257,6 +975,37 @@ int levels_per_block(long long tiles, int nz, long long target) {
   const long long parts = tiles >= target ? 1 : (target + tiles - 1) / tiles;
   const int n = (int)((nz + parts - 1) / parts);
   return n < 1 ? 1 : n;
+}
+
+void launch_tracers(bool mixed, hipStream_t s, Dims d, StepParams p, Geo geo, const double* T,
+                    const double* S, const double* b, const double* u, const double* v,
+                    const double* w, const double* Kh, double* cst, double* T_out,
+                    double* S_out, double* b_out) {
+  const int gx = (d.nx + TX - 1) / TX, gy = (d.ny + TY - 1) / TY;
+  const int parts = p.tracers_ts ? 2 : 1;
+  // 1024 workgroups, as many as are resident (4 per CU). Measured with 1024 / 2048 / 4096,
+  // both tracer kernels: 128 x 128 x 30 63 / 68 / 77 us, 256 x 256 x 30 112 / 119 / 129,
+  // 512 x 512 x 40 and 1000 x 1000 x 30 equal.
+  const int nk = levels_per_block((long long)parts * gx * gy, d.nz, 1024);
+  const unsigned grid = (unsigned)parts * gx * gy * ((d.nz + nk - 1) / nk);
+  const bool tvd = p.advection == ADV_UP3_TVD;
+  auto rhs = [&](auto kernel) {
+    kernel<<<grid, TILE_THREADS, 0, s>>>(d, p, geo, nk, T, S, b, u, v, w, Kh, T_out, S_out,
+                                         b_out);
+  };
+  auto solve = [&](auto kernel) {
+    const unsigned nb = (unsigned)((d.n2 + SOLVE_THREADS - 1) / SOLVE_THREADS);
+    kernel<<<nb, SOLVE_THREADS, 0, s>>>(d, p, geo, geo.zs, Kh, cst, T_out, S_out, b_out);
+  };
+  if (p.zcol) {
+    if (mixed) rhs(tvd ? k_tracer_rhs<float, true, true> : k_tracer_rhs<float, true, false>);
+    else rhs(tvd ? k_tracer_rhs<double, true, true> : k_tracer_rhs<double, true, false>);
+    solve(k_tracer_solve<true>);
+  } else {
+    if (mixed) rhs(k_tracer_rhs<float, false, false>);
+    else rhs(tvd ? k_tracer_rhs<double, false, true> : k_tracer_rhs<double, false, false>);
+    solve(k_tracer_solve<false>);
+  }
 }
 
 void launch_momentum_explicit_tiled(bool mixed, hipStream_t s, Dims d, StepParams p, Geo geo,
