@@ -769,6 +769,53 @@ double* vcycle_jacobi(hoc_stepper* h, int l, const double* b, double* x, double*
   return x;
 }
 
+// One V-cycle of the hierarchy with S sweeps per side in fused legs: one
+// launch down and one up per level above the first level of at most
+// MG_COARSE_MAX cells; from there to the last level the cycle runs in one
+// workgroup in LDS. rb: red-black Gauss-Seidel sweeps, else damped Jacobi.
+// b: level 0's right-hand side, x_in its starting field (null: zero; rb with
+// two sweeps only), out the result.
+int vcycle_fused(hoc_stepper* h, int S, bool rb, const double* b, const double* x_in, double* out,
+                 hipStream_t s) {
+  const int last = h->nlev - 1;
+  const double om = h->cfg.mg_omega;
+  auto level_b = [&](int l) -> const double* { return l == 0 ? b : h->mg_b[l]; };
+  const int l0 = h->mg_cycle_l0 >= 0 ? h->mg_cycle_l0 : last;
+  for (int l = 0; l < l0; ++l) {
+    if (rb)
+      launch_mg_down_rb(S, h->mg_tile_shape, s, h->lev[l], h->lev[l + 1],
+                        l == 0 ? x_in : nullptr, level_b(l), h->mg_x[l], h->mg_b[l + 1], h->sc);
+    else
+      launch_mg_down(S, h->mg_tile_shape, s, h->lev[l], h->lev[l + 1], om, level_b(l),
+                     h->mg_x[l], h->mg_b[l + 1], h->sc);
+  }
+  double* ec = l0 == 0 ? out : h->mg_x[l0];
+  if (h->mg_cycle_l0 >= 0) {
+    MgCycle C{};
+    C.nl = last - l0 + 1;
+    C.rb = rb ? 1 : 0;
+    for (int l = 0; l < C.nl; ++l) C.lev[l] = h->lev[l0 + l];
+    const size_t lds = mg_cycle_layout(C);
+    launch_mg_coarse_cycle(C, lds, om, S, level_b(l0), l0 == 0 ? x_in : nullptr, ec, h->sc, s);
+  } else if (rb) {
+    // the last level alone: S forward and S reverse sweeps from zero
+    k_mg_zero<<<blocks(h->lev[last].n), TPB, 0, s>>>(h->lev[last].n, ec, h->sc);
+    for (int k = 0; k < 2 * S; ++k) rbgs_sweep(h, last, level_b(last), ec, k >= S, s);
+  } else {
+    double* res = vcycle_jacobi(h, last, level_b(last), ec, h->mg_t[last], s);
+    if (res != ec) return fail(HOC_ERR_DEVICE, "pcg_mg: coarse result left its buffer");
+  }
+  for (int l = l0 - 1; l >= 0; --l) {
+    double* to = l == 0 ? out : h->mg_t[l];
+    if (rb)
+      launch_mg_up_rb(S, h->mg_tile_shape, s, h->lev[l], h->mg_x[l], ec, level_b(l), to, h->sc);
+    else
+      launch_mg_up(S, h->mg_tile_shape, s, h->lev[l], om, h->mg_x[l], ec, level_b(l), to, h->sc);
+    ec = to;
+  }
+  return HOC_OK;
+}
+
 // z = M^-1 r for pcg_rbgs (symmetric RBGS sweep pair from zero,
 // solvers_var.py:154-160) and pcg_mg.
 int precondition(hoc_stepper* h, const double* r, double* z, hipStream_t s) {
@@ -783,7 +830,7 @@ int precondition(hoc_stepper* h, const double* r, double* z, hipStream_t s) {
     const float om = (float)h->cfg.mg_omega;
     if (l0 < 0) return fail(HOC_ERR_DEVICE, "mixed pcg_mg: no one-workgroup coarse cycle");
     for (int l = 0; l < l0; ++l)
-      launch_mg_down_f32(S, mg_tile_grid(h->levf[l]), s, h->levf[l], h->levf[l + 1], om,
+      launch_mg_down_f32(S, h->mg_tile_shape, s, h->levf[l], h->levf[l + 1], om,
                          l == 0 ? r : nullptr, l == 0 ? nullptr : h->mgf_b[l], h->mgf_x[l],
                          h->mgf_b[l + 1], h->sc);
     {
@@ -797,54 +844,12 @@ int precondition(hoc_stepper* h, const double* r, double* z, hipStream_t s) {
     }
     const float* ec = h->mgf_x[l0];
     for (int l = l0 - 1; l >= 0; --l) {
-      launch_mg_up_f32(S, mg_tile_grid(h->levf[l]), s, h->levf[l], h->levf[l + 1].nx, om,
-                       h->mgf_x[l], ec, l == 0 ? r : nullptr, l == 0 ? nullptr : h->mgf_b[l],
+      launch_mg_up_f32(S, h->mg_tile_shape, s, h->levf[l], om, h->mgf_x[l], ec, l == 0 ? r : nullptr, l == 0 ? nullptr : h->mgf_b[l],
                        l == 0 ? z : nullptr, l == 0 ? nullptr : h->mgf_t[l], h->sc);
       ec = h->mgf_t[l];
     }
   } else if (h->cfg.mg_sweeps <= MG_FUSED_MAX_SWEEPS) {
-    // fused legs: one launch down and one up per level above the first level
-    // of at most MG_COARSE_MAX cells; from there to the last level the cycle
-    // runs in one workgroup in LDS
-    const int S = h->cfg.mg_sweeps, last = h->nlev - 1;
-    const double om = h->cfg.mg_omega;
-    const bool rb = h->cfg.mg_smoother == 1;
-    auto level_b = [&](int l) -> const double* { return l == 0 ? r : h->mg_b[l]; };
-    const int l0 = h->mg_cycle_l0 >= 0 ? h->mg_cycle_l0 : last;
-    for (int l = 0; l < l0; ++l) {
-      if (rb)
-        launch_mg_down_rb(S, h->mg_tile_shape, s, h->lev[l], h->lev[l + 1], level_b(l),
-                          h->mg_x[l], h->mg_b[l + 1], h->sc);
-      else
-        launch_mg_down(S, h->mg_tile_shape, s, h->lev[l], h->lev[l + 1], om, level_b(l),
-                       h->mg_x[l], h->mg_b[l + 1], h->sc);
-    }
-    double* ec = l0 == 0 ? z : h->mg_x[l0];
-    if (h->mg_cycle_l0 >= 0) {
-      MgCycle C{};
-      C.nl = last - l0 + 1;
-      C.rb = rb ? 1 : 0;
-      for (int l = 0; l < C.nl; ++l) C.lev[l] = h->lev[l0 + l];
-      const size_t lds = mg_cycle_layout(C);
-      launch_mg_coarse_cycle(C, lds, om, S, level_b(l0), ec, h->sc, s);
-    } else if (rb) {
-      // the last level alone: S forward and S reverse sweeps from zero
-      k_mg_zero<<<blocks(h->lev[last].n), TPB, 0, s>>>(h->lev[last].n, ec, h->sc);
-      for (int k = 0; k < 2 * S; ++k) rbgs_sweep(h, last, level_b(last), ec, k >= S, s);
-    } else {
-      double* out = vcycle_jacobi(h, last, level_b(last), ec, h->mg_t[last], s);
-      if (out != ec) return fail(HOC_ERR_DEVICE, "pcg_mg: coarse result left its buffer");
-    }
-    for (int l = l0 - 1; l >= 0; --l) {
-      double* out = l == 0 ? z : h->mg_t[l];
-      if (rb)
-        launch_mg_up_rb(S, h->mg_tile_shape, s, h->lev[l], h->lev[l + 1].nx, h->mg_x[l], ec,
-                        level_b(l), out, h->sc);
-      else
-        launch_mg_up(S, h->mg_tile_shape, s, h->lev[l], h->lev[l + 1].nx, om, h->mg_x[l], ec,
-                     level_b(l), out, h->sc);
-      ec = out;
-    }
+    TRY(vcycle_fused(h, h->cfg.mg_sweeps, h->cfg.mg_smoother == 1, r, nullptr, z, s));
   } else {
     // 2 * mg_sweeps buffer swaps per level: the result is back in z
     double* out = vcycle_jacobi(h, 0, r, z, h->mg_t[0], s);
@@ -965,8 +970,9 @@ int helmholtz_solve(hoc_stepper* h, const double* Ku, const double* Kv, const do
       int batch = std::max(1, std::min(h->last_iters, max_iter));
       while (true) {
         for (int b = 0; b < batch && it <= max_iter; ++b, ++it) {
-          if (kind == SOLVER_MULTIGRID) vcycle_rbgs(h, 0, x, h->r, s);
-          else rbgs_sweep(h, 0, h->r, x, false, s);
+          if (kind == SOLVER_RBGS) rbgs_sweep(h, 0, h->r, x, false, s);
+          else if (h->mg_cycle_l0 >= 0) TRY(vcycle_fused(h, 2, true, h->r, x, x, s));
+          else vcycle_rbgs(h, 0, x, h->r, s);
           k_mg_res_parts<<<np, PCG_WG, 0, s>>>(ar, h->lev[0], x);
           k_mg_check<<<1, PCG_WG, 0, s>>>(ar, it);
         }
@@ -1870,7 +1876,8 @@ int hoc_stepper_create(const hoc_config* cfg, const hoc_geometry* g, hoc_stepper
       ldy = ldy * 2.0;
     }
   }
-  if (cfg->solver == SOLVER_PCG_MG && cfg->mg_sweeps <= MG_FUSED_MAX_SWEEPS) {
+  if ((cfg->solver == SOLVER_PCG_MG && cfg->mg_sweeps <= MG_FUSED_MAX_SWEEPS) ||
+      cfg->solver == SOLVER_MULTIGRID) {
     int l0 = -1;
     for (int l = 0; l < h->nlev; ++l)
       if (h->lev[l].n <= MG_COARSE_MAX) {
@@ -1881,14 +1888,14 @@ int hoc_stepper_create(const hoc_config* cfg, const hoc_geometry* g, hoc_stepper
     if (l0 >= 0 && h->nlev - l0 <= MG_CYCLE_LEVELS) {
       MgCycle C{};
       C.nl = h->nlev - l0;
-      C.rb = cfg->mg_smoother == 1 ? 1 : 0;
+      C.rb = cfg->mg_smoother == 1 || cfg->solver == SOLVER_MULTIGRID ? 1 : 0;
       for (int l = 0; l < C.nl; ++l) C.lev[l] = h->lev[l0 + l];
-      if (mg_cycle_prepare(mg_cycle_layout(C)) == 0) h->mg_cycle_l0 = l0;
+      if (mg_cycle_prepare(C, mg_cycle_layout(C)) == 0) h->mg_cycle_l0 = l0;
       if (cfg->precision >= 1) {
         MgCycleF CF{};
         CF.nl = C.nl;
         for (int l = 0; l < CF.nl; ++l) CF.lev[l] = h->levf[l0 + l];
-        if (mg_cycle_prepare_f32(mg_cycle_layout(CF)) != 0) h->mg_cycle_l0 = -1;
+        if (mg_cycle_prepare_f32(CF, mg_cycle_layout(CF)) != 0) h->mg_cycle_l0 = -1;
       }
     }
     if (cfg->precision >= 1 && h->mg_cycle_l0 < 0)

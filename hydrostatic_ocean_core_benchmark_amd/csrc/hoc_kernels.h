@@ -426,12 +426,10 @@ __global__ void k_mg_check(PcgArgs a, int it);
 __global__ void k_mg_start(PcgArgs a);
 constexpr int MG_COARSE_MAX = 1024;      // cells of a level solved in one workgroup
 constexpr int MG_COARSE_LAST_MAX = 4096; // ... also when it is the hierarchy's last level
-constexpr int MG_COARSE_THREADS = 1024;
 constexpr int MG_FUSED_MAX_SWEEPS = 3;   // fused V-cycle legs for 1..3 sweeps per side
 // The coarse end of a V-cycle solved in one workgroup (levels of at most
-// MG_COARSE_MAX cells, all vectors in LDS). Measured at 512 x 512: taking
-// the 64 x 64 level into the workgroup as well (4096 cells) costs 28 us per
-// cycle against 19 us for its two tiled launches plus the 32 x 32 cycle.
+// MG_COARSE_MAX cells): with one level more the half-sweeps of its 4096 cells
+// on one compute unit cost more than its two tiled launches.
 // A last level of up to MG_COARSE_LAST_MAX cells (the 64 x 64 end of a
 // 5-level hierarchy on 1024 x 1024) is one workgroup's 2S sweeps instead of
 // 2S + 1 launches.
@@ -442,9 +440,9 @@ struct MgCycleT {
   MgLevelT<R> lev[MG_CYCLE_LEVELS];
   int boff[MG_CYCLE_LEVELS], xoff[MG_CYCLE_LEVELS];  // LDS offsets (elements) of b, x_S
   int nl;
-  int rb;  // 1: red-black Gauss-Seidel sweeps (a third work vector in LDS), 0: damped Jacobi
-  // 1: the levels' Ku, Kv, 1/diag (at coff, elements) and masks (at moff, bytes) are
-  // copied into LDS too, when they fit beside the vectors
+  int rb;  // 1: red-black Gauss-Seidel sweeps, 0: damped Jacobi
+  // 1: the Ku, Kv, 1/diag (at coff, elements) and masks (at moff, bytes) of the levels below
+  // the first are copied into LDS too, when they fit beside the vectors
   int stage;
   int coff[MG_CYCLE_LEVELS], moff[MG_CYCLE_LEVELS];
 };
@@ -452,21 +450,22 @@ using MgCycle = MgCycleT<double>;
 using MgCycleF = MgCycleT<float>;
 template <class R>
 size_t mg_cycle_layout(MgCycleT<R>& C);  // fills boff/xoff, returns the LDS bytes
-int mg_cycle_prepare(size_t lds);        // < 0 if the fp64 cycle does not fit one workgroup
-int mg_cycle_prepare_f32(size_t lds);    // the same for the fp32 cycles
+// < 0 if the cycle does not fit one workgroup
+int mg_cycle_prepare(const MgCycle& C, size_t lds);
+int mg_cycle_prepare_f32(const MgCycleF& C, size_t lds);
 void launch_mg_coarse_cycle(const MgCycle& C, size_t lds, double omega, int S, const double* b0,
-                            double* out, const PcgScalars* sc, hipStream_t s);
+                            const double* x0, double* out, const PcgScalars* sc, hipStream_t s);
 constexpr int MG_TILE_SHAPES = 4;  // fused-leg tile shapes (32x16, 64x8, 16x16, 64x16)
 // The pcg_mg V-cycle legs with red-black Gauss-Seidel smoothing (S = 1..3).
 void launch_mg_down_rb(int S, int shape, hipStream_t s, const MgLevel& L, const MgLevel& C,
-                       const double* b, double* xs_out, double* bc, const PcgScalars* sc);
-void launch_mg_up_rb(int S, int shape, hipStream_t s, const MgLevel& L, int cnx,
-                     const double* xs_in, const double* ec, const double* b, double* out,
-                     const PcgScalars* sc);
+                       const double* x_in, const double* b, double* xs_out, double* bc,
+                       const PcgScalars* sc);
+void launch_mg_up_rb(int S, int shape, hipStream_t s, const MgLevel& L, const double* xs_in,
+                     const double* ec, const double* b, double* out, const PcgScalars* sc);
 void launch_mg_down(int S, int shape, hipStream_t s, const MgLevel& L, const MgLevel& C,
                     double omega, const double* b, double* xs_out, double* bc,
                     const PcgScalars* sc);
-void launch_mg_up(int S, int shape, hipStream_t s, const MgLevel& L, int cnx, double omega,
+void launch_mg_up(int S, int shape, hipStream_t s, const MgLevel& L, double omega,
                   const double* xs_in, const double* ec, const double* b, double* out,
                   const PcgScalars* sc);
 // fp32 V-cycle of the mixed-precision preconditioner: level 0 reads the fp64
@@ -474,19 +473,14 @@ void launch_mg_up(int S, int shape, hipStream_t s, const MgLevel& L, int cnx, do
 void launch_mg_coarse_cycle_f32(const MgCycleF& C, size_t lds, float omega, int S,
                                 const double* b0_d, const float* b0_f, double* out_d,
                                 float* out_f, const PcgScalars* sc, hipStream_t s);
-void launch_mg_down_f32(int S, dim3 grid, hipStream_t s, const MgLevelF& L, const MgLevelF& C,
+void launch_mg_down_f32(int S, int shape, hipStream_t s, const MgLevelF& L, const MgLevelF& C,
                         float omega, const double* b_d, const float* b_f, float* xs_out,
                         float* bc, const PcgScalars* sc);
-void launch_mg_up_f32(int S, dim3 grid, hipStream_t s, const MgLevelF& L, int cnx, float omega,
+void launch_mg_up_f32(int S, int shape, hipStream_t s, const MgLevelF& L, float omega,
                       const float* xs_in, const float* ec, const double* b_d, const float* b_f,
                       double* out_d, float* out_f, const PcgScalars* sc);
 __global__ void k_mg_to_f32(long long n, const double* Ku, const double* Kv, const double* inv,
                             float* fKu, float* fKv, float* finv);
-constexpr int MG_TW = 32, MG_TH = 16, MG_THREADS = 256;  // fused-leg tile and workgroup
-template <class R>
-dim3 mg_tile_grid(const MgLevelT<R>& L) {
-  return dim3((unsigned)((L.nx + MG_TW - 1) / MG_TW), (unsigned)((L.ny + MG_TH - 1) / MG_TH));
-}
 __global__ void k_pcg_init(PcgArgs a);
 __global__ void k_pcg_init_z(PcgArgs a);
 __global__ void k_pcg_ap(PcgArgs a, int it);

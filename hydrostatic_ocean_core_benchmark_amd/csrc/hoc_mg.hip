@@ -5,6 +5,8 @@
 //   piecewise-constant prolongation. Elementwise only -- every kernel is one
 //   pass over a level -- and in the reference's operand order, so the
 //   iterates are bitwise those of the oracle.
+#include <type_traits>
+
 #include "hoc_device.h"
 #include "hoc_kernels.h"
 #include "hoc_reduce.h"
@@ -53,15 +55,6 @@ __device__ __forceinline__ R apply_vals(const MgLevelT<R>& L, long long c, long 
                        mkr<R>(L.mask[cn]), mkr<R>(L.mask[cs]), x0, x_e, x_w, x_n, x_s);
 }
 
-// Damped Jacobi at c: x + omega (inv_diag (b - A x)) mask.
-template <class R>
-__device__ __forceinline__ R jacobi_vals(const MgLevelT<R>& L, R omega, long long c, long long ce,
-                                         long long cw, long long cn, long long cs, R x0, R x_e,
-                                         R x_w, R x_n, R x_s, R b) {
-  const R ax = apply_vals<R>(L, c, ce, cw, cn, cs, x0, x_e, x_w, x_n, x_s);
-  return x0 + omega * (L.inv_diag[c] * (b - ax)) * mkr<R>(L.mask[c]);
-}
-
 // Red-black Gauss-Seidel update at c: inv_diag (b + neighbour_sum(x)), the
 // neighbours' values unmasked (solvers_var.py:55-69), in the operand order
 // of mg_neighbour_sum.
@@ -69,13 +62,6 @@ template <class R>
 __device__ __forceinline__ R rbgs_from(R inv, R b, R cx, R cy, R ku_c, R ku_w, R kv_c, R kv_s,
                                        R x_e, R x_w, R x_n, R x_s) {
   return inv * (b + (cx * (ku_c * x_e + ku_w * x_w) + cy * (kv_c * x_n + kv_s * x_s)));
-}
-
-template <class R>
-__device__ __forceinline__ R rbgs_vals(const MgLevelT<R>& L, long long c, long long cw,
-                                       long long cs, R b, R x_e, R x_w, R x_n, R x_s) {
-  return rbgs_from<R>(L.inv_diag[c], b, L.cx, L.cy, L.Ku[c], L.Ku[cw], L.Kv[c], L.Kv[cs], x_e,
-                      x_w, x_n, x_s);
 }
 
 struct Nbr {
@@ -403,495 +389,678 @@ __global__ __launch_bounds__(PCG_WG) void k_mg_start(PcgArgs a) {
   }
 }
 
-// ------------------------------------------------- fused pcg_mg V-cycle legs
+// x wrapped into [0, n) for x in [-H, n + TW + H).
+template <int H, int TW>
+__device__ __forceinline__ int tile_wrap(int x, int n) {
+  if (n >= TW + H) {  // one period either way (the same for every thread)
+    if (x < 0) x += n;
+    return x >= n ? x - n : x;
+  }
+  return mg_pmod(x, n);
+}
+
+// ------------------------------ fused pcg_mg V-cycle legs, damped Jacobi
 // The pcg_mg preconditioner with S damped-Jacobi sweeps per side, as LDS
-// tiles of MG_TW x MG_TH fine cells. Each sweep is evaluated on the tile
-// plus the halo the later steps still need (radius 1 per remaining sweep,
-// neighbours wrapping like the operator), so one launch replaces the
-// zero / S sweeps / residual-restrict launches of the way down and the
-// prolong / S sweeps launches of the way up, with the same arithmetic per
-// cell (apply_vals, jacobi_vals). R is the arithmetic and storage type of
-// the level's vectors; RB the type of the right-hand side read (double on
-// level 0 of the fp32 cycle, where it is the fp64 PCG residual), RO the
-// type of the way-up result (double on level 0 of the fp32 cycle).
+// tiles of TW x TH fine cells plus the halo the later steps still need
+// (radius 1 per remaining step, neighbours wrapping like the operator), so one
+// launch replaces the zero / S sweeps / residual-restrict launches of the way
+// down and the prolong / S sweeps launches of the way up, with the same
+// arithmetic per cell. A thread owns its cells (one; two for the largest tile)
+// for the whole leg, coefficients, right-hand side and value in registers, and
+// a sweep reads only the four neighbours' values from LDS; from zero the first
+// sweep reads none, so the way down needs no halo for it. R is the arithmetic
+// and storage type of the level's vectors; RB the type of the right-hand side
+// read (double on level 0 of the fp32 cycle, where it is the fp64 PCG
+// residual), RO the type of the way-up result (double on level 0 of the fp32
+// cycle).
+// Bound: latency, that of the loads before the first sweep and of one barrier,
+// four LDS reads and five dependent operations per sweep; with the region
+// walked in several rounds by 256 threads, coefficients re-read and divisions
+// by the spacings, a leg down and up took 5.5 and 4.5 us on average under
+// 128 x 128 and 6.0 and 5.6 us in fp32 under 640 x 512; so it is 3.7 and 3.7,
+// 3.7 and 3.6 us. A level can be smaller than a tile and its halo: positions
+// wrap round it as often as needed.
+// The cells of a TW x TH tile with a halo of H: Q per thread.
+template <int H, int TW, int TH>
+struct JacRegion {
+  static constexpr int RW = TW + 2 * H, RH = TH + 2 * H, RN = RW * RH;
+  static constexpr int Q = (RN + 1023) / 1024;
+  static constexpr int NT = ((RN + Q - 1) / Q + 63) / 64 * 64;
+};
+
+// One cell of a thread: its coefficients, right-hand side, 1/diag and mask,
+// the LDS positions of its neighbours and of itself, its index on the level
+// and its place in the tile. A cell's neighbours beyond the region are itself
+// (a value that no valid cell uses).
+template <class R>
+struct JacCell {
+  R inv, b, ke, kw, kn, ks, m;
+  int q, e, w, n, s, g, up, ti, tj;
+};
+
+template <class R, class RB, int H, int TW, int TH>
+__device__ __forceinline__ JacCell<R> jac_cell(const MgLevelT<R>& L, const RB* __restrict__ b,
+                                               int i0, int j0, int t) {
+  using Rg = JacRegion<H, TW, TH>;
+  const int lj = t / Rg::RW, li = t % Rg::RW;
+  const int ui = i0 - H + li, uj = j0 - H + lj;
+  const int i = tile_wrap<H, TW>(ui, L.nx), iw = tile_wrap<H + 1, TW>(ui - 1, L.nx);
+  const int j = tile_wrap<H, TH>(uj, L.ny), js = tile_wrap<H + 1, TH>(uj - 1, L.ny);
+  JacCell<R> K;
+  K.g = j * L.nx + i;
+  K.inv = L.inv_diag[K.g];
+  K.b = (R)b[K.g];
+  K.ke = L.Ku[K.g];
+  K.kw = L.Ku[j * L.nx + iw];
+  K.kn = L.Kv[K.g];
+  K.ks = L.Kv[js * L.nx + i];
+  K.m = mkr<R>(L.mask[K.g]);
+  K.q = t;
+  K.e = li + 1 < Rg::RW ? t + 1 : t;
+  K.w = li > 0 ? t - 1 : t;
+  K.n = lj + 1 < Rg::RH ? t + Rg::RW : t;
+  K.s = lj > 0 ? t - Rg::RW : t;
+  K.up = (j / 2) * (L.nx / 2) + i / 2;
+  K.ti = li - H;
+  K.tj = lj - H;
+  return K;
+}
+
+// A x at a cell in apply_from's order; the values are masked already, so its
+// multiplications by the masks are exact no-ops.
+template <class R>
+__device__ __forceinline__ R jac_apply(const JacCell<R>& K, R coef, const Divisor<R>& by_dx2,
+                                       const Divisor<R>& by_dy2, R xc, R xe, R xw, R xn, R xs) {
+  const R lap = by_dx2(K.ke * (xe - xc) - K.kw * (xc - xw)) +
+                by_dy2(K.kn * (xn - xc) - K.ks * (xc - xs));
+  return (xc - coef * lap) * K.m + xc * (R(1) - K.m);
+}
 
 // Way down on one level: x_S = S sweeps from zero (written out for the way
 // up) and bc = restrict((b - A x_S) mask).
-template <int S, class R, class RB, int TW = MG_TW, int TH = MG_TH>
-__global__ __launch_bounds__(MG_THREADS) void k_mg_down(MgLevelT<R> L, MgLevelT<R> C, R omega,
-                                                        const RB* __restrict__ b,
-                                                        R* __restrict__ xs_out,
-                                                        R* __restrict__ bc,
-                                                        const PcgScalars* sc) {
+template <int S, class R, class RB, int TW, int TH>
+__global__ __launch_bounds__((JacRegion<S, TW, TH>::NT)) void k_mg_down(
+    MgLevelT<R> L, MgLevelT<R> C, R omega, const RB* __restrict__ b, R* __restrict__ xs_out,
+    R* __restrict__ bc, const PcgScalars* sc) {
   if (finished(sc)) return;
-  constexpr int RW = TW + 2 * S, RH = TH + 2 * S;
-  __shared__ R buf[2][RH * RW];
+  constexpr int H = S;
+  using Rg = JacRegion<H, TW, TH>;
+  constexpr int Q = Rg::Q;
+  __shared__ R buf[2][Rg::RN];
   const int i0 = blockIdx.x * TW, j0 = blockIdx.y * TH;
+  const Divisor<R> by_dx2 = uniform_divisor<R>(L.dx2), by_dy2 = uniform_divisor<R>(L.dy2);
+  JacCell<R> K[Q];
+  R v[Q];
+  bool on[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int t = threadIdx.x + q * Rg::NT;
+    on[q] = t < Rg::RN;
+    K[q] = jac_cell<R, RB, H, TW, TH>(L, b, i0, j0, on[q] ? t : 0);
+    v[q] = R(0);
+  }
+#pragma unroll
   for (int k = 1; k <= S; ++k) {
-    const int h = S - k + 1;  // halo of x_k
-    const int w = TW + 2 * h, hh = TH + 2 * h;
-    R* dst = buf[(k - 1) & 1];
     const R* src = buf[k & 1];
-    for (int t = threadIdx.x; t < w * hh; t += MG_THREADS) {
-      const int li = S - h + t % w, lj = S - h + t / w;
-      const Nbr n = nbr_of(L, mg_pmod(i0 - S + li, L.nx), mg_pmod(j0 - S + lj, L.ny));
-      const int q = lj * RW + li;
-      const R bb = (R)b[n.c];
-      dst[q] = (k == 1)
-                   ? jacobi_vals<R>(L, omega, n.c, n.ce, n.cw, n.cn, n.cs, R(0), R(0), R(0), R(0),
-                                    R(0), bb)
-                   : jacobi_vals<R>(L, omega, n.c, n.ce, n.cw, n.cn, n.cs, src[q], src[q + 1],
-                                    src[q - 1], src[q + RW], src[q - RW], bb);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const R z = R(0);
+      const R ax = k == 1 ? jac_apply(K[q], L.coef, by_dx2, by_dy2, z, z, z, z, z)
+                          : jac_apply(K[q], L.coef, by_dx2, by_dy2, v[q], src[K[q].e],
+                                      src[K[q].w], src[K[q].n], src[K[q].s]);
+      v[q] = v[q] + omega * (K[q].inv * (K[q].b - ax)) * K[q].m;
+      if (on[q]) buf[(k - 1) & 1][K[q].q] = v[q];
     }
     __syncthreads();
   }
   const R* xs = buf[(S - 1) & 1];
-  for (int t = threadIdx.x; t < TW * TH; t += MG_THREADS) {
-    const int gi = i0 + t % TW, gj = j0 + t / TW;
-    if (gi < L.nx && gj < L.ny)
-      xs_out[(long long)gj * L.nx + gi] = xs[(S + t / TW) * RW + S + t % TW];
+  R* res = buf[S & 1];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    if (!on[q] || K[q].ti < 0 || K[q].ti >= TW || K[q].tj < 0 || K[q].tj >= TH) continue;
+    if (i0 + K[q].ti < L.nx && j0 + K[q].tj < L.ny) xs_out[K[q].g] = v[q];
+    const R ax = jac_apply(K[q], L.coef, by_dx2, by_dy2, v[q], xs[K[q].e], xs[K[q].w],
+                           xs[K[q].n], xs[K[q].s]);
+    res[K[q].q] = (K[q].b - ax) * K[q].m;
   }
+  __syncthreads();
   constexpr int CW = TW / 2, CH = TH / 2;
-  for (int t = threadIdx.x; t < CW * CH; t += MG_THREADS) {
-    const int I = i0 / 2 + t % CW, J = j0 / 2 + t / CW;
+  for (int u = threadIdx.x; u < CW * CH; u += Rg::NT) {
+    const int I = i0 / 2 + u % CW, J = j0 / 2 + u / CW;
     if (I >= C.nx || J >= C.ny) continue;
-    R r[4];
-    for (int qd = 0; qd < 4; ++qd) {  // [0::2,0::2], [0::2,1::2], [1::2,0::2], [1::2,1::2]
-      const int a = qd & 1, bq = qd >> 1;
-      const int gi = 2 * I + a, gj = 2 * J + bq;
-      const Nbr n = nbr_of(L, gi, gj);
-      const int q = (S + gj - j0) * RW + S + gi - i0;
-      const R ax = apply_vals<R>(L, n.c, n.ce, n.cw, n.cn, n.cs, xs[q], xs[q + 1], xs[q - 1],
-                                 xs[q + RW], xs[q - RW]);
-      r[qd] = ((R)b[n.c] - ax) * mkr<R>(L.mask[n.c]);
-    }
-    bc[(long long)J * C.nx + I] = R(0.25) * (r[0] + r[1] + r[2] + r[3]);
+    const int q = (H + 2 * (u / CW)) * Rg::RW + H + 2 * (u % CW);
+    bc[(long long)J * C.nx + I] =
+        R(0.25) * (res[q] + res[q + 1] + res[q + Rg::RW] + res[q + Rg::RW + 1]);
   }
 }
 
 // Way up on one level: x = x_S + prolong(ec) mask, then S sweeps; out = x.
-template <int S, class R, class RB, class RO, int TW = MG_TW, int TH = MG_TH>
-__global__ __launch_bounds__(MG_THREADS) void k_mg_up(MgLevelT<R> L, int cnx, R omega,
-                                                      const R* __restrict__ xs_in,
-                                                      const R* __restrict__ ec,
-                                                      const RB* __restrict__ b,
-                                                      RO* __restrict__ out,
-                                                      const PcgScalars* sc) {
+template <int S, class R, class RB, class RO, int TW, int TH>
+__global__ __launch_bounds__((JacRegion<S, TW, TH>::NT)) void k_mg_up(
+    MgLevelT<R> L, R omega, const R* __restrict__ xs_in, const R* __restrict__ ec,
+    const RB* __restrict__ b, RO* __restrict__ out, const PcgScalars* sc) {
   if (finished(sc)) return;
-  constexpr int RW = TW + 2 * S, RH = TH + 2 * S;
-  __shared__ R buf[2][RH * RW];
+  constexpr int H = S;
+  using Rg = JacRegion<H, TW, TH>;
+  constexpr int Q = Rg::Q;
+  __shared__ R buf[2][Rg::RN];
   const int i0 = blockIdx.x * TW, j0 = blockIdx.y * TH;
-  for (int t = threadIdx.x; t < RW * RH; t += MG_THREADS) {
-    const int gi = mg_pmod(i0 - S + t % RW, L.nx), gj = mg_pmod(j0 - S + t / RW, L.ny);
-    const long long c = (long long)gj * L.nx + gi;
-    buf[0][t] = xs_in[c] + ec[(long long)(gj / 2) * cnx + gi / 2] * mkr<R>(L.mask[c]);
+  const Divisor<R> by_dx2 = uniform_divisor<R>(L.dx2), by_dy2 = uniform_divisor<R>(L.dy2);
+  JacCell<R> K[Q];
+  R v[Q];
+  bool on[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int t = threadIdx.x + q * Rg::NT;
+    on[q] = t < Rg::RN;
+    K[q] = jac_cell<R, RB, H, TW, TH>(L, b, i0, j0, on[q] ? t : 0);
+    v[q] = xs_in[K[q].g] + ec[K[q].up] * K[q].m;
+    if (on[q]) buf[0][K[q].q] = v[q];
   }
   __syncthreads();
+#pragma unroll
   for (int k = 1; k <= S; ++k) {
-    const int h = S - k;
-    const int w = TW + 2 * h, hh = TH + 2 * h;
-    R* dst = buf[k & 1];
     const R* src = buf[(k - 1) & 1];
-    for (int t = threadIdx.x; t < w * hh; t += MG_THREADS) {
-      const int li = S - h + t % w, lj = S - h + t / w;
-      const Nbr n = nbr_of(L, mg_pmod(i0 - S + li, L.nx), mg_pmod(j0 - S + lj, L.ny));
-      const int q = lj * RW + li;
-      dst[q] = jacobi_vals<R>(L, omega, n.c, n.ce, n.cw, n.cn, n.cs, src[q], src[q + 1],
-                              src[q - 1], src[q + RW], src[q - RW], (R)b[n.c]);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const R ax = jac_apply(K[q], L.coef, by_dx2, by_dy2, v[q], src[K[q].e], src[K[q].w],
+                             src[K[q].n], src[K[q].s]);
+      v[q] = v[q] + omega * (K[q].inv * (K[q].b - ax)) * K[q].m;
+      if (k < S && on[q]) buf[k & 1][K[q].q] = v[q];
     }
-    __syncthreads();
+    if (k < S) __syncthreads();
   }
-  const R* x = buf[S & 1];
-  for (int t = threadIdx.x; t < TW * TH; t += MG_THREADS) {
-    const int gi = i0 + t % TW, gj = j0 + t / TW;
-    if (gi < L.nx && gj < L.ny)
-      out[(long long)gj * L.nx + gi] = (RO)x[(S + t / TW) * RW + S + t % TW];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    if (!on[q] || K[q].ti < 0 || K[q].ti >= TW || K[q].tj < 0 || K[q].tj >= TH) continue;
+    if (i0 + K[q].ti < L.nx && j0 + K[q].tj < L.ny) out[K[q].g] = (RO)v[q];
   }
 }
 
-// ---------------------------------------- fused legs, RBGS smoothing
-// The pcg_mg V-cycle with S red-black Gauss-Seidel sweeps per side (red then
-// black on the way down, black then red on the way up; the wet mask after
-// each sweep, as rbgs_sweep): each half-sweep updates one colour from the
-// values of the previous half-sweep, evaluated on the tile plus the halo the
-// later half-sweeps still need (radius 1 per remaining half-sweep), with the
-// two LDS buffers alternating per half-sweep. The level's coefficients and
-// right-hand side over the tile's region are staged in LDS once, so the
-// half-sweeps read no global memory. Each thread takes a pair of
-// neighbouring cells along x, one of each colour: one update per thread and
-// half-sweep, no lane idles on the other colour. These legs run on the
-// levels above the coarse cycle, which are all coarsened and so have even
-// sides: a cell's colour is then the parity of its unwrapped coordinates.
-
-// A tile region's copy of the level: face coefficients, 1/diag, right-hand
-// side, wet mask (0/1).
-template <int RN>
-struct RbStage {
-  double ku[RN], kv[RN], inv[RN], b[RN], m[RN];
+// ---------------------------------- fused V-cycle legs, red-black smoother
+// The legs of a V-cycle whose smoother is red-black Gauss-Seidel: S sweeps
+// red-black on the way down and S sweeps black-red on the way up, each
+// half-sweep evaluated on the tile plus the halo that the later ones still
+// need, so a leg is one launch with the arithmetic of k_mg_rbgs per cell.
+// These legs run on the levels above the coarse cycle, which are all
+// coarsened and so have even sides: a cell's colour is then the parity of its
+// unwrapped coordinates.
+//
+// Bound by the latency of one chain (launch, loads, 2S half-sweeps with a
+// barrier each, residual, stores), not by work. So one thread owns one pair
+// of neighbouring cells along x, one of each colour, for the whole leg: both
+// cells' coefficients, right-hand sides and values stay in its registers, and
+// a half-sweep reads only the updated cell's three other neighbours from LDS.
+// Against both colours walked in rounds by 256 threads, a leg down and up fell
+// from 5.1 and 4.9 us to 4.3 and 4.2 on average under 128 x 128 (16 x 16
+// tiles) and from 6.1 and 5.7 to 5.2 and 5.1 under 512 x 512. The stationary
+// multigrid's level-0 sweeps start from x_in with one more cell of halo; in
+// legs its cycle on 400 x 400 takes 4 launches fewer per level, and a solve
+// 0.55 instead of 1.28 ms.
+// One cell of a thread's pair: its coefficients towards the horizontal
+// neighbour outside the pair and to the north and south, its right-hand
+// side, 1/diag and mask, the LDS positions of those neighbours and of itself.
+struct RbCell {
+  double inv, b, kh, kn, ks, m;
+  int h, n, s, q;
 };
 
-// Stage the region of halo H around the tile at (i0, j0), positions wrapping
-// like the operator.
+// The pairs of a TW x TH tile with a halo of H cells: one thread each.
 template <int H, int TW, int TH>
-__device__ __forceinline__ void rb_stage(RbStage<(TW + 2 * H) * (TH + 2 * H)>& st,
-                                         const MgLevel& L, const double* __restrict__ b, int i0,
-                                         int j0) {
-  constexpr int RW = TW + 2 * H, RN = RW * (TH + 2 * H);
-  for (int t = threadIdx.x; t < RN; t += MG_THREADS) {
-    const int gi = mg_pmod(i0 - H + t % RW, L.nx), gj = mg_pmod(j0 - H + t / RW, L.ny);
-    const long long c = (long long)gj * L.nx + gi;
-    st.ku[t] = L.Ku[c];
-    st.kv[t] = L.Kv[c];
-    st.inv[t] = L.inv_diag[c];
-    st.b[t] = b[c];
-    st.m[t] = mkr<double>(L.mask[c]);
+struct RbRegion {
+  static constexpr int RW = TW + 2 * H, RH = TH + 2 * H, RN = RW * RH, PW = RW / 2;
+  static constexpr int PAIRS = PW * RH, NT = (PAIRS + 63) / 64 * 64;
+  static_assert(NT <= 1024, "one thread per pair");
+};
+
+// This thread's pair: [0] the red cell, [1] the black one; kp is the face
+// between them, g the cells' indices on the level, (gi, gj) the first cell's
+// unwrapped position.
+struct RbPair {
+  RbCell c[2];
+  double kp, x[2];
+  int g[2], up[2];  // indices on the level and, of the cell holding it, on the coarser one
+  int ti[2], tj;    // columns and row in the tile
+};
+
+template <int H, int TW, int TH>
+__device__ __forceinline__ RbPair rb_pair(const MgLevel& L, const double* __restrict__ b, int i0,
+                                          int j0, int t) {
+  using Rg = RbRegion<H, TW, TH>;
+  const int lj = t / Rg::PW, li = 2 * (t % Rg::PW);
+  const int ui = i0 - H + li, uj = j0 - H + lj;
+  const int ia = tile_wrap<H, TW>(ui, L.nx), ib = tile_wrap<H, TW>(ui + 1, L.nx);
+  const int iw = tile_wrap<H + 1, TW>(ui - 1, L.nx);
+  const int jj = tile_wrap<H, TH>(uj, L.ny), js = tile_wrap<H + 1, TH>(uj - 1, L.ny);
+  const int row = jj * L.nx, rs = js * L.nx;
+  const int ga = row + ia, gb = row + ib;
+  const int q = lj * Rg::RW + li;
+  const int qn = lj + 1 < Rg::RH ? Rg::RW : 0, qs = lj > 0 ? Rg::RW : 0;
+  RbCell A, B;
+  A.inv = L.inv_diag[ga];
+  B.inv = L.inv_diag[gb];
+  A.b = b[ga];
+  B.b = b[gb];
+  A.kh = L.Ku[row + iw];
+  B.kh = L.Ku[gb];
+  A.kn = L.Kv[ga];
+  B.kn = L.Kv[gb];
+  A.ks = L.Kv[rs + ia];
+  B.ks = L.Kv[rs + ib];
+  A.m = mkr<double>(L.mask[ga]);
+  B.m = mkr<double>(L.mask[gb]);
+  RbPair P;
+  P.kp = L.Ku[ga];
+  A.q = q;
+  A.h = li > 0 ? q - 1 : q;  // beyond the region: a value that no valid cell uses
+  A.n = q + qn;
+  A.s = q - qs;
+  B.q = q + 1;
+  B.h = li + 2 < Rg::RW ? q + 2 : q + 1;
+  B.n = q + 1 + qn;
+  B.s = q + 1 - qs;
+  const bool black_first = ((ui + uj) & 1) != 0;
+  P.c[0] = black_first ? B : A;
+  P.c[1] = black_first ? A : B;
+  P.g[0] = black_first ? gb : ga;
+  P.g[1] = black_first ? ga : gb;
+  const int ur = (jj / 2) * (L.nx / 2);
+  P.up[0] = ur + (black_first ? ib : ia) / 2;
+  P.up[1] = ur + (black_first ? ia : ib) / 2;
+  P.ti[0] = li - H + (black_first ? 1 : 0);
+  P.ti[1] = li - H + (black_first ? 0 : 1);
+  P.tj = lj - H;
+  P.x[0] = P.x[1] = 0.0;
+  return P;
+}
+
+// One half-sweep of colour `col` from the neighbours in src; the wet mask
+// over both cells after the sweep's second colour (mask_all).
+__device__ __forceinline__ void rb_update(RbPair& P, double cx, double cy, int col, bool mask_all,
+                                          const double* src) {
+  const RbCell& c = P.c[col];
+  P.x[col] = rbgs_from<double>(c.inv, c.b, cx, cy, P.kp, c.kh, c.kn, c.ks, P.x[1 - col],
+                               src[c.h], src[c.n], src[c.s]);
+  if (mask_all) {
+    P.x[0] = P.x[0] * P.c[0].m;
+    P.x[1] = P.x[1] * P.c[1].m;
   }
 }
 
-// One half-sweep of colour `colour` on the region of halo h, src -> dst; the
-// wet mask applied after the sweep's second colour (mask_all).
-template <int H, int TW, int TH>
-__device__ __forceinline__ void rb_half_sweep(const RbStage<(TW + 2 * H) * (TH + 2 * H)>& st,
-                                              double cx, double cy, int i0, int j0, int h,
-                                              int colour, bool mask_all, const double* src,
-                                              double* dst) {
-  constexpr int RW = TW + 2 * H;
-  const int w2 = (TW + 2 * h) / 2, hh = TH + 2 * h;
-  for (int t = threadIdx.x; t < w2 * hh; t += MG_THREADS) {
-    const int lj = H - h + t / w2;
-    const int li0 = H - h + 2 * (t % w2);
-    const int a = ((i0 + li0 + j0 + lj) & 1) == colour ? 0 : 1;  // the pair's cell of this colour
-    const int q = lj * RW + li0 + a, qo = lj * RW + li0 + 1 - a;
-    const double v = rbgs_from<double>(st.inv[q], st.b[q], cx, cy, st.ku[q], st.ku[q - 1],
-                                       st.kv[q], st.kv[q - RW], src[q + 1], src[q - 1],
-                                       src[q + RW], src[q - RW]);
-    const double vo = src[qo];
-    dst[q] = mask_all ? v * st.m[q] : v;
-    dst[qo] = mask_all ? vo * st.m[qo] : vo;
-  }
+__device__ __forceinline__ void rb_put(const RbPair& P, double* dst) {
+  dst[P.c[0].q] = P.x[0];
+  dst[P.c[1].q] = P.x[1];
 }
 
-// Way down: x_S = S sweeps from zero (written out for the way up) and
-// bc = restrict((b - A x_S) mask).
-template <int S, int TW = MG_TW, int TH = MG_TH>
-__global__ __launch_bounds__(MG_THREADS) void k_mg_down_rb(MgLevel L, MgLevel C,
-                                                           const double* __restrict__ b,
-                                                           double* __restrict__ xs_out,
-                                                           double* __restrict__ bc,
-                                                           const PcgScalars* sc) {
+// Way down: x_S = S sweeps (from zero, or from x_in with FROM_X: level 0 of
+// the stationary multigrid) written out for the way up, and
+// bc = restrict((b - A x_S) mask). From zero the first half-sweep reads no
+// neighbour, so the halo is one cell narrower.
+template <int S, bool FROM_X, int TW, int TH>
+__global__ __launch_bounds__((RbRegion<2 * S + (FROM_X ? 1 : 0), TW, TH>::NT)) void k_mg_down_rb(
+    MgLevel L, MgLevel C, const double* __restrict__ x_in, const double* __restrict__ b,
+    double* __restrict__ xs_out, double* __restrict__ bc, const PcgScalars* sc) {
   if (finished(sc)) return;
-  constexpr int H = 2 * S + 1;  // 2S half-sweeps, then the residual's stencil
-  constexpr int RW = TW + 2 * H, RN = RW * (TH + 2 * H);
-  __shared__ RbStage<RN> st;
-  __shared__ double buf[2][RN];
+  constexpr int H = 2 * S + (FROM_X ? 1 : 0);
+  using Rg = RbRegion<H, TW, TH>;
+  __shared__ double buf[2][Rg::RN];
   const int i0 = blockIdx.x * TW, j0 = blockIdx.y * TH;
-  rb_stage<H, TW, TH>(st, L, b, i0, j0);
-  for (int t = threadIdx.x; t < RN; t += MG_THREADS) buf[0][t] = 0.0;
+  const int t = threadIdx.x;
+  const bool on = t < Rg::PAIRS;
+  RbPair P = rb_pair<H, TW, TH>(L, b, i0, j0, on ? t : 0);
+  if (FROM_X) {
+    P.x[0] = x_in[P.g[0]];
+    P.x[1] = x_in[P.g[1]];
+    if (on) rb_put(P, buf[0]);
+    __syncthreads();
+    rb_update(P, L.cx, L.cy, 0, false, buf[0]);
+  } else {
+    const RbCell& c = P.c[0];
+    P.x[0] = rbgs_from<double>(c.inv, c.b, L.cx, L.cy, P.kp, c.kh, c.kn, c.ks, 0.0, 0.0, 0.0,
+                               0.0);
+  }
+  if (on) rb_put(P, buf[1]);
   __syncthreads();
-  for (int ph = 1; ph <= 2 * S; ++ph) {  // red first
-    rb_half_sweep<H, TW, TH>(st, L.cx, L.cy, i0, j0, H - ph, (ph - 1) & 1, (ph & 1) == 0,
-                             buf[(ph - 1) & 1], buf[ph & 1]);
+#pragma unroll
+  for (int ph = 2; ph <= 2 * S; ++ph) {  // red first
+    rb_update(P, L.cx, L.cy, (ph - 1) & 1, (ph & 1) == 0, buf[(ph - 1) & 1]);
+    if (on) rb_put(P, buf[ph & 1]);
     __syncthreads();
   }
   const double* xs = buf[0];  // 2S half-sweeps end in buf[0]
-  for (int t = threadIdx.x; t < TW * TH; t += MG_THREADS) {
-    const int gi = i0 + t % TW, gj = j0 + t / TW;
-    if (gi < L.nx && gj < L.ny)
-      xs_out[(long long)gj * L.nx + gi] = xs[(H + t / TW) * RW + H + t % TW];
-  }
-  constexpr int CW = TW / 2, CH = TH / 2;
-  for (int t = threadIdx.x; t < CW * CH; t += MG_THREADS) {
-    const int I = i0 / 2 + t % CW, J = j0 / 2 + t / CW;
-    if (I >= C.nx || J >= C.ny) continue;
-    double r[4];
-    for (int qd = 0; qd < 4; ++qd) {  // [0::2,0::2], [0::2,1::2], [1::2,0::2], [1::2,1::2]
-      const int gi = 2 * I + (qd & 1), gj = 2 * J + (qd >> 1);
-      const int q = (H + gj - j0) * RW + H + gi - i0;
-      const double ax = apply_from<double>(
-          L.coef, L.dx2, L.dy2, st.ku[q], st.ku[q - 1], st.kv[q], st.kv[q - RW], st.m[q],
-          st.m[q + 1], st.m[q - 1], st.m[q + RW], st.m[q - RW], xs[q], xs[q + 1], xs[q - 1],
-          xs[q + RW], xs[q - RW]);
-      r[qd] = (st.b[q] - ax) * st.m[q];
+  double* res = buf[1];
+  const Divisor<double> by_dx2 = uniform_divisor<double>(L.dx2),
+                        by_dy2 = uniform_divisor<double>(L.dy2);
+  if (on) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const RbCell& c = P.c[k];
+      if (P.ti[k] < 0 || P.ti[k] >= TW || P.tj < 0 || P.tj >= TH) continue;
+      if (i0 + P.ti[k] < L.nx && j0 + P.tj < L.ny) xs_out[P.g[k]] = P.x[k];
+      // the residual in apply_from's order; the values are masked already
+      // (x m m = x m for a 0/1 mask). The pair's cell to the east is the
+      // other one for the western cell, and the sums of two commute.
+      const double xc = P.x[k], xp = P.x[1 - k], xh = xs[c.h], xn = xs[c.n], xsv = xs[c.s];
+      const bool west = P.ti[k] < P.ti[1 - k];
+      const double fe = west ? P.kp * (xp - xc) : c.kh * (xh - xc);
+      const double fw = west ? c.kh * (xc - xh) : P.kp * (xc - xp);
+      const double fn = c.kn * (xn - xc), fs = c.ks * (xc - xsv);
+      const double lap = by_dx2(fe - fw) + by_dy2(fn - fs);
+      const double ax = (xc - L.coef * lap) * c.m + xc * (1.0 - c.m);
+      res[c.q] = (c.b - ax) * c.m;
     }
-    bc[(long long)J * C.nx + I] = 0.25 * (r[0] + r[1] + r[2] + r[3]);
+  }
+  __syncthreads();
+  constexpr int CW = TW / 2, CH = TH / 2;
+  for (int u = t; u < CW * CH; u += Rg::NT) {
+    const int I = i0 / 2 + u % CW, J = j0 / 2 + u / CW;
+    if (I >= C.nx || J >= C.ny) continue;
+    const int q = (H + 2 * (u / CW)) * Rg::RW + H + 2 * (u % CW);
+    bc[(long long)J * C.nx + I] =
+        0.25 * (res[q] + res[q + 1] + res[q + Rg::RW] + res[q + Rg::RW + 1]);
   }
 }
 
 // Way up: x = x_S + prolong(ec) mask, then S reversed sweeps; out = x.
-template <int S, int TW = MG_TW, int TH = MG_TH>
-__global__ __launch_bounds__(MG_THREADS) void k_mg_up_rb(MgLevel L, int cnx,
-                                                         const double* __restrict__ xs_in,
-                                                         const double* __restrict__ ec,
-                                                         const double* __restrict__ b,
-                                                         double* __restrict__ out,
-                                                         const PcgScalars* sc) {
+template <int S, int TW, int TH>
+__global__ __launch_bounds__((RbRegion<2 * S, TW, TH>::NT)) void k_mg_up_rb(
+    MgLevel L, const double* __restrict__ xs_in, const double* __restrict__ ec,
+    const double* __restrict__ b, double* __restrict__ out, const PcgScalars* sc) {
   if (finished(sc)) return;
   constexpr int H = 2 * S;
-  constexpr int RW = TW + 2 * H, RN = RW * (TH + 2 * H);
-  __shared__ RbStage<RN> st;
-  __shared__ double buf[2][RN];
+  using Rg = RbRegion<H, TW, TH>;
+  __shared__ double buf[2][Rg::RN];
   const int i0 = blockIdx.x * TW, j0 = blockIdx.y * TH;
-  rb_stage<H, TW, TH>(st, L, b, i0, j0);
-  for (int t = threadIdx.x; t < RN; t += MG_THREADS) {  // st.m[t] was written by this thread
-    const int gi = mg_pmod(i0 - H + t % RW, L.nx), gj = mg_pmod(j0 - H + t / RW, L.ny);
-    const long long c = (long long)gj * L.nx + gi;
-    buf[0][t] = xs_in[c] + ec[(long long)(gj / 2) * cnx + gi / 2] * st.m[t];
+  const int t = threadIdx.x;
+  const bool on = t < Rg::PAIRS;
+  RbPair P = rb_pair<H, TW, TH>(L, b, i0, j0, on ? t : 0);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) P.x[k] = xs_in[P.g[k]] + ec[P.up[k]] * P.c[k].m;
+  if (on) rb_put(P, buf[0]);
+  __syncthreads();
+#pragma unroll
+  for (int ph = 1; ph <= 2 * S; ++ph) {  // black first
+    rb_update(P, L.cx, L.cy, ph & 1, (ph & 1) == 0, buf[(ph - 1) & 1]);
+    if (ph == 2 * S) break;
+    if (on) rb_put(P, buf[ph & 1]);
+    __syncthreads();
+  }
+  if (!on) return;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    if (P.ti[k] < 0 || P.ti[k] >= TW || P.tj < 0 || P.tj >= TH) continue;
+    if (i0 + P.ti[k] < L.nx && j0 + P.tj < L.ny) out[P.g[k]] = P.x[k];
+  }
+}
+
+// The coarse end of the pcg_mg V-cycle (and of the stationary multigrid's) in
+// one workgroup: levels C.lev[0..nl) (the first with at most MG_COARSE_MAX
+// cells, or the last level alone), S sweeps from zero + residual restriction
+// down, 2S sweeps from zero on the last level (the second S reversed),
+// prolongation + S sweeps up; the same arithmetic per cell as the tiled legs.
+// With C.rb the sweeps are red-black Gauss-Seidel, reversed (black first) on
+// the way up and in the last level's second S. b0 is level 0's right-hand
+// side, out receives its result; x0, when given, is level 0's starting field
+// (the stationary multigrid on a grid small enough to need no legs).
+//
+// Bound by latency: a chain of about 10 half-sweeps per level, each a round of
+// LDS reads, five dependent fp64 operations and a barrier. So a thread owns
+// its cells for a whole visit of a level, their coefficients, right-hand sides
+// and values in registers (level 0's for the whole cycle), and a half-sweep
+// reads only the four neighbours' values from LDS; the levels below the first
+// have at most one cell per thread. Sweeps are out of place between two
+// buffers, because a level with an odd periodic side has same-colour
+// neighbours across the wrap, whose old values the reference reads.
+// The three levels from 32 x 32 down: 11.2 us against 14.9 with every field
+// in LDS and 1024 threads (rbgs), 10.4 against 14.7 (Jacobi).
+template <class R>
+struct CycCell {
+  R inv, b, ke, kw, kn, ks, m;
+  int c, ce, cw, cn, cs;
+  int up;  // the coarser level's cell that holds this one
+  int par;
+  bool on;
+};
+
+// Neighbours and colour of cell c of level L (n cells; off when c >= n).
+template <class R>
+__device__ __forceinline__ CycCell<R> cyc_index(const MgLevelT<R>& L, int c) {
+  CycCell<R> K;
+  K.on = c < (int)L.n;
+  K.c = K.on ? c : 0;
+  const int j = K.c / L.nx, i = K.c - j * L.nx;
+  K.ce = j * L.nx + wrap(i, 1, L.nx);
+  K.cw = j * L.nx + wrap(i, -1, L.nx);
+  K.cn = wrap(j, 1, L.ny) * L.nx + i;
+  K.cs = wrap(j, -1, L.ny) * L.nx + i;
+  K.up = (j / 2) * (L.nx / 2) + i / 2;
+  K.par = (i + j) & 1;
+  return K;
+}
+template <class R>
+__device__ __forceinline__ void cyc_coefficients(CycCell<R>& K, const R* ku, const R* kv,
+                                                 const R* inv, const uint8_t* m) {
+  K.inv = inv[K.c];
+  K.ke = ku[K.c];
+  K.kw = ku[K.cw];
+  K.kn = kv[K.c];
+  K.ks = kv[K.cs];
+  K.m = mkr<R>(m[K.c]);
+}
+
+// A x at a cell from its own value and its neighbours' (all masked already,
+// so apply_from's multiplications by the masks are exact no-ops).
+template <class R>
+__device__ __forceinline__ R cyc_apply(const CycCell<R>& K, R coef, const Divisor<R>& by_dx2,
+                                       const Divisor<R>& by_dy2, R xc, R xe, R xw, R xn, R xs) {
+  const R lap = by_dx2(K.ke * (xe - xc) - K.kw * (xc - xw)) +
+                by_dy2(K.kn * (xn - xc) - K.ks * (xc - xs));
+  return (xc - coef * lap) * K.m + xc * (R(1) - K.m);
+}
+
+// The two field buffers of the cycle; `cur` holds the last field written.
+template <class R>
+struct CycField {
+  R *cur, *next;
+  __device__ __forceinline__ void swap() {
+    R* t = cur;
+    cur = next;
+    next = t;
+  }
+};
+
+// S sweeps on the cells of one level, from f.cur (or from zero), the own
+// values in v; the result in v and in f.cur.
+template <class R, int Q>
+__device__ __forceinline__ void cyc_sweeps(const MgLevelT<R>& L, CycCell<R>* K, R* v,
+                                           CycField<R>& f, R omega, bool rb, int S, bool zero,
+                                           bool reverse) {
+  // all cells' loads, then all updates, then all stores: a thread's cells
+  // overlap, and a cell that is off or of the other colour computes a value
+  // that is not kept
+  R xe[Q], xw[Q], xn[Q], xs[Q];
+  auto neighbours = [&](bool z) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      xe[q] = z ? R(0) : f.cur[K[q].ce];
+      xw[q] = z ? R(0) : f.cur[K[q].cw];
+      xn[q] = z ? R(0) : f.cur[K[q].cn];
+      xs[q] = z ? R(0) : f.cur[K[q].cs];
+    }
+  };
+  auto put = [&] {
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      if (K[q].on) f.next[K[q].c] = v[q];
+    __syncthreads();
+    f.swap();
+  };
+  if (rb) {
+    auto half = [&](int col, bool last, bool z) {
+      neighbours(z);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const R u = rbgs_from<R>(K[q].inv, K[q].b, L.cx, L.cy, K[q].ke, K[q].kw, K[q].kn,
+                                 K[q].ks, xe[q], xw[q], xn[q], xs[q]);
+        v[q] = K[q].par == col ? u : v[q];
+        if (last) v[q] = v[q] * K[q].m;
+      }
+      put();
+    };
+    const int first = reverse ? 1 : 0;
+    for (int s = 0; s < S; ++s) {
+      half(first, false, zero && s == 0);
+      half(1 - first, true, false);
+    }
+  } else {
+    const Divisor<R> by_dx2 = uniform_divisor<R>(L.dx2), by_dy2 = uniform_divisor<R>(L.dy2);
+    for (int s = 0; s < S; ++s) {
+      neighbours(zero && s == 0);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const R ax = cyc_apply(K[q], L.coef, by_dx2, by_dy2, v[q], xe[q], xw[q], xn[q], xs[q]);
+        v[q] = v[q] + omega * (K[q].inv * (K[q].b - ax)) * K[q].m;
+      }
+      put();
+    }
+  }
+}
+
+// The masked residual of the level's field (f.cur, own values v) into res.
+template <class R, int Q>
+__device__ __forceinline__ void cyc_residual(const MgLevelT<R>& L, const CycCell<R>* K,
+                                             const R* v, const CycField<R>& f, R* res) {
+  const Divisor<R> by_dx2 = uniform_divisor<R>(L.dx2), by_dy2 = uniform_divisor<R>(L.dy2);
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    if (!K[q].on) continue;
+    const R ax = cyc_apply(K[q], L.coef, by_dx2, by_dy2, v[q], f.cur[K[q].ce], f.cur[K[q].cw],
+                           f.cur[K[q].cn], f.cur[K[q].cs]);
+    res[K[q].c] = (K[q].b - ax) * K[q].m;
   }
   __syncthreads();
-  for (int ph = 1; ph <= 2 * S; ++ph) {  // black first
-    rb_half_sweep<H, TW, TH>(st, L.cx, L.cy, i0, j0, H - ph, ph & 1, (ph & 1) == 0,
-                             buf[(ph - 1) & 1], buf[ph & 1]);
-    __syncthreads();
-  }
-  const double* x = buf[0];
-  for (int t = threadIdx.x; t < TW * TH; t += MG_THREADS) {
-    const int gi = i0 + t % TW, gj = j0 + t / TW;
-    if (gi < L.nx && gj < L.ny) out[(long long)gj * L.nx + gi] = x[(H + t / TW) * RW + H + t % TW];
-  }
 }
 
-// The coarse end of the pcg_mg V-cycle in one workgroup, every vector in
-// LDS: levels C.lev[0..nl) (the first with at most MG_COARSE_MAX cells, or
-// the last level alone), S sweeps from zero + residual restriction down, 2S
-// sweeps from zero on the last level, prolongation + S sweeps up; the same
-// arithmetic per cell as the tiled legs (jacobi_vals or rbgs_vals,
-// apply_vals, from their operands). With C.rb the sweeps are red-black
-// Gauss-Seidel, reversed (black first) on the way up and in the last level's
-// second S. b0 is level 0's right-hand side (staged in LDS), out receives
-// level 0's result.
-
-// One level's operands inside the cycle: its coefficients from their LDS
-// copies (STAGED) or from the level's arrays, never a mix, so that the
-// compiler addresses the copies as LDS.
-template <class R, bool STAGED>
-struct CycLevel {
-  int nx, ny, n;
-  R coef, cx, cy, dx2, dy2;
-  const R *ku, *kv, *inv;
-  const uint8_t* m;
-};
-
-// One cell of a level with its neighbours and colour (the parity of i + j).
-struct CycCell {
-  int c, ce, cw, cn, cs, par;
-};
-
-template <class R, bool STAGED>
-__device__ __forceinline__ CycCell cyc_cell(const CycLevel<R, STAGED>& L, int c) {
-  const int i = c % L.nx, j = c / L.nx;
-  return CycCell{c, j * L.nx + wrap(i, 1, L.nx), j * L.nx + wrap(i, -1, L.nx),
-                 wrap(j, 1, L.ny) * L.nx + i, wrap(j, -1, L.ny) * L.nx + i, (i + j) & 1};
-}
-
-template <class R, bool STAGED>
-__device__ __forceinline__ R cyc_apply(const CycLevel<R, STAGED>& L, int c, int ce, int cw,
-                                       int cn, int cs, R x0, R x_e, R x_w, R x_n, R x_s) {
-  return apply_from<R>(L.coef, L.dx2, L.dy2, L.ku[c], L.ku[cw], L.kv[c], L.kv[cs],
-                       mkr<R>(L.m[c]), mkr<R>(L.m[ce]), mkr<R>(L.m[cw]), mkr<R>(L.m[cn]),
-                       mkr<R>(L.m[cs]), x0, x_e, x_w, x_n, x_s);
-}
-
-template <class R, class RB, class RO, bool STAGED>
-__device__ __forceinline__ void coarse_cycle(const MgCycleT<R>& C, R omega, int S,
-                                             const RB* __restrict__ b0, RO* __restrict__ out,
-                                             unsigned char* cyc_raw) {
-  R* cyc = reinterpret_cast<R*>(cyc_raw);
-  const int n0 = (int)C.lev[0].n;
-  const int tid = threadIdx.x;
-  auto lev = [&](int l) {
-    const MgLevelT<R>& G = C.lev[l];
-    CycLevel<R, STAGED> L;
-    L.nx = G.nx;
-    L.ny = G.ny;
-    L.n = (int)G.n;
-    L.coef = G.coef;
-    L.cx = G.cx;
-    L.cy = G.cy;
-    L.dx2 = G.dx2;
-    L.dy2 = G.dy2;
-    if (STAGED) {
-      L.ku = cyc + C.coff[l];
-      L.kv = cyc + C.coff[l] + L.n;
-      L.inv = cyc + C.coff[l] + 2 * L.n;
-      L.m = cyc_raw + C.moff[l];
-    } else {
-      L.ku = G.Ku;
-      L.kv = G.Kv;
-      L.inv = G.inv_diag;
-      L.m = G.mask;
-    }
-    return L;
-  };
-  R* wA = cyc;
-  R* wB = cyc + n0;
-  R* wC = cyc + 2 * n0;  // red-black sweeps only: the field between the two colours
-  // one sweep on level L from src (zero when `zero`) into dst: damped
-  // Jacobi, or red-black Gauss-Seidel (red first unless reverse) through wC.
-  // K0 is the thread's first cell (tid), formed once per visit of the
-  // level; the others (levels of more than MG_COARSE_THREADS cells) are
-  // formed as they come.
-  auto for_cells = [&](const CycLevel<R, STAGED>& L, const CycCell& K0, auto&& f) {
-    if (tid < L.n) f(K0);
-    for (int c = tid + MG_COARSE_THREADS; c < L.n; c += MG_COARSE_THREADS) f(cyc_cell(L, c));
-  };
-  auto sweep = [&](const CycLevel<R, STAGED>& L, const CycCell& K0, const R* b, const R* src,
-                   bool zero, R* dst, bool reverse) {
-    if (!C.rb) {
-      for_cells(L, K0, [&](const CycCell& K) {
-        const int c = K.c;
-        const R x0 = zero ? R(0) : src[c], xe = zero ? R(0) : src[K.ce];
-        const R xw = zero ? R(0) : src[K.cw], xn = zero ? R(0) : src[K.cn];
-        const R xs = zero ? R(0) : src[K.cs];
-        const R ax = cyc_apply(L, c, K.ce, K.cw, K.cn, K.cs, x0, xe, xw, xn, xs);
-        dst[c] = x0 + omega * (L.inv[c] * (b[c] - ax)) * mkr<R>(L.m[c]);
-      });
-      __syncthreads();
-      return;
-    }
-    const int first = reverse ? 1 : 0;
-    for_cells(L, K0, [&](const CycCell& K) {
-      const int c = K.c;
-      R v = zero ? R(0) : src[c];
-      if (K.par == first) {
-        const R xe = zero ? R(0) : src[K.ce], xw = zero ? R(0) : src[K.cw];
-        const R xn = zero ? R(0) : src[K.cn], xs = zero ? R(0) : src[K.cs];
-        v = rbgs_from<R>(L.inv[c], b[c], L.cx, L.cy, L.ku[c], L.ku[K.cw], L.kv[c], L.kv[K.cs],
-                         xe, xw, xn, xs);
-      }
-      wC[c] = v;
-    });
-    __syncthreads();
-    for_cells(L, K0, [&](const CycCell& K) {
-      const int c = K.c;
-      R v = wC[c];
-      if (K.par != first)
-        v = rbgs_from<R>(L.inv[c], b[c], L.cx, L.cy, L.ku[c], L.ku[K.cw], L.kv[c], L.kv[K.cs],
-                         wC[K.ce], wC[K.cw], wC[K.cn], wC[K.cs]);
-      dst[c] = v * mkr<R>(L.m[c]);
-    });
-    __syncthreads();
-  };
-  // level 0's right-hand side, staged (the restriction of the levels below
-  // overwrites nothing of it), and the levels' coefficients when staged
-  {
-    R* st = cyc + C.boff[0];
-    for (int c = tid; c < n0; c += MG_COARSE_THREADS) st[c] = (R)b0[c];
-    if (STAGED) {
-      for (int l = 0; l < C.nl; ++l) {
-        const MgLevelT<R>& G = C.lev[l];
-        const int n = (int)G.n;
-        R* k = cyc + C.coff[l];
-        unsigned char* m = cyc_raw + C.moff[l];
-        for (int c = tid; c < n; c += MG_COARSE_THREADS) {
-          k[c] = G.Ku[c];
-          k[n + c] = G.Kv[c];
-          k[2 * n + c] = G.inv_diag[c];
-          m[c] = G.mask[c];
-        }
-      }
-    }
-    __syncthreads();
-  }
-  auto level_b = [&](int l) -> const R* { return cyc + C.boff[l]; };
-  // down: x_S into XS[l], restricted residual into B[l + 1]
-  for (int l = 0; l + 1 < C.nl; ++l) {
-    const CycLevel<R, STAGED> L = lev(l);
-    const CycCell K0 = cyc_cell(L, tid);
-    const R* b = level_b(l);
-    R* xs = cyc + C.xoff[l];
-    const R* src = wA;
-    for (int k = 1; k <= S; ++k) {
-      R* dst = (k == S) ? xs : ((k & 1) ? wA : wB);
-      sweep(L, K0, b, src, k == 1, dst, false);
-      src = dst;
-    }
-    const MgLevelT<R>& Cl = C.lev[l + 1];  // sizes only
-    R* bc = cyc + C.boff[l + 1];
-    const int nc = (int)Cl.n;
-    for (int t = tid; t < nc; t += MG_COARSE_THREADS) {
-      const int I = t % Cl.nx, J = t / Cl.nx;
-      R r[4];
-      for (int qd = 0; qd < 4; ++qd) {  // [0::2,0::2], [0::2,1::2], [1::2,0::2], [1::2,1::2]
-        const int gi = 2 * I + (qd & 1), gj = 2 * J + (qd >> 1);
-        const int c = gj * L.nx + gi;
-        const int ce = gj * L.nx + wrap(gi, 1, L.nx), cw = gj * L.nx + wrap(gi, -1, L.nx);
-        const int cn = wrap(gj, 1, L.ny) * L.nx + gi, cs = wrap(gj, -1, L.ny) * L.nx + gi;
-        const R ax = cyc_apply(L, c, ce, cw, cn, cs, xs[c], xs[ce], xs[cw], xs[cn], xs[cs]);
-        r[qd] = (b[c] - ax) * mkr<R>(L.m[c]);
-      }
-      bc[t] = R(0.25) * (r[0] + r[1] + r[2] + r[3]);
-    }
-    __syncthreads();
-  }
-  // the last level: 2S sweeps from zero (the second S reversed)
-  R* e = wA;
-  {
-    const int l = C.nl - 1;
-    const CycLevel<R, STAGED> L = lev(l);
-    const CycCell K0 = cyc_cell(L, tid);
-    const R* b = level_b(l);
-    const R* src = wB;
-    for (int k = 1; k <= 2 * S; ++k) {
-      R* dst = (k & 1) ? wA : wB;
-      sweep(L, K0, b, src, k == 1, dst, k > S);
-      src = dst;
-      e = dst;
-    }
-  }
-  // up: x = XS[l] + prolong(e) mask, then S sweeps
-  for (int l = C.nl - 2; l >= 0; --l) {
-    const CycLevel<R, STAGED> L = lev(l);
-    const CycCell K0 = cyc_cell(L, tid);
-    const R* b = level_b(l);
-    const R* xs = cyc + C.xoff[l];
-    const int cnx = C.lev[l + 1].nx;
-    R* xp = (e == wA) ? wB : wA;
-    R* other = (e == wA) ? wA : wB;
-    for (int c = tid; c < L.n; c += MG_COARSE_THREADS) {
-      const int i = c % L.nx, j = c / L.nx;
-      xp[c] = xs[c] + e[(j / 2) * cnx + i / 2] * mkr<R>(L.m[c]);
-    }
-    __syncthreads();
-    const R* src = xp;
-    for (int k = 1; k <= S; ++k) {
-      R* dst = (k & 1) ? other : xp;
-      sweep(L, K0, b, src, false, dst, true);
-      src = dst;
-      e = dst;
-    }
-  }
-  for (int c = tid; c < n0; c += MG_COARSE_THREADS) out[c] = (RO)e[c];
-}
-
-template <class R, class RB, class RO>
-__global__ __launch_bounds__(MG_COARSE_THREADS) void k_mg_coarse_cycle(
-    MgCycleT<R> C, R omega, int S, const RB* __restrict__ b0, RO* __restrict__ out,
-    const PcgScalars* sc) {
+template <class R, class RB, class RO, int NT, int Q>
+__global__ __launch_bounds__(NT) void k_mg_coarse_cycle(MgCycleT<R> C, R omega, int S,
+                                                        const RB* __restrict__ b0,
+                                                        const R* x0, RO* out,
+                                                        const PcgScalars* sc) {
   if (finished(sc)) return;
   extern __shared__ __align__(16) unsigned char cyc_raw[];
+  R* cyc = reinterpret_cast<R*>(cyc_raw);
+  const int tid = threadIdx.x;
+  const int n0 = (int)C.lev[0].n;
+  const bool rb = C.rb != 0;
+  CycField<R> f{cyc, cyc + n0};
+  R* res = cyc + 2 * n0;
+  // level 0's cells, for the whole cycle; the levels below copied into LDS
+  // when they fit
+  CycCell<R> K0[Q];
+  R v0[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    K0[q] = cyc_index(C.lev[0], tid + q * NT);
+    cyc_coefficients(K0[q], C.lev[0].Ku, C.lev[0].Kv, C.lev[0].inv_diag, C.lev[0].mask);
+    K0[q].b = (R)b0[K0[q].c];
+    v0[q] = x0 ? x0[K0[q].c] : R(0);
+  }
   if (C.stage)
-    coarse_cycle<R, RB, RO, true>(C, omega, S, b0, out, cyc_raw);
-  else
-    coarse_cycle<R, RB, RO, false>(C, omega, S, b0, out, cyc_raw);
+    for (int l = 1; l < C.nl; ++l) {
+      const MgLevelT<R>& G = C.lev[l];
+      const int n = (int)G.n;
+      if (tid < n) {
+        R* k = cyc + C.coff[l];
+        k[tid] = G.Ku[tid];
+        k[n + tid] = G.Kv[tid];
+        k[2 * n + tid] = G.inv_diag[tid];
+        cyc_raw[C.moff[l] + tid] = G.mask[tid];
+      }
+    }
+  if (x0) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      if (K0[q].on) f.cur[K0[q].c] = v0[q];
+  }
+  __syncthreads();
+  auto level = [&](int l) {  // this thread's cell of a level below the first
+    const MgLevelT<R>& G = C.lev[l];
+    CycCell<R> K = cyc_index(G, tid);
+    if (C.stage) {
+      const R* k = cyc + C.coff[l];
+      cyc_coefficients(K, k, k + (int)G.n, k + 2 * (int)G.n, cyc_raw + C.moff[l]);
+    } else {
+      cyc_coefficients(K, G.Ku, G.Kv, G.inv_diag, G.mask);
+    }
+    return K;
+  };
+  const int last = C.nl - 1;
+  cyc_sweeps<R, Q>(C.lev[0], K0, v0, f, omega, rb, S, x0 == nullptr, false);
+  if (last == 0) {
+    cyc_sweeps<R, Q>(C.lev[0], K0, v0, f, omega, rb, S, false, true);
+  } else {
+    cyc_residual<R, Q>(C.lev[0], K0, v0, f, res);
+    for (int l = 1; l <= last; ++l) {
+      CycCell<R> K = level(l);
+      // the restricted residual of the level above (its cells by rows)
+      const int fnx = C.lev[l - 1].nx;
+      const int j = K.c / C.lev[l].nx, i = K.c - j * C.lev[l].nx;
+      const int q = 2 * j * fnx + 2 * i;
+      K.b = R(0.25) * (res[q] + res[q + 1] + res[q + fnx] + res[q + fnx + 1]);
+      R v = R(0);
+      cyc_sweeps<R, 1>(C.lev[l], &K, &v, f, omega, rb, S, true, false);
+      if (l == last) {
+        cyc_sweeps<R, 1>(C.lev[l], &K, &v, f, omega, rb, S, false, true);
+      } else {
+        if (K.on) {
+          cyc[C.boff[l] + K.c] = K.b;
+          cyc[C.xoff[l] + K.c] = v;
+        }
+        cyc_residual<R, 1>(C.lev[l], &K, &v, f, res);
+      }
+    }
+    for (int l = last - 1; l >= 1; --l) {
+      CycCell<R> K = level(l);
+      K.b = cyc[C.boff[l] + K.c];
+      R v = cyc[C.xoff[l] + K.c] + f.cur[K.up] * K.m;
+      if (K.on) f.next[K.c] = v;
+      __syncthreads();
+      f.swap();
+      cyc_sweeps<R, 1>(C.lev[l], &K, &v, f, omega, rb, S, false, true);
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      if (!K0[q].on) continue;
+      v0[q] = v0[q] + f.cur[K0[q].up] * K0[q].m;
+      f.next[K0[q].c] = v0[q];
+    }
+    __syncthreads();
+    f.swap();
+    cyc_sweeps<R, Q>(C.lev[0], K0, v0, f, omega, rb, S, false, true);
+  }
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (K0[q].on) out[K0[q].c] = (RO)v0[q];
 }
 
+// LDS of a cycle: two field buffers and the residual, the lower levels'
+// right-hand sides and x_S, and their coefficients when they fit.
 template <class R>
 size_t mg_cycle_layout(MgCycleT<R>& C) {
-  const int n0 = (int)C.lev[0].n;
-  int off = (C.rb ? 3 : 2) * n0;
-  for (int l = 0; l < C.nl; ++l) {
+  int off = 3 * (int)C.lev[0].n;
+  for (int l = 1; l < C.nl; ++l) {
     C.boff[l] = off;
     off += (int)C.lev[l].n;
     C.xoff[l] = off;
     off += (int)C.lev[l].n;
   }
   const size_t vectors = (size_t)off * sizeof(R);
-  for (int l = 0; l < C.nl; ++l) {
+  for (int l = 1; l < C.nl; ++l) {
     C.coff[l] = off;
     off += 3 * (int)C.lev[l].n;
   }
   size_t bytes = (size_t)off * sizeof(R);
-  for (int l = 0; l < C.nl; ++l) {
+  for (int l = 1; l < C.nl; ++l) {
     C.moff[l] = (int)bytes;
     bytes += (size_t)C.lev[l].n;
   }
@@ -903,171 +1072,163 @@ template size_t mg_cycle_layout<double>(MgCycle&);
 template size_t mg_cycle_layout<float>(MgCycleF&);
 
 namespace {
-int set_cycle_lds(const void* fn, size_t lds) {
-  if (lds > MG_CYCLE_LDS) return -1;
-  return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) ==
-                 hipSuccess
+// Threads and cells per thread by the first level's cells: 256 x 4 up to 1024
+// cells (one wave per SIMD: the barriers of 16 waves cost more than their
+// parallelism gives), 1024 x 2 and 1024 x 4 beyond (a last level alone).
+template <class R, class RB, class RO>
+const void* cycle_kernel(long long n0) {
+  if (n0 <= 1024) return (const void*)k_mg_coarse_cycle<R, RB, RO, 256, 4>;
+  if (n0 <= 2048) return (const void*)k_mg_coarse_cycle<R, RB, RO, 1024, 2>;
+  return (const void*)k_mg_coarse_cycle<R, RB, RO, 1024, 4>;
+}
+template <class R, class RB, class RO>
+int cycle_lds(long long n0, size_t lds) {
+  if (lds > MG_CYCLE_LDS || n0 > MG_COARSE_LAST_MAX) return -1;
+  return hipFuncSetAttribute(cycle_kernel<R, RB, RO>(n0),
+                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)lds) == hipSuccess
              ? 0
              : -2;
 }
+template <class R, class RB, class RO>
+void launch_cycle(const MgCycleT<R>& C, size_t lds, R omega, int S, const RB* b0, const R* x0,
+                  RO* out, const PcgScalars* sc, hipStream_t s) {
+  const long long n0 = C.lev[0].n;
+  if (n0 <= 1024)
+    k_mg_coarse_cycle<R, RB, RO, 256, 4><<<1, 256, lds, s>>>(C, omega, S, b0, x0, out, sc);
+  else if (n0 <= 2048)
+    k_mg_coarse_cycle<R, RB, RO, 1024, 2><<<1, 1024, lds, s>>>(C, omega, S, b0, x0, out, sc);
+  else
+    k_mg_coarse_cycle<R, RB, RO, 1024, 4><<<1, 1024, lds, s>>>(C, omega, S, b0, x0, out, sc);
+}
 }  // namespace
 
-int mg_cycle_prepare(size_t lds) {
-  return set_cycle_lds((const void*)k_mg_coarse_cycle<double, double, double>, lds);
+int mg_cycle_prepare(const MgCycle& C, size_t lds) {
+  return cycle_lds<double, double, double>(C.lev[0].n, lds);
 }
 
-int mg_cycle_prepare_f32(size_t lds) {
-  int rc = set_cycle_lds((const void*)k_mg_coarse_cycle<float, double, double>, lds);
-  return rc ? rc : set_cycle_lds((const void*)k_mg_coarse_cycle<float, float, float>, lds);
+int mg_cycle_prepare_f32(const MgCycleF& C, size_t lds) {
+  const int rc = cycle_lds<float, double, double>(C.lev[0].n, lds);
+  return rc ? rc : cycle_lds<float, float, float>(C.lev[0].n, lds);
 }
 
 void launch_mg_coarse_cycle(const MgCycle& C, size_t lds, double omega, int S, const double* b0,
-                            double* out, const PcgScalars* sc, hipStream_t s) {
-  k_mg_coarse_cycle<double, double, double>
-      <<<1, MG_COARSE_THREADS, lds, s>>>(C, omega, S, b0, out, sc);
+                            const double* x0, double* out, const PcgScalars* sc, hipStream_t s) {
+  launch_cycle<double, double, double>(C, lds, omega, S, b0, x0, out, sc, s);
 }
 
 void launch_mg_coarse_cycle_f32(const MgCycleF& C, size_t lds, float omega, int S,
                                 const double* b0_d, const float* b0_f, double* out_d,
                                 float* out_f, const PcgScalars* sc, hipStream_t s) {
   if (b0_d)
-    k_mg_coarse_cycle<float, double, double>
-        <<<1, MG_COARSE_THREADS, lds, s>>>(C, omega, S, b0_d, out_d, sc);
+    launch_cycle<float, double, double>(C, lds, omega, S, b0_d, nullptr, out_d, sc, s);
   else
-    k_mg_coarse_cycle<float, float, float>
-        <<<1, MG_COARSE_THREADS, lds, s>>>(C, omega, S, b0_f, out_f, sc);
+    launch_cycle<float, float, float>(C, lds, omega, S, b0_f, nullptr, out_f, sc, s);
 }
 
 // Fused-leg tile shapes (cells per workgroup tile; every shape gives the
 // same values, they differ only in halo recomputation and occupancy):
 // 0: 32 x 16, 1: 64 x 8, 2: 16 x 16, 3: 64 x 16. Shapes 1-3 are built for
 // 2 sweeps per side (the default), other sweep counts use shape 0.
-dim3 mg_tile_grid_shape(const MgLevel& L, int shape) {
-  static const int tw[MG_TILE_SHAPES] = {32, 64, 16, 64}, th[MG_TILE_SHAPES] = {16, 8, 16, 16};
-  const int q = (shape >= 0 && shape < MG_TILE_SHAPES) ? shape : 0;
-  return dim3((unsigned)((L.nx + tw[q] - 1) / tw[q]), (unsigned)((L.ny + th[q] - 1) / th[q]));
+constexpr int SHAPE_W[MG_TILE_SHAPES] = {32, 64, 16, 64}, SHAPE_H[MG_TILE_SHAPES] = {16, 8, 16, 16};
+template <class R>
+dim3 mg_tile_grid_shape(const MgLevelT<R>& L, int shape) {
+  return dim3((unsigned)((L.nx + SHAPE_W[shape] - 1) / SHAPE_W[shape]),
+              (unsigned)((L.ny + SHAPE_H[shape] - 1) / SHAPE_H[shape]));
 }
+
+namespace {
+// One leg kernel per sweep count and tile shape.
+template <class Go>
+void leg_dispatch(int S, int shape, const Go& go) {
+  if (S == 1) go(std::integral_constant<int, 1>{}, std::integral_constant<int, 0>{});
+  else if (S == 3) go(std::integral_constant<int, 3>{}, std::integral_constant<int, 0>{});
+  else if (shape == 1) go(std::integral_constant<int, 2>{}, std::integral_constant<int, 1>{});
+  else if (shape == 2) go(std::integral_constant<int, 2>{}, std::integral_constant<int, 2>{});
+  else if (shape == 3) go(std::integral_constant<int, 2>{}, std::integral_constant<int, 3>{});
+  else go(std::integral_constant<int, 2>{}, std::integral_constant<int, 0>{});
+}
+int leg_shape(int S, int shape) { return S == 2 && shape >= 0 && shape < MG_TILE_SHAPES ? shape : 0; }
+
+template <class R, class RB>
+void leg_down(int S, int shape, hipStream_t s, const MgLevelT<R>& L, const MgLevelT<R>& C, R omega,
+              const RB* b, R* xs_out, R* bc, const PcgScalars* sc) {
+  shape = leg_shape(S, shape);
+  const dim3 grid = mg_tile_grid_shape(L, shape);
+  leg_dispatch(S, shape, [&](auto sv, auto qv) {
+    constexpr int SS = decltype(sv)::value, W = SHAPE_W[decltype(qv)::value],
+                  T = SHAPE_H[decltype(qv)::value];
+    k_mg_down<SS, R, RB, W, T><<<grid, JacRegion<SS, W, T>::NT, 0, s>>>(L, C, omega, b, xs_out, bc,
+                                                                       sc);
+  });
+}
+template <class R, class RB, class RO>
+void leg_up(int S, int shape, hipStream_t s, const MgLevelT<R>& L, R omega, const R* xs_in,
+            const R* ec, const RB* b, RO* out, const PcgScalars* sc) {
+  shape = leg_shape(S, shape);
+  const dim3 grid = mg_tile_grid_shape(L, shape);
+  leg_dispatch(S, shape, [&](auto sv, auto qv) {
+    constexpr int SS = decltype(sv)::value, W = SHAPE_W[decltype(qv)::value],
+                  T = SHAPE_H[decltype(qv)::value];
+    k_mg_up<SS, R, RB, RO, W, T><<<grid, JacRegion<SS, W, T>::NT, 0, s>>>(L, omega, xs_in, ec, b,
+                                                                         out, sc);
+  });
+}
+}  // namespace
 
 void launch_mg_down(int S, int shape, hipStream_t s, const MgLevel& L, const MgLevel& C,
                     double omega, const double* b, double* xs_out, double* bc,
                     const PcgScalars* sc) {
-  if (S != 2) shape = 0;
-  const dim3 grid = mg_tile_grid_shape(L, shape);
-  if (S == 1)
-    k_mg_down<1, double, double><<<grid, MG_THREADS, 0, s>>>(L, C, omega, b, xs_out, bc, sc);
-  else if (S == 3)
-    k_mg_down<3, double, double><<<grid, MG_THREADS, 0, s>>>(L, C, omega, b, xs_out, bc, sc);
-  else if (shape == 1)
-    k_mg_down<2, double, double, 64, 8><<<grid, MG_THREADS, 0, s>>>(L, C, omega, b, xs_out, bc, sc);
-  else if (shape == 2)
-    k_mg_down<2, double, double, 16, 16><<<grid, MG_THREADS, 0, s>>>(L, C, omega, b, xs_out, bc,
-                                                                    sc);
-  else if (shape == 3)
-    k_mg_down<2, double, double, 64, 16><<<grid, MG_THREADS, 0, s>>>(L, C, omega, b, xs_out, bc,
-                                                                    sc);
-  else
-    k_mg_down<2, double, double><<<grid, MG_THREADS, 0, s>>>(L, C, omega, b, xs_out, bc, sc);
+  leg_down<double, double>(S, shape, s, L, C, omega, b, xs_out, bc, sc);
 }
-
-void launch_mg_up(int S, int shape, hipStream_t s, const MgLevel& L, int cnx, double omega,
+void launch_mg_up(int S, int shape, hipStream_t s, const MgLevel& L, double omega,
                   const double* xs_in, const double* ec, const double* b, double* out,
                   const PcgScalars* sc) {
-  if (S != 2) shape = 0;
-  const dim3 grid = mg_tile_grid_shape(L, shape);
-  if (S == 1)
-    k_mg_up<1, double, double, double><<<grid, MG_THREADS, 0, s>>>(L, cnx, omega, xs_in, ec, b,
-                                                                   out, sc);
-  else if (S == 3)
-    k_mg_up<3, double, double, double><<<grid, MG_THREADS, 0, s>>>(L, cnx, omega, xs_in, ec, b,
-                                                                   out, sc);
-  else if (shape == 1)
-    k_mg_up<2, double, double, double, 64, 8><<<grid, MG_THREADS, 0, s>>>(L, cnx, omega, xs_in, ec,
-                                                                          b, out, sc);
-  else if (shape == 2)
-    k_mg_up<2, double, double, double, 16, 16><<<grid, MG_THREADS, 0, s>>>(L, cnx, omega, xs_in,
-                                                                           ec, b, out, sc);
-  else if (shape == 3)
-    k_mg_up<2, double, double, double, 64, 16><<<grid, MG_THREADS, 0, s>>>(L, cnx, omega, xs_in,
-                                                                           ec, b, out, sc);
-  else
-    k_mg_up<2, double, double, double><<<grid, MG_THREADS, 0, s>>>(L, cnx, omega, xs_in, ec, b,
-                                                                   out, sc);
+  leg_up<double, double, double>(S, shape, s, L, omega, xs_in, ec, b, out, sc);
 }
-
-void launch_mg_down_rb(int S, int shape, hipStream_t s, const MgLevel& L, const MgLevel& C,
-                       const double* b, double* xs_out, double* bc, const PcgScalars* sc) {
-  if (S != 2) shape = 0;
-  const dim3 grid = mg_tile_grid_shape(L, shape);
-  if (S == 1)
-    k_mg_down_rb<1><<<grid, MG_THREADS, 0, s>>>(L, C, b, xs_out, bc, sc);
-  else if (S == 3)
-    k_mg_down_rb<3><<<grid, MG_THREADS, 0, s>>>(L, C, b, xs_out, bc, sc);
-  else if (shape == 1)
-    k_mg_down_rb<2, 64, 8><<<grid, MG_THREADS, 0, s>>>(L, C, b, xs_out, bc, sc);
-  else if (shape == 2)
-    k_mg_down_rb<2, 16, 16><<<grid, MG_THREADS, 0, s>>>(L, C, b, xs_out, bc, sc);
-  else if (shape == 3)
-    k_mg_down_rb<2, 64, 16><<<grid, MG_THREADS, 0, s>>>(L, C, b, xs_out, bc, sc);
-  else
-    k_mg_down_rb<2><<<grid, MG_THREADS, 0, s>>>(L, C, b, xs_out, bc, sc);
-}
-
-void launch_mg_up_rb(int S, int shape, hipStream_t s, const MgLevel& L, int cnx,
-                     const double* xs_in, const double* ec, const double* b, double* out,
-                     const PcgScalars* sc) {
-  if (S != 2) shape = 0;
-  const dim3 grid = mg_tile_grid_shape(L, shape);
-  if (S == 1)
-    k_mg_up_rb<1><<<grid, MG_THREADS, 0, s>>>(L, cnx, xs_in, ec, b, out, sc);
-  else if (S == 3)
-    k_mg_up_rb<3><<<grid, MG_THREADS, 0, s>>>(L, cnx, xs_in, ec, b, out, sc);
-  else if (shape == 1)
-    k_mg_up_rb<2, 64, 8><<<grid, MG_THREADS, 0, s>>>(L, cnx, xs_in, ec, b, out, sc);
-  else if (shape == 2)
-    k_mg_up_rb<2, 16, 16><<<grid, MG_THREADS, 0, s>>>(L, cnx, xs_in, ec, b, out, sc);
-  else if (shape == 3)
-    k_mg_up_rb<2, 64, 16><<<grid, MG_THREADS, 0, s>>>(L, cnx, xs_in, ec, b, out, sc);
-  else
-    k_mg_up_rb<2><<<grid, MG_THREADS, 0, s>>>(L, cnx, xs_in, ec, b, out, sc);
-}
-
-namespace {
-template <int S>
-void down_f32(dim3 grid, hipStream_t s, const MgLevelF& L, const MgLevelF& C, float omega,
-              const double* b_d, const float* b_f, float* xs_out, float* bc,
-              const PcgScalars* sc) {
-  if (b_d)
-    k_mg_down<S, float, double><<<grid, MG_THREADS, 0, s>>>(L, C, omega, b_d, xs_out, bc, sc);
-  else
-    k_mg_down<S, float, float><<<grid, MG_THREADS, 0, s>>>(L, C, omega, b_f, xs_out, bc, sc);
-}
-template <int S>
-void up_f32(dim3 grid, hipStream_t s, const MgLevelF& L, int cnx, float omega, const float* xs_in,
-            const float* ec, const double* b_d, const float* b_f, double* out_d, float* out_f,
-            const PcgScalars* sc) {
-  if (b_d)
-    k_mg_up<S, float, double, double><<<grid, MG_THREADS, 0, s>>>(L, cnx, omega, xs_in, ec, b_d,
-                                                                  out_d, sc);
-  else
-    k_mg_up<S, float, float, float><<<grid, MG_THREADS, 0, s>>>(L, cnx, omega, xs_in, ec, b_f,
-                                                                out_f, sc);
-}
-}  // namespace
-
-void launch_mg_down_f32(int S, dim3 grid, hipStream_t s, const MgLevelF& L, const MgLevelF& C,
+void launch_mg_down_f32(int S, int shape, hipStream_t s, const MgLevelF& L, const MgLevelF& C,
                         float omega, const double* b_d, const float* b_f, float* xs_out,
                         float* bc, const PcgScalars* sc) {
-  if (S == 1) down_f32<1>(grid, s, L, C, omega, b_d, b_f, xs_out, bc, sc);
-  else if (S == 2) down_f32<2>(grid, s, L, C, omega, b_d, b_f, xs_out, bc, sc);
-  else down_f32<3>(grid, s, L, C, omega, b_d, b_f, xs_out, bc, sc);
+  if (b_d) leg_down<float, double>(S, shape, s, L, C, omega, b_d, xs_out, bc, sc);
+  else leg_down<float, float>(S, shape, s, L, C, omega, b_f, xs_out, bc, sc);
 }
-
-void launch_mg_up_f32(int S, dim3 grid, hipStream_t s, const MgLevelF& L, int cnx, float omega,
+void launch_mg_up_f32(int S, int shape, hipStream_t s, const MgLevelF& L, float omega,
                       const float* xs_in, const float* ec, const double* b_d, const float* b_f,
                       double* out_d, float* out_f, const PcgScalars* sc) {
-  if (S == 1) up_f32<1>(grid, s, L, cnx, omega, xs_in, ec, b_d, b_f, out_d, out_f, sc);
-  else if (S == 2) up_f32<2>(grid, s, L, cnx, omega, xs_in, ec, b_d, b_f, out_d, out_f, sc);
-  else up_f32<3>(grid, s, L, cnx, omega, xs_in, ec, b_d, b_f, out_d, out_f, sc);
+  if (b_d) leg_up<float, double, double>(S, shape, s, L, omega, xs_in, ec, b_d, out_d, sc);
+  else leg_up<float, float, float>(S, shape, s, L, omega, xs_in, ec, b_f, out_f, sc);
+}
+
+// x_in: the level's starting field (null: zero; 2 sweeps only otherwise).
+void launch_mg_down_rb(int S, int shape, hipStream_t s, const MgLevel& L, const MgLevel& C,
+                       const double* x_in, const double* b, double* xs_out, double* bc,
+                       const PcgScalars* sc) {
+  shape = leg_shape(S, shape);
+  const dim3 grid = mg_tile_grid_shape(L, shape);
+  leg_dispatch(S, shape, [&](auto sv, auto qv) {
+    constexpr int SS = decltype(sv)::value, W = SHAPE_W[decltype(qv)::value],
+                  T = SHAPE_H[decltype(qv)::value];
+    if constexpr (SS == 2) {
+      if (x_in) {
+        k_mg_down_rb<SS, true, W, T><<<grid, RbRegion<2 * SS + 1, W, T>::NT, 0, s>>>(
+            L, C, x_in, b, xs_out, bc, sc);
+        return;
+      }
+    }
+    k_mg_down_rb<SS, false, W, T><<<grid, RbRegion<2 * SS, W, T>::NT, 0, s>>>(
+        L, C, nullptr, b, xs_out, bc, sc);
+  });
+}
+
+void launch_mg_up_rb(int S, int shape, hipStream_t s, const MgLevel& L, const double* xs_in,
+                     const double* ec, const double* b, double* out, const PcgScalars* sc) {
+  shape = leg_shape(S, shape);
+  const dim3 grid = mg_tile_grid_shape(L, shape);
+  leg_dispatch(S, shape, [&](auto sv, auto qv) {
+    constexpr int SS = decltype(sv)::value, W = SHAPE_W[decltype(qv)::value],
+                  T = SHAPE_H[decltype(qv)::value];
+    k_mg_up_rb<SS, W, T><<<grid, RbRegion<2 * SS, W, T>::NT, 0, s>>>(L, xs_in, ec, b, out, sc);
+  });
 }
 
 // fp32 copies of one level's face coefficients and inverse diagonal
