@@ -172,7 +172,7 @@ struct hoc_stepper {
   double *r, *z, *pp, *pp2, *Ap, *part_a, *part_b, *part_c;
   unsigned* bar = nullptr;      // persistent-solver grid barrier [GRID_BAR_WORDS]
   int* bar_err = nullptr;
-  int pcg_sub = 1;        // subtrees per full 8192-element chunk
+  int pcg_tail_slots = 0;  // slots of the trailing chunk's tree (a power of two)
   int pcg_parts_all = 0;  // workgroups of one PCG phase
   int pcg_parts = 0;      // == pcg_parts_all when the cooperative launch is usable
   PcgScalars* sc = nullptr;
@@ -612,11 +612,10 @@ PcgArgs pcg_args(hoc_stepper* h, const HelmOp& op, const double* inv_diag, const
   a.part_a = h->part_a;
   a.part_b = h->part_b;
   a.part_c = h->part_c;
-  a.plans = h->red.plans;
   a.nfull = h->red.nfull;
-  a.sub = h->pcg_sub;
-  a.tail = (int)(h->red.nchunks - h->red.nfull);
-  a.nparts = h->pcg_parts;
+  a.tail = (int)(h->d.n2 % PW_CHUNK);
+  a.tail_slots = h->pcg_tail_slots;
+  a.nparts = h->pcg_parts_all;
   a.nchunks = (int)h->red.nchunks;
   a.rtol = h->p.rtol;
   a.max_iter = h->p.max_iter;
@@ -624,9 +623,11 @@ PcgArgs pcg_args(hoc_stepper* h, const HelmOp& op, const double* inv_diag, const
   a.err = h->bar_err;
   a.sc = h->sc;
   a.counters = h->dcount;
-  // beyond 256 chunks (2M cells) the phases' scalars are formed once per
-  // grid (k_pcg_totals) instead of in every workgroup
-  a.central = a.nchunks > 256 ? 1 : 0;
+  // beyond 96 chunks (786432 cells) the phases' scalars are formed once per
+  // grid (k_pcg_totals) instead of in every workgroup: a solve on 704 x 704
+  // (61 chunks) takes 929 us that way against 892, on 1024 x 1024 (128
+  // chunks) 1305 us against 1360
+  a.central = a.nchunks > 96 ? 1 : 0;
   return a;
 }
 
@@ -1767,15 +1768,11 @@ int hoc_stepper_create(const hoc_config* cfg, const hoc_geometry* g, hoc_stepper
     if (rc != HOC_OK) return cleanup(rc);
     h->part_a = pa;
     h->part_b = pb;
-    // persistent solver: split each full chunk into `sub` subtrees so that
-    // about 256-512 single-wave workgroups share the work
+    // parts: 512-element subtrees of the full chunks and the slots of the
+    // trailing chunk's tree, filled up to its depth
     const long long nfull = h->red.nfull;
-    // parts of 8192 / PCG_MAX_SUB = 512 elements: one element per thread
-    // in two passes at most, ~8 waves per CU at 512 x 512
-    const int sub = PCG_MAX_SUB;
-    PwPlan tail_plan = make_plan((int)(d.n2 % PW_CHUNK));
-    const long long parts = nfull * sub + (h->red.nchunks > nfull ? tail_plan.nleaves : 0);
-    h->pcg_sub = sub;
+    if (d.n2 % PW_CHUNK) h->pcg_tail_slots = 1 << make_plan((int)(d.n2 % PW_CHUNK)).nlevels;
+    const long long parts = nfull * PCG_SUB + h->pcg_tail_slots;
     h->pcg_parts_all = (int)parts;
     int dev = 0, ncu = 0, coop = 0, per_cu = 0;
     if (hipGetDevice(&dev) == hipSuccess &&

@@ -9,10 +9,10 @@
 // into 8192-element chunks; each chunk is summed pairwise (recursive halving
 // to blocks of <= 128 elements, each block with eight interleaved
 // accumulators combined as ((r0+r1)+(r2+r3))+((r4+r5)+(r6+r7)), then its
-// remainder); the chunk sums are then added in order. One workgroup owns one
-// chunk: eight lanes per block accumulate, a 3-step xor-shuffle combines the
-// eight accumulators in exactly that order, and the blocks' tree is walked
-// level by level in LDS from a host-built plan.
+// remainder); the chunk sums are then added in order. The solver's workgroups
+// own subtrees of chunks (hoc_reduce.h); the stand-alone dot product
+// (k_pw_dot) has one workgroup per chunk, eight lanes per block, and walks the
+// blocks' tree level by level in LDS from a host-built plan.
 #include "hoc_device.h"
 #include "hoc_kernels.h"
 #include "hoc_reduce.h"
@@ -256,14 +256,21 @@ __device__ bool grid_barrier(unsigned* bar, int* err, unsigned nblocks) {
   return s_ok != 0;
 }
 
+// Column and row of flat index e (at most PCG_MAX_CHUNKS chunks: 32 bits).
+__device__ __forceinline__ void cell_ij(const Dims& d, long long e, int& i, int& j) {
+  j = (int)((unsigned)e / (unsigned)d.nx);
+  i = (int)((unsigned)e - (unsigned)j * (unsigned)d.nx);
+}
+
 // Per-element work of the A phase: p_new at the five stencil points (z +
 // beta p_old; p itself on the first iteration), A p_new at e, store p_new
 // and Ap; returns p_new * Ap for the p.Ap sum.
-__device__ __forceinline__ Two pcg_apply_elem(const PcgArgs& a, long long e, bool first,
+__device__ __forceinline__ double pcg_apply_elem(const PcgArgs& a, long long e, bool first,
                                               double bt, double* pnew, const double* pold) {
   const Dims& d = a.d;
   const HelmOp& op = a.op;
-  const int i = (int)(e % d.nx), j = (int)(e / d.nx);
+  int i, j;
+  cell_ij(d, e, i, j);
   const long long ce = at2(d, j, wrap(i, 1, d.nx)), cw = at2(d, j, wrap(i, -1, d.nx));
   const long long cn = at2(d, wrap(j, 1, d.ny), i), cs = at2(d, wrap(j, -1, d.ny), i);
   auto pv = [&](long long q) -> double { return first ? pnew[q] : a.z[q] + bt * pold[q]; };
@@ -282,7 +289,7 @@ __device__ __forceinline__ Two pcg_apply_elem(const PcgArgs& a, long long e, boo
   const double ap = (xc - op.coef * lap) * mc + xc * (1.0 - mc);
   if (!first) pnew[e] = pc;
   a.Ap[e] = ap;
-  return Two{pc * ap, 0.0};
+  return pc * ap;
 }
 
 // Per-element work of the update phase: x += alpha p, r -= alpha Ap,
@@ -308,7 +315,8 @@ __device__ __forceinline__ ApLoads ap_load(const PcgArgs& a, long long e, bool f
                                            const double* pnew, const double* pold) {
   const Dims& d = a.d;
   const HelmOp& op = a.op;
-  const int i = (int)(e % d.nx), j = (int)(e / d.nx);
+  int i, j;
+  cell_ij(d, e, i, j);
   const long long ce = at2(d, j, wrap(i, 1, d.nx)), cw = at2(d, j, wrap(i, -1, d.nx));
   const long long cn = at2(d, wrap(j, 1, d.ny), i), cs = at2(d, wrap(j, -1, d.ny), i);
   ApLoads L;
@@ -341,7 +349,9 @@ __device__ __forceinline__ ApLoads ap_load(const PcgArgs& a, long long e, bool f
 
 // pcg_apply_elem from preloaded operands (same arithmetic).
 __device__ __forceinline__ double ap_finish(const PcgArgs& a, long long e, bool first, double bt,
-                                            double* pnew, const ApLoads& L) {
+                                            double* pnew, const ApLoads& L,
+                                            const Divisor<double>& by_dx2,
+                                            const Divisor<double>& by_dy2) {
   const HelmOp& op = a.op;
   const double pc = first ? L.p0 : L.z0 + bt * L.p0;
   const double pe = first ? L.p1 : L.z1 + bt * L.p1;
@@ -357,7 +367,7 @@ __device__ __forceinline__ double ap_finish(const PcgArgs& a, long long e, bool 
   const double fxw = L.kuw * (xc - xw);
   const double fy = L.kv * (xn - xc);
   const double fys = L.kvs * (xc - xs);
-  const double lap = (fx - fxw) / op.dx2 + (fy - fys) / op.dy2;
+  const double lap = by_dx2(fx - fxw) + by_dy2(fy - fys);
   const double ap = (xc - op.coef * lap) * L.mc + xc * (1.0 - L.mc);
   if (!first) pnew[e] = pc;
   a.Ap[e] = ap;
@@ -374,8 +384,7 @@ __device__ __forceinline__ int logical_block(int nb) {
 
 __global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
   __shared__ double lds[2 * PCG_STAGE];
-  __shared__ double leafs[128];
-  __shared__ double cs[PCG_MAX_CHUNKS];
+  __shared__ double cs[2 * PCG_CS];
   const unsigned nb = gridDim.x;
   const int part = logical_block((int)nb);
   const HelmOp& op = a.op;
@@ -386,13 +395,13 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
 
   // r = rhs * mask, x = 0; ||rhs||
   {
-    const Two s = part_sum<1>(a, part, [&](long long e) -> Two {
+    const double s = part_sum(a, part, [&](long long e) -> double {
       const double r = a.rhs[e] * mk(op.mask[e]);
       a.r[e] = r;
       a.x[e] = 0.0;
-      return Two{r * r, 0.0};
-    }, lds, leafs);
-    if (threadIdx.x == 0) a.part_a[part] = s.a;
+      return r * r;
+    }, lds);
+    if (threadIdx.x == 0) a.part_a[part] = s;
   }
   ok = grid_barrier(a.bar, a.err, nb);
   if (ok) {
@@ -403,13 +412,13 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
   }
   if (ok && !done) {
     // z = M^-1 r, p = z (into pb1, the buffer iteration 1 uses); r.z
-    const Two s = part_sum<1>(a, part, [&](long long e) -> Two {
+    const double s = part_sum(a, part, [&](long long e) -> double {
       const double z = a.inv_diag[e] * a.r[e];
       a.z[e] = z;
       a.pb1[e] = z;
-      return Two{a.r[e] * z, 0.0};
-    }, lds, leafs);
-    if (threadIdx.x == 0) a.part_b[part] = s.a;
+      return a.r[e] * z;
+    }, lds);
+    if (threadIdx.x == 0) a.part_b[part] = s;
     ok = grid_barrier(a.bar, a.err, nb);
     if (ok) rz = total_from_parts(a, a.part_b, cs);
   }
@@ -420,33 +429,38 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
     const bool first = it == 1;
     const double bt = beta;
     {
-      const Two s = part_sum<1>(a, part, [&](long long e) -> Two {
+      const double s = part_sum(a, part, [&](long long e) -> double {
         return pcg_apply_elem(a, e, first, bt, pnew, pold);
-      }, lds, leafs);
-      if (threadIdx.x == 0) a.part_a[part] = s.a;
+      }, lds);
+      if (threadIdx.x == 0) a.part_a[part] = s;
     }
     ok = grid_barrier(a.bar, a.err, nb);
     if (!ok) break;
     alpha = rz / total_from_parts(a, a.part_a, cs);
     {
       const double al = alpha;
-      const Two s = part_sum<2>(a, part, [&](long long e) -> Two {
-        return pcg_update_elem(a, e, al, pnew);
-      }, lds, leafs);
-      if (threadIdx.x == 0) {
-        a.part_b[part] = s.a;
-        a.part_c[part] = s.b;
+      const PartRange pr = part_range(a, part);
+      for (int t = threadIdx.x; t < pr.nel; t += PCG_WG) {
+        const Two v = pcg_update_elem(a, pr.base + t, al, pnew);
+        lds[stage_at(t)] = v.a;
+        lds[PCG_STAGE + stage_at(t)] = v.b;
       }
+      const double s = part_reduce<2>(pr, lds);
+      if (threadIdx.x == 0) a.part_b[part] = s;
+      if (threadIdx.x == 32) a.part_c[part] = s;
     }
     ok = grid_barrier(a.bar, a.err, nb);
     if (!ok) break;
-    res = sqrt(total_from_parts(a, a.part_b, cs));
+    const double* parts[2] = {a.part_b, a.part_c};
+    double tot[2];
+    totals_from_parts<2>(a, parts, cs, tot);
+    res = sqrt(tot[0]);
     if (res <= tol) {
       done = 1;
       conv = 1;
       break;
     }
-    const double rz_new = total_from_parts(a, a.part_c, cs);
+    const double rz_new = tot[1];
     beta = rz_new / rz;
     rz = rz_new;
     if (it >= a.max_iter) {
@@ -479,23 +493,21 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
 
 // r = rhs * mask, x = 0; partial sums of r*r
 __global__ __launch_bounds__(PCG_WG) void k_pcg_init(PcgArgs a) {
-  __shared__ double lds[2 * PCG_STAGE];
-  __shared__ double leafs[128];
+  __shared__ double lds[PCG_STAGE];
   const int part = blockIdx.x;
-  const Two s = part_sum<1>(a, part, [&](long long e) -> Two {
+  const double s = part_sum(a, part, [&](long long e) -> double {
     const double r = a.rhs[e] * mk(a.op.mask[e]);
     a.r[e] = r;
     a.x[e] = 0.0;
-    return Two{r * r, 0.0};
-  }, lds, leafs);
-  if (threadIdx.x == 0) a.part_a[part] = s.a;
+    return r * r;
+  }, lds);
+  if (threadIdx.x == 0) a.part_a[part] = s;
 }
 
 // ||rhs|| (zero: done in 0 iterations); z = M^-1 r, p = z; partials of r*z
 __global__ __launch_bounds__(PCG_WG) void k_pcg_init_z(PcgArgs a) {
-  __shared__ double lds[2 * PCG_STAGE];
-  __shared__ double leafs[128];
-  __shared__ double cs[PCG_MAX_CHUNKS];
+  __shared__ double lds[PCG_STAGE];
+  __shared__ double cs[PCG_CS];
   const double nb = sqrt(total_from_parts(a, a.part_a, cs));
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     a.sc->norm_b = nb;
@@ -507,13 +519,13 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_init_z(PcgArgs a) {
   }
   if (nb == 0.0) return;
   const int part = blockIdx.x;
-  const Two s = part_sum<1>(a, part, [&](long long e) -> Two {
+  const double s = part_sum(a, part, [&](long long e) -> double {
     const double z = a.inv_diag[e] * a.r[e];
     a.z[e] = z;
     a.pb1[e] = z;
-    return Two{a.r[e] * z, 0.0};
-  }, lds, leafs);
-  if (threadIdx.x == 0) a.part_b[part] = s.a;
+    return a.r[e] * z;
+  }, lds);
+  if (threadIdx.x == 0) a.part_b[part] = s;
 }
 
 // The scalars the next phase needs from the last phase's partial sums,
@@ -525,7 +537,7 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_init_z(PcgArgs a) {
 // part_c (r.z).
 __global__ __launch_bounds__(PCG_WG) void k_pcg_totals(PcgArgs a, int which) {
   if (a.sc->done) return;
-  __shared__ double cs[2 * PCG_MAX_CHUNKS];
+  __shared__ double cs[2 * PCG_CS];
   if (which == 0) {
     const double t = total_from_parts(a, a.part_a, cs);
     if (threadIdx.x == 0) a.sc->tot[0] = t;
@@ -545,37 +557,42 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_totals(PcgArgs a, int which) {
 
 // Iteration `it` (1-based), phase A. For it > 1 it first finishes
 // iteration it-1: the convergence test on ||r||, then beta and the new rz.
+// All loads that need no other (the solve's state, the partial sums, the
+// elements' operands) are issued before any is used.
 __global__ __launch_bounds__(PCG_WG) void k_pcg_ap(PcgArgs a, int it) {
-  if (a.sc->done) return;
-  __shared__ double lds[2 * PCG_STAGE];
-  __shared__ double leafs[128];
-  __shared__ double cs[2 * PCG_MAX_CHUNKS];
+  __shared__ double lds[PCG_STAGE];
+  __shared__ double cs[2 * PCG_CS];
   const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
   const bool first = it == 1;
   double* pnew = (it & 1) ? a.pb1 : a.pb0;
   const double* pold = (it & 1) ? a.pb0 : a.pb1;
   const int part = blockIdx.x;
   const PartRange pr = part_range(a, part);
-  // operands of this part's (at most two per thread) elements first
-  const int t0 = threadIdx.x, t1 = threadIdx.x + PCG_WG;
-  const bool h0 = t0 < pr.nel, h1 = t1 < pr.nel;
-  const ApLoads L0 = ap_load(a, pr.base + (h0 ? t0 : 0), first, pnew, pold);
-  const ApLoads L1 = ap_load(a, pr.base + (h1 ? t1 : 0), first, pnew, pold);
-  double beta = 0.0;
-  if (first) {
-    const double rz = a.central ? a.sc->tot[1] : total_from_parts(a, a.part_b, cs);
-    if (lead) a.sc->rz2[1] = rz;
+  const int done = a.sc->done;
+  const double tol = a.sc->tol, rz_old = a.sc->rz2[(it - 1) & 1];
+  const double* parts[2] = {a.part_b, a.part_c};
+  TotalsLoads<2> T;
+  if (!a.central) T = totals_load<2>(a, parts);
+  ApLoads L[PCG_EPT];
+#pragma unroll
+  for (int k = 0; k < PCG_EPT; ++k) {
+    const int t = threadIdx.x + k * PCG_WG;
+    if (t < pr.nel) L[k] = ap_load(a, pr.base + t, first, pnew, pold);
+  }
+  double tot[2] = {0.0, 0.0};
+  if (a.central) {
+    tot[0] = a.sc->tot[1];
+    tot[1] = a.sc->tot[2];
   } else {
-    const double* parts[2] = {a.part_b, a.part_c};
-    double tot[2];
-    if (a.central) {
-      tot[0] = a.sc->tot[1];
-      tot[1] = a.sc->tot[2];
-    } else {
-      totals_from_parts<2>(a, parts, cs, tot);
-    }
+    totals_finish<2>(a, parts, T, cs, tot);  // the first iteration uses only part_b's
+  }
+  if (done) return;
+  const double beta = first ? 0.0 : tot[1] / rz_old;
+  if (first) {
+    if (lead) a.sc->rz2[1] = tot[0];
+  } else {
     const double res = sqrt(tot[0]);
-    if (res <= a.sc->tol) {
+    if (res <= tol) {
       if (lead) {
         a.sc->res = res;
         a.sc->done = 1;
@@ -596,14 +613,18 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_ap(PcgArgs a, int it) {
       }
       return;
     }
-    const double rz_new = tot[1];
-    beta = rz_new / a.sc->rz2[(it - 1) & 1];
-    if (lead) a.sc->rz2[it & 1] = rz_new;
+    if (lead) a.sc->rz2[it & 1] = tot[1];
   }
-  if (h0) lds[t0] = ap_finish(a, pr.base + t0, first, beta, pnew, L0);
-  if (h1) lds[t1] = ap_finish(a, pr.base + t1, first, beta, pnew, L1);
-  const Two s = part_reduce<1>(pr, lds, leafs);
-  if (threadIdx.x == 0) a.part_a[part] = s.a;
+  const Divisor<double> by_dx2 = uniform_divisor<double>(a.op.dx2);
+  const Divisor<double> by_dy2 = uniform_divisor<double>(a.op.dy2);
+#pragma unroll
+  for (int k = 0; k < PCG_EPT; ++k) {
+    const int t = threadIdx.x + k * PCG_WG;
+    if (t < pr.nel)
+      lds[stage_at(t)] = ap_finish(a, pr.base + t, first, beta, pnew, L[k], by_dx2, by_dy2);
+  }
+  const double s = part_reduce<1>(pr, lds);
+  if (threadIdx.x == 0) a.part_a[part] = s;
 }
 
 // Iteration `it`, phase B: alpha = rz / (p.Ap); x += alpha p; r -= alpha Ap;
@@ -611,63 +632,64 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_ap(PcgArgs a, int it) {
 // of r*r and r*z, otherwise only r*r (the preconditioner follows in its own
 // launches and then k_pcg_rz).
 __global__ __launch_bounds__(PCG_WG) void k_pcg_update(PcgArgs a, int it, int jacobi) {
-  if (a.sc->done) return;
   __shared__ double lds[2 * PCG_STAGE];
-  __shared__ double leafs[128];
-  __shared__ double cs[PCG_MAX_CHUNKS];
+  __shared__ double cs[PCG_CS];
   const double* pnew = (it & 1) ? a.pb1 : a.pb0;
   const int part = blockIdx.x;
   const PartRange pr = part_range(a, part);
-  // element operands first (independent of alpha); element base + t for
-  // t = tid and tid + PCG_WG (a part has at most 2 * PCG_WG elements)
-  const int t0 = threadIdx.x, t1 = threadIdx.x + PCG_WG;
-  const bool h0 = t0 < pr.nel, h1 = t1 < pr.nel;
-  const long long e0 = pr.base + (h0 ? t0 : 0), e1 = pr.base + (h1 ? t1 : 0);
-  const double x0 = a.x[e0], p0 = pnew[e0], r0 = a.r[e0], ap0 = a.Ap[e0];
-  const double x1 = a.x[e1], p1 = pnew[e1], r1 = a.r[e1], ap1 = a.Ap[e1];
-  const double d0 = jacobi ? a.inv_diag[e0] : 0.0, d1 = jacobi ? a.inv_diag[e1] : 0.0;
-  const double al =
-      a.sc->rz2[it & 1] / (a.central ? a.sc->tot[0] : total_from_parts(a, a.part_a, cs));
-  auto fin = [&](bool h, int t, long long e, double xv, double pv, double rv, double av,
-                 double dv) {
-    if (!h) return;
-    a.x[e] = xv + al * pv;
-    const double r = rv - al * av;
-    a.r[e] = r;
-    lds[t] = r * r;
-    if (jacobi) {
-      const double z = dv * r;
-      a.z[e] = z;
-      lds[PCG_STAGE + t] = r * z;
-    }
+  const int done = a.sc->done;
+  const double rz = a.sc->rz2[it & 1];
+  const double* parts[1] = {a.part_a};
+  TotalsLoads<1> T;
+  if (!a.central) T = totals_load<1>(a, parts);
+  struct Loads {
+    double x, p, r, ap, d;
   };
-  fin(h0, t0, e0, x0, p0, r0, ap0, d0);
-  fin(h1, t1, e1, x1, p1, r1, ap1, d1);
-  if (jacobi) {
-    const Two s = part_reduce<2>(pr, lds, leafs);
-    if (threadIdx.x == 0) {
-      a.part_b[part] = s.a;
-      a.part_c[part] = s.b;
-    }
-  } else {
-    const Two s = part_reduce<1>(pr, lds, leafs);
-    if (threadIdx.x == 0) a.part_b[part] = s.a;
+  Loads L[PCG_EPT];
+#pragma unroll
+  for (int k = 0; k < PCG_EPT; ++k) {
+    const int t = threadIdx.x + k * PCG_WG;
+    if (t >= pr.nel) continue;
+    const long long e = pr.base + t;
+    L[k] = Loads{a.x[e], pnew[e], a.r[e], a.Ap[e], jacobi ? a.inv_diag[e] : 0.0};
   }
+  double pap;
+  if (a.central) pap = a.sc->tot[0];
+  else totals_finish<1>(a, parts, T, cs, &pap);
+  if (done) return;
+  const double al = rz / pap;
+#pragma unroll
+  for (int k = 0; k < PCG_EPT; ++k) {
+    const int t = threadIdx.x + k * PCG_WG;
+    if (t >= pr.nel) continue;
+    const long long e = pr.base + t;
+    a.x[e] = L[k].x + al * L[k].p;
+    const double r = L[k].r - al * L[k].ap;
+    a.r[e] = r;
+    lds[stage_at(t)] = r * r;
+    if (jacobi) {
+      const double z = L[k].d * r;
+      a.z[e] = z;
+      lds[PCG_STAGE + stage_at(t)] = r * z;
+    }
+  }
+  const double s = jacobi ? part_reduce<2>(pr, lds) : part_reduce<1>(pr, lds);
+  if (threadIdx.x == 0) a.part_b[part] = s;
+  if (jacobi && threadIdx.x == 32) a.part_c[part] = s;
 }
 
 // Partial sums of r*z after a preconditioner application; into_b = 1 on the
 // first application (also p = z into pb1), 0 in the iterations (part_c).
 __global__ __launch_bounds__(PCG_WG) void k_pcg_rz(PcgArgs a, int into_b) {
   if (a.sc->done) return;
-  __shared__ double lds[2 * PCG_STAGE];
-  __shared__ double leafs[128];
+  __shared__ double lds[PCG_STAGE];
   const int part = blockIdx.x;
-  const Two s = part_sum<1>(a, part, [&](long long e) -> Two {
+  const double s = part_sum(a, part, [&](long long e) -> double {
     const double z = a.z[e];
     if (into_b) a.pb1[e] = z;
-    return Two{a.r[e] * z, 0.0};
-  }, lds, leafs);
-  if (threadIdx.x == 0) (into_b ? a.part_b : a.part_c)[part] = s.a;
+    return a.r[e] * z;
+  }, lds);
+  if (threadIdx.x == 0) (into_b ? a.part_b : a.part_c)[part] = s;
 }
 
 // After a sync-free solve of n_it launched iterations: a solve whose done

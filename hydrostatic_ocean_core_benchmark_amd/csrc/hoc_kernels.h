@@ -357,9 +357,9 @@ struct PcgArgs {
   const double* inv_diag;
   double *x, *r, *z, *pb0, *pb1, *Ap;
   double *part_a, *part_b, *part_c;
-  const PwPlan* plans;  // [0] full chunk, [1] trailing chunk
   long long nfull;
-  int sub, tail, nparts, nchunks;
+  int tail, tail_slots;  // elements of the trailing chunk, slots of its tree
+  int nparts, nchunks;
   double rtol;
   int max_iter;
   unsigned* bar;        // grid barrier block, GRID_BAR_WORDS words
@@ -372,8 +372,10 @@ struct PcgArgs {
 constexpr int PCG_WG = 256;         // threads per workgroup of a PCG phase
 constexpr int GRID_BAR_LINE = 64;   // words per counter line of the grid barrier
 constexpr int GRID_BAR_WORDS = 10 * GRID_BAR_LINE;  // 8 group counters, leaders, generation
-constexpr int PCG_STAGE = 512;      // elements staged per part (8192 / sub)
-constexpr int PCG_MAX_SUB = 16;     // subtrees per full chunk
+constexpr int PCG_SUB = 16;         // subtrees (parts) per full chunk
+constexpr int PCG_PART = 512;       // elements of one: 8192 / PCG_SUB
+constexpr int PCG_EPT = PCG_PART / PCG_WG;  // elements of a part per thread
+constexpr int PCG_STAGE = 544;      // LDS values that stage a part (stage_at)
 constexpr int PCG_MAX_CHUNKS = 1024;
 
 // One level of the multigrid hierarchy (level 0 is the model grid).

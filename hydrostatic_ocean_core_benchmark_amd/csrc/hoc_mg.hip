@@ -15,8 +15,8 @@ namespace hoc {
 
 template <class R>
 __device__ __forceinline__ void lvl_ij(const MgLevelT<R>& L, long long c, int& i, int& j) {
-  i = (int)(c % L.nx);
-  j = (int)(c / L.nx);
+  j = (int)((unsigned)c / (unsigned)L.nx);  // a level has fewer than 2^31 cells
+  i = (int)((unsigned)c - (unsigned)j * (unsigned)L.nx);
 }
 
 template <class R>
@@ -343,20 +343,19 @@ __global__ void k_mg_prolong(MgLevel f, const double* __restrict__ xc, int cnx,
 __global__ __launch_bounds__(PCG_WG) void k_mg_res_parts(PcgArgs a, MgLevel L,
                                                          const double* __restrict__ x) {
   if (a.sc->done) return;
-  __shared__ double lds[2 * PCG_STAGE];
-  __shared__ double leafs[128];
+  __shared__ double lds[PCG_STAGE];
   const int part = blockIdx.x;
-  const Two s = part_sum<1>(a, part, [&](long long e) -> Two {
+  const double s = part_sum(a, part, [&](long long e) -> double {
     const double r = a.rhs[e] - mg_apply(L, x, e);
-    return Two{r * r, 0.0};
-  }, lds, leafs);
-  if (threadIdx.x == 0) a.part_b[part] = s.a;
+    return r * r;
+  }, lds);
+  if (threadIdx.x == 0) a.part_b[part] = s;
 }
 
 // Stationary-solver bookkeeping after iteration `it`: ||rhs - A x|| <= tol.
 __global__ __launch_bounds__(PCG_WG) void k_mg_check(PcgArgs a, int it) {
   if (a.sc->done) return;
-  __shared__ double cs[PCG_MAX_CHUNKS];
+  __shared__ double cs[PCG_CS];
   const double res = sqrt(total_from_parts(a, a.part_b, cs));
   if (threadIdx.x != 0) return;
   PcgScalars* sc = a.sc;
@@ -377,7 +376,7 @@ __global__ __launch_bounds__(PCG_WG) void k_mg_check(PcgArgs a, int it) {
 
 // ||rhs|| and the zero-rhs shortcut for the stationary solvers; x = 0.
 __global__ __launch_bounds__(PCG_WG) void k_mg_start(PcgArgs a) {
-  __shared__ double cs[PCG_MAX_CHUNKS];
+  __shared__ double cs[PCG_CS];
   const double nb = sqrt(total_from_parts(a, a.part_a, cs));
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     a.sc->norm_b = nb;

@@ -1,5 +1,14 @@
 // NumPy-order float64 reductions over a PCG partition (see PcgArgs in
 // hoc_kernels.h): per-part pairwise sums and the in-order total.
+//
+// Both are chains of latencies (load, a few adds, LDS, barrier), so they are
+// cut to the fewest links: adds between lanes are DPP moves, the accumulators'
+// sixteen LDS reads are issued together, the trees have one shape for every
+// length (an absent leaf is -0.0, which adds as nothing), and each has one
+// barrier. With the trailing chunk's tree walked from a plan in memory, LDS
+// read by read and with a barrier per tree level, the A phase of 131 x 77 took
+// 8.3 us and its update 5.8, of 128 x 128 6.5 and 4.4; so they are 5.8 and
+// 3.9, 5.2 and 3.5.
 #pragma once
 
 #include "hoc_device.h"
@@ -13,167 +22,199 @@ struct Two {
   double a, b;
 };
 
-// The elements of one part: [base, base + nel), nleaves leaves of leaf_len.
-// Parts: full 8192-element chunks are cut into `sub` aligned subtrees of
-// 8192/sub elements (each a perfect tree of 128-element leaves); the
-// trailing partial chunk contributes one part per leaf of its plan.
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), CTRL, 0xf, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// Pairwise sums over groups of 8 and of 16 neighbouring lanes, in every lane:
+// lane ^ 1, lane ^ 2, then the mirrored lane of the 8 and of the 16, whose
+// value is that of lane ^ 4 and lane ^ 8 once quads and eights agree. All
+// lanes of the group must be active.
+__device__ __forceinline__ double sum8(double v) {
+  v = v + dpp_d<0xB1>(v);
+  v = v + dpp_d<0x4E>(v);
+  return v + dpp_d<0x141>(v);
+}
+__device__ __forceinline__ double sum16(double v) {
+  v = sum8(v);
+  return v + dpp_d<0x140>(v);
+}
+
+// The elements of one part: [base, base + nel). Full 8192-element chunks are
+// cut into PCG_SUB aligned subtrees of 512 elements (four 128-element leaves).
+// The trailing partial chunk is one part per slot of its halving tree filled
+// up to a perfect one: a slot whose leaf lies higher up is empty (nel = 0).
 struct PartRange {
   long long base;
-  int nel, nleaves, leaf_len;
+  int nel;
 };
 
 __device__ __forceinline__ PartRange part_range(const PcgArgs& a, int part) {
-  const long long nfp = a.nfull * a.sub;
-  PartRange r;
-  if (part < nfp) {
-    const long long c = part / a.sub;
-    const int s = part % a.sub;
-    r.nel = (int)(PW_CHUNK / a.sub);
-    r.base = c * PW_CHUNK + (long long)s * r.nel;
-    r.nleaves = r.nel / 128;
-    r.leaf_len = 128;
-  } else {
-    const PwPlan* tp = &a.plans[1];
-    const int l = (int)(part - nfp);
-    r.base = a.nfull * PW_CHUNK + tp->leaf_off[l];
-    r.nel = tp->leaf_len[l];
-    r.nleaves = 1;
-    r.leaf_len = r.nel;
+  const int nfp = (int)a.nfull * PCG_SUB;
+  if (part < nfp) return PartRange{(long long)part * PCG_PART, PCG_PART};
+  // halve as the pairwise sum does (the left half a multiple of 8)
+  int off = 0, len = a.tail;
+  for (int bit = a.tail_slots >> 1; bit > 0; bit >>= 1) {
+    const bool right = ((part - nfp) & bit) != 0;
+    if (len > 128) {
+      const int half = (len / 2) & ~7;
+      off += right ? half : 0;
+      len = right ? len - half : half;
+    } else if (right) {
+      len = 0;
+    }
   }
-  return r;
+  return PartRange{a.nfull * PW_CHUNK + off, len};
 }
 
-// Pairwise sum(s) in NumPy's order over values staged in lds[0..nel)
-// (and lds[PCG_STAGE..] for the second sum): eight lanes per leaf
-// accumulate with NumPy's eight interleaved accumulators, then the leaves
-// are combined pairwise. Starts with a barrier (the staging must be done).
+// Where element t of a part is staged in LDS: the leaves 8 values apart from
+// a common bank.
+__device__ __forceinline__ int stage_at(int t) { return t + (t >> 7) * 8; }
+
+// Pairwise sum(s) in NumPy's order over values staged at lds[stage_at(0..nel)]
+// (and lds[PCG_STAGE + ..] for the second sum): the first wave's lanes 0-31
+// form the first sum, lanes 32-63 the second, eight lanes per leaf with
+// NumPy's eight interleaved accumulators, then the leaves pairwise. Starts with
+// a barrier (the staging must be done). The sums are in threads 0 and 32.
 template <int NS>
-__device__ Two part_reduce(const PartRange& pr, double* lds, double* leafs /* [2][64] */) {
+__device__ __forceinline__ double part_reduce(const PartRange& pr, const double* lds) {
   const int tid = threadIdx.x;
-  const int nleaves = pr.nleaves, leaf_len = pr.leaf_len;
   __syncthreads();
-  const int g = tid >> 3, lane = tid & 7;
-  if (g < nleaves) {
-    const int lo = g * leaf_len;
-    const int len = leaf_len;
-    Two res{0.0, 0.0};
-    if (len >= 8) {
-      const int fl = len - (len % 8);
-      Two acc{lds[lo + lane], NS > 1 ? lds[PCG_STAGE + lo + lane] : 0.0};
-      for (int t = 8; t < fl; t += 8) {
-        acc.a = acc.a + lds[lo + t + lane];
-        if (NS > 1) acc.b = acc.b + lds[PCG_STAGE + lo + t + lane];
-      }
-      for (int m = 1; m < 8; m <<= 1) {
-        acc.a = acc.a + shfl_xor_d(acc.a, m);
-        if (NS > 1) acc.b = acc.b + shfl_xor_d(acc.b, m);
-      }
-      res = acc;
-      if (lane == 0) {
-        for (int t = fl; t < len; ++t) {
-          res.a = res.a + lds[lo + t];
-          if (NS > 1) res.b = res.b + lds[PCG_STAGE + lo + t];
-        }
-      }
-    } else if (lane == 0) {
-      for (int t = 0; t < len; ++t) {
-        res.a = res.a + lds[lo + t];
-        if (NS > 1) res.b = res.b + lds[PCG_STAGE + lo + t];
-      }
-    }
-    if (lane == 0) {
-      leafs[g] = res.a;
-      if (NS > 1) leafs[64 + g] = res.b;
-    }
+  if (tid >= 64) return 0.0;
+  const int g = (tid >> 3) & 3, lane = tid & 7;
+  const double* v = lds + (NS > 1 ? (tid >> 5) * PCG_STAGE : 0) + g * 136;
+  double w[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) w[t] = v[8 * t + lane];
+  double s;
+  if (pr.nel == PCG_PART) {
+    s = w[0];
+#pragma unroll
+    for (int t = 1; t < 16; ++t) s = s + w[t];
+    s = sum8(s);
+  } else {
+    const int len = min(max(pr.nel - 128 * g, 0), 128), fl = len & ~7;
+    double rem[7];
+#pragma unroll
+    for (int t = 0; t < 7; ++t) rem[t] = v[fl + t];
+    s = fl ? w[0] : len ? 0.0 : -0.0;
+#pragma unroll
+    for (int t = 1; t < 16; ++t) s = 8 * t < fl ? s + w[t] : s;
+    s = sum8(s);
+#pragma unroll
+    for (int t = 0; t < 7; ++t) s = fl + t < len ? s + rem[t] : s;
   }
-  __syncthreads();
-  // perfect pairwise tree over the part's leaves (1, 2, 4, ... leaves)
-  for (int w = 1; w < nleaves; w <<= 1) {
-    if (tid < nleaves / (2 * w)) {
-      leafs[2 * w * tid] = leafs[2 * w * tid] + leafs[2 * w * tid + w];
-      if (NS > 1) leafs[64 + 2 * w * tid] = leafs[64 + 2 * w * tid] + leafs[64 + 2 * w * tid + w];
-    }
-    __syncthreads();
-  }
-  Two out{leafs[0], NS > 1 ? leafs[64] : 0.0};
-  __syncthreads();
-  return out;
+  s = s + dpp_d<0x140>(s);
+  return s + __shfl_xor(s, 16, 64);
 }
 
-// This workgroup's part and the pairwise sum(s) over it in NumPy's order.
-// Each thread evaluates elements independently (`elem(e)` may store
+// This workgroup's part and the pairwise sum over it in NumPy's order (in
+// thread 0). Each thread evaluates elements independently (`elem(e)` may store
 // per-element results; it runs exactly once per index) and the values are
-// staged in LDS for part_reduce.
-template <int NS, class F>
-__device__ Two part_sum(const PcgArgs& a, int part, F elem, double* lds /* [2][PCG_STAGE] */,
-                        double* leafs /* [2][64] */) {
+// staged in LDS for part_reduce; a thread's elements are evaluated before
+// any is staged, so their loads are in flight together.
+template <class F>
+__device__ __forceinline__ double part_sum(const PcgArgs& a, int part, F elem,
+                                           double* lds /* [PCG_STAGE] */) {
   const PartRange pr = part_range(a, part);
-  for (int t = threadIdx.x; t < pr.nel; t += PCG_WG) {
-    const Two v = elem(pr.base + t);
-    lds[t] = v.a;
-    if (NS > 1) lds[PCG_STAGE + t] = v.b;
+  double v[PCG_EPT];
+#pragma unroll
+  for (int k = 0; k < PCG_EPT; ++k) {
+    const int t = threadIdx.x + k * PCG_WG;
+    v[k] = t < pr.nel ? elem(pr.base + t) : 0.0;
   }
-  return part_reduce<NS>(pr, lds, leafs);
+#pragma unroll
+  for (int k = 0; k < PCG_EPT; ++k) lds[stage_at(threadIdx.x + k * PCG_WG)] = v[k];
+  return part_reduce<1>(pr, lds);
 }
 
-// In-order float64 sums of whole vectors from their per-part partials: each
-// full chunk's top tree levels over its `sub` subtree sums, the trailing
-// chunk's tree from its plan over its leaf sums, then the chunk sums added
-// sequentially. Every workgroup computes them identically; NV vectors
-// (1 or 2) are summed in one pass.
+// In-order float64 sums of whole vectors from their per-part partials: sixteen
+// lanes sum a full chunk's subtrees pairwise, the trailing chunk's slots are
+// rows of sixteen of its tree, then the chunk sums are added sequentially.
+// Every thread forms them identically; NV vectors (1 or 2) are summed in one
+// pass. The first rows' loads are apart (totals_load), for a kernel to issue
+// before its other loads. cs must not be in use (its last readers a barrier
+// ago).
+constexpr int PCG_CS = PCG_MAX_CHUNKS + 8;  // rows of one vector
+constexpr int PCG_ROWS = PCG_WG / 16;       // rows of one pass, two in flight
 template <int NV>
-__device__ void totals_from_parts(const PcgArgs& a, const double* const* part, double* cs,
-                                  double* out) {
-  const int tid = threadIdx.x;
-  __shared__ double s_tot[2];
-  __shared__ double tail_v[2][256];
-  const long long nfp = a.nfull * a.sub;
-  for (int c = tid; c < a.nfull; c += PCG_WG) {
+struct TotalsLoads {
+  double v[2][NV];
+};
+
+// The trailing chunk's first row, behind fillers of -0.0, and all rows.
+__device__ __forceinline__ int totals_tail_row(const PcgArgs& a) { return ((int)a.nfull + 7) & ~7; }
+__device__ __forceinline__ int totals_rows(const PcgArgs& a) {
+  return totals_tail_row(a) + (a.tail_slots + 15) / 16;
+}
+
+template <int NV>
+__device__ __forceinline__ TotalsLoads<NV> totals_load(const PcgArgs& a,
+                                                       const double* const* part, int c0 = 0) {
+  const int nfull = (int)a.nfull, trow = totals_tail_row(a), rows = totals_rows(a);
+  const int row = threadIdx.x >> 4, lane = threadIdx.x & 15;
+  TotalsLoads<NV> L;
 #pragma unroll
-    for (int q = 0; q < NV; ++q) {
-      double t[PCG_MAX_SUB];
+  for (int k = 0; k < 2; ++k) {
+    const int c = c0 + k * PCG_ROWS + row;
+    const int slot = c < trow ? c * 16 + lane : (nfull + c - trow) * 16 + lane;
+    const bool on = c < rows && (c < trow ? c < nfull : slot < a.nparts);
 #pragma unroll
-      for (int s = 0; s < PCG_MAX_SUB; ++s)
-        if (s < a.sub) t[s] = part[q][(long long)c * a.sub + s];
-#pragma unroll
-      for (int w = 1; w < PCG_MAX_SUB; w <<= 1)
-#pragma unroll
-        for (int s = 0; s + w < PCG_MAX_SUB; s += 2 * w)
-          if (s + w < a.sub) t[s] = t[s] + t[s + w];
-      cs[q * PCG_MAX_CHUNKS + c] = t[0];
-    }
+    for (int q = 0; q < NV; ++q) L.v[k][q] = on ? part[q][slot] : -0.0;
   }
-  if (a.tail) {
-    const PwPlan* tp = &a.plans[1];
-    const int L = tp->nleaves;
-    for (int l = tid; l < L; l += PCG_WG)
+  return L;
+}
+
+template <int NV>
+__device__ __forceinline__ void totals_finish(const PcgArgs& a, const double* const* part,
+                                              TotalsLoads<NV> L, double* cs /* [NV][PCG_CS] */,
+                                              double* out) {
+  const int trow = totals_tail_row(a), rows = totals_rows(a);
+  const int row = threadIdx.x >> 4, lane = threadIdx.x & 15;
+  for (int c0 = 0; c0 < rows; c0 += 2 * PCG_ROWS) {
+    if (c0) L = totals_load<NV>(a, part, c0);
 #pragma unroll
-      for (int q = 0; q < NV; ++q) tail_v[q][l] = part[q][nfp + l];
-    __syncthreads();
-    int start = 0;
-    for (int lv = 0; lv < tp->nlevels; ++lv) {
-      const int end = tp->level_end[lv];
-      for (int n = start + tid; n < end; n += PCG_WG)
+    for (int k = 0; k < 2; ++k) {
+      const int c = c0 + k * PCG_ROWS + row;
+      if (c0 + k * PCG_ROWS >= rows) break;
 #pragma unroll
-        for (int q = 0; q < NV; ++q)
-          tail_v[q][L + n] = tail_v[q][tp->node_l[n]] + tail_v[q][tp->node_r[n]];
-      start = end;
-      __syncthreads();
+      for (int q = 0; q < NV; ++q) {
+        const double s = sum16(L.v[k][q]);
+        if (lane == 0 && c < rows) cs[q * PCG_CS + c] = s;
+      }
     }
-    if (tid < NV)
-      cs[tid * PCG_MAX_CHUNKS + a.nfull] =
-          tp->nnodes > 0 ? tail_v[tid][L + tp->nnodes - 1] : tail_v[tid][0];
   }
   __syncthreads();
-  if (tid < NV) {
+#pragma unroll
+  for (int q = 0; q < NV; ++q) {
+    const double* v = cs + q * PCG_CS;
     double s = 0.0;
-    for (int c = 0; c < a.nchunks; ++c) s = s + cs[tid * PCG_MAX_CHUNKS + c];
-    s_tot[tid] = s;
-  }
-  __syncthreads();
+    for (int c = 0; c < trow; c += 8) {
+      double w[8];
 #pragma unroll
-  for (int q = 0; q < NV; ++q) out[q] = s_tot[q];
-  __syncthreads();
+      for (int k = 0; k < 8; ++k) w[k] = v[c + k];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) s = s + w[k];
+    }
+    if (a.tail) {
+      double w[8];
+      const int n = rows - trow;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) w[k] = k < n ? v[trow + k] : -0.0;
+      s = s + (((w[0] + w[1]) + (w[2] + w[3])) + ((w[4] + w[5]) + (w[6] + w[7])));
+    }
+    out[q] = s;
+  }
+}
+
+template <int NV>
+__device__ __forceinline__ void totals_from_parts(const PcgArgs& a, const double* const* part,
+                                                  double* cs, double* out) {
+  totals_finish<NV>(a, part, totals_load<NV>(a, part), cs, out);
 }
 
 __device__ __forceinline__ double total_from_parts(const PcgArgs& a, const double* part,
