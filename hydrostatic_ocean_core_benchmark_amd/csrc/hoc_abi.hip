@@ -576,11 +576,10 @@ int build_coefficients(hoc_stepper* h, hipStream_t s) {
   if (!h->Km || !h->Kh) return fail(HOC_ERR_INVALID, "bind K_m / K_h before building");
   const Dims d = h->d;
   { ProfScope _ps(h, "k_coefficients", s);
-  k_coefficients<<<blocks(d.n2), TPB, 0, s>>>(d, h->p, h->geo, h->Km, h->sub_m, h->den_m,
-                                              h->cst_m, h->q); }
+  launch_coefficients(s, d, h->p, h->geo, h->Km, h->sub_m, h->den_m, h->cst_m, h->q); }
   LAUNCH_CHECK("k_coefficients");
   { ProfScope _ps(h, "k_kukv", s);
-  k_kukv<<<blocks(d.n2), TPB, 0, s>>>(d, h->p, h->geo, h->q, h->Ku, h->Kv); }
+  launch_kukv(s, d, h->p, h->geo, h->q, h->Ku, h->Kv); }
   LAUNCH_CHECK("k_kukv");
   h->tridiagonal_solves += 1;
   h->coeff_gen += 1;  // Ku, Kv and 1/diag are new: the multigrid levels follow them
@@ -2014,7 +2013,7 @@ int hoc_stepper_tke_step(hoc_stepper* h, const double* e_in, const double* u, co
     launch_closure_lengths(d, h->p, h->geo, e_in, u, v, b, h->s_n2, h->s_sh, h->s_l, h->s_le, s);
   }
   { ProfScope _ps(h, "k_closure", s);
-  k_closure<<<blocks(d.n2), TPB, 0, s>>>(d, h->p, h->geo, e_in, h->Km, h->Kh, e_out, h->s_n2,
+  launch_closure(s, d, h->p, h->geo, e_in, h->Km, h->Kh, e_out, h->s_n2,
                                          h->s_sh, h->s_l, h->s_le, h->s_c); }
   LAUNCH_CHECK("k_closure");
   return HOC_OK;
@@ -2147,7 +2146,7 @@ static int step_impl(hoc_stepper* h, const hoc_state* in, hoc_state* out, void* 
   // phi, the transports of the state (theta, split_explicit) and, unless the
   // previous step formed it, w of the state: one column pass
   { ProfScope _ps(h, "k_prologue", s);
-  k_prologue<<<blocks(d.n2), TPB, 0, s>>>(d, p, geo, in->u, in->v, in->b, h->phi,
+  launch_prologue(s, d, p, geo, in->u, in->v, in->b, h->phi,
                                           (theta || split) ? h->U0 : nullptr, h->V0,
                                           w_ready ? nullptr : h->w); }
   if (tape)
@@ -2164,16 +2163,9 @@ static int step_impl(hoc_stepper* h, const hoc_state* in, hoc_state* out, void* 
     double* gu = tape ? tape->gh_u[it] : h->gh_u[it & 1];
     double* gv = tape ? tape->gh_v[it] : h->gh_v[it & 1];
     { ProfScope _ps(h, "k_predictor", s);
-    if (p.zcol)
-      k_predictor_col<<<blocks(d.n2), TPB, 0, s>>>(d, p, geo, in->u, in->v, in->eta, u_it, v_it,
-                                                   h->pgx, h->pgy, h->dzu, h->dzv, h->stu,
-                                                   h->stv, h->sub_m, h->den_m, h->cst_m, gu, gv,
-                                                   h->Ug, h->Vg);
-    else
-      k_predictor<<<blocks(d.n2), TPB, 0, s>>>(d, p, geo, in->u, in->v, in->eta, u_it, v_it,
-                                               h->pgx, h->pgy, h->dzu, h->dzv, h->stu, h->stv,
-                                               h->sub_m, h->den_m, h->cst_m, gu, gv, h->Ug,
-                                               h->Vg); }
+    launch_predictor(s, d, p, geo, in->u, in->v, in->eta, u_it, v_it, h->pgx, h->pgy, h->dzu,
+                     h->dzv, h->stu, h->stv, h->sub_m, h->den_m, h->cst_m, gu, gv, h->Ug,
+                     h->Vg); }
     LAUNCH_CHECK("k_predictor");
     h->tridiagonal_solves += 2;
     if (theta) {
@@ -2202,7 +2194,7 @@ static int step_impl(hoc_stepper* h, const hoc_state* in, hoc_state* out, void* 
         // the last pass: back-substitution and w of the new velocity in one
         // column pass (the tracers read w next)
         ProfScope _ps(h, "k_backsub_w", s);
-        k_backsub_w<<<blocks(d.n2), TPB, 0, s>>>(d, p, geo, gu, gv, h->q, out->eta, out->u,
+        launch_backsub_w(s, d, p, geo, gu, gv, h->q, out->eta, out->u,
                                                  out->v, h->w);
       } else {
         ProfScope _ps(h, "k_backsub", s);
@@ -2228,7 +2220,7 @@ static int step_impl(hoc_stepper* h, const hoc_state* in, hoc_state* out, void* 
   }
   if (!theta) {  // the theta scheme's last back-substitution formed w already
     ProfScope _ps(h, "k_w_diag", s);
-    k_w_diag<<<blocks(d.n2), TPB, 0, s>>>(d, p, geo, out->u, out->v, h->w);
+    launch_w_diag(s, d, p, geo, out->u, out->v, h->w);
   }
   { ProfScope _ps(h, "k_tracers", s);
   launch_tracers((h->fp32_parts & HOC_FP32_TRACER_FLUX) != 0, s, d, p, geo, in->T, in->S,
@@ -2546,7 +2538,7 @@ int hoc_stepper_w_diag(hoc_stepper* h, const double* u, const double* v, double*
                        void* stream) {
   if (!h || !u || !v || !w) return fail(HOC_ERR_INVALID, "null argument");
   const Dims d = h->d;
-  k_w_diag<<<blocks(d.n2), TPB, 0, (hipStream_t)stream>>>(d, h->p, h->geo, u, v, w);
+  launch_w_diag((hipStream_t)stream, d, h->p, h->geo, u, v, w);
   LAUNCH_CHECK("k_w_diag");
   return HOC_OK;
 }

@@ -169,6 +169,29 @@ struct FaceGeo {
   }
 };
 
+// The same east or north face of a static z-level geometry by its number of
+// wet levels: every level above the last wet one is the face rule of two full
+// cells, which is formed once.
+struct FaceCol {
+  int n;
+  double full, last;
+  __device__ __forceinline__ double dz(int k) const {
+    return k < n - 1 ? full : (k == n - 1 ? last : 0.0);
+  }
+  __device__ __forceinline__ bool wet(int k) const { return k < n; }
+};
+__device__ __forceinline__ FaceCol face_col(const Geo& geo, const StepParams& p, long long c0,
+                                            long long c1, int axis) {
+  const int a = geo.nw[c0], b = geo.nw[c1];
+  FaceCol f;
+  f.n = (axis == 0 ? geo.mu2[c0] : geo.mv2[c0]) ? (a < b ? a : b) : 0;
+  f.full = face_value(p.face_rule, p.dzr, p.dzr);
+  f.last = f.n > 0 ? face_value(p.face_rule, cg_dz(p.dzr, a, geo.hb[c0], f.n - 1),
+                                cg_dz(p.dzr, b, geo.hb[c1], f.n - 1))
+                   : 0.0;
+  return f;
+}
+
 // Tile of this workgroup in a 2D grid, remapped so that each of the 8 XCDs
 // (workgroups are dispatched to them round-robin by linear id) owns one
 // contiguous band of tile rows: neighbouring tiles then share their halo
@@ -201,6 +224,68 @@ __device__ __forceinline__ BlockTile xcd_block(int gx, int gy, int parts) {
   t.y = L % gy;
   t.z = L / gy;
   return t;
+}
+
+// Value of a plane at a byte offset. The plane's address is the same in every
+// lane and is kept in scalar registers, so that one vector register holds the
+// offset for every array (a plane is below 2^32 bytes). Without the empty asm
+// the compiler keeps a 64-bit vector address per array across the march, 30
+// registers in the momentum kernel.
+template <class T>
+__device__ __forceinline__ T at_byte(const T* plane, unsigned off) {
+  unsigned long long a = (unsigned long long)plane;
+  __asm__("" : "+s"(a));
+  using G = const __attribute__((address_space(1))) char;
+  return *(const __attribute__((address_space(1))) T*)((G*)a + off);
+}
+__device__ __forceinline__ void put_byte(double* plane, unsigned off, double v) {
+  unsigned long long a = (unsigned long long)plane;
+  __asm__("" : "+s"(a));
+  using G = __attribute__((address_space(1))) char;
+  *(__attribute__((address_space(1))) double*)((G*)a + off) = v;
+}
+
+// A column march whose operands are loaded W levels ahead: the loads of levels k + W .. k + 2W
+// are issued before levels k .. k + W are used, so a march waits for memory once per W levels
+// and not at every level. load(k) returns a level's operands, use(k, operands) advances the
+// recurrence. `load` may be called for a level again (the last one, in place of those beyond
+// it) and up to 2W levels before `use` reaches it: an array that `use` writes is read only at levels
+// that the march has yet to write.
+template <int W, class L, class U>
+__device__ __forceinline__ void march_down(int n, const L& load, const U& use) {
+  using V = decltype(load(0));
+  V A[W], B[W];
+  auto fill = [&](V* v, int kb) {
+#pragma unroll
+    for (int q = 0; q < W; ++q) v[q] = load(kb + q < n ? kb + q : n - 1);
+  };
+  fill(A, 0);
+  for (int kb = 0; kb < n; kb += W) {
+    if (kb + W < n) fill(B, kb + W);
+#pragma unroll
+    for (int q = 0; q < W; ++q) {
+      if (kb + q >= n) break;
+      use(kb + q, A[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < W; ++q) A[q] = B[q];
+  }
+}
+// The same from level n - 1 up to level 0.
+template <int W, class L, class U>
+__device__ __forceinline__ void march_up(int n, const L& load, const U& use) {
+  march_down<W>(
+      n, [&](int k) { return load(n - 1 - k); },
+      [&](int k, const decltype(load(0))& v) { use(n - 1 - k, v); });
+}
+
+// Linear workgroup id remapped so that each of the 8 XCDs (workgroups are dispatched to them
+// round-robin) owns one contiguous range: columns that share neighbour rows then meet in one
+// L2. A bijection for any number of workgroups.
+__device__ __forceinline__ unsigned xcd_linear() {
+  const unsigned nb = gridDim.x, id = blockIdx.x;
+  const unsigned x = id % 8, q = nb / 8, r = nb % 8;
+  return x * q + (x < r ? x : r) + id / 8;
 }
 
 // Half the Superbee limiter, phi(r) / 2 = max(0, max(min(r, 1/2), min(r / 2, 1))), with

@@ -42,9 +42,10 @@ struct PcgScalars {
 __global__ void k_geometry(Dims d, StepParams p, const double* dz3, const uint8_t* m3u,
                            const uint8_t* m3v, const double* tau_x, const double* tau_y,
                            double* dzi, double* tau_u, double* tau_v);
-__global__ void k_closure(Dims d, StepParams p, Geo geo, const double* e_in, double* Km,
-                          double* Kh, double* e_out, const double* s_n2, const double* s_sh,
-                          const double* s_l, const double* s_le, double* s_c);
+void launch_closure(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                    const double* e_in, double* Km, double* Kh, double* e_out,
+                    const double* s_n2, const double* s_sh, const double* s_l,
+                    const double* s_le, double* s_c);
 __global__ void k_closure_shear(Dims d, StepParams p, Geo geo, const double* u, const double* v,
                                 const double* b, double* s_n2, double* s_sh);
 __global__ void k_mixing_recursive(Dims d, StepParams p, Geo geo, const double* e_in,
@@ -56,15 +57,18 @@ void launch_closure_lengths(const Dims& d, const StepParams& p, const Geo& geo,
 // Sets the LDS limit of the integral-length kernel for nz levels; < 0 if
 // its staging does not fit one workgroup's LDS.
 int closure_lengths_prepare(int nz);
-__global__ void k_coefficients(Dims d, StepParams p, Geo geo, const double* Km,
-                               double* sub_m, double* den_m, double* cst_m, double* q);
-__global__ void k_kukv(Dims d, StepParams p, Geo geo, const double* q, double* Ku, double* Kv);
+void launch_coefficients(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                         const double* Km, double* sub_m, double* den_m, double* cst_m,
+                         double* q);
+void launch_kukv(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                 const double* q, double* Ku, double* Kv);
 __global__ void k_phi(Dims d, StepParams p, Geo geo, const double* b, double* phi);
-// k_phi, k_depth_sum (U0 set) and k_w_diag (w set) in one column pass
-__global__ void k_prologue(Dims d, StepParams p, Geo geo, const double* u, const double* v,
-                           const double* b, double* phi, double* U0, double* V0, double* w);
-__global__ void k_w_diag(Dims d, StepParams p, Geo geo, const double* u, const double* v,
-                         double* w);
+// phi, the transports (U0 set) and w (w set) of a state in one launch
+void launch_prologue(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                     const double* u, const double* v, const double* b, double* phi, double* U0,
+                     double* V0, double* w);
+void launch_w_diag(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                   const double* u, const double* v, double* w);
 __global__ void k_momentum_explicit(Dims d, StepParams p, Geo geo, const double* u,
                                     const double* v, const double* b, const double* phi,
                                     const double* w, const double* Km, double* pgx,
@@ -98,22 +102,15 @@ __global__ void k_split_final(Dims d, Geo geo, const double* gh_u, const double*
                               const double* V, const double* Hu, const double* Hv, double* u,
                               double* v);
 __global__ void k_face_depth(Dims d, Geo geo, double* Hu, double* Hv);
-__global__ void k_predictor(Dims d, StepParams p, Geo geo, const double* u, const double* v,
-                            const double* eta, const double* u_it, const double* v_it,
-                            const double* pgx, const double* pgy, const double* dzu,
-                            const double* dzv, const double* stu, const double* stv,
-                            const double* sub,
-                            const double* den, const double* cst, double* gh_u, double* gh_v,
-                            double* Ug, double* Vg);
-__global__ void k_predictor_col(Dims d, StepParams p, Geo geo, const double* u, const double* v,
-                                const double* eta, const double* u_it, const double* v_it,
-                                const double* pgx, const double* pgy, const double* dzu,
-                                const double* dzv, const double* stu, const double* stv,
-                                const double* sub, const double* den, const double* cst,
-                                double* gh_u, double* gh_v, double* Ug, double* Vg);
-__global__ void k_backsub_w(Dims d, StepParams p, Geo geo, const double* gh_u,
-                            const double* gh_v, const double* q, const double* eta_n, double* u,
-                            double* v, double* w);
+void launch_predictor(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                      const double* u, const double* v, const double* eta, const double* u_it,
+                      const double* v_it, const double* pgx, const double* pgy,
+                      const double* dzu, const double* dzv, const double* stu,
+                      const double* stv, const double* sub, const double* den,
+                      const double* cst, double* gh_u, double* gh_v, double* Ug, double* Vg);
+void launch_backsub_w(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                      const double* gh_u, const double* gh_v, const double* q,
+                      const double* eta_n, double* u, double* v, double* w);
 __global__ void k_backsub(Dims d, StepParams p, Geo geo, const double* gh_u,
                           const double* gh_v, const double* q, const double* eta_n,
                           double* u_it, double* v_it);

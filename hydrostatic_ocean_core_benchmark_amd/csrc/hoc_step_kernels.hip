@@ -3,18 +3,43 @@
 //
 // Two launch shapes:
 //   column kernels: one lane per (j, i) column, marching k; lanes are
-//     consecutive in i, so every level's load is one coalesced row segment.
+//     consecutive in i, so every level's load is one coalesced row segment,
+//     issued a few levels before it is used (march_down, march_up).
 //     Used where the work is a recurrence in k (tridiagonal sweeps, prefix
 //     sums, the TKE mixing-length march) and the horizontal stencil at each
 //     level is fused into the same pass.
 //   cell kernels: one lane per (k, j, i) for the pure 3D stencils.
 //
-// Column recurrences keep their forward-sweep values (c*, d*) in global
-// scratch rather than registers so that any nz runs through the same code.
+// Column recurrences keep their forward-sweep values (c*, d*) in LDS where the
+// column fits (COL_LDS_MAX), in global scratch for deeper ones.
+#include <type_traits>
+
 #include "hoc_device.h"
 #include "hoc_kernels.h"
 
 namespace hoc {
+
+// Columns of a column kernel's workgroup: one wave, so that a grid of few
+// columns spreads over as many compute units as it can.
+constexpr int COLS = 64;
+// Sweeps keep a column in LDS up to here (two or more workgroups per compute
+// unit); deeper columns use the global work arrays.
+constexpr size_t COL_LDS_MAX = 64 * 1024;
+static unsigned column_blocks(const Dims& d) { return (unsigned)((d.n2 + COLS - 1) / COLS); }
+
+// go(zc, stage) with the two flags as compile-time constants.
+template <class Go>
+static void with_column_form(bool zcol, bool stage, const Go& go) {
+  using T = std::true_type;
+  using F = std::false_type;
+  if (zcol) {
+    if (stage) go(T{}, T{});
+    else go(T{}, F{});
+  } else {
+    if (stage) go(F{}, T{});
+    else go(F{}, F{});
+  }
+}
 
 // ------------------------------------------------------------ geometry
 // Interface thickness of dz3 (libs/core/vertical_var.py:21-32) and the
@@ -308,167 +333,336 @@ __global__ void k_mixing_recursive(Dims d, StepParams p, Geo geo, const double* 
 }
 
 // The interface tridiagonal for e and the eddy coefficients, one lane per
-// column, from s_n2, s_sh, s_l = l_k and s_le = l_eps.
-__global__ void k_closure(Dims d, StepParams p, Geo geo, const double* __restrict__ e_in,
-                          double* __restrict__ Km, double* __restrict__ Kh,
-                          double* __restrict__ e_out, const double* __restrict__ s_n2,
-                          const double* __restrict__ s_sh, const double* __restrict__ s_l,
-                          const double* __restrict__ s_le, double* __restrict__ s_c) {
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+// column, from s_n2, s_sh, s_l = l_k and s_le = l_eps. ZC: thicknesses and wet
+// flags from the column form. STAGE: c* and d* stay in LDS between the sweeps
+// instead of in s_c and e_out.
+// Bound: latency of the march on small grids, then memory (10 fields) and the
+// roots and divisions at the few waves that LDS leaves. Per launch, against no
+// loads ahead and c*, d* in memory: 128 x 4 x 20 33 -> 18 us, 128 x 128 x 30
+// 51 -> 26, 512 x 512 x 40 212 -> 214, 640 x 512 x 48 326 -> 289, 1000 x 1000
+// x 30 676 -> 495.
+template <bool ZC, bool STAGE>
+__global__ __launch_bounds__(COLS) void k_closure(
+    Dims d, StepParams p, Geo geo, const double* __restrict__ e_in, double* __restrict__ Km,
+    double* __restrict__ Kh, double* __restrict__ e_out, const double* __restrict__ s_n2,
+    const double* __restrict__ s_sh, const double* __restrict__ s_l,
+    const double* __restrict__ s_le, double* __restrict__ s_c) {
+  extern __shared__ double clo_lds[];  // STAGE: [2][nz + 1][COLS], a thread's own column
+  const long long c = (long long)xcd_linear() * COLS + threadIdx.x;
   if (c >= d.n2) return;
   const int nz = d.nz;
   const long long n2 = d.n2;
-  const ColumnGeo cg(geo, p, d, c);
+  const unsigned bc = 8u * (unsigned)c;
   const double kb = geo.kappa_b[c];
   const double dt = p.dt;
-  double c_prev = 0.0, d_prev = 0.0;
-  double rhs0 = 0.0;
-  // K_m at interfaces k-1, k, k+1 and the wet flag of the cell above
-  // interface k, carried down the column
-  double km_up = 0.0, km_0 = Km[c], km_dn = nz >= 1 ? Km[n2 + c] : 0.0;
-  bool wet_above = false;
-  for (int k = 0; k <= nz; ++k) {
-    const bool wet_below = k < nz && cg.wet(k);
-    const double wet = (k >= 1 && k < nz) ? (wet_above ? 1.0 : 0.0) * (wet_below ? 1.0 : 0.0)
-                                          : 0.0;
-    const double ek = e_in[k * n2 + c];
-    const double n2k = s_n2[k * n2 + c];
-    const double l_eps = s_le[k * n2 + c];
-    const double kmo = km_0;
-    const double kho = Kh[k * n2 + c];
-    const double prod = (kmo - p.nu_b) * s_sh[k * n2 + c] - (kho - kb) * n2k;
-    const double diss = p.c_eps * sqrt(nmax(ek, p.e_min)) / l_eps;
-    double a_up = 0.0, a_dn = 0.0;
-    if (k >= 1 && k < nz) {
-      const double idzi = safe_inv(cg.dzi(k));
-      const double klay_up = 0.5 * (km_up + kmo);
-      const double klay_dn = 0.5 * (kmo + km_dn);
-      a_up = dt * klay_up * safe_inv(cg.dz(k - 1)) * idzi;
-      a_dn = dt * klay_dn * safe_inv(cg.dz(k)) * idzi;
-    }
-    double sub = -a_up, sup = -a_dn;
-    double diag = 1.0 + a_up + a_dn + dt * diss;
-    double rhs = ek + dt * prod;
-    if (wet <= 0.0) {
-      diag = 1.0;
-      sub = 0.0;
-      sup = 0.0;
-      rhs = p.e_min;
-    }
-    if (k == 0) {
-      rhs = wet_below ? p.e_bb * geo.ustar2[c] : p.e_min;
-      rhs0 = rhs;
-    }
-    double cst, dst;
-    if (k == 0) {
-      cst = sup / diag;
-      dst = rhs / diag;
-    } else {
-      const double den = diag - sub * c_prev;
-      cst = sup / den;
-      dst = (rhs - sub * d_prev) / den;
-    }
-    s_c[k * n2 + c] = cst;
-    e_out[k * n2 + c] = dst;
-    c_prev = cst;
-    d_prev = dst;
-    km_up = km_0;
-    km_0 = km_dn;
-    km_dn = k + 2 <= nz ? Km[(k + 2) * n2 + c] : 0.0;
-    wet_above = wet_below;
+  double* lc = clo_lds + threadIdx.x;
+  double* ld = lc + (size_t)(nz + 1) * COLS;
+  int nwc = 0;
+  InvCol ic{};
+  if constexpr (ZC) {
+    nwc = geo.nw[c];
+    ic = inv_col(nwc, p.dzr, nwc > 0 ? geo.hb[c] : 0.0);
   }
+  auto wet_at = [&](int k, uint8_t m) { return k >= 0 && k < nz && (ZC ? k < nwc : m != 0); };
+  struct Level {
+    double e, n2, sh, le, kh, km, dzi, dz;
+    uint8_t m;
+  };
+  double c_prev = 0.0, d_prev = 0.0, rhs0 = 0.0;
+  // K_m at interfaces k - 1 and k, the inverse thickness and the wet flag of
+  // the cell above interface k, carried down the column
+  double km_up = 0.0, km_0 = Km[c], inv_up = 0.0;
+  bool wet_above = false;
+  march_down<4>(
+      nz + 1,
+      [&](int k) {
+        const long long o = k * n2;
+        Level L;
+        L.e = at_byte(e_in + o, bc);
+        L.n2 = at_byte(s_n2 + o, bc);
+        L.sh = at_byte(s_sh + o, bc);
+        L.le = at_byte(s_le + o, bc);
+        L.kh = at_byte(Kh + o, bc);
+        L.km = at_byte(Km + (k < nz ? o + n2 : o), bc);
+        if constexpr (!ZC) {
+          const long long oc = k < nz ? o : o - n2;
+          L.dzi = at_byte(geo.dzi + o, bc);
+          L.dz = at_byte(geo.dz3 + oc, bc);
+          L.m = at_byte(geo.m3 + oc, (unsigned)c);
+        }
+        return L;
+      },
+      [&](int k, const Level& L) {
+        const bool wet_below = wet_at(k, L.m);
+        const double wet = wet_above && wet_below ? 1.0 : 0.0;
+        const double kmo = km_0, km_dn = L.km;
+        const double prod = (kmo - p.nu_b) * L.sh - (L.kh - kb) * L.n2;
+        const double diss = p.c_eps * sqrt(nmax(L.e, p.e_min)) / L.le;
+        const double inv_dn = ZC ? ic.inv(k) : safe_inv(L.dz);
+        double a_up = 0.0, a_dn = 0.0;
+        if (k >= 1 && k < nz) {
+          const double idzi = ZC ? ic.idzi(k) : safe_inv(L.dzi);
+          const double klay_up = 0.5 * (km_up + kmo);
+          const double klay_dn = 0.5 * (kmo + km_dn);
+          a_up = dt * klay_up * inv_up * idzi;
+          a_dn = dt * klay_dn * inv_dn * idzi;
+        }
+        double sub = -a_up, sup = -a_dn;
+        double diag = 1.0 + a_up + a_dn + dt * diss;
+        double rhs = L.e + dt * prod;
+        if (wet <= 0.0) {
+          diag = 1.0;
+          sub = 0.0;
+          sup = 0.0;
+          rhs = p.e_min;
+        }
+        if (k == 0) {
+          rhs = wet_below ? p.e_bb * geo.ustar2[c] : p.e_min;
+          rhs0 = rhs;
+        }
+        const Divisor<double> by_den(k == 0 ? diag : diag - sub * c_prev);
+        const double cst = by_den(sup);
+        const double dst = k == 0 ? by_den(rhs) : by_den(rhs - sub * d_prev);
+        if constexpr (STAGE) {
+          lc[k * COLS] = cst;
+          ld[k * COLS] = dst;
+        } else {
+          put_byte(s_c + k * n2, bc, cst);
+          put_byte(e_out + k * n2, bc, dst);
+        }
+        c_prev = cst;
+        d_prev = dst;
+        km_up = km_0;
+        km_0 = km_dn;
+        inv_up = inv_dn;
+        wet_above = wet_below;
+      });
 
   // back-substitution, floors, eddy coefficients
+  struct Back {
+    double cst, dst, l;
+    uint8_t m;
+  };
+  const Divisor<double> by_pr = uniform_divisor<double>(p.pr_t);
   double x_next = 0.0;
   bool wet_below = false;  // cell k (below interface k)
-  for (int k = nz; k >= 0; --k) {
-    const bool wet_above = k >= 1 && cg.wet(k - 1);
-    const double dst = e_out[k * n2 + c];
-    const double x = (k == nz) ? dst : dst - s_c[k * n2 + c] * x_next;
-    x_next = x;
-    const double wet = (k >= 1 && k < nz) ? (wet_above ? 1.0 : 0.0) * (wet_below ? 1.0 : 0.0)
-                                          : 0.0;
-    double en = nmax(x, p.e_min);
-    en = wet > 0.0 ? en : p.e_min;
-    if (k == 0) en = rhs0;
-    const double km = p.c_k * s_l[k * n2 + c] * sqrt(en) * wet + p.nu_b;
-    const double kh = (km - p.nu_b) / p.pr_t + kb;
-    e_out[k * n2 + c] = en;
-    Km[k * n2 + c] = km;
-    Kh[k * n2 + c] = kh;
-    wet_below = wet_above;
-  }
+  march_up<4>(
+      nz + 1,
+      [&](int k) {
+        const long long o = k * n2;
+        Back B;
+        if constexpr (STAGE) {
+          B.cst = lc[k * COLS];
+          B.dst = ld[k * COLS];
+        } else {
+          B.cst = at_byte(s_c + o, bc);
+          B.dst = at_byte(e_out + o, bc);
+        }
+        B.l = at_byte(s_l + o, bc);
+        if constexpr (!ZC) B.m = at_byte(geo.m3 + (k > 0 ? o - n2 : o), (unsigned)c);
+        return B;
+      },
+      [&](int k, const Back& B) {
+        const bool wet_above = wet_at(k - 1, B.m);
+        const double x = (k == nz) ? B.dst : B.dst - B.cst * x_next;
+        x_next = x;
+        const double wet = wet_above && wet_below ? 1.0 : 0.0;
+        double en = nmax(x, p.e_min);
+        en = wet > 0.0 ? en : p.e_min;
+        if (k == 0) en = rhs0;
+        const double km = p.c_k * B.l * sqrt(en) * wet + p.nu_b;
+        const double kh = by_pr(km - p.nu_b) + kb;
+        put_byte(e_out + k * n2, bc, en);
+        put_byte(Km + k * n2, bc, km);
+        put_byte(Kh + k * n2, bc, kh);
+        wet_below = wet_above;
+      });
+}
+
+void launch_closure(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                    const double* e_in, double* Km, double* Kh, double* e_out,
+                    const double* s_n2, const double* s_sh, const double* s_l,
+                    const double* s_le, double* s_c) {
+  const size_t lds = (size_t)2 * (d.nz + 1) * COLS * sizeof(double);
+  with_column_form(p.zcol != 0, lds <= COL_LDS_MAX, [&](auto zc, auto sg) {
+    constexpr bool SG = decltype(sg)::value;
+    k_closure<decltype(zc)::value, SG><<<column_blocks(d), COLS, SG ? lds : 0, s>>>(
+        d, p, geo, e_in, Km, Kh, e_out, s_n2, s_sh, s_l, s_le, s_c);
+  });
 }
 
 // ------------------------------------------------ vertical coefficients
 // tri_m (viscosity Km, bottom drag), factored, then q = A_m^-1 1
 // (libs/core/model3d_v05.py:141-153); tri_b is factored by the tracer
-// kernels from the K_h they read anyway.
-__global__ void k_coefficients(Dims d, StepParams p, Geo geo, const double* __restrict__ Km,
-                               double* __restrict__ sub_m, double* __restrict__ den_m,
-                               double* __restrict__ cst_m, double* __restrict__ q) {
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+// kernels from the K_h they read anyway. The factorization and the forward
+// sweep of q are one pass over the column; STAGE: c* and d* are kept in LDS
+// for the back-substitution. Memory-bound on large grids (5 fields instead of
+// 8), latency-bound on small ones: 128 x 128 x 30 29 -> 16 us, 512 x 512 x 40
+// 126 -> 93, 1000 x 1000 x 30 350 -> 243.
+template <bool ZC, bool STAGE>
+__global__ __launch_bounds__(COLS) void k_coefficients(
+    Dims d, StepParams p, Geo geo, const double* __restrict__ Km, double* __restrict__ sub_m,
+    double* __restrict__ den_m, double* __restrict__ cst_m, double* __restrict__ q) {
+  extern __shared__ double coe_lds[];  // STAGE: [2][nz][COLS], a thread's own column
+  const long long c = (long long)xcd_linear() * COLS + threadIdx.x;
   if (c >= d.n2) return;
   const int nz = d.nz;
   const long long n2 = d.n2;
-  // the factorization and the forward sweep of q in one pass over the
-  // column, so the geometry is read once and tri_m is not read back
-  const ColumnGeo cg(geo, p, d, c);
-  double cm_prev = 0.0, d_prev = 0.0;
-  double idzi_t = safe_inv(cg.dzi(0));
-  double km_t = Km[c];
-  bool wet = cg.wet(0);
-  for (int k = 0; k < nz; ++k) {
-    const long long o = k * n2 + c;
-    const double inv_dz = safe_inv(cg.dz(k));
-    const double idzi_b = safe_inv(cg.dzi(k + 1));
-    const double km_b = Km[o + n2];
-    const bool below = (k + 1 < nz) && cg.wet(k + 1);
-    double sm, dm, cm;
-    factor_row(p, k, inv_dz, km_t, km_b, idzi_t, idzi_b, wet, below, p.thv_dt_drag, cm_prev,
-               sm, dm, cm);
-    sub_m[o] = sm;
-    den_m[o] = dm;
-    cst_m[o] = cm;
-    const double dst = (k == 0) ? 1.0 / dm : (1.0 - sm * d_prev) / dm;
-    q[o] = dst;
-    d_prev = dst;
-    cm_prev = cm;
-    idzi_t = idzi_b;
-    km_t = km_b;
-    wet = below;
+  const unsigned bc = 8u * (unsigned)c;
+  double* lc = coe_lds + threadIdx.x;
+  double* ld = lc + (size_t)nz * COLS;
+  InvCol ic{};
+  int nwc = 0;
+  double idzi_t;
+  bool wet;
+  if constexpr (ZC) {
+    nwc = geo.nw[c];
+    ic = inv_col(nwc, p.dzr, nwc > 0 ? geo.hb[c] : 0.0);
+    idzi_t = ic.inv(0);
+    wet = nwc > 0;
+  } else {
+    idzi_t = safe_inv(geo.dzi[c]);
+    wet = geo.m3[c] != 0;
   }
-  double x_next = q[(nz - 1) * n2 + c];
-  for (int k = nz - 2; k >= 0; --k) {
-    const long long o = k * n2 + c;
-    const double x = q[o] - cst_m[o] * x_next;
-    q[o] = x;
-    x_next = x;
-  }
+  struct Level {
+    double km, dz, dzi;
+    uint8_t m;
+  };
+  double cm_prev = 0.0, d_prev = 0.0, km_t = Km[c];
+  march_down<8>(
+      nz,
+      [&](int k) {
+        const long long o = k * n2;
+        Level L;
+        L.km = at_byte(Km + o + n2, bc);
+        if constexpr (!ZC) {
+          L.dz = at_byte(geo.dz3 + o, bc);
+          L.dzi = at_byte(geo.dzi + o + n2, bc);
+          L.m = at_byte(geo.m3 + (k + 1 < nz ? o + n2 : o), (unsigned)c);
+        }
+        return L;
+      },
+      [&](int k, const Level& L) {
+        const long long o = k * n2;
+        double inv_dz, idzi_b;
+        bool below = k + 1 < nz;
+        if constexpr (ZC) {
+          inv_dz = ic.inv(k);
+          idzi_b = k + 1 == nz ? inv_dz : ic.idzi(k + 1);
+          below = below && k + 1 < nwc;
+        } else {
+          inv_dz = safe_inv(L.dz);
+          idzi_b = safe_inv(L.dzi);
+          below = below && L.m != 0;
+        }
+        double sub, sup, den;
+        matrix_row(p, k, inv_dz, km_t, L.km, idzi_t, idzi_b, wet, below, p.thv_dt_drag, cm_prev,
+                   sub, sup, den);
+        const Divisor<double> by_den(den);
+        const double cm = by_den(sup);
+        const double dst = k == 0 ? by_den(1.0) : by_den(1.0 - sub * d_prev);
+        put_byte(sub_m + o, bc, sub);
+        put_byte(den_m + o, bc, den);
+        put_byte(cst_m + o, bc, cm);
+        if constexpr (STAGE) {
+          lc[k * COLS] = cm;
+          ld[k * COLS] = dst;
+        } else {
+          put_byte(q + o, bc, dst);
+        }
+        d_prev = dst;
+        cm_prev = cm;
+        idzi_t = idzi_b;
+        km_t = L.km;
+        wet = below;
+      });
+  struct Back {
+    double cm, dst;
+  };
+  double x = 0.0;
+  march_up<8>(
+      nz,
+      [&](int k) {
+        const long long o = k * n2;
+        Back B;
+        if constexpr (STAGE) {
+          B.cm = lc[k * COLS];
+          B.dst = ld[k * COLS];
+        } else {
+          B.cm = at_byte(cst_m + o, bc);
+          B.dst = at_byte(q + o, bc);
+        }
+        return B;
+      },
+      [&](int k, const Back& B) {
+        x = k == nz - 1 ? B.dst : B.dst - B.cm * x;
+        put_byte(q + k * n2, bc, x);
+      });
+}
+
+void launch_coefficients(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                         const double* Km, double* sub_m, double* den_m, double* cst_m,
+                         double* q) {
+  const size_t lds = (size_t)2 * d.nz * COLS * sizeof(double);
+  with_column_form(p.zcol != 0, lds <= COL_LDS_MAX, [&](auto zc, auto sg) {
+    constexpr bool SG = decltype(sg)::value;
+    k_coefficients<decltype(zc)::value, SG><<<column_blocks(d), COLS, SG ? lds : 0, s>>>(
+        d, p, geo, Km, sub_m, den_m, cst_m, q);
+  });
 }
 
 // Helmholtz face coefficients Ku = sum_k dz3u min(q, q_east) mask_u and Kv
 // (libs/core/model3d_v05.py:154-157), summed in k order like NumPy's
-// axis-0 reduction.
-__global__ void k_kukv(Dims d, StepParams p, Geo geo, const double* __restrict__ q,
-                       double* __restrict__ Ku, double* __restrict__ Kv) {
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+// axis-0 reduction. 128 x 128 x 30 24 -> 10 us, 512 x 512 x 40 39 -> 35.
+template <bool ZC>
+__global__ __launch_bounds__(COLS) void k_kukv(Dims d, StepParams p, Geo geo,
+                                               const double* __restrict__ q,
+                                               double* __restrict__ Ku,
+                                               double* __restrict__ Kv) {
+  const long long c = (long long)xcd_linear() * COLS + threadIdx.x;
   if (c >= d.n2) return;
-  const int i = (int)(c % d.nx), j = (int)(c / d.nx);
+  const int j = (int)((unsigned)c / (unsigned)d.nx), i = (int)((unsigned)c - (unsigned)j * d.nx);
   const long long ce = at2(d, j, wrap(i, 1, d.nx));
   const long long cn = at2(d, wrap(j, 1, d.ny), i);
   const long long n2 = d.n2;
-  const FaceGeo fu(geo, p, d, c, ce, 0), fv(geo, p, d, c, cn, 1);
-  double su = 0.0, sv = 0.0;
-  for (int k = 0; k < d.nz; ++k) {
-    const double qc = q[k * n2 + c];
-    const double tu = fu.dz(k) * nmin(qc, q[k * n2 + ce]);
-    const double tv = fv.dz(k) * nmin(qc, q[k * n2 + cn]);
-    su = (k == 0) ? tu : su + tu;
-    sv = (k == 0) ? tv : sv + tv;
+  const unsigned bc = 8u * (unsigned)c, be = 8u * (unsigned)ce, bn = 8u * (unsigned)cn;
+  FaceCol fu{}, fv{};
+  if constexpr (ZC) {
+    fu = face_col(geo, p, c, ce, 0);
+    fv = face_col(geo, p, c, cn, 1);
   }
+  struct Level {
+    double c, e, n, du, dv;
+  };
+  double su = 0.0, sv = 0.0;
+  march_down<3>(
+      d.nz,
+      [&](int k) {
+        const long long o = k * n2;
+        Level L;
+        L.c = at_byte(q + o, bc);
+        L.e = at_byte(q + o, be);
+        L.n = at_byte(q + o, bn);
+        if constexpr (!ZC) {
+          L.du = at_byte(geo.dz3u + o, bc);
+          L.dv = at_byte(geo.dz3v + o, bc);
+        }
+        return L;
+      },
+      [&](int k, const Level& L) {
+        const double tu = (ZC ? fu.dz(k) : L.du) * nmin(L.c, L.e);
+        const double tv = (ZC ? fv.dz(k) : L.dv) * nmin(L.c, L.n);
+        su = (k == 0) ? tu : su + tu;
+        sv = (k == 0) ? tv : sv + tv;
+      });
   Ku[c] = su * mk(geo.mu2[c]);
   Kv[c] = sv * mk(geo.mv2[c]);
+}
+
+void launch_kukv(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                 const double* q, double* Ku, double* Kv) {
+  if (p.zcol) k_kukv<true><<<column_blocks(d), COLS, 0, s>>>(d, p, geo, q, Ku, Kv);
+  else k_kukv<false><<<column_blocks(d), COLS, 0, s>>>(d, p, geo, q, Ku, Kv);
 }
 
 // --------------------------------------------------- pressure potential
@@ -501,98 +695,203 @@ __global__ void k_phi(Dims d, StepParams p, Geo geo, const double* __restrict__ 
   }
 }
 
-// ------------------------------------------------- vertical velocity
+// ------------------------------------- transports and vertical velocity
+// Of one column: the transports U0 = sum dz3u u, V0 = sum dz3v v (TR) and
 // w_k = -sum_{k'>=k} div(dz3u u, dz3v v), w_nz = 0, summed from the bottom
-// (libs/core/vertical_var.py:109-121 with model3d_v05.py:232-235).
-__global__ void k_w_diag(Dims d, StepParams p, Geo geo, const double* __restrict__ u,
-                         const double* __restrict__ v, double* __restrict__ w) {
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= d.n2) return;
-  const int i = (int)(c % d.nx), j = (int)(c / d.nx);
-  const long long cw = at2(d, j, wrap(i, -1, d.nx));
-  const long long cs = at2(d, wrap(j, -1, d.ny), i);
-  const long long n2 = d.n2;
-  const int nz = d.nz;
-  const ColumnGeo cg(geo, p, d, c);
-  const FaceGeo fe(geo, p, d, c, at2(d, j, wrap(i, 1, d.nx)), 0), fw(geo, p, d, cw, c, 0);
-  const FaceGeo fn(geo, p, d, c, at2(d, wrap(j, 1, d.ny), i), 1), fs(geo, p, d, cs, c, 1);
-  double s = 0.0;
-  for (int k = nz - 1; k >= 0; --k) {
-    const long long o = k * n2;
-    const double U = fe.dz(k) * u[o + c];
-    const double Uw = fw.dz(k) * u[o + cw];
-    const double V = fn.dz(k) * v[o + c];
-    const double Vs = fs.dz(k) * v[o + cs];
-    const double dv = (cg.wet(k) ? 1.0 : 0.0) * ((U - Uw) / p.dx + (V - Vs) / p.dy);
-    s = (k == nz - 1) ? dv : s + dv;
-    w[o + c] = -s;
-  }
-  w[(long long)nz * n2 + c] = 0.0;
-}
-
-// ------------------------------------------------- the step's prologue
-// k_phi, k_depth_sum and k_w_diag of one column in one pass over it (the
-// same operations in the same order, so the same bits): the top-down march
-// forms phi from b and the transports U0 = sum dz3u u, V0 = sum dz3v v
-// (when U0 is set), then the bottom-up march forms w (when w is set) from u
-// and the west u, v and the south v, the column's own velocities in cache.
-__global__ void k_prologue(Dims d, StepParams p, Geo geo, const double* __restrict__ u,
-                           const double* __restrict__ v, const double* __restrict__ b,
-                           double* __restrict__ phi, double* __restrict__ U0,
-                           double* __restrict__ V0, double* __restrict__ w) {
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= d.n2) return;
-  const long long n2 = d.n2;
-  const int nz = d.nz;
-  const int i = (int)(c % d.nx), j = (int)(c / d.nx);
+// (libs/core/vertical_var.py:109-121 with model3d_v05.py:232-235) (WW), in one
+// march down that reads u and v once: the divergences wait in LDS (STAGE: a
+// thread's own [nz] values, COLS apart) or in w for the sum upwards.
+template <bool ZC, bool STAGE, bool TR, bool WW>
+__device__ __forceinline__ void transports_column(const Dims& d, const StepParams& p,
+                                                  const Geo& geo, const double* __restrict__ u,
+                                                  const double* __restrict__ v,
+                                                  double* __restrict__ U0,
+                                                  double* __restrict__ V0,
+                                                  double* __restrict__ w, double* lds,
+                                                  long long c) {
+  const int j = (int)((unsigned)c / (unsigned)d.nx), i = (int)((unsigned)c - (unsigned)j * d.nx);
   const long long ce = at2(d, j, wrap(i, 1, d.nx)), cn = at2(d, wrap(j, 1, d.ny), i);
-  const ColumnGeo cg(geo, p, d, c);
-  const FaceGeo fe(geo, p, d, c, ce, 0), fn(geo, p, d, c, cn, 1);
-  double above = 0.0, su = 0.0, sv = 0.0;
-  for (int k = 0; k < nz; ++k) {
-    const long long t = k * n2 + c;
-    const double dz = cg.dz(k);
-    const double bk = b[t];
-    phi[t] = 0.5 * dz * bk + above;
-    const double tb = dz * bk;
-    above = (k == 0) ? tb : above + tb;
-    if (U0) {
-      const double tu = fe.dz(k) * u[t];
-      const double tv = fn.dz(k) * v[t];
-      su = (k == 0) ? tu : su + tu;
-      sv = (k == 0) ? tv : sv + tv;
+  const long long cw = at2(d, j, wrap(i, -1, d.nx)), cs = at2(d, wrap(j, -1, d.ny), i);
+  const unsigned bc = 8u * (unsigned)c, bw = 8u * (unsigned)cw, bs = 8u * (unsigned)cs;
+  const long long n2 = d.n2;
+  const int nz = d.nz;
+  FaceCol fe{}, fw{}, fn{}, fs{};
+  int nwc = 0;
+  if constexpr (ZC) {
+    fe = face_col(geo, p, c, ce, 0);
+    fn = face_col(geo, p, c, cn, 1);
+    if constexpr (WW) {
+      nwc = geo.nw[c];
+      fw = face_col(geo, p, cw, c, 0);
+      fs = face_col(geo, p, cs, c, 1);
     }
   }
-  if (U0) {
+  const Divisor<double> by_dx = uniform_divisor<double>(p.dx), by_dy = uniform_divisor<double>(p.dy);
+  struct Level {
+    double u, uw, v, vs, de, dw, dn, ds;
+    uint8_t m;
+  };
+  double su = 0.0, sv = 0.0;
+  march_down<ZC ? 4 : 3>(
+      nz,
+      [&](int k) {
+        const long long o = k * n2;
+        Level L;
+        L.u = at_byte(u + o, bc);
+        L.v = at_byte(v + o, bc);
+        if constexpr (WW) {
+          L.uw = at_byte(u + o, bw);
+          L.vs = at_byte(v + o, bs);
+        }
+        if constexpr (!ZC) {
+          L.de = at_byte(geo.dz3u + o, bc);
+          L.dn = at_byte(geo.dz3v + o, bc);
+          if constexpr (WW) {
+            L.dw = at_byte(geo.dz3u + o, bw);
+            L.ds = at_byte(geo.dz3v + o, bs);
+            L.m = at_byte(geo.m3 + o, (unsigned)c);
+          }
+        }
+        return L;
+      },
+      [&](int k, const Level& L) {
+        const double U = (ZC ? fe.dz(k) : L.de) * L.u;
+        const double V = (ZC ? fn.dz(k) : L.dn) * L.v;
+        if constexpr (TR) {
+          su = (k == 0) ? U : su + U;
+          sv = (k == 0) ? V : sv + V;
+        }
+        if constexpr (WW) {
+          const double Uw = (ZC ? fw.dz(k) : L.dw) * L.uw;
+          const double Vs = (ZC ? fs.dz(k) : L.ds) * L.vs;
+          const double wet = (ZC ? k < nwc : L.m != 0) ? 1.0 : 0.0;
+          const double dv = wet * (by_dx(U - Uw) + by_dy(V - Vs));
+          if constexpr (STAGE) lds[k * COLS] = dv;
+          else put_byte(w + k * n2, bc, dv);
+        }
+      });
+  if constexpr (TR) {
     U0[c] = su;
     V0[c] = sv;
   }
+  if constexpr (WW) {
+    double s = 0.0;
+    march_up<8>(
+        nz,
+        [&](int k) {
+          if constexpr (STAGE) return lds[k * COLS];
+          else return at_byte(w + k * n2, bc);
+        },
+        [&](int k, double dv) {
+          s = (k == nz - 1) ? dv : s + dv;
+          put_byte(w + k * n2, bc, -s);
+        });
+    w[(long long)nz * n2 + c] = 0.0;
+  }
+}
+
+template <bool ZC, bool STAGE>
+__global__ __launch_bounds__(COLS) void k_w_diag(Dims d, StepParams p, Geo geo,
+                                                 const double* __restrict__ u,
+                                                 const double* __restrict__ v,
+                                                 double* __restrict__ w) {
+  extern __shared__ double wd_lds[];
+  const long long c = (long long)xcd_linear() * COLS + threadIdx.x;
+  if (c < d.n2)
+    transports_column<ZC, STAGE, false, true>(d, p, geo, u, v, nullptr, nullptr, w,
+                                              wd_lds + threadIdx.x, c);
+}
+
+void launch_w_diag(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                   const double* u, const double* v, double* w) {
+  const size_t lds = (size_t)d.nz * COLS * sizeof(double);
+  with_column_form(p.zcol != 0, lds <= COL_LDS_MAX, [&](auto zc, auto sg) {
+    constexpr bool SG = decltype(sg)::value;
+    k_w_diag<decltype(zc)::value, SG><<<column_blocks(d), COLS, SG ? lds : 0, s>>>(d, p, geo, u,
+                                                                                  v, w);
+  });
+}
+
+// ------------------------------------------------- the step's prologue
+// phi as k_phi forms it and, independently, the transports (U0 set) and w (w
+// set): two waves over the same columns (`part`).
+// Against one lane marching down for phi and the transports and up again for
+// w: 128 x 128 x 30 40 -> 12.5 us, 512 x 512 x 40 117 -> 102, 1000 x 1000 x 30
+// 290 -> 250. (The waves in workgroups of their own would each hold the LDS of
+// the second: 322 us.)
+template <bool ZC, bool STAGE, bool TR, bool WW>
+__global__ __launch_bounds__(2 * COLS) void k_prologue(
+    Dims d, StepParams p, Geo geo, const double* __restrict__ u, const double* __restrict__ v,
+    const double* __restrict__ b, double* __restrict__ phi, double* __restrict__ U0,
+    double* __restrict__ V0, double* __restrict__ w) {
+  extern __shared__ double pro_lds[];
+  const int lane = threadIdx.x % COLS;
+  const long long c = (long long)xcd_linear() * COLS + lane;
+  if (c >= d.n2) return;
+  if constexpr (TR || WW) {
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x / COLS) == 1) {
+      transports_column<ZC, STAGE, TR, WW>(d, p, geo, u, v, U0, V0, w, pro_lds + lane, c);
+      return;
+    }
+  }
+  const long long n2 = d.n2;
+  const int nz = d.nz;
+  const unsigned bc = 8u * (unsigned)c;
+  struct Level {
+    double x, dz;
+  };
+  const ColumnGeo cg(geo, p, d, c);
+  auto level = [&](const double* f, int k) {
+    return Level{at_byte(f + k * n2, bc), ZC ? 0.0 : at_byte(geo.dz3 + k * n2, bc)};
+  };
+  double above = 0.0;
+  march_down<8>(
+      nz, [&](int k) { return level(b, k); },
+      [&](int k, const Level& L) {
+        const double dz = ZC ? cg.dz(k) : L.dz;
+        put_byte(phi + k * n2, bc, 0.5 * dz * L.x + above);
+        const double t = dz * L.x;
+        above = (k == 0) ? t : above + t;
+      });
   if (p.pgf_remove) {
     double tot = 0.0, wsum = 0.0;
-    for (int k = 0; k < nz; ++k) {
-      const double dz = cg.dz(k);
-      const double t = dz * phi[k * n2 + c];
-      tot = (k == 0) ? dz : tot + dz;
-      wsum = (k == 0) ? t : wsum + t;
-    }
+    march_down<8>(
+        nz, [&](int k) { return level(phi, k); },
+        [&](int k, const Level& L) {
+          const double dz = ZC ? cg.dz(k) : L.dz;
+          const double t = dz * L.x;
+          tot = (k == 0) ? dz : tot + dz;
+          wsum = (k == 0) ? t : wsum + t;
+        });
     const double mean = wsum * safe_inv(tot);
-    for (int k = 0; k < nz; ++k) phi[k * n2 + c] = phi[k * n2 + c] - mean;
+    march_down<8>(
+        nz, [&](int k) { return at_byte(phi + k * n2, bc); },
+        [&](int k, double x) { put_byte(phi + k * n2, bc, x - mean); });
   }
-  if (!w) return;
-  const long long cw = at2(d, j, wrap(i, -1, d.nx)), cs = at2(d, wrap(j, -1, d.ny), i);
-  const FaceGeo fw(geo, p, d, cw, c, 0), fs(geo, p, d, cs, c, 1);
-  double sw = 0.0;
-  for (int k = nz - 1; k >= 0; --k) {
-    const long long o = k * n2;
-    const double U = fe.dz(k) * u[o + c];
-    const double Uw = fw.dz(k) * u[o + cw];
-    const double V = fn.dz(k) * v[o + c];
-    const double Vs = fs.dz(k) * v[o + cs];
-    const double dv = (cg.wet(k) ? 1.0 : 0.0) * ((U - Uw) / p.dx + (V - Vs) / p.dy);
-    sw = (k == nz - 1) ? dv : sw + dv;
-    w[o + c] = -sw;
-  }
-  w[(long long)nz * n2 + c] = 0.0;
+}
+
+void launch_prologue(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                     const double* u, const double* v, const double* b, double* phi, double* U0,
+                     double* V0, double* w) {
+  const size_t lds = w ? (size_t)d.nz * COLS * sizeof(double) : 0;
+  with_column_form(p.zcol != 0, lds <= COL_LDS_MAX, [&](auto zc, auto sg) {
+    constexpr bool ZC = decltype(zc)::value, SG = decltype(sg)::value;
+    auto go = [&](auto tr, auto ww) {
+      constexpr bool TR = decltype(tr)::value, WW = decltype(ww)::value;
+      k_prologue<ZC, SG, TR, WW>
+          <<<column_blocks(d), TR || WW ? 2 * COLS : COLS, SG ? lds : 0, s>>>(d, p, geo, u, v, b,
+                                                                              phi, U0, V0, w);
+    };
+    using T = std::true_type;
+    using F = std::false_type;
+    if (U0) {
+      if (w) go(T{}, T{});
+      else go(T{}, F{});
+    } else {
+      if (w) go(F{}, T{});
+      else go(F{}, F{});
+    }
+  });
 }
 
 // ------------------------------------------------ explicit momentum terms
@@ -1081,114 +1380,48 @@ __global__ void k_face_depth(Dims d, Geo geo, double* __restrict__ Hu, double* _
 }
 
 // ------------------------------------------- predictor and column solves
-// One lane per column, one Picard pass (model3d_v05.py:387-396):
+// Mean over the open ones of four faces (libs/core/operators_masked.py:46-61):
+// the weighted sum over the number of open faces, in the reference's order.
+// The quotient by 1, 2, 3 or 4 is formed like Divisor's, whose reciprocals are
+// the constants here.
+__device__ __forceinline__ double avg4(const double* a, const bool* f, bool own) {
+  const double w0 = f[0] ? 1.0 : 0.0, w1 = f[1] ? 1.0 : 0.0;
+  const double w2 = f[2] ? 1.0 : 0.0, w3 = f[3] ? 1.0 : 0.0;
+  const double num = 0.0 + w0 * a[0] + w1 * a[1] + w2 * a[2] + w3 * a[3];
+  const int n = (int)f[0] + (int)f[1] + (int)f[2] + (int)f[3];
+  const double den = (double)n;
+  const double y = n == 4 ? 0.25 : n == 3 ? 1.0 / 3.0 : n == 2 ? 0.5 : 1.0;
+  const double q = num * y;
+  const double r = __builtin_fma(-den, q, num);
+  const double m = __builtin_amdgcn_div_fixup(__builtin_fma(r, y, q), den, num);
+  return (n > 0 ? m : 0.0) * (own ? 1.0 : 0.0);
+}
+
+// One Picard pass (model3d_v05.py:387-396), one wave per 64 columns and
+// velocity component:
 //   v_cor = (1-tc) avg_v_to_u(v) + tc avg_v_to_u(v_it),  u_cor likewise
-// (both partners formed here, from the state and from the iterate)
+// (both partners formed here, from the state and from the iterate; FIRST: the
+// iterate is the state)
 //   gu = u + dt (f v_cor + pgx) - g dt (1-th) Gx(eta) + (1-thv) dt dzu
 //   gh_u = A_m^-1 (gu + stu) * mask3, and the same for v,
 // then the depth sums Ug = sum dz3u gh_u, Vg = sum dz3v gh_v for the
-// Helmholtz right-hand side. gh_u / gh_v hold d* between the sweeps.
-__global__ void k_predictor(Dims d, StepParams p, Geo geo, const double* __restrict__ u,
-                            const double* __restrict__ v, const double* __restrict__ eta,
-                            const double* __restrict__ u_it, const double* __restrict__ v_it,
-                            const double* __restrict__ pgx, const double* __restrict__ pgy,
-                            const double* __restrict__ dzu, const double* __restrict__ dzv,
-                            const double* __restrict__ stu, const double* __restrict__ stv,
-                            const double* __restrict__ sub, const double* __restrict__ den,
-                            const double* __restrict__ cst, double* __restrict__ gh_u,
-                            double* __restrict__ gh_v, double* __restrict__ Ug,
-                            double* __restrict__ Vg) {
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= d.n2) return;
-  const int i = (int)(c % d.nx), j = (int)(c / d.nx);
-  const Nb q = neighbours(d, j, i);
-  const long long n2 = d.n2;
-  const int nz = d.nz;
-  const bool split = p.scheme == SCHEME_SPLIT;
-  const double gx2 = mk(geo.mu2[c]) * (eta[q.e] - eta[c]) / p.dx;
-  const double gy2 = mk(geo.mv2[c]) * (eta[q.n] - eta[c]) / p.dy;
-  double du_prev = 0.0, dv_prev = 0.0;
-  for (int k = 0; k < nz; ++k) {
-    const long long o = k * n2;
-    const long long t = o + c;
-    // Coriolis partners of the old state, formed here from u and v (their
-    // neighbours are in cache) instead of stored and re-read; in the first
-    // Picard pass the iterate is the old state itself
-    const double av_v = avg_v_to_u(v, geo.m3v, geo.m3u, o, q);
-    const double av_u = avg_u_to_v(u, geo.m3u, geo.m3v, o, q);
-    const double av_v_it = v_it == v ? av_v : avg_v_to_u(v_it, geo.m3v, geo.m3u, o, q);
-    const double av_u_it = u_it == u ? av_u : avg_u_to_v(u_it, geo.m3u, geo.m3v, o, q);
-    const double vcor = p.one_m_tc * av_v + p.theta_cor * av_v_it;
-    const double ucor = p.one_m_tc * av_u + p.theta_cor * av_u_it;
-    const double gxe = gx2 * mk(geo.m3u[t]);
-    const double gye = gy2 * mk(geo.m3v[t]);
-    // split_explicit leaves the surface gradient to the barotropic substeps
-    // (model3d_v05.py:431-432)
-    const double gu = split ? u[t] + p.dt * (p.f * vcor + pgx[t]) + p.c_dzd * dzu[t]
-                            : u[t] + p.dt * (p.f * vcor + pgx[t]) - p.c_gx * gxe + p.c_dzd * dzu[t];
-    const double gv = split ? v[t] + p.dt * (p.neg_f * ucor + pgy[t]) + p.c_dzd * dzv[t]
-                            : v[t] + p.dt * (p.neg_f * ucor + pgy[t]) - p.c_gx * gye +
-                                  p.c_dzd * dzv[t];
-    const double ru = gu + stu[t];
-    const double rv = gv + stv[t];
-    double du, dv;
-    if (k == 0) {
-      du = ru / den[t];
-      dv = rv / den[t];
-    } else {
-      du = (ru - sub[t] * du_prev) / den[t];
-      dv = (rv - sub[t] * dv_prev) / den[t];
-    }
-    gh_u[t] = du;
-    gh_v[t] = dv;
-    du_prev = du;
-    dv_prev = dv;
-  }
-  double xu = 0.0, xv = 0.0;
-  for (int k = nz - 1; k >= 0; --k) {
-    const long long t = k * n2 + c;
-    if (k == nz - 1) {
-      xu = gh_u[t];
-      xv = gh_v[t];
-    } else {
-      xu = gh_u[t] - cst[t] * xu;
-      xv = gh_v[t] - cst[t] * xv;
-    }
-    const double mm = mk(geo.m3[t]);
-    gh_u[t] = xu * mm;
-    gh_v[t] = xv * mm;
-  }
-  double su = 0.0, sv = 0.0;
-  for (int k = 0; k < nz; ++k) {
-    const long long t = k * n2 + c;
-    const double tu = geo.dz3u[t] * gh_u[t];
-    const double tv = geo.dz3v[t] * gh_v[t];
-    su = (k == 0) ? tu : su + tu;
-    sv = (k == 0) ? tv : sv + tv;
-  }
-  Ug[c] = su;
-  Vg[c] = sv;
-}
-
-// Coriolis partners with the face masks given as flags: the same sums in
-// the same order as avg_v_to_u / avg_u_to_v.
-__device__ __forceinline__ double avg4(double a0, double a1, double a2, double a3, bool f0,
-                                       bool f1, bool f2, bool f3, bool own) {
-  const double w0 = f0 ? 1.0 : 0.0, w1 = f1 ? 1.0 : 0.0, w2 = f2 ? 1.0 : 0.0, w3 = f3 ? 1.0 : 0.0;
-  const double num = 0.0 + w0 * a0 + w1 * a1 + w2 * a2 + w3 * a3;
-  const double den = 0.0 + w0 + w1 + w2 + w3;
-  const double out = den > 0.0 ? num / den : 0.0;
-  return out * (own ? 1.0 : 0.0);
-}
-
-// k_predictor for a static z-level geometry in column form: the same
-// operations on the same operands in the same order (the same bits), with
-// the cell and face masks of the Coriolis averages and the face thicknesses
-// of the depth sums formed from the wet-level counts of the column and its
-// neighbours instead of read per cell. At most 128 VGPRs, so that a 512 x
-// 512 plane of columns is resident at once (4 waves per SIMD): the column
-// march is latency-bound.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_predictor_col(
+// Helmholtz right-hand side. ZC: masks and thicknesses from the columns' wet
+// levels (a face mask at level k is k < its threshold: the 2D face mask and
+// the shallower of the face's two cells) instead of the arrays, the same bits.
+// STAGE: d* and the solution stay in LDS between the three sweeps instead of
+// in gh_u / gh_v.
+//
+// Bound: memory on large grids (16 fields of the grid in a first pass, 20 in
+// a later one, and the neighbour rows of two), latency of the
+// march on small ones. One wave per component, operands two levels ahead and
+// d* in LDS, against one lane for both components, no loads ahead and d*, x in
+// memory, per launch (mean of both passes): 128 x 4 x 20 47 -> 17 us, 128 x
+// 128 x 30 84 -> 25, 512 x 512 x 40 322 -> 305, 640 x 512 x 48 584 -> 449,
+// 1000 x 1000 x 30 930 -> 795. Four levels ahead cost more in registers than
+// they hide (1000 x 1000 x 30: 891).
+constexpr int PRED_AHEAD = 2;
+template <bool ZC, bool FIRST, bool STAGE>
+__global__ __launch_bounds__(2 * COLS) void k_predictor(
     Dims d, StepParams p, Geo geo, const double* __restrict__ u, const double* __restrict__ v,
     const double* __restrict__ eta, const double* __restrict__ u_it,
     const double* __restrict__ v_it, const double* __restrict__ pgx,
@@ -1197,90 +1430,157 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
     const double* __restrict__ stv, const double* __restrict__ sub,
     const double* __restrict__ den, const double* __restrict__ cst, double* __restrict__ gh_u,
     double* __restrict__ gh_v, double* __restrict__ Ug, double* __restrict__ Vg) {
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  extern __shared__ double pred_lds[];  // STAGE: [2][nz][COLS], a thread's own column
+  const int comp = __builtin_amdgcn_readfirstlane(threadIdx.x / COLS);
+  const int lane = threadIdx.x % COLS;
+  const long long c = (long long)xcd_linear() * COLS + lane;
   if (c >= d.n2) return;
-  const int i = (int)(c % d.nx), j = (int)(c / d.nx);
+  const int j = (int)((unsigned)c / (unsigned)d.nx), i = (int)((unsigned)c - (unsigned)j * d.nx);
   const Nb q = neighbours(d, j, i);
   const long long n2 = d.n2;
   const int nz = d.nz;
   const bool split = p.scheme == SCHEME_SPLIT;
-  // a face mask at level k is k < its threshold: the 2D face mask and the
-  // shallower of the face's two cells
-  const int nwc = geo.nw[q.c], nwe = geo.nw[q.e], nwn = geo.nw[q.n], nwne = geo.nw[q.ne];
-  auto thr = [](uint8_t open, int a, int b) { return open ? (a < b ? a : b) : 0; };
-  const int tu_c = thr(geo.mu2[q.c], nwc, nwe), tu_w = thr(geo.mu2[q.w], geo.nw[q.w], nwc);
-  const int tu_n = thr(geo.mu2[q.n], nwn, nwne), tu_nw = thr(geo.mu2[q.nw], geo.nw[q.nw], nwn);
-  const int tv_c = thr(geo.mv2[q.c], nwc, nwn), tv_s = thr(geo.mv2[q.s], geo.nw[q.s], nwc);
-  const int tv_e = thr(geo.mv2[q.e], nwe, nwne), tv_se = thr(geo.mv2[q.se], geo.nw[q.se], nwe);
-  const double gx2 = mk(geo.mu2[c]) * (eta[q.e] - eta[c]) / p.dx;
-  const double gy2 = mk(geo.mv2[c]) * (eta[q.n] - eta[c]) / p.dy;
-  const bool first = u_it == u;
-  double du_prev = 0.0, dv_prev = 0.0;
-  for (int k = 0; k < nz; ++k) {
-    const long long o = k * n2;
-    const long long t = o + c;
-    // Coriolis partners of the old state, and of the iterate in a second pass
-    const bool fv0 = k < tv_c, fv1 = k < tv_s, fv2 = k < tv_e, fv3 = k < tv_se;
-    const bool fu0 = k < tu_c, fu1 = k < tu_w, fu2 = k < tu_n, fu3 = k < tu_nw;
-    const double av_v = avg4(v[t], v[o + q.s], v[o + q.e], v[o + q.se], fv0, fv1, fv2, fv3, fu0);
-    const double av_u = avg4(u[t], u[o + q.w], u[o + q.n], u[o + q.nw], fu0, fu1, fu2, fu3, fv0);
-    const double av_v_it = first ? av_v
-                                 : avg4(v_it[t], v_it[o + q.s], v_it[o + q.e], v_it[o + q.se],
-                                        fv0, fv1, fv2, fv3, fu0);
-    const double av_u_it = first ? av_u
-                                 : avg4(u_it[t], u_it[o + q.w], u_it[o + q.n], u_it[o + q.nw],
-                                        fu0, fu1, fu2, fu3, fv0);
-    const double vcor = p.one_m_tc * av_v + p.theta_cor * av_v_it;
-    const double ucor = p.one_m_tc * av_u + p.theta_cor * av_u_it;
-    const double gxe = gx2 * (fu0 ? 1.0 : 0.0);
-    const double gye = gy2 * (fv0 ? 1.0 : 0.0);
-    // split_explicit leaves the surface gradient to the barotropic substeps
-    // (model3d_v05.py:431-432)
-    const double gu = split ? u[t] + p.dt * (p.f * vcor + pgx[t]) + p.c_dzd * dzu[t]
-                            : u[t] + p.dt * (p.f * vcor + pgx[t]) - p.c_gx * gxe + p.c_dzd * dzu[t];
-    const double gv = split ? v[t] + p.dt * (p.neg_f * ucor + pgy[t]) + p.c_dzd * dzv[t]
-                            : v[t] + p.dt * (p.neg_f * ucor + pgy[t]) - p.c_gx * gye +
-                                  p.c_dzd * dzv[t];
-    const double ru = gu + stu[t];
-    const double rv = gv + stv[t];
-    double du, dv;
-    if (k == 0) {
-      du = ru / den[t];
-      dv = rv / den[t];
-    } else {
-      du = (ru - sub[t] * du_prev) / den[t];
-      dv = (rv - sub[t] * dv_prev) / den[t];
+  // this component's field and, of the other one's, the four faces round it
+  const double* f = comp ? v : u;
+  const double* g = comp ? u : v;
+  const double* gi = comp ? u_it : v_it;
+  const double* pg = comp ? pgy : pgx;
+  const double* dzf = comp ? dzv : dzu;
+  const double* st = comp ? stv : stu;
+  double* gh = comp ? gh_v : gh_u;
+  const uint8_t* mo = comp ? geo.m3v : geo.m3u;
+  const uint8_t* mg = comp ? geo.m3u : geo.m3v;
+  const int o4[4] = {q.c, comp ? q.w : q.s, comp ? q.n : q.e, comp ? q.nw : q.se};
+  const double fc = comp ? p.neg_f : p.f;
+  const int far = comp ? q.n : q.e;
+  const uint8_t* m2o = comp ? geo.mv2 : geo.mu2;
+  const double ge = mk(m2o[c]) * (eta[far] - eta[c]) / (comp ? p.dy : p.dx);
+  int th[4] = {}, tho = 0, nwc = 0;
+  if constexpr (ZC) {
+    nwc = geo.nw[c];
+    const uint8_t* m2g = comp ? geo.mu2 : geo.mv2;
+    const int far4[4] = {comp ? q.e : q.n, q.c, q.ne, comp ? q.n : q.e};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int a = geo.nw[o4[t]], b = geo.nw[far4[t]];
+      th[t] = m2g[o4[t]] ? (a < b ? a : b) : 0;
     }
-    gh_u[t] = du;
-    gh_v[t] = dv;
-    du_prev = du;
-    dv_prev = dv;
+    const int b = geo.nw[far];
+    tho = m2o[c] ? (nwc < b ? nwc : b) : 0;
   }
-  double xu = 0.0, xv = 0.0;
-  for (int k = nz - 1; k >= 0; --k) {
-    const long long t = k * n2 + c;
-    if (k == nz - 1) {
-      xu = gh_u[t];
-      xv = gh_v[t];
-    } else {
-      xu = gh_u[t] - cst[t] * xu;
-      xv = gh_v[t] - cst[t] * xv;
-    }
-    const double mm = k < nwc ? 1.0 : 0.0;
-    gh_u[t] = xu * mm;
-    gh_v[t] = xv * mm;
-  }
-  const FaceGeo fu(geo, p, d, c, q.e, 0), fv(geo, p, d, c, q.n, 1);
-  double su = 0.0, sv = 0.0;
-  for (int k = 0; k < nz; ++k) {
-    const long long t = k * n2 + c;
-    const double tu = fu.dz(k) * gh_u[t];
-    const double tv = fv.dz(k) * gh_v[t];
-    su = (k == 0) ? tu : su + tu;
-    sv = (k == 0) ? tv : sv + tv;
-  }
-  Ug[c] = su;
-  Vg[c] = sv;
+  struct Level {
+    double f, g[4], gi[FIRST ? 1 : 4], pg, dz, st, sub, den;
+    uint8_t m[ZC ? 1 : 5];
+  };
+  double* lds = STAGE ? pred_lds + (size_t)comp * nz * COLS + lane : nullptr;
+  const unsigned bc = 8u * (unsigned)c;
+  double prev = 0.0;
+  march_down<PRED_AHEAD>(
+      nz,
+      [&](int k) {
+        const long long o = k * n2;
+        Level L;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          L.g[s] = at_byte(g + o, 8u * (unsigned)o4[s]);
+          if constexpr (!FIRST) L.gi[s] = at_byte(gi + o, 8u * (unsigned)o4[s]);
+          if constexpr (!ZC) L.m[s] = at_byte(mg + o, (unsigned)o4[s]);
+        }
+        if constexpr (!ZC) L.m[4] = at_byte(mo + o, (unsigned)c);
+        L.f = at_byte(f + o, bc);
+        L.pg = at_byte(pg + o, bc);
+        L.dz = at_byte(dzf + o, bc);
+        L.st = at_byte(st + o, bc);
+        L.sub = at_byte(sub + o, bc);
+        L.den = at_byte(den + o, bc);
+        return L;
+      },
+      [&](int k, const Level& L) {
+        bool open[4], own;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          if constexpr (ZC) open[s] = k < th[s];
+          else open[s] = L.m[s] != 0;
+        }
+        if constexpr (ZC) own = k < tho;
+        else own = L.m[4] != 0;
+        const double av = avg4(L.g, open, own);
+        const double av_it = FIRST ? av : avg4(L.gi, open, own);
+        const double cor = p.one_m_tc * av + p.theta_cor * av_it;
+        const double gxe = ge * (own ? 1.0 : 0.0);
+        // split_explicit leaves the surface gradient to the barotropic substeps
+        // (model3d_v05.py:431-432)
+        const double r0 = L.f + p.dt * (fc * cor + L.pg);
+        const double r1 = split ? r0 : r0 - p.c_gx * gxe;
+        const double rhs = (r1 + p.c_dzd * L.dz) + L.st;
+        const Divisor<double> by_den(L.den);
+        prev = k == 0 ? by_den(rhs) : by_den(rhs - L.sub * prev);
+        if constexpr (STAGE) lds[k * COLS] = prev;
+        else put_byte(gh + k * n2, bc, prev);
+      });
+  struct Back {
+    double cst, d;
+    uint8_t m;
+  };
+  double x = 0.0;
+  march_up<8>(
+      nz,
+      [&](int k) {
+        const long long o = k * n2;
+        Back B;
+        B.cst = at_byte(cst + o, bc);
+        if constexpr (STAGE) B.d = lds[k * COLS];
+        else B.d = at_byte(gh + o, bc);
+        if constexpr (ZC) B.m = k < nwc;
+        else B.m = at_byte(geo.m3 + o, (unsigned)c);
+        return B;
+      },
+      [&](int k, const Back& B) {
+        x = k == nz - 1 ? B.d : B.d - B.cst * x;
+        const double xm = x * mk(B.m);
+        if constexpr (STAGE) lds[k * COLS] = xm;
+        put_byte(gh + k * n2, bc, xm);
+      });
+  FaceCol face{};
+  if constexpr (ZC) face = face_col(geo, p, c, far, comp);
+  const double* dzface = comp ? geo.dz3v : geo.dz3u;
+  struct Sum {
+    double dz, x;
+  };
+  double s = 0.0;
+  march_down<8>(
+      nz,
+      [&](int k) {
+        Sum S;
+        S.dz = ZC ? 0.0 : at_byte(dzface + k * n2, bc);
+        if constexpr (STAGE) S.x = lds[k * COLS];
+        else S.x = at_byte(gh + k * n2, bc);
+        return S;
+      },
+      [&](int k, const Sum& S) {
+        const double t = (ZC ? face.dz(k) : S.dz) * S.x;
+        s = k == 0 ? t : s + t;
+      });
+  (comp ? Vg : Ug)[c] = s;
+}
+
+void launch_predictor(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                      const double* u, const double* v, const double* eta, const double* u_it,
+                      const double* v_it, const double* pgx, const double* pgy,
+                      const double* dzu, const double* dzv, const double* stu,
+                      const double* stv, const double* sub, const double* den,
+                      const double* cst, double* gh_u, double* gh_v, double* Ug, double* Vg) {
+  const size_t lds = (size_t)2 * d.nz * COLS * sizeof(double);
+  with_column_form(p.zcol != 0, lds <= COL_LDS_MAX, [&](auto zc, auto sg) {
+    constexpr bool ZC = decltype(zc)::value, SG = decltype(sg)::value;
+    auto go = [&](auto fi) {
+      k_predictor<ZC, decltype(fi)::value, SG><<<column_blocks(d), 2 * COLS, SG ? lds : 0, s>>>(
+          d, p, geo, u, v, eta, u_it, v_it, pgx, pgy, dzu, dzv, stu, stv, sub, den, cst, gh_u,
+          gh_v, Ug, Vg);
+    };
+    if (u_it == u && v_it == v) go(std::true_type{});
+    else go(std::false_type{});
+  });
 }
 
 // u_it = (gh_u - g dt th q Gx(eta_new) mask3u) mask3 (model3d_v05.py:404-406)
@@ -1319,13 +1619,17 @@ __global__ void k_backsub(Dims d, StepParams p, Geo geo, const double* __restric
 // as k_backsub forms them; the west u and the south v that the transport
 // divergence needs are formed again from the same operands (the same bits),
 // so w is k_w_diag's of the stored fields without reading them back.
-__global__ void k_backsub_w(Dims d, StepParams p, Geo geo, const double* __restrict__ gh_u,
-                            const double* __restrict__ gh_v, const double* __restrict__ q,
-                            const double* __restrict__ eta_n, double* __restrict__ u,
-                            double* __restrict__ v, double* __restrict__ w) {
-  const long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+// Two levels ahead, spacings divided by a reciprocal: 128 x 128 x 30 45 -> 20
+// us, 512 x 512 x 40 112 -> 103, 640 x 512 x 48 198 -> 160.
+template <bool ZC>
+__global__ __launch_bounds__(COLS) void k_backsub_w(
+    Dims d, StepParams p, Geo geo, const double* __restrict__ gh_u,
+    const double* __restrict__ gh_v, const double* __restrict__ q,
+    const double* __restrict__ eta_n, double* __restrict__ u, double* __restrict__ v,
+    double* __restrict__ w) {
+  const long long c = (long long)xcd_linear() * COLS + threadIdx.x;
   if (c >= d.n2) return;
-  const int i = (int)(c % d.nx), j = (int)(c / d.nx);
+  const int j = (int)((unsigned)c / (unsigned)d.nx), i = (int)((unsigned)c - (unsigned)j * d.nx);
   const long long ce = at2(d, j, wrap(i, 1, d.nx)), cw = at2(d, j, wrap(i, -1, d.nx));
   const long long cn = at2(d, wrap(j, 1, d.ny), i), cs = at2(d, wrap(j, -1, d.ny), i);
   const long long n2 = d.n2;
@@ -1336,30 +1640,82 @@ __global__ void k_backsub_w(Dims d, StepParams p, Geo geo, const double* __restr
   const double gx_w = mk(geo.mu2[cw]) * (eta_n[c] - eta_n[cw]) / p.dx;
   const double gy_c = mk(geo.mv2[c]) * (eta_n[cn] - eta_n[c]) / p.dy;
   const double gy_s = mk(geo.mv2[cs]) * (eta_n[c] - eta_n[cs]) / p.dy;
-  const ColumnGeo gc(geo, p, d, c), gw(geo, p, d, cw), gs(geo, p, d, cs);
-  const FaceGeo fe(geo, p, d, c, ce, 0), fw(geo, p, d, cw, c, 0);
-  const FaceGeo fn(geo, p, d, c, cn, 1), fs(geo, p, d, cs, c, 1);
-  double sum = 0.0;
-  for (int k = nz - 1; k >= 0; --k) {
-    const long long o = (long long)k * n2;
-    const double mc = gc.wet(k) ? 1.0 : 0.0;
-    const double uc = (gh_u[o + c] - p.c_bs * q[o + c] * gx_c * (fe.wet(k) ? 1.0 : 0.0)) * mc;
-    const double vc = (gh_v[o + c] - p.c_bs * q[o + c] * gy_c * (fn.wet(k) ? 1.0 : 0.0)) * mc;
-    const double uw = (gh_u[o + cw] - p.c_bs * q[o + cw] * gx_w * (fw.wet(k) ? 1.0 : 0.0)) *
-                      (gw.wet(k) ? 1.0 : 0.0);
-    const double vs = (gh_v[o + cs] - p.c_bs * q[o + cs] * gy_s * (fs.wet(k) ? 1.0 : 0.0)) *
-                      (gs.wet(k) ? 1.0 : 0.0);
-    u[o + c] = uc;
-    v[o + c] = vc;
-    const double U = fe.dz(k) * uc;
-    const double Uw = fw.dz(k) * uw;
-    const double V = fn.dz(k) * vc;
-    const double Vs = fs.dz(k) * vs;
-    const double dv = mc * ((U - Uw) / p.dx + (V - Vs) / p.dy);
-    sum = (k == nz - 1) ? dv : sum + dv;
-    w[o + c] = -sum;
+  const unsigned bc = 8u * (unsigned)c, bw = 8u * (unsigned)cw, bs = 8u * (unsigned)cs;
+  FaceCol fe{}, fw{}, fn{}, fs{};
+  int nwc = 0, nww = 0, nws = 0;
+  if constexpr (ZC) {
+    fe = face_col(geo, p, c, ce, 0);
+    fw = face_col(geo, p, cw, c, 0);
+    fn = face_col(geo, p, c, cn, 1);
+    fs = face_col(geo, p, cs, c, 1);
+    nwc = geo.nw[c];
+    nww = geo.nw[cw];
+    nws = geo.nw[cs];
   }
+  const Divisor<double> by_dx = uniform_divisor<double>(p.dx), by_dy = uniform_divisor<double>(p.dy);
+  struct Level {
+    double u, v, uw, vs, q, qw, qs, de, dw, dn, ds;
+    uint8_t m, mw, ms, me, mfw, mn, mfs;
+  };
+  double sum = 0.0;
+  march_up<2>(
+      nz,
+      [&](int k) {
+        const long long o = k * n2;
+        Level L;
+        L.u = at_byte(gh_u + o, bc);
+        L.v = at_byte(gh_v + o, bc);
+        L.uw = at_byte(gh_u + o, bw);
+        L.vs = at_byte(gh_v + o, bs);
+        L.q = at_byte(q + o, bc);
+        L.qw = at_byte(q + o, bw);
+        L.qs = at_byte(q + o, bs);
+        if constexpr (!ZC) {
+          L.de = geo.dz3u[o + c];
+          L.dw = geo.dz3u[o + cw];
+          L.dn = geo.dz3v[o + c];
+          L.ds = geo.dz3v[o + cs];
+          L.m = geo.m3[o + c];
+          L.mw = geo.m3[o + cw];
+          L.ms = geo.m3[o + cs];
+          L.me = geo.m3u[o + c];
+          L.mfw = geo.m3u[o + cw];
+          L.mn = geo.m3v[o + c];
+          L.mfs = geo.m3v[o + cs];
+        }
+        return L;
+      },
+      [&](int k, const Level& L) {
+        const double mc = (ZC ? k < nwc : L.m != 0) ? 1.0 : 0.0;
+        const double mw = (ZC ? k < nww : L.mw != 0) ? 1.0 : 0.0;
+        const double ms = (ZC ? k < nws : L.ms != 0) ? 1.0 : 0.0;
+        const double me = (ZC ? fe.wet(k) : L.me != 0) ? 1.0 : 0.0;
+        const double mfw = (ZC ? fw.wet(k) : L.mfw != 0) ? 1.0 : 0.0;
+        const double mn = (ZC ? fn.wet(k) : L.mn != 0) ? 1.0 : 0.0;
+        const double mfs = (ZC ? fs.wet(k) : L.mfs != 0) ? 1.0 : 0.0;
+        const double uc = (L.u - p.c_bs * L.q * gx_c * me) * mc;
+        const double vc = (L.v - p.c_bs * L.q * gy_c * mn) * mc;
+        const double uw = (L.uw - p.c_bs * L.qw * gx_w * mfw) * mw;
+        const double vs = (L.vs - p.c_bs * L.qs * gy_s * mfs) * ms;
+        put_byte(u + k * n2, bc, uc);
+        put_byte(v + k * n2, bc, vc);
+        const double U = (ZC ? fe.dz(k) : L.de) * uc;
+        const double Uw = (ZC ? fw.dz(k) : L.dw) * uw;
+        const double V = (ZC ? fn.dz(k) : L.dn) * vc;
+        const double Vs = (ZC ? fs.dz(k) : L.ds) * vs;
+        const double dv = mc * (by_dx(U - Uw) + by_dy(V - Vs));
+        sum = (k == nz - 1) ? dv : sum + dv;
+        put_byte(w + k * n2, bc, -sum);
+      });
   w[(long long)nz * n2 + c] = 0.0;
+}
+
+void launch_backsub_w(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo,
+                      const double* gh_u, const double* gh_v, const double* q,
+                      const double* eta_n, double* u, double* v, double* w) {
+  const unsigned nb = column_blocks(d);
+  if (p.zcol) k_backsub_w<true><<<nb, COLS, 0, s>>>(d, p, geo, gh_u, gh_v, q, eta_n, u, v, w);
+  else k_backsub_w<false><<<nb, COLS, 0, s>>>(d, p, geo, gh_u, gh_v, q, eta_n, u, v, w);
 }
 
 // ------------------------------------------------------------- tracers

@@ -54,25 +54,6 @@ __device__ __forceinline__ R tracer_face_z(int adv, int kk, int nz, R far_up, R 
                          hu, hd, adv == ADV_UP3_TVD);
 }
 
-// Value of a plane at a byte offset. The plane's address is the same in every
-// lane and is kept in scalar registers, so that one vector register holds the
-// offset for every array (a plane is below 2^32 bytes). Without the empty asm
-// the compiler keeps a 64-bit vector address per array across the march, 30
-// registers in the momentum kernel.
-template <class T>
-__device__ __forceinline__ T at_byte(const T* plane, unsigned off) {
-  unsigned long long a = (unsigned long long)plane;
-  __asm__("" : "+s"(a));
-  using G = const __attribute__((address_space(1))) char;
-  return *(const __attribute__((address_space(1))) T*)((G*)a + off);
-}
-__device__ __forceinline__ void put_byte(double* plane, unsigned off, double v) {
-  unsigned long long a = (unsigned long long)plane;
-  __asm__("" : "+s"(a));
-  using G = __attribute__((address_space(1))) char;
-  *(__attribute__((address_space(1))) double*)((G*)a + off) = v;
-}
-
 struct NoTile {};
 
 // First threads that form the tile's west column of faces (TY of them) and
