@@ -681,15 +681,15 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_update(PcgArgs a, int it, int ja
 // Partial sums of r*z after a preconditioner application; into_b = 1 on the
 // first application (also p = z into pb1), 0 in the iterations (part_c).
 __global__ __launch_bounds__(PCG_WG) void k_pcg_rz(PcgArgs a, int into_b) {
-  if (a.sc->done) return;
+  const int done = a.sc->done;
   __shared__ double lds[PCG_STAGE];
   const int part = blockIdx.x;
   const double s = part_sum(a, part, [&](long long e) -> double {
     const double z = a.z[e];
-    if (into_b) a.pb1[e] = z;
+    if (into_b && !done) a.pb1[e] = z;
     return a.r[e] * z;
   }, lds);
-  if (threadIdx.x == 0) (into_b ? a.part_b : a.part_c)[part] = s;
+  if (threadIdx.x == 0 && !done) (into_b ? a.part_b : a.part_c)[part] = s;
 }
 
 // After a sync-free solve of n_it launched iterations: a solve whose done

@@ -342,22 +342,22 @@ __global__ void k_mg_prolong(MgLevel f, const double* __restrict__ xc, int cnx,
 // solvers, solvers_var.py:176).
 __global__ __launch_bounds__(PCG_WG) void k_mg_res_parts(PcgArgs a, MgLevel L,
                                                          const double* __restrict__ x) {
-  if (a.sc->done) return;
+  const int done = a.sc->done;
   __shared__ double lds[PCG_STAGE];
   const int part = blockIdx.x;
   const double s = part_sum(a, part, [&](long long e) -> double {
     const double r = a.rhs[e] - mg_apply(L, x, e);
     return r * r;
   }, lds);
-  if (threadIdx.x == 0) a.part_b[part] = s;
+  if (threadIdx.x == 0 && !done) a.part_b[part] = s;
 }
 
 // Stationary-solver bookkeeping after iteration `it`: ||rhs - A x|| <= tol.
 __global__ __launch_bounds__(PCG_WG) void k_mg_check(PcgArgs a, int it) {
-  if (a.sc->done) return;
+  const int done = a.sc->done;
   __shared__ double cs[PCG_CS];
   const double res = sqrt(total_from_parts(a, a.part_b, cs));
-  if (threadIdx.x != 0) return;
+  if (threadIdx.x != 0 || done) return;
   PcgScalars* sc = a.sc;
   sc->res = res;
   if (res <= sc->tol) {
@@ -481,7 +481,7 @@ template <int S, class R, class RB, int TW, int TH>
 __global__ __launch_bounds__((JacRegion<S, TW, TH>::NT)) void k_mg_down(
     MgLevelT<R> L, MgLevelT<R> C, R omega, const RB* __restrict__ b, R* __restrict__ xs_out,
     R* __restrict__ bc, const PcgScalars* sc) {
-  if (finished(sc)) return;
+  const bool done = finished(sc);  // tested once the loads are on their way
   constexpr int H = S;
   using Rg = JacRegion<H, TW, TH>;
   constexpr int Q = Rg::Q;
@@ -511,6 +511,7 @@ __global__ __launch_bounds__((JacRegion<S, TW, TH>::NT)) void k_mg_down(
       if (on[q]) buf[(k - 1) & 1][K[q].q] = v[q];
     }
     __syncthreads();
+    if (k == 1 && done) return;
   }
   const R* xs = buf[(S - 1) & 1];
   R* res = buf[S & 1];
@@ -538,7 +539,7 @@ template <int S, class R, class RB, class RO, int TW, int TH>
 __global__ __launch_bounds__((JacRegion<S, TW, TH>::NT)) void k_mg_up(
     MgLevelT<R> L, R omega, const R* __restrict__ xs_in, const R* __restrict__ ec,
     const RB* __restrict__ b, RO* __restrict__ out, const PcgScalars* sc) {
-  if (finished(sc)) return;
+  const bool done = finished(sc);  // tested once the loads are on their way
   constexpr int H = S;
   using Rg = JacRegion<H, TW, TH>;
   constexpr int Q = Rg::Q;
@@ -557,6 +558,7 @@ __global__ __launch_bounds__((JacRegion<S, TW, TH>::NT)) void k_mg_up(
     if (on[q]) buf[0][K[q].q] = v[q];
   }
   __syncthreads();
+  if (done) return;
 #pragma unroll
   for (int k = 1; k <= S; ++k) {
     const R* src = buf[(k - 1) & 1];
@@ -699,7 +701,7 @@ template <int S, bool FROM_X, int TW, int TH>
 __global__ __launch_bounds__((RbRegion<2 * S + (FROM_X ? 1 : 0), TW, TH>::NT)) void k_mg_down_rb(
     MgLevel L, MgLevel C, const double* __restrict__ x_in, const double* __restrict__ b,
     double* __restrict__ xs_out, double* __restrict__ bc, const PcgScalars* sc) {
-  if (finished(sc)) return;
+  const bool done = finished(sc);  // tested once the loads are on their way
   constexpr int H = 2 * S + (FROM_X ? 1 : 0);
   using Rg = RbRegion<H, TW, TH>;
   __shared__ double buf[2][Rg::RN];
@@ -720,6 +722,7 @@ __global__ __launch_bounds__((RbRegion<2 * S + (FROM_X ? 1 : 0), TW, TH>::NT)) v
   }
   if (on) rb_put(P, buf[1]);
   __syncthreads();
+  if (done) return;
 #pragma unroll
   for (int ph = 2; ph <= 2 * S; ++ph) {  // red first
     rb_update(P, L.cx, L.cy, (ph - 1) & 1, (ph & 1) == 0, buf[(ph - 1) & 1]);
@@ -765,7 +768,7 @@ template <int S, int TW, int TH>
 __global__ __launch_bounds__((RbRegion<2 * S, TW, TH>::NT)) void k_mg_up_rb(
     MgLevel L, const double* __restrict__ xs_in, const double* __restrict__ ec,
     const double* __restrict__ b, double* __restrict__ out, const PcgScalars* sc) {
-  if (finished(sc)) return;
+  const bool done = finished(sc);  // tested once the loads are on their way
   constexpr int H = 2 * S;
   using Rg = RbRegion<H, TW, TH>;
   __shared__ double buf[2][Rg::RN];
@@ -777,6 +780,7 @@ __global__ __launch_bounds__((RbRegion<2 * S, TW, TH>::NT)) void k_mg_up_rb(
   for (int k = 0; k < 2; ++k) P.x[k] = xs_in[P.g[k]] + ec[P.up[k]] * P.c[k].m;
   if (on) rb_put(P, buf[0]);
   __syncthreads();
+  if (done) return;
 #pragma unroll
   for (int ph = 1; ph <= 2 * S; ++ph) {  // black first
     rb_update(P, L.cx, L.cy, ph & 1, (ph & 1) == 0, buf[(ph - 1) & 1]);
@@ -945,7 +949,7 @@ __global__ __launch_bounds__(NT) void k_mg_coarse_cycle(MgCycleT<R> C, R omega, 
                                                         const RB* __restrict__ b0,
                                                         const R* x0, RO* out,
                                                         const PcgScalars* sc) {
-  if (finished(sc)) return;
+  const bool done = finished(sc);  // tested once the loads are on their way
   extern __shared__ __align__(16) unsigned char cyc_raw[];
   R* cyc = reinterpret_cast<R*>(cyc_raw);
   const int tid = threadIdx.x;
@@ -982,6 +986,7 @@ __global__ __launch_bounds__(NT) void k_mg_coarse_cycle(MgCycleT<R> C, R omega, 
       if (K0[q].on) f.cur[K0[q].c] = v0[q];
   }
   __syncthreads();
+  if (done) return;
   auto level = [&](int l) {  // this thread's cell of a level below the first
     const MgLevelT<R>& G = C.lev[l];
     CycCell<R> K = cyc_index(G, tid);
