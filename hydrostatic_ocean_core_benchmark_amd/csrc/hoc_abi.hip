@@ -128,6 +128,33 @@ struct Reducer {
 }  // namespace
 
 // ------------------------------------------------------------ the handle
+// PCG-Jacobi iterations recorded as HIP graphs of 2 << q iterations each, on
+// the step's own operands (see jacobi_iterations).
+struct IterGraphs {
+  static constexpr int SIZES = 6;
+  // Recording costs about as much as three steps gain (131 x 77): not before
+  // this many solves in a row on the same operands.
+  static constexpr int WARM_SOLVES = 8;
+  PcgArgs key{};
+  int solves = 0;       // solves in a row on key
+  bool failed = false;  // recording failed: launches only
+  hipGraph_t graph[SIZES] = {};
+  hipGraphExec_t exec[SIZES] = {};
+  bool any() const {
+    for (hipGraphExec_t e : exec)
+      if (e) return true;
+    return false;
+  }
+  void clear() {
+    for (int q = 0; q < SIZES; ++q) {
+      if (exec[q]) (void)hipGraphExecDestroy(exec[q]);
+      if (graph[q]) (void)hipGraphDestroy(graph[q]);
+      exec[q] = nullptr;
+      graph[q] = nullptr;
+    }
+  }
+};
+
 struct hoc_stepper {
   hoc_config cfg{};
   Dims d{};
@@ -188,6 +215,8 @@ struct hoc_stepper {
   const void* sf_key[5] = {};
   int sf_key_budget = 0, sf_key_tile = -1;
   double* sf_x = nullptr;  // fixed solution buffer of the step's graph-replayed solves
+  IterGraphs it_graphs;
+  hipStream_t record = nullptr;  // the iterations' graphs are recorded on it; runs nothing
   int mg_tile_shape = 0;     // fused V-cycle leg tile shape (0..MG_TILE_SHAPES-1)
                              // default by size: 16x16 up to 512x512 columns
                              // (5.50 vs 5.66 ms/step at 512x512x40), else 32x16
@@ -231,6 +260,8 @@ struct hoc_stepper {
   ~hoc_stepper() {
     if (sf_exec) (void)hipGraphExecDestroy(sf_exec);
     if (sf_graph) (void)hipGraphDestroy(sf_graph);
+    it_graphs.clear();
+    if (record) (void)hipStreamDestroy(record);
     for (hipEvent_t e : prof_ev) (void)hipEventDestroy(e);
     for (void* v : allocs) (void)hipFree(v);
     if (host_flag) (void)hipHostFree(host_flag);
@@ -859,28 +890,110 @@ int precondition(hoc_stepper* h, const double* r, double* z, hipStream_t s) {
   return HOC_OK;
 }
 
+// One PCG iteration: the launches of iteration `it` on s; it = -1 or -2 stands
+// for any odd or even one whose number the device knows (Jacobi only).
+int pcg_iteration(hoc_stepper* h, const PcgArgs& a, hipStream_t s, int it) {
+  const unsigned np = (unsigned)h->pcg_parts_all;
+  const int jacobi = h->cfg.solver == SOLVER_PCG_JACOBI ? 1 : 0;
+  if (a.central) k_pcg_totals<<<1, PCG_WG, 0, s>>>(a, it == 1 ? 1 : 2);
+  { ProfScope _ps(h, "k_pcg_ap", s); k_pcg_ap<<<np, PCG_WG, 0, s>>>(a, it); }
+  if (it > h->p.max_iter) return HOC_OK;  // only finishes the last iteration
+  if (a.central) k_pcg_totals<<<1, PCG_WG, 0, s>>>(a, 0);
+  { ProfScope _ps(h, "k_pcg_update", s); k_pcg_update<<<np, PCG_WG, 0, s>>>(a, it, jacobi); }
+  if (!jacobi) {
+    TRY(precondition(h, h->r, h->z, s));
+    k_pcg_rz<<<np, PCG_WG, 0, s>>>(a, 0);
+  }
+  return HOC_OK;
+}
+
+// Whether the Jacobi iterations with operands a (x and rhs left out) may be
+// replayed on stream s: after WARM_SOLVES solves in a row with them, not while a
+// phase is profiled by name or the caller captures the stream.
+bool iteration_graphs_usable(hoc_stepper* h, const PcgArgs& a, hipStream_t s) {
+  IterGraphs& g = h->it_graphs;
+  if (h->prof_name == "k_pcg_ap" || h->prof_name == "k_pcg_update") return false;
+  if (s != nullptr) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
+      return false;
+  }
+  PcgArgs key;
+  std::memcpy(&key, &a, sizeof(a));  // compared byte by byte
+  key.rhs = nullptr;
+  key.x = nullptr;
+  if (std::memcmp(&g.key, &key, sizeof(key)) != 0) {
+    if (g.any()) (void)hipDeviceSynchronize();  // a replay of the old ones may still run
+    g.clear();
+    std::memcpy(&g.key, &key, sizeof(key));
+    g.solves = 0;
+  }
+  return ++g.solves > IterGraphs::WARM_SOLVES && !g.failed;
+}
+
+// The graph of 2 << q iterations, recorded on first use; null if that fails.
+hipGraphExec_t iteration_graph(hoc_stepper* h, const PcgArgs& a, int q) {
+  IterGraphs& g = h->it_graphs;
+  if (g.exec[q] || g.failed) return g.exec[q];
+  bool ok = h->record || hipStreamCreateWithFlags(&h->record, hipStreamNonBlocking) == hipSuccess;
+  ok = ok && hipStreamBeginCapture(h->record, hipStreamCaptureModeRelaxed) == hipSuccess;
+  if (ok) {
+    for (int i = 0; i < (2 << q) && ok; ++i)
+      ok = pcg_iteration(h, a, h->record, (i & 1) ? -1 : -2) == HOC_OK;
+    ok = hipStreamEndCapture(h->record, &g.graph[q]) == hipSuccess && g.graph[q] && ok;
+  }
+  ok = ok && hipGraphInstantiate(&g.exec[q], g.graph[q], nullptr, nullptr, 0) == hipSuccess;
+  if (!ok) {
+    (void)hipGetLastError();
+    g.exec[q] = nullptr;
+    g.failed = true;
+  }
+  return g.exec[q];
+}
+
+// PCG iterations it .. it + count - 1 (it is advanced). replay: runs of Jacobi
+// iterations with an even first number are replayed from graphs of 64, 32, ..,
+// 2 iterations and only the rest is launched; the replayed kernels take the
+// iteration's number from the device. A launch costs the host 4 to 4.4 us, as
+// much as one of these kernels runs on a grid up to ITER_GRAPH_CELLS: per solve
+// launched and replayed, 64 x 64 1732 and 1509 us, 131 x 77 (195 iterations)
+// 1861 and 1654, 256 x 256 1870 and 1743, 512 x 512 2828 and 2829, 1024 x 1024
+// 8309 and 8384. The V-cycle's iterations (8 kernels and more, 10 to 20 of
+// them) gain nothing: 128 x 128 438 and 427, 512 x 512 676 and 692.
+constexpr long long ITER_GRAPH_CELLS = 1 << 17;
+int pcg_iterations(hoc_stepper* h, const PcgArgs& a, bool replay, hipStream_t s, int& it,
+                   int count) {
+  while (count > 0) {
+    const int room = std::min(count, h->p.max_iter - it + 1);  // whole iterations
+    hipGraphExec_t e = nullptr;
+    int q = 0;
+    if (replay && (it & 1) == 0 && room >= 2) {
+      while (q + 1 < IterGraphs::SIZES && (4 << q) <= room) ++q;
+      e = iteration_graph(h, a, q);
+    }
+    if (e) HIP_TRY(hipGraphLaunch(e, s));
+    else TRY(pcg_iteration(h, a, s, it));
+    const int n = e ? 2 << q : 1;
+    it += n;
+    count -= n;
+  }
+  LAUNCH_CHECK("pcg iteration");
+  return HOC_OK;
+}
+
 // The sync-free PCG of pcg_mg / pcg_rbgs: a fixed launch sequence with no
 // host read-back (capturable in a HIP graph). Every phase returns at once
 // after the device `done` flag is set, and a solve that has not converged
 // within the budget counts as a failure.
 int pcg_sync_free(hoc_stepper* h, const PcgArgs& a, unsigned np, hipStream_t s, int* iters_out,
                   int* conv_out) {
-  const int max_iter = h->p.max_iter;
   k_pcg_init<<<np, PCG_WG, 0, s>>>(a);   // r = rhs * mask, x = 0, ||rhs||^2 parts
   k_mg_start<<<1, PCG_WG, 0, s>>>(a);
   TRY(precondition(h, h->r, h->z, s));
   k_pcg_rz<<<np, PCG_WG, 0, s>>>(a, 1);
-  const int n_it = std::min(h->sync_free_budget, max_iter + 1);
-  for (int it = 1; it <= n_it; ++it) {
-    if (a.central) k_pcg_totals<<<1, PCG_WG, 0, s>>>(a, it == 1 ? 1 : 2);
-    k_pcg_ap<<<np, PCG_WG, 0, s>>>(a, it);
-    if (it <= max_iter) {
-      if (a.central) k_pcg_totals<<<1, PCG_WG, 0, s>>>(a, 0);
-      k_pcg_update<<<np, PCG_WG, 0, s>>>(a, it, 0);
-      TRY(precondition(h, h->r, h->z, s));
-      k_pcg_rz<<<np, PCG_WG, 0, s>>>(a, 0);
-    }
-  }
+  const int n_it = std::min(h->sync_free_budget, h->p.max_iter + 1);
+  int it = 1;
+  TRY(pcg_iterations(h, a, false, s, it, n_it));
   k_pcg_budget_check<<<1, 64, 0, s>>>(a, n_it);
   LAUNCH_CHECK("pcg iteration (sync-free)");
   if (iters_out) *iters_out = -1;
@@ -921,7 +1034,6 @@ int helmholtz_solve(hoc_stepper* h, const double* Ku, const double* Kv, const do
       TRY(mg_build(h, Ku, Kv, inv_diag, s));
       h->mg_gen = own ? h->coeff_gen : -1;
     }
-    const int max_iter = h->p.max_iter;
     if (h->sync_free_budget > 0 && kind != SOLVER_RBGS && kind != SOLVER_MULTIGRID) {
       bool replay = false;
       TRY(sf_graph_usable(h, s, &replay));
@@ -959,58 +1071,8 @@ int helmholtz_solve(hoc_stepper* h, const double* Ku, const double* Kv, const do
       if (conv_out) *conv_out = -1;
       return HOC_OK;
     }
-    k_pcg_init<<<np, PCG_WG, 0, s>>>(a);   // r = rhs * mask, x = 0, ||rhs||^2 parts
-    k_mg_start<<<1, PCG_WG, 0, s>>>(a);
-    LAUNCH_CHECK("solver init");
-    if (kind == SOLVER_RBGS || kind == SOLVER_MULTIGRID) {
-      // stationary iteration on x with the masked rhs (a.r); ||rhs - A x||
-      PcgArgs ar = a;
-      ar.rhs = h->r;
-      int it = 1;
-      int batch = std::max(1, std::min(h->last_iters, max_iter));
-      while (true) {
-        for (int b = 0; b < batch && it <= max_iter; ++b, ++it) {
-          if (kind == SOLVER_RBGS) rbgs_sweep(h, 0, h->r, x, false, s);
-          else if (h->mg_cycle_l0 >= 0) TRY(vcycle_fused(h, 2, true, h->r, x, x, s));
-          else vcycle_rbgs(h, 0, x, h->r, s);
-          k_mg_res_parts<<<np, PCG_WG, 0, s>>>(ar, h->lev[0], x);
-          k_mg_check<<<1, PCG_WG, 0, s>>>(ar, it);
-        }
-        LAUNCH_CHECK("stationary iteration");
-        int done = 0;
-        TRY(poll_done(h, s, &done));
-        if (done) break;
-        if (it > max_iter) return fail(HOC_ERR_DEVICE, "solver did not report completion");
-        batch = std::min(2 * batch, 64);  // slow stationary convergence: fewer polls
-      }
-      return pcg_finish(h, s, false, iters_out, conv_out, true);
-    }
-    // PCG with the RBGS or multigrid preconditioner
-    TRY(precondition(h, h->r, h->z, s));
-    k_pcg_rz<<<np, PCG_WG, 0, s>>>(a, 1);
-    int it = 1;
-    int batch = std::max(1, std::min(h->last_iters + 1, max_iter + 1));
-    while (true) {
-      for (int b = 0; b < batch && it <= max_iter + 1; ++b, ++it) {
-        if (a.central) k_pcg_totals<<<1, PCG_WG, 0, s>>>(a, it == 1 ? 1 : 2);
-        { ProfScope _ps(h, "k_pcg_ap", s); k_pcg_ap<<<np, PCG_WG, 0, s>>>(a, it); }
-        if (it <= max_iter) {
-          if (a.central) k_pcg_totals<<<1, PCG_WG, 0, s>>>(a, 0);
-          { ProfScope _ps(h, "k_pcg_update", s); k_pcg_update<<<np, PCG_WG, 0, s>>>(a, it, 0); }
-          TRY(precondition(h, h->r, h->z, s));
-          k_pcg_rz<<<np, PCG_WG, 0, s>>>(a, 0);
-        }
-      }
-      LAUNCH_CHECK("pcg iteration");
-      int done = 0;
-      TRY(poll_done(h, s, &done));
-      if (done) break;
-      if (it > max_iter + 1) return fail(HOC_ERR_DEVICE, "Helmholtz solve did not report completion");
-      batch = 4;
-    }
-    return pcg_finish(h, s, false, iters_out, conv_out, true);
   }
-  if (h->pcg_parts > 0 && !h->force_multikernel) {
+  if (kind == SOLVER_PCG_JACOBI && h->pcg_parts > 0 && !h->force_multikernel) {
     a.sc = h->sc;
     void* args[] = {&a};
     { ProfScope _ps(h, "k_pcg_persistent", s);
@@ -1018,31 +1080,57 @@ int helmholtz_solve(hoc_stepper* h, const double* Ku, const double* Kv, const do
                                          dim3(PCG_WG), args, 0, s)); }
     return pcg_finish(h, s, true, iters_out, conv_out);
   }
-  k_pcg_init<<<np, PCG_WG, 0, s>>>(a);
-  k_pcg_init_z<<<np, PCG_WG, 0, s>>>(a);
-  LAUNCH_CHECK("pcg init");
   const int max_iter = h->p.max_iter;
-  // Iteration it's A launch also finishes iteration it-1, so max_iter
-  // iterations need max_iter + 1 A launches; the device flag stops early.
-  int it = 1;
-  int batch = std::max(1, std::min(h->last_iters + 1, max_iter + 1));
-  while (true) {
-    for (int b = 0; b < batch && it <= max_iter + 1; ++b, ++it) {
-      if (a.central) k_pcg_totals<<<1, PCG_WG, 0, s>>>(a, it == 1 ? 1 : 2);
-      { ProfScope _ps(h, "k_pcg_ap", s); k_pcg_ap<<<np, PCG_WG, 0, s>>>(a, it); }
-      if (it <= max_iter) {
-        if (a.central) k_pcg_totals<<<1, PCG_WG, 0, s>>>(a, 0);
-        ProfScope _ps(h, "k_pcg_update", s);
-        k_pcg_update<<<np, PCG_WG, 0, s>>>(a, it, 1);
-      }
+  const bool stationary = kind == SOLVER_RBGS || kind == SOLVER_MULTIGRID;
+  // replayed iterations solve into a buffer of the handle's, copied to x
+  bool replay = false;
+  if (kind == SOLVER_PCG_JACOBI && h->d.n2 <= ITER_GRAPH_CELLS && Ku == h->Ku && Kv == h->Kv &&
+      inv_diag == h->inv_diag && iteration_graphs_usable(h, a, s)) {
+    if (!h->sf_x) TRY(h->alloc(&h->sf_x, h->d.n2));
+    a.x = h->sf_x;
+    replay = true;
+  }
+  k_pcg_init<<<np, PCG_WG, 0, s>>>(a);  // r = rhs * mask, x = 0, ||rhs||^2 parts
+  if (kind == SOLVER_PCG_JACOBI) {
+    k_pcg_init_z<<<np, PCG_WG, 0, s>>>(a);
+  } else {
+    k_mg_start<<<1, PCG_WG, 0, s>>>(a);
+    if (!stationary) {
+      TRY(precondition(h, h->r, h->z, s));
+      k_pcg_rz<<<np, PCG_WG, 0, s>>>(a, 1);
     }
-    LAUNCH_CHECK("pcg iteration");
+  }
+  LAUNCH_CHECK("solver init");
+  // A PCG iteration's A launch also finishes the iteration before, so max_iter
+  // iterations need max_iter + 1 A launches; the device flag stops early.
+  const int last = stationary ? max_iter : max_iter + 1;
+  int it = 1;
+  int batch = std::max(1, std::min(stationary ? h->last_iters : h->last_iters + 1, last));
+  while (true) {
+    const int count = std::min(batch, last - it + 1);
+    if (!stationary) {
+      TRY(pcg_iterations(h, a, replay, s, it, count));
+    } else {
+      // stationary iteration on x with the masked rhs (r); ||rhs - A x||
+      PcgArgs ar = a;
+      ar.rhs = h->r;
+      for (int b = 0; b < count; ++b, ++it) {
+        if (kind == SOLVER_RBGS) rbgs_sweep(h, 0, h->r, x, false, s);
+        else if (h->mg_cycle_l0 >= 0) TRY(vcycle_fused(h, 2, true, h->r, x, x, s));
+        else vcycle_rbgs(h, 0, x, h->r, s);
+        k_mg_res_parts<<<np, PCG_WG, 0, s>>>(ar, h->lev[0], x);
+        k_mg_check<<<1, PCG_WG, 0, s>>>(ar, it);
+      }
+      LAUNCH_CHECK("stationary iteration");
+    }
+    if (a.x != x)
+      HIP_TRY(hipMemcpyAsync(x, a.x, h->d.n2 * sizeof(double), hipMemcpyDeviceToDevice, s));
     int done = 0;
     TRY(poll_done(h, s, &done));
     if (done) break;
-    if (it > max_iter + 1)
-      return fail(HOC_ERR_DEVICE, "Helmholtz solve did not report completion");
-    batch = 4;
+    if (it > last) return fail(HOC_ERR_DEVICE, "Helmholtz solve did not report completion");
+    batch = stationary ? std::min(2 * batch, 64)  // slow stationary convergence: fewer polls
+                       : 4;
   }
   return pcg_finish(h, s, false, iters_out, conv_out, true);
 }

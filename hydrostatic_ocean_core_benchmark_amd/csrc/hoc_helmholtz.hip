@@ -512,6 +512,7 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_init_z(PcgArgs a) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     a.sc->norm_b = nb;
     a.sc->tol = a.rtol * nb;
+    a.sc->it = 1;
     a.sc->iters = 0;
     a.sc->converged = 1;
     a.sc->done = (nb == 0.0) ? 1 : 0;
@@ -557,7 +558,8 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_totals(PcgArgs a, int which) {
 
 // Iteration `it` (1-based), phase A. For it > 1 it first finishes
 // iteration it-1: the convergence test on ||r||, then beta and the new rz.
-// All loads that need no other (the solve's state, the partial sums, the
+// it < 0 (a recorded launch, never the first iteration): the number is sc->it,
+// -1 for odd ones and -2 for even ones. All loads that need no other (the solve's state, the partial sums, the
 // elements' operands) are issued before any is used.
 __global__ __launch_bounds__(PCG_WG) void k_pcg_ap(PcgArgs a, int it) {
   __shared__ double lds[PCG_STAGE];
@@ -569,6 +571,7 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_ap(PcgArgs a, int it) {
   const int part = blockIdx.x;
   const PartRange pr = part_range(a, part);
   const int done = a.sc->done;
+  const int n = it > 0 ? it : a.sc->it;
   const double tol = a.sc->tol, rz_old = a.sc->rz2[(it - 1) & 1];
   const double* parts[2] = {a.part_b, a.part_c};
   TotalsLoads<2> T;
@@ -597,12 +600,12 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_ap(PcgArgs a, int it) {
         a.sc->res = res;
         a.sc->done = 1;
         a.sc->converged = 1;
-        a.sc->iters = it - 1;
-        a.counters[0] += it - 1;
+        a.sc->iters = n - 1;
+        a.counters[0] += n - 1;
       }
       return;
     }
-    if (it - 1 >= a.max_iter) {
+    if (n - 1 >= a.max_iter) {
       if (lead) {
         a.sc->res = res;
         a.sc->done = 1;
@@ -638,6 +641,7 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_update(PcgArgs a, int it, int ja
   const int part = blockIdx.x;
   const PartRange pr = part_range(a, part);
   const int done = a.sc->done;
+  const int n = it > 0 ? it : a.sc->it;
   const double rz = a.sc->rz2[it & 1];
   const double* parts[1] = {a.part_a};
   TotalsLoads<1> T;
@@ -657,6 +661,7 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_update(PcgArgs a, int it, int ja
   if (a.central) pap = a.sc->tot[0];
   else totals_finish<1>(a, parts, T, cs, &pap);
   if (done) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) a.sc->it = n + 1;
   const double al = rz / pap;
 #pragma unroll
   for (int k = 0; k < PCG_EPT; ++k) {
