@@ -2117,17 +2117,30 @@ int split_barotropic(hoc_stepper* h, const double* eta, const double* gh_u, cons
   const Geo& geo = h->geo;
   const unsigned nb = blocks(d.n2);
   k_split_forcing<<<nb, TPB, 0, s>>>(d, p, geo, h->U0, h->V0, h->Ug, h->Vg, h->bfx, h->bfy);
-  if (p.bt_mean) {
-    HIP_TRY(hipMemsetAsync(h->acc_u, 0, d.n2 * sizeof(double), s));
-    HIP_TRY(hipMemsetAsync(h->acc_v, 0, d.n2 * sizeof(double), s));
-  }
   // transports rotate over three buffers: the substep's start and two
   // Picard iterates; the levels over two, the last substep writing out->eta
   const double* U = h->U0;
   const double* V = h->V0;
   const double* e = eta;
   int cur = -1;  // buffer index holding U, V (-1: U0, V0)
-  for (int n = 0; n < p.n_split; ++n) {
+  int n = 0;
+  while (n < p.n_split) {  // several substeps per launch
+    const int ns = std::min(BT_SUBSTEPS, p.n_split - n), q = cur == 0 ? 1 : 0;
+    double* e_new = n + ns == p.n_split ? out->eta : h->be[q];
+    if (!launch_bt_substeps(s, d, p, geo, n, ns, U, V, e, h->bfx, h->bfy, h->Ku, h->Kv, h->bU[q],
+                            h->bV[q], e_new, p.bt_mean ? h->acc_u : nullptr, h->acc_v))
+      break;
+    U = h->bU[q];
+    V = h->bV[q];
+    e = e_new;
+    cur = q;
+    n += ns;
+  }
+  if (n < p.n_split && p.bt_mean) {
+    HIP_TRY(hipMemsetAsync(h->acc_u, 0, d.n2 * sizeof(double), s));
+    HIP_TRY(hipMemsetAsync(h->acc_v, 0, d.n2 * sizeof(double), s));
+  }
+  for (; n < p.n_split; ++n) {  // more Picard passes than that: launch by launch
     const double* Ui = U;
     const double* Vi = V;
     int slot = -1;

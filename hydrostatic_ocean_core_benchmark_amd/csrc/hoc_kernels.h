@@ -95,6 +95,13 @@ __global__ void k_bt_picard(Dims d, StepParams p, Geo geo, const double* U, cons
                             const double* Kv, double* Uo, double* Vo);
 __global__ void k_bt_eta(Dims d, StepParams p, Geo geo, const double* e, const double* U,
                          const double* V, double* e_new, double* acc_u, double* acc_v);
+constexpr int BT_SUBSTEPS = 2;  // barotropic substeps of one launch
+// Substeps n0 .. n0 + ns - 1, ns <= BT_SUBSTEPS, from U, V, e into Uo, Vo, eo (buffers of their
+// own); false where there is no such kernel for the number of Picard passes.
+bool launch_bt_substeps(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo, int n0,
+                        int ns, const double* U, const double* V, const double* e, const double* fx,
+                        const double* fy, const double* Ku, const double* Kv, double* Uo,
+                        double* Vo, double* eo, double* acc_u, double* acc_v);
 __global__ void k_bt_mean(Dims d, StepParams p, const double* acc_u, const double* acc_v,
                           double* U, double* V);
 __global__ void k_split_final(Dims d, Geo geo, const double* gh_u, const double* gh_v,

@@ -942,6 +942,37 @@ __device__ __forceinline__ double avg_u_to_v(const double* u, const uint8_t* mu,
   return out * mk(mv[o + q.c]);
 }
 
+// Mean over the open ones of four faces (libs/core/operators_masked.py:46-61):
+// the weighted sum over the number of open faces, in the reference's order.
+// The quotient by 1, 2, 3 or 4 is formed like Divisor's, whose reciprocals are
+// the constants here.
+struct Avg4 {
+  double w[4], den, y, own;
+  bool any;
+  __device__ __forceinline__ Avg4(const bool* f, bool own_) {
+    int n = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      w[q] = f[q] ? 1.0 : 0.0;
+      n += (int)f[q];
+    }
+    den = (double)n;
+    y = n == 4 ? 0.25 : n == 3 ? 1.0 / 3.0 : n == 2 ? 0.5 : 1.0;
+    own = own_ ? 1.0 : 0.0;
+    any = n > 0;
+  }
+  __device__ __forceinline__ double operator()(double a0, double a1, double a2, double a3) const {
+    const double num = 0.0 + w[0] * a0 + w[1] * a1 + w[2] * a2 + w[3] * a3;
+    const double q = num * y;
+    const double r = __builtin_fma(-den, q, num);
+    const double m = __builtin_amdgcn_div_fixup(__builtin_fma(r, y, q), den, num);
+    return (any ? m : 0.0) * own;
+  }
+};
+__device__ __forceinline__ double avg4(const double* a, const bool* f, bool own) {
+  return Avg4(f, own)(a[0], a[1], a[2], a[3]);
+}
+
 // Explicit vertical diffusion Dz[f] at layer k with surface flux sflux, no
 // flux through a column's bottom interface and linear drag on the bottom
 // cell (libs/core/vertical_var.py:80-106). dzf is the thickness of f's
@@ -1341,6 +1372,156 @@ __global__ void k_bt_eta(Dims d, StepParams p, Geo geo, const double* __restrict
   }
 }
 
+// Up to S barotropic substeps of P Picard passes each in one launch, the same
+// operations per cell as k_bt_picard and k_bt_eta: a tile of BT_W x BT_H cells
+// with the halo that S substeps need (one cell per pass and one for the
+// level), one thread per cell of the region, its coefficients and own values in
+// registers and the fields that neighbours read in LDS. A cell beyond the halo
+// reads itself; no cell of the tile sees its value. From U, V, e into Uo, Vo,
+// eo; acc_u, acc_v: the transports summed for the averaged mode (from substep
+// 0 on; n0 is this launch's first), or null.
+//
+// Bound: latency (launch, loads, P + 1 barriers per substep). Two substeps of
+// two passes on 197 x 131 take 7.2 us against 24 in six launches; a step on 64 x
+// 64 x 12 188 us against 271, on 400 x 400 x 12 796 against 871, on 1000 x 1000
+// x 12 4429 against 4477. Tiles of 16 x 8 gain 1 to 3% on the small grids and
+// lose as much on the 400 x 400 one; three substeps per launch likewise.
+constexpr int BT_W = 16, BT_H = 16;
+template <int S, int P>
+struct BtRegion {
+  static constexpr int H = S * (P + 1), RW = BT_W + 2 * H, RH = BT_H + 2 * H, RN = RW * RH;
+  static constexpr int NT = (RN + 63) / 64 * 64;
+};
+template <int S, int P>
+__global__ __launch_bounds__((BtRegion<S, P>::NT)) void k_bt_substeps(
+    Dims d, StepParams p, Geo geo, int n0, int ns, const double* __restrict__ U,
+    const double* __restrict__ V, const double* __restrict__ e, const double* __restrict__ fx,
+    const double* __restrict__ fy, const double* __restrict__ Ku,
+    const double* __restrict__ Kv, double* __restrict__ Uo, double* __restrict__ Vo,
+    double* __restrict__ eo, double* __restrict__ acc_u, double* __restrict__ acc_v) {
+  using Rg = BtRegion<S, P>;
+  constexpr int RW = Rg::RW, RH = Rg::RH, H = Rg::H;
+  __shared__ double lu[3][Rg::RN], lv[3][Rg::RN], le[Rg::RN];
+  const bool on = (int)threadIdx.x < Rg::RN;
+  const int t = on ? (int)threadIdx.x : 0;
+  const int li = t % RW, lj = t / RW;
+  const int nx = d.nx, ny = d.ny;
+  auto wrapped = [](int x, int n) {
+    x %= n;
+    return x < 0 ? x + n : x;
+  };
+  const int ui = (int)blockIdx.x * BT_W + li - H, uj = (int)blockIdx.y * BT_H + lj - H;
+  const int i = wrapped(ui, nx), j = wrapped(uj, ny);
+  const Nb q = neighbours(d, j, i);
+  const int c = q.c;
+  // the region's neighbours
+  const int te = li + 1 < RW ? t + 1 : t, tw = li > 0 ? t - 1 : t;
+  const int tn = lj + 1 < RH ? t + RW : t, ts = lj > 0 ? t - RW : t;
+  const int tse = lj > 0 && li + 1 < RW ? t - RW + 1 : t;
+  const int tnw = lj + 1 < RH && li > 0 ? t + RW - 1 : t;
+  const bool ov = geo.mv2[c] != 0, ou = geo.mu2[c] != 0;
+  const bool fv[4] = {ov, geo.mv2[q.s] != 0, geo.mv2[q.e] != 0, geo.mv2[q.se] != 0};
+  const bool fu[4] = {ou, geo.mu2[q.w] != 0, geo.mu2[q.n] != 0, geo.mu2[q.nw] != 0};
+  const double mu = ou ? 1.0 : 0.0, mv = ov ? 1.0 : 0.0, m = mk(geo.m2[c]);
+  const double fxc = fx[c], fyc = fy[c], gKu = p.g * Ku[c], gKv = p.g * Kv[c];
+  const double cg = p.open_x || p.open_y ? sqrt(p.g * nmax(geo.H[c], 1.0)) : 0.0;
+  const Divisor<double> by_dx = uniform_divisor<double>(p.dx), by_dy = uniform_divisor<double>(p.dy);
+  const Avg4 to_u(fv, ou), to_v(fu, ov);
+  double u0 = U[c], v0 = V[c], ec = e[c];
+  const bool own = on && li >= H && li < H + BT_W && lj >= H && lj < H + BT_H && ui < nx && uj < ny;
+  double au = 0.0, av = 0.0;
+  if (acc_u && own && n0 > 0) {
+    au = acc_u[c];
+    av = acc_v[c];
+  }
+  int start = 0;  // the buffers of the substep's start and of the last iterate
+  if (on) {
+    lu[0][t] = u0;
+    lv[0][t] = v0;
+    le[t] = ec;
+  }
+  __syncthreads();
+  for (int n = 0; n < ns; ++n) {
+    const double gxe = by_dx(mu * (le[te] - ec)), gye = by_dy(mv * (le[tn] - ec));
+    auto avg_v = [&](const double* f, double own_v) { return to_u(own_v, f[ts], f[te], f[tse]); };
+    auto avg_u = [&](const double* f, double own_u) { return to_v(own_u, f[tw], f[tn], f[tnw]); };
+    const double av0 = avg_v(lv[start], v0), au0 = avg_u(lu[start], u0);
+    double un = u0, vn = v0;
+    int it = start;
+#pragma unroll
+    for (int m_ = 0; m_ < P; ++m_) {
+      const double v_cor = p.one_m_tc * av0 + p.theta_cor * (m_ == 0 ? av0 : avg_v(lv[it], vn));
+      const double u_cor = p.one_m_tc * au0 + p.theta_cor * (m_ == 0 ? au0 : avg_u(lu[it], un));
+      un = (u0 + p.ddt * (p.f * v_cor - gKu * gxe + fxc)) * mu;
+      vn = (v0 + p.ddt * (p.neg_f * u_cor - gKv * gye + fyc)) * mv;
+      int nxt = 0;  // the buffer that is neither the start's nor the last iterate's
+      while (nxt == start || nxt == it) ++nxt;
+      if (on) {
+        lu[nxt][t] = un;
+        lv[nxt][t] = vn;
+      }
+      it = nxt;
+      __syncthreads();
+    }
+    // e - ddt div(U, V) as div_bt forms it
+    const double uw = lu[it][tw], vs = lv[it][ts];
+    double dv = m * (by_dx(un - uw) + by_dy(vn - vs));
+    if (p.open_x || p.open_y) {
+      if (p.open_x && i == 0) {
+        const double bw = p.u_ext - cg * (ec - p.eta_ext);
+        dv = dv + (by_dx(un - bw) - by_dx(un - uw));
+      }
+      if (p.open_x && i == nx - 1) {
+        const double be = p.u_ext + cg * (ec - p.eta_ext);
+        dv = dv + (by_dx(be - uw) - by_dx(un - uw));
+      }
+      if (p.open_y && j == 0) {
+        const double bs = p.u_ext - cg * (ec - p.eta_ext);
+        dv = dv + (by_dy(vn - bs) - by_dy(vn - vs));
+      }
+      if (p.open_y && j == ny - 1) {
+        const double bn = p.u_ext + cg * (ec - p.eta_ext);
+        dv = dv + (by_dy(bn - vs) - by_dy(vn - vs));
+      }
+      dv = dv * m;
+    }
+    ec = ec - p.ddt * dv;
+    if (on) le[t] = ec;
+    u0 = un;
+    v0 = vn;
+    start = it;
+    au = au + un;
+    av = av + vn;
+    if (n + 1 < ns) __syncthreads();
+  }
+  if (!own) return;
+  Uo[c] = u0;
+  Vo[c] = v0;
+  eo[c] = ec;
+  if (acc_u) {
+    acc_u[c] = au;
+    acc_v[c] = av;
+  }
+}
+
+bool launch_bt_substeps(hipStream_t s, const Dims& d, const StepParams& p, const Geo& geo, int n0,
+                        int ns, const double* U, const double* V, const double* e, const double* fx,
+                        const double* fy, const double* Ku, const double* Kv, double* Uo,
+                        double* Vo, double* eo, double* acc_u, double* acc_v) {
+  const dim3 grid((unsigned)((d.nx + BT_W - 1) / BT_W), (unsigned)((d.ny + BT_H - 1) / BT_H));
+  auto go = [&](auto pp) {
+    constexpr int P = decltype(pp)::value;
+    k_bt_substeps<BT_SUBSTEPS, P><<<grid, BtRegion<BT_SUBSTEPS, P>::NT, 0, s>>>(
+        d, p, geo, n0, ns, U, V, e, fx, fy, Ku, Kv, Uo, Vo, eo, acc_u, acc_v);
+  };
+  // a region of up to 1024 cells: three passes at most
+  if (p.n_picard == 1) go(std::integral_constant<int, 1>{});
+  else if (p.n_picard == 2) go(std::integral_constant<int, 2>{});
+  else if (p.n_picard == 3) go(std::integral_constant<int, 3>{});
+  else return false;
+  return true;
+}
+
 __global__ void k_bt_mean(Dims d, StepParams p, const double* __restrict__ acc_u,
                           const double* __restrict__ acc_v, double* __restrict__ U,
                           double* __restrict__ V) {
@@ -1380,23 +1561,6 @@ __global__ void k_face_depth(Dims d, Geo geo, double* __restrict__ Hu, double* _
 }
 
 // ------------------------------------------- predictor and column solves
-// Mean over the open ones of four faces (libs/core/operators_masked.py:46-61):
-// the weighted sum over the number of open faces, in the reference's order.
-// The quotient by 1, 2, 3 or 4 is formed like Divisor's, whose reciprocals are
-// the constants here.
-__device__ __forceinline__ double avg4(const double* a, const bool* f, bool own) {
-  const double w0 = f[0] ? 1.0 : 0.0, w1 = f[1] ? 1.0 : 0.0;
-  const double w2 = f[2] ? 1.0 : 0.0, w3 = f[3] ? 1.0 : 0.0;
-  const double num = 0.0 + w0 * a[0] + w1 * a[1] + w2 * a[2] + w3 * a[3];
-  const int n = (int)f[0] + (int)f[1] + (int)f[2] + (int)f[3];
-  const double den = (double)n;
-  const double y = n == 4 ? 0.25 : n == 3 ? 1.0 / 3.0 : n == 2 ? 0.5 : 1.0;
-  const double q = num * y;
-  const double r = __builtin_fma(-den, q, num);
-  const double m = __builtin_amdgcn_div_fixup(__builtin_fma(r, y, q), den, num);
-  return (n > 0 ? m : 0.0) * (own ? 1.0 : 0.0);
-}
-
 // One Picard pass (model3d_v05.py:387-396), one wave per 64 columns and
 // velocity component:
 //   v_cor = (1-tc) avg_v_to_u(v) + tc avg_v_to_u(v_it),  u_cor likewise
