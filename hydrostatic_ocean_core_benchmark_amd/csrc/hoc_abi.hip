@@ -1867,7 +1867,7 @@ int hoc_stepper_create(const hoc_config* cfg, const hoc_geometry* g, hoc_stepper
         hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) == hipSuccess &&
         hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void*)k_pcg_persistent,
                                                      PCG_WG, 0) == hipSuccess &&
-        coop && parts <= (long long)ncu * per_cu) {
+        coop && h->red.nchunks <= PCG_COOP_CHUNKS && parts <= (long long)ncu * per_cu) {
       h->pcg_parts = (int)parts;
     }
     if (cfg->closure_tke && !cfg->mxl_recursive) {

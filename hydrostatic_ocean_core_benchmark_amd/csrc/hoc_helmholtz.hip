@@ -384,7 +384,7 @@ __device__ __forceinline__ int logical_block(int nb) {
 
 __global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
   __shared__ double lds[2 * PCG_STAGE];
-  __shared__ double cs[2 * PCG_CS];
+  __shared__ double cs[2 * PCG_COOP_CS];  // its workgroups must all be resident
   const unsigned nb = gridDim.x;
   const int part = logical_block((int)nb);
   const HelmOp& op = a.op;
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
     if (!ok) break;
     const double* parts[2] = {a.part_b, a.part_c};
     double tot[2];
-    totals_from_parts<2>(a, parts, cs, tot);
+    totals_from_parts<2, PCG_COOP_CS>(a, parts, cs, tot);
     res = sqrt(tot[0]);
     if (res <= tol) {
       done = 1;

@@ -381,6 +381,8 @@ constexpr int PCG_PART = 512;       // elements of one: 8192 / PCG_SUB
 constexpr int PCG_EPT = PCG_PART / PCG_WG;  // elements of a part per thread
 constexpr int PCG_STAGE = 544;      // LDS values that stage a part (stage_at)
 constexpr int PCG_MAX_CHUNKS = 1024;
+constexpr int PCG_COOP_CHUNKS = 256;  // ... of the cooperative launch
+constexpr int PCG_COOP_CS = PCG_COOP_CHUNKS + 8;
 
 // One level of the multigrid hierarchy (level 0 is the model grid).
 // One multigrid level: face coefficients, diagonal and constants in the

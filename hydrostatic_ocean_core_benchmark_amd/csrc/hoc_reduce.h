@@ -169,9 +169,9 @@ __device__ __forceinline__ TotalsLoads<NV> totals_load(const PcgArgs& a,
   return L;
 }
 
-template <int NV>
+template <int NV, int CS = PCG_CS>
 __device__ __forceinline__ void totals_finish(const PcgArgs& a, const double* const* part,
-                                              TotalsLoads<NV> L, double* cs /* [NV][PCG_CS] */,
+                                              TotalsLoads<NV> L, double* cs /* [NV][CS] */,
                                               double* out) {
   const int trow = totals_tail_row(a), rows = totals_rows(a);
   const int row = threadIdx.x >> 4, lane = threadIdx.x & 15;
@@ -184,14 +184,14 @@ __device__ __forceinline__ void totals_finish(const PcgArgs& a, const double* co
 #pragma unroll
       for (int q = 0; q < NV; ++q) {
         const double s = sum16(L.v[k][q]);
-        if (lane == 0 && c < rows) cs[q * PCG_CS + c] = s;
+        if (lane == 0 && c < rows) cs[q * CS + c] = s;
       }
     }
   }
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < NV; ++q) {
-    const double* v = cs + q * PCG_CS;
+    const double* v = cs + q * CS;
     double s = 0.0;
     for (int c = 0; c < trow; c += 8) {
       double w[8];
@@ -211,10 +211,10 @@ __device__ __forceinline__ void totals_finish(const PcgArgs& a, const double* co
   }
 }
 
-template <int NV>
+template <int NV, int CS = PCG_CS>
 __device__ __forceinline__ void totals_from_parts(const PcgArgs& a, const double* const* part,
                                                   double* cs, double* out) {
-  totals_finish<NV>(a, part, totals_load<NV>(a, part), cs, out);
+  totals_finish<NV, CS>(a, part, totals_load<NV>(a, part), cs, out);
 }
 
 __device__ __forceinline__ double total_from_parts(const PcgArgs& a, const double* part,
