@@ -192,22 +192,11 @@ __device__ __forceinline__ FaceCol face_col(const Geo& geo, const StepParams& p,
   return f;
 }
 
-// Tile of this workgroup in a 2D grid, remapped so that each of the 8 XCDs
-// (workgroups are dispatched to them round-robin by linear id) owns one
-// contiguous band of tile rows: neighbouring tiles then share their halo
-// rows in the same L2. A bijection for any grid size.
-__device__ __forceinline__ void xcd_tile(int& bx, int& by) {
-  const int gx = (int)gridDim.x;
-  const int nb = gx * (int)gridDim.y;
-  const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x);
-  const int x = id % 8, q = nb / 8, r = nb % 8;
-  const int L = x * q + (x < r ? x : r) + id / 8;
-  bx = L % gx;
-  by = L / gx;
-}
-
-// The same for a 1D grid of gx x gy tiles by `parts` workgroups per tile and
-// range of levels: part fastest (a tile's parts read the same fields, so they
+// Tile of this workgroup in a 1D grid of gx x gy tiles by `parts` workgroups per
+// tile and range of levels, remapped so that each of the 8 XCDs (workgroups are
+// dispatched to them round-robin) owns one contiguous run of them: neighbouring
+// tiles then share their halo rows in one L2. A bijection for any grid size; part
+// fastest (a tile's parts read the same fields, so they
 // run side by side on one XCD), then x, y and the range of levels z.
 struct BlockTile {
   int part, x, y, z;
@@ -483,17 +472,6 @@ __device__ __forceinline__ void matrix_row(const StepParams& p, int k, double in
   den_o = (k == 0) ? diag : diag - sub * c_prev;
   sub_o = sub;
   sup_o = sup;
-}
-// The same factored: sub, den and c* = sup / den.
-__device__ __forceinline__ void factor_row(const StepParams& p, int k, double inv_dz,
-                                           double nu_t, double nu_b, double idzi_t,
-                                           double idzi_b, bool wet, bool below,
-                                           double drag_term, double c_prev, double& sub_o,
-                                           double& den_o, double& cst_o) {
-  double sup;
-  matrix_row(p, k, inv_dz, nu_t, nu_b, idzi_t, idzi_b, wet, below, drag_term, c_prev, sub_o, sup,
-             den_o);
-  cst_o = sup / den_o;
 }
 
 // ------------------------------------------------------------------ EOS

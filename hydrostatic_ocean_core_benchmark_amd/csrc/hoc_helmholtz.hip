@@ -382,7 +382,10 @@ __device__ __forceinline__ int logical_block(int nb) {
   return (w % 8) * (nb / 8) + (w / 8);
 }
 
-__global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
+// Seven workgroups per compute unit: the launch takes grids of up to 1792 parts.
+// Per iteration 12.0 us on 128 x 128, 33.9 on 512 x 512 and 72.8 on 1000 x 512
+// (13.8, 36.5 and 85.1 with the sums walked leaf by leaf, six per compute unit).
+__global__ __launch_bounds__(PCG_WG, 7) void k_pcg_persistent(PcgArgs a) {
   __shared__ double lds[2 * PCG_STAGE];
   __shared__ double cs[2 * PCG_COOP_CS];  // its workgroups must all be resident
   const unsigned nb = gridDim.x;
@@ -395,7 +398,7 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
 
   // r = rhs * mask, x = 0; ||rhs||
   {
-    const double s = part_sum(a, part, [&](long long e) -> double {
+    const double s = part_sum_each(a, part, [&](long long e) -> double {
       const double r = a.rhs[e] * mk(op.mask[e]);
       a.r[e] = r;
       a.x[e] = 0.0;
@@ -412,7 +415,7 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
   }
   if (ok && !done) {
     // z = M^-1 r, p = z (into pb1, the buffer iteration 1 uses); r.z
-    const double s = part_sum(a, part, [&](long long e) -> double {
+    const double s = part_sum_each(a, part, [&](long long e) -> double {
       const double z = a.inv_diag[e] * a.r[e];
       a.z[e] = z;
       a.pb1[e] = z;
@@ -429,7 +432,7 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
     const bool first = it == 1;
     const double bt = beta;
     {
-      const double s = part_sum(a, part, [&](long long e) -> double {
+      const double s = part_sum_each(a, part, [&](long long e) -> double {
         return pcg_apply_elem(a, e, first, bt, pnew, pold);
       }, lds);
       if (threadIdx.x == 0) a.part_a[part] = s;
@@ -440,6 +443,7 @@ __global__ __launch_bounds__(PCG_WG) void k_pcg_persistent(PcgArgs a) {
     {
       const double al = alpha;
       const PartRange pr = part_range(a, part);
+#pragma unroll 1
       for (int t = threadIdx.x; t < pr.nel; t += PCG_WG) {
         const Two v = pcg_update_elem(a, pr.base + t, al, pnew);
         lds[stage_at(t)] = v.a;

@@ -132,6 +132,16 @@ __device__ __forceinline__ double part_sum(const PcgArgs& a, int part, F elem,
   return part_reduce<1>(pr, lds);
 }
 
+// The same, one element after the other: half the registers, for the
+// cooperative kernel, whose workgroups must all be resident.
+template <class F>
+__device__ __forceinline__ double part_sum_each(const PcgArgs& a, int part, F elem, double* lds) {
+  const PartRange pr = part_range(a, part);
+#pragma unroll 1
+  for (int t = threadIdx.x; t < pr.nel; t += PCG_WG) lds[stage_at(t)] = elem(pr.base + t);
+  return part_reduce<1>(pr, lds);
+}
+
 // In-order float64 sums of whole vectors from their per-part partials: sixteen
 // lanes sum a full chunk's subtrees pairwise, the trailing chunk's slots are
 // rows of sixteen of its tree, then the chunk sums are added sequentially.
