@@ -1960,8 +1960,9 @@ int hoc_stepper_create(const hoc_config* cfg, const hoc_geometry* g, hoc_stepper
       ldy = ldy * 2.0;
     }
   }
+  // (a mixed handle of any other solver name belongs to a scheme that solves nothing)
   if ((cfg->solver == SOLVER_PCG_MG && cfg->mg_sweeps <= MG_FUSED_MAX_SWEEPS) ||
-      cfg->solver == SOLVER_MULTIGRID) {
+      (cfg->solver == SOLVER_MULTIGRID && cfg->precision == 0)) {
     int l0 = -1;
     for (int l = 0; l < h->nlev; ++l)
       if (h->lev[l].n <= MG_COARSE_MAX) {

@@ -97,3 +97,25 @@ def test_mixed_rejects_other_solvers(hoc):
     prob = basin(nx=64, nz=40, solver="pcg_jacobi")
     with pytest.raises(ValueError, match="pcg_mg only"):
         hoc.HipStepper(prob.domain, prob.physics, prob.params, prob.dt, precision="mixed")
+
+
+@pytest.mark.parametrize("scheme", ["fb", "split_explicit"])
+@pytest.mark.parametrize("nx,ny", [(131, 77), (140, 100), (64, 48)])
+def test_mixed_without_a_solve_takes_any_solver_name(hoc, nx, ny, scheme):
+    """The schemes that solve nothing take mixed precision with every solver
+    name, also where that solver's hierarchy would end in a level too large for
+    one workgroup (131 x 77 has 10087 cells and no coarser level). Two steps,
+    the same bits whatever the name."""
+    import dataclasses
+    from test_gpu_level_ranges import _problem
+    from hydrostatic_ocean_core_benchmark_amd.types import State3D
+    dom, phys, params, f = _problem(nx, ny, 3, "zlevel", "up3_tvd")
+    out = {}
+    for solver in ("pcg_jacobi", "multigrid", "rbgs"):
+        p = dataclasses.replace(params, name=scheme, solver=solver)
+        with hoc.HipStepper(dom, phys, p, 60.0, precision="mixed") as st:
+            s = st.step(st.step(State3D(**f)))
+            out[solver] = {k: _np(getattr(s, k)) for k in ("u", "v", "eta", "T", "S", "b", "e")}
+    for solver in ("multigrid", "rbgs"):
+        for k, want in out["pcg_jacobi"].items():
+            assert np.array_equal(out[solver][k], want), (solver, k)
