@@ -128,29 +128,21 @@ struct Reducer {
 }  // namespace
 
 // ------------------------------------------------------------ the handle
-// PCG-Jacobi iterations recorded as HIP graphs of 2 << q iterations each, on
-// the step's own operands (see jacobi_iterations).
+// PCG-Jacobi iterations as HIP graphs of 2 << q iterations each, on the step's
+// own operands, which a handle never moves (see pcg_iterations).
 struct IterGraphs {
   static constexpr int SIZES = 6;
-  // Recording costs about as much as three steps gain (131 x 77): not before
-  // this many solves in a row on the same operands.
+  // Building costs about as much as three steps gain (131 x 77): not before
+  // this many solves on those operands.
   static constexpr int WARM_SOLVES = 8;
-  PcgArgs key{};
-  int solves = 0;       // solves in a row on key
-  bool failed = false;  // recording failed: launches only
+  int solves = 0;
+  bool failed = false;  // building failed: launches only
   hipGraph_t graph[SIZES] = {};
   hipGraphExec_t exec[SIZES] = {};
-  bool any() const {
-    for (hipGraphExec_t e : exec)
-      if (e) return true;
-    return false;
-  }
   void clear() {
     for (int q = 0; q < SIZES; ++q) {
       if (exec[q]) (void)hipGraphExecDestroy(exec[q]);
       if (graph[q]) (void)hipGraphDestroy(graph[q]);
-      exec[q] = nullptr;
-      graph[q] = nullptr;
     }
   }
 };
@@ -216,7 +208,6 @@ struct hoc_stepper {
   int sf_key_budget = 0, sf_key_tile = -1;
   double* sf_x = nullptr;  // fixed solution buffer of the step's graph-replayed solves
   IterGraphs it_graphs;
-  hipStream_t record = nullptr;  // the iterations' graphs are recorded on it; runs nothing
   int mg_tile_shape = 0;     // fused V-cycle leg tile shape (0..MG_TILE_SHAPES-1)
                              // default by size: 16x16 up to 512x512 columns
                              // (5.50 vs 5.66 ms/step at 512x512x40), else 32x16
@@ -261,7 +252,6 @@ struct hoc_stepper {
     if (sf_exec) (void)hipGraphExecDestroy(sf_exec);
     if (sf_graph) (void)hipGraphDestroy(sf_graph);
     it_graphs.clear();
-    if (record) (void)hipStreamDestroy(record);
     for (hipEvent_t e : prof_ev) (void)hipEventDestroy(e);
     for (void* v : allocs) (void)hipFree(v);
     if (host_flag) (void)hipHostFree(host_flag);
@@ -890,8 +880,8 @@ int precondition(hoc_stepper* h, const double* r, double* z, hipStream_t s) {
   return HOC_OK;
 }
 
-// One PCG iteration: the launches of iteration `it` on s; it = -1 or -2 stands
-// for any odd or even one whose number the device knows (Jacobi only).
+// One PCG iteration: the launches of iteration `it` on s (iteration_graph's
+// nodes are those of the Jacobi one).
 int pcg_iteration(hoc_stepper* h, const PcgArgs& a, hipStream_t s, int it) {
   const unsigned np = (unsigned)h->pcg_parts_all;
   const int jacobi = h->cfg.solver == SOLVER_PCG_JACOBI ? 1 : 0;
@@ -907,10 +897,10 @@ int pcg_iteration(hoc_stepper* h, const PcgArgs& a, hipStream_t s, int it) {
   return HOC_OK;
 }
 
-// Whether the Jacobi iterations with operands a (x and rhs left out) may be
-// replayed on stream s: after WARM_SOLVES solves in a row with them, not while a
-// phase is profiled by name or the caller captures the stream.
-bool iteration_graphs_usable(hoc_stepper* h, const PcgArgs& a, hipStream_t s) {
+// Whether the Jacobi iterations on the step's own operands may be replayed on
+// stream s: after WARM_SOLVES solves with them, not while a phase is profiled
+// by name or the caller captures the stream.
+bool iteration_graphs_usable(hoc_stepper* h, hipStream_t s) {
   IterGraphs& g = h->it_graphs;
   if (h->prof_name == "k_pcg_ap" || h->prof_name == "k_pcg_update") return false;
   if (s != nullptr) {
@@ -918,29 +908,34 @@ bool iteration_graphs_usable(hoc_stepper* h, const PcgArgs& a, hipStream_t s) {
     if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
       return false;
   }
-  PcgArgs key;
-  std::memcpy(&key, &a, sizeof(a));  // compared byte by byte
-  key.rhs = nullptr;
-  key.x = nullptr;
-  if (std::memcmp(&g.key, &key, sizeof(key)) != 0) {
-    if (g.any()) (void)hipDeviceSynchronize();  // a replay of the old ones may still run
-    g.clear();
-    std::memcpy(&g.key, &key, sizeof(key));
-    g.solves = 0;
-  }
   return ++g.solves > IterGraphs::WARM_SOLVES && !g.failed;
 }
 
-// The graph of 2 << q iterations, recorded on first use; null if that fails.
-hipGraphExec_t iteration_graph(hoc_stepper* h, const PcgArgs& a, int q) {
+// The graph of 2 << q iterations from an even one on, built on first use; null
+// if that fails. A chain of kernel nodes, added one by one: nothing is
+// captured or allocated, which another thread's capture could forbid.
+hipGraphExec_t iteration_graph(hoc_stepper* h, PcgArgs a, int q) {
   IterGraphs& g = h->it_graphs;
   if (g.exec[q] || g.failed) return g.exec[q];
-  bool ok = h->record || hipStreamCreateWithFlags(&h->record, hipStreamNonBlocking) == hipSuccess;
-  ok = ok && hipStreamBeginCapture(h->record, hipStreamCaptureModeRelaxed) == hipSuccess;
-  if (ok) {
-    for (int i = 0; i < (2 << q) && ok; ++i)
-      ok = pcg_iteration(h, a, h->record, (i & 1) ? -1 : -2) == HOC_OK;
-    ok = hipStreamEndCapture(h->record, &g.graph[q]) == hipSuccess && g.graph[q] && ok;
+  bool ok = hipGraphCreate(&g.graph[q], 0) == hipSuccess;
+  hipGraphNode_t last = nullptr;
+  auto add = [&](void* kernel, void** args) {
+    hipKernelNodeParams node{};
+    node.func = kernel;
+    node.gridDim = dim3((unsigned)h->pcg_parts_all);
+    node.blockDim = dim3(PCG_WG);
+    node.kernelParams = args;
+    hipGraphNode_t n = nullptr;
+    ok = ok && hipGraphAddKernelNode(&n, g.graph[q], last ? &last : nullptr, last ? 1 : 0,
+                                     &node) == hipSuccess;
+    last = n;
+  };
+  int it, jacobi = 1;
+  void* args[3] = {&a, &it, &jacobi};
+  for (int i = 0; i < (2 << q) && ok; ++i) {
+    it = (i & 1) ? -1 : -2;
+    add((void*)k_pcg_ap, args);
+    add((void*)k_pcg_update, args);
   }
   ok = ok && hipGraphInstantiate(&g.exec[q], g.graph[q], nullptr, nullptr, 0) == hipSuccess;
   if (!ok) {
@@ -1085,8 +1080,7 @@ int helmholtz_solve(hoc_stepper* h, const double* Ku, const double* Kv, const do
   // replayed iterations solve into a buffer of the handle's, copied to x
   bool replay = false;
   if (kind == SOLVER_PCG_JACOBI && h->d.n2 <= ITER_GRAPH_CELLS && Ku == h->Ku && Kv == h->Kv &&
-      inv_diag == h->inv_diag && iteration_graphs_usable(h, a, s)) {
-    if (!h->sf_x) TRY(h->alloc(&h->sf_x, h->d.n2));
+      inv_diag == h->inv_diag && iteration_graphs_usable(h, s)) {
     a.x = h->sf_x;
     replay = true;
   }
@@ -1844,6 +1838,8 @@ int hoc_stepper_create(const hoc_config* cfg, const hoc_geometry* g, hoc_stepper
   A(h->bar_err, 1);
   A(h->sc, 1);
   A(h->dcount, 4);
+  if (cfg->scheme == 0 && cfg->solver == SOLVER_PCG_JACOBI && d.n2 <= ITER_GRAPH_CELLS)
+    A(h->sf_x, d.n2);
 #undef A
   {
     int rc = h->red.init(d.n2);

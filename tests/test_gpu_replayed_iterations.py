@@ -48,3 +48,53 @@ def test_steps_match_oracle(hoc, max_iter, side_stream):
             for k in ("u", "v", "eta", "T", "S"):
                 g, w = getattr(got, k).cpu().numpy(), getattr(want, k)
                 assert np.array_equal(g, w), (n, k, rel_l2(g, w))
+
+
+def test_steps_while_another_thread_captures(hoc):
+    """A handle stepped through its first replayed solves while another thread
+    captures a graph (in the thread-local mode: in the global one a polled
+    step's synchronisation is refused, with or without replays): the state and
+    the graph come out right."""
+    import threading
+    dom, phys, params, f = _problem(37, 22, 6, "zlevel", "up3_tvd")
+    params = dataclasses.replace(params, name="theta")
+    got, err = {}, []
+    with hoc.HipStepper(dom, phys, params, 300.0) as st, \
+            hoc.HipStepper(dom, phys, params, 300.0) as plain:
+        runs = []
+        for h in (st, plain):
+            a, b = h._new_state_buffers(), h._new_state_buffers()
+            for k, buf in a.items():
+                buf.copy_(torch.as_tensor(f[k]))
+            runs.append((a, b))
+        want = plain._step_n_into(*runs[1], 8)
+        side, cap = torch.cuda.Stream(), torch.cuda.Stream()
+        y = torch.zeros(1000, device="cuda")
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+
+        def steps():
+            try:
+                with torch.cuda.stream(side):
+                    got.update(st._step_n_into(*runs[0], 8))
+            except Exception as e:
+                err.append(e)
+
+        with torch.cuda.stream(cap):
+            graph.capture_begin(capture_error_mode="thread_local")
+            y.add_(1.0)
+            t = threading.Thread(target=steps)
+            t.start()
+            t.join()
+            try:
+                graph.capture_end()
+            except Exception as e:
+                err.append(e)
+        assert not err, err
+        torch.cuda.synchronize()
+        for n in range(3):
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.all(y == n + 1.0), n
+        for k, w in want.items():
+            assert torch.equal(got[k], w), k
