@@ -25,6 +25,7 @@ constexpr int COLS = 64;
 // Sweeps keep a column in LDS up to here (two or more workgroups per compute
 // unit); deeper columns use the global work arrays.
 constexpr size_t COL_LDS_MAX = 64 * 1024;
+constexpr long long CUS = 256, CU_LDS = 160 * 1024;  // compute units, LDS of one
 static unsigned column_blocks(const Dims& d) { return (unsigned)((d.n2 + COLS - 1) / COLS); }
 
 // go(zc, stage) with the two flags as compile-time constants.
@@ -335,20 +336,24 @@ __global__ void k_mixing_recursive(Dims d, StepParams p, Geo geo, const double* 
 // The interface tridiagonal for e and the eddy coefficients, one lane per
 // column, from s_n2, s_sh, s_l = l_k and s_le = l_eps. ZC: thicknesses and wet
 // flags from the column form. STAGE: c* and d* stay in LDS between the sweeps
-// instead of in s_c and e_out.
-// Bound: latency of the march on small grids, then memory (10 fields) and the
-// roots and divisions at the few waves that LDS leaves. Per launch, against no
-// loads ahead and c*, d* in memory: 128 x 4 x 20 33 -> 18 us, 128 x 128 x 30
-// 51 -> 26, 512 x 512 x 40 212 -> 214, 640 x 512 x 48 326 -> 289, 1000 x 1000
-// x 30 676 -> 495.
-template <bool ZC, bool STAGE>
-__global__ __launch_bounds__(COLS) void k_closure(
+// instead of in s_c and e_out. NT: threads of a workgroup.
+// Bound: latency of the march on small grids, then memory (10 fields, 14
+// unstaged) and the roots and divisions at the few waves that LDS leaves. Per
+// launch, against no loads ahead and c*, d* in memory: 128 x 4 x 20 33 -> 18
+// us, 128 x 128 x 30 51 -> 26, 640 x 512 x 48 326 -> 308, 1000 x 1000 x 30
+// 675 -> 513; 512 x 512 x 40 212 -> 219, whose levels are exactly 2 MiB apart
+// (448 x 448 x 40 175 -> 172, 576 x 576 x 40 302 -> 266); where launch_closure
+// leaves it unstaged 384 x 384 x 60 210 -> 190, 512 x 512 x 60 318 -> 316, 800 x
+// 800 x 60 846 -> 826.
+template <bool ZC, bool STAGE, int NT>
+__global__ __launch_bounds__(NT) void k_closure(
     Dims d, StepParams p, Geo geo, const double* __restrict__ e_in, double* __restrict__ Km,
     double* __restrict__ Kh, double* __restrict__ e_out, const double* __restrict__ s_n2,
     const double* __restrict__ s_sh, const double* __restrict__ s_l,
     const double* __restrict__ s_le, double* __restrict__ s_c) {
   extern __shared__ double clo_lds[];  // STAGE: [2][nz + 1][COLS], a thread's own column
-  const long long c = (long long)xcd_linear() * COLS + threadIdx.x;
+  static_assert(!STAGE || NT == COLS, "a staged column per lane of one wave");
+  const long long c = (long long)(NT == COLS ? xcd_linear() : blockIdx.x) * NT + threadIdx.x;
   if (c >= d.n2) return;
   const int nz = d.nz;
   const long long n2 = d.n2;
@@ -373,7 +378,7 @@ __global__ __launch_bounds__(COLS) void k_closure(
   // the cell above interface k, carried down the column
   double km_up = 0.0, km_0 = Km[c], inv_up = 0.0;
   bool wet_above = false;
-  march_down<4>(
+  march_down<STAGE ? 4 : 3>(  // 3: four unstaged waves per SIMD instead of three
       nz + 1,
       [&](int k) {
         const long long o = k * n2;
@@ -484,9 +489,29 @@ void launch_closure(hipStream_t s, const Dims& d, const StepParams& p, const Geo
                     const double* s_n2, const double* s_sh, const double* s_l,
                     const double* s_le, double* s_c) {
   const size_t lds = (size_t)2 * (d.nz + 1) * COLS * sizeof(double);
-  with_column_form(p.zcol != 0, lds <= COL_LDS_MAX, [&](auto zc, auto sg) {
-    constexpr bool SG = decltype(sg)::value;
-    k_closure<decltype(zc)::value, SG><<<column_blocks(d), COLS, SG ? lds : 0, s>>>(
+  const long long waves = column_blocks(d), per_cu = CU_LDS / (long long)lds;
+  // Staged where LDS holds three workgroups per compute unit, or the whole grid
+  // at once; with two of them (53 levels and more) a large grid gains less from
+  // the four passes saved than it loses in waves. Staged and not: 384 x 384 x
+  // 40 126 and 124 us, 640 x 512 x 48 308 and 340, 128 x 128 x 60 45 and 50,
+  // 320 x 320 x 60 174 and 132, 512 x 512 x 60 370 and 316, 800 x 800 x 60 880
+  // and 826.
+  const bool stage = lds <= COL_LDS_MAX && (per_cu >= 3 || waves <= CUS * per_cu);
+  // Unstaged, workgroups of four waves from four per compute unit on; fewer
+  // spread unevenly. One wave and four: 384 x 384 x 60 190 and 210 us, 448 x
+  // 448 x 40 177 and 185, 512 x 512 x 60 340 and 316, 704 x 704 x 40 434 and 421.
+  const bool wide = waves >= 16 * CUS;
+  with_column_form(p.zcol != 0, stage, [&](auto zc, auto sg) {
+    constexpr bool ZC = decltype(zc)::value, SG = decltype(sg)::value;
+    constexpr int WIDE = 4 * COLS;
+    if constexpr (!SG) {
+      if (wide) {
+        k_closure<ZC, SG, WIDE><<<(unsigned)((d.n2 + WIDE - 1) / WIDE), WIDE, 0, s>>>(
+            d, p, geo, e_in, Km, Kh, e_out, s_n2, s_sh, s_l, s_le, s_c);
+        return;
+      }
+    }
+    k_closure<ZC, SG, COLS><<<column_blocks(d), COLS, SG ? lds : 0, s>>>(
         d, p, geo, e_in, Km, Kh, e_out, s_n2, s_sh, s_l, s_le, s_c);
   });
 }
