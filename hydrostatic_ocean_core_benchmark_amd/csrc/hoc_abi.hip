@@ -2134,8 +2134,8 @@ int split_barotropic(hoc_stepper* h, const double* eta, const double* gh_u, cons
     n += ns;
   }
   if (n < p.n_split && p.bt_mean) {
-    HIP_TRY(hipMemsetAsync(h->acc_u, 0, d.n2 * sizeof(double), s));
-    HIP_TRY(hipMemsetAsync(h->acc_v, 0, d.n2 * sizeof(double), s));
+    k_fill<<<nb, TPB, 0, s>>>(d.n2, 0.0, h->acc_u);
+    k_fill<<<nb, TPB, 0, s>>>(d.n2, 0.0, h->acc_v);
   }
   for (; n < p.n_split; ++n) {  // more Picard passes than that: launch by launch
     const double* Ui = U;
@@ -2622,8 +2622,8 @@ int hoc_stepper_pressure_gradients(hoc_stepper* h, const double* b, double* pgx,
   const Dims d = h->d;
   // The explicit-momentum kernel computes the gradient along with the other
   // start-of-step terms; u = v = 0 and w = 0 make those terms harmless here.
-  HIP_TRY(hipMemsetAsync(h->gh_u[0], 0, d.n3 * sizeof(double), s));
-  HIP_TRY(hipMemsetAsync(h->s_n2, 0, d.ni * sizeof(double), s));
+  k_fill<<<blocks(d.n3), TPB, 0, s>>>(d.n3, 0.0, h->gh_u[0]);
+  k_fill<<<blocks(d.ni), TPB, 0, s>>>(d.ni, 0.0, h->s_n2);
   k_phi<<<blocks(d.n2), TPB, 0, s>>>(d, h->p, h->geo, b, h->phi);
   k_momentum_explicit<<<blocks(d.n3), TPB, 0, s>>>(d, h->p, h->geo, h->gh_u[0], h->gh_u[0], b,
                                                    h->phi, h->s_n2, h->Km, pgx, pgy, h->avu,

@@ -47,3 +47,42 @@ def test_steps_match_oracle(hoc, nx, ny, edges, n_split, n_picard):
         for k in ("u", "v", "eta", "T", "S"):
             g, w = getattr(got, k).cpu().numpy(), getattr(want, k)
             assert np.array_equal(g, w), (k, rel_l2(g, w))
+
+
+@pytest.mark.parametrize("n_picard", [2, 4])
+def test_captured_step_replays(hoc, n_picard):
+    """A split step and the pressure gradients in a graph of the caller's,
+    replayed four times with eager steps and a synchronisation between the
+    replays, each time bitwise the eager result: what is cleared inside (the
+    averaged transports from four passes on, the pressure gradients' zero
+    fields) is cleared by kernels."""
+    from hydrostatic_ocean_core_benchmark_amd.types import State3D
+    dom, phys, params, f = _problem(33, 15, 3, "zlevel", "up3")
+    params = dataclasses.replace(params, name="split_explicit", n_split=3, n_picard=n_picard,
+                                 barotropic_average="mean")
+    with hoc.HipStepper(dom, phys, params, 60.0) as st:
+        fin, out = st._inputs(State3D(**f)), st._new_state_buffers()
+        want, other = st._new_state_buffers(), st._new_state_buffers()
+        nu, kappa = st.nu.clone(), st.kappa.clone()
+
+        def eager(src, dst):
+            st.nu.copy_(nu)
+            st.kappa.copy_(kappa)
+            st._step_into(src, dst)
+
+        eager(fin, want)
+        px, py = st.pressure_gradients(fin["b"])
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            eager(fin, out)
+            gx, gy = st.pressure_gradients(fin["b"])
+        for n in range(4):
+            eager(want, other)
+            st.pressure_gradients(other["b"])
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(gx, px) and torch.equal(gy, py), n
+            for k, w in want.items():
+                assert torch.equal(out[k], w), (n, k)
