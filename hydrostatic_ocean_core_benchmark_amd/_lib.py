@@ -172,6 +172,7 @@ PROTOTYPES = {
     "hoc_helm_divgrad": ([i32, i32, f64, f64, VP, VP, VP, VP, VP, VP], i32),
     "hoc_stepper_set_solver_path": ([VP, i32], i32),
     "hoc_stepper_solver_path": ([VP], i32),
+    "hoc_stepper_replayed_iterations": ([VP, C.POINTER(i64)], i32),
     "hoc_stepper_profile_kernel": ([VP, C.c_char_p], i32),
     "hoc_stepper_profile_read": ([VP, C.POINTER(i64), C.POINTER(f64)], i32),
     "hoc_last_error": ([], C.c_char_p),

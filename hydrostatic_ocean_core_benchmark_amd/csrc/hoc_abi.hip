@@ -136,7 +136,8 @@ struct IterGraphs {
   // this many solves on those operands.
   static constexpr int WARM_SOLVES = 8;
   int solves = 0;
-  bool failed = false;  // building failed: launches only
+  long long replayed = 0;  // iterations replayed so far
+  bool failed = false;     // building failed: launches only
   hipGraph_t graph[SIZES] = {};
   hipGraphExec_t exec[SIZES] = {};
   void clear() {
@@ -969,6 +970,7 @@ int pcg_iterations(hoc_stepper* h, const PcgArgs& a, bool replay, hipStream_t s,
     if (e) HIP_TRY(hipGraphLaunch(e, s));
     else TRY(pcg_iteration(h, a, s, it));
     const int n = e ? 2 << q : 1;
+    if (e) h->it_graphs.replayed += n;
     it += n;
     count -= n;
   }
@@ -2566,6 +2568,12 @@ int hoc_stepper_set_solver_path(hoc_stepper* h, int32_t path) {
 int32_t hoc_stepper_solver_path(hoc_stepper* h) {
   if (!h) return -1;
   return (h->pcg_parts > 0 && !h->force_multikernel) ? 0 : 1;
+}
+
+int hoc_stepper_replayed_iterations(hoc_stepper* h, int64_t* n) {
+  if (!h || !n) return fail(HOC_ERR_INVALID, "null argument");
+  *n = h->it_graphs.replayed;
+  return HOC_OK;
 }
 
 int hoc_stepper_profile_kernel(hoc_stepper* h, const char* name) {

@@ -425,6 +425,13 @@ class HipStepper:
         _lib.check(self.lib.hoc_stepper_set_solver_path(self._h, 0 if path == "persistent"
                                                         else 1))
 
+    @property
+    def replayed_iterations(self) -> int:
+        """PCG-Jacobi iterations replayed from graphs so far."""
+        n = C.c_int64()
+        _lib.check(self.lib.hoc_stepper_replayed_iterations(self._h, C.byref(n)))
+        return int(n.value)
+
     # --------------------------------------------------------- measurement
     def profile_kernel(self, name: str | None) -> None:
         """Time every launch of one step kernel with HIP events on its stream."""

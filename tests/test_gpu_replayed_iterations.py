@@ -43,6 +43,8 @@ def test_steps_match_oracle(hoc, max_iter, side_stream):
             other.step(State3D(**f))
             got = st.step(got)
             stream.synchronize()
+            # two solves a step; a run of two needs a third iteration
+            assert (st.replayed_iterations > 0) == (n >= 4 and max_iter >= 3), n
             assert st.solver_iterations == ref.solver_iterations, n
             assert st.solver_failures == ref.solver_failures, n
             for k in ("u", "v", "eta", "T", "S"):
@@ -91,6 +93,7 @@ def test_steps_while_another_thread_captures(hoc):
             except Exception as e:
                 err.append(e)
         assert not err, err
+        assert st.replayed_iterations > 0
         torch.cuda.synchronize()
         for n in range(3):
             graph.replay()
