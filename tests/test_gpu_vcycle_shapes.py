@@ -2,8 +2,9 @@
 where their regions can go wrong: levels smaller than a tile plus its halo
 (the region wraps round the level more than once), partial tiles, coarse
 levels with odd sides, and first levels of the coarse cycle just below and
-above each thread count's cells. Solves from random coefficients, bitwise
-against the oracle and with its iteration counts."""
+above each thread count's cells, with one to three sweeps per side. Solves
+from random coefficients, bitwise against the oracle and with its iteration
+counts."""
 
 from __future__ import annotations
 
@@ -42,15 +43,16 @@ def _stepper(hoc, shape, bc, tile=None, precision="fp64", seed=17, **kw):
     return st, grid, mask, Ku, Kv, rhs
 
 
-@pytest.mark.parametrize("kind,smoother", [("pcg_mg", "rbgs"), ("pcg_mg", "jacobi"),
-                                           ("multigrid", None)])
+@pytest.mark.parametrize("kind,smoother,sweeps", [
+    ("pcg_mg", "rbgs", 2), ("pcg_mg", "jacobi", 2), ("multigrid", None, 2), ("pcg_mg", "rbgs", 1),
+    ("pcg_mg", "rbgs", 3), ("pcg_mg", "jacobi", 1), ("pcg_mg", "jacobi", 3)])
 @pytest.mark.parametrize("shape,levels", SHAPES)
-def test_cycle_matches_oracle(hoc, kind, smoother, shape, levels):
+def test_cycle_matches_oracle(hoc, kind, smoother, sweeps, shape, levels):
     from oracle.helmholtz import HelmholtzVar
     kw = {"solver": kind}
     okw = {}
     if kind == "pcg_mg":
-        okw = {"mg_levels": levels, "mg_smoother": smoother}
+        okw = {"mg_levels": levels, "mg_smoother": smoother, "mg_sweeps": sweeps}
     for tile, bc in ((0, "closed"), (2, "periodic")):
         st, grid, mask, Ku, Kv, rhs = _stepper(hoc, shape, bc, tile, **kw, **okw)
         ny, nx = shape
@@ -63,15 +65,47 @@ def test_cycle_matches_oracle(hoc, kind, smoother, shape, levels):
         assert np.array_equal(got, want), (tile, rel_l2(got, want))
 
 
+def _fp32_oracle(*args, **kw):
+    """The oracle's PCG with its V-cycle in float32: coefficients, masks and
+    every operation (scalars are rounded to the arrays' type), from the
+    rounded residual to the correction, which goes back to float64."""
+    import copy
+
+    from oracle.helmholtz import HelmholtzVar
+
+    class Mixed(HelmholtzVar):
+        def _precondition(self, r):
+            fine = self.levels
+            self.levels = []
+            for op in fine:
+                op = copy.copy(op)
+                for k in ("Ku", "Kv", "mask", "inv_diag"):
+                    setattr(op, k, getattr(op, k).astype(np.float32))
+                self.levels.append(op)
+            z = self._mg_precond(r.astype(np.float32))
+            self.levels = fine
+            assert z.dtype == np.float32
+            return z.astype(np.float64)
+
+    return Mixed(*args, **kw)
+
+
 @pytest.mark.parametrize("sweeps", [1, 2, 3])
-def test_fp32_legs_do_not_depend_on_the_tile(hoc, sweeps):
-    """The fp32 preconditioner: every tile shape gives the same bits."""
-    outs = []
-    for tile in range(4):
-        st, *_, Ku, Kv, rhs = _stepper(hoc, (160, 232), "periodic", tile, "mixed", solver="pcg_mg",
-                                       mg_levels=3, mg_sweeps=sweeps)
+@pytest.mark.parametrize("shape,levels", [((160, 232), 3), ((40, 20), 2), ((24, 512), 5),
+                                          ((130, 64), 2)])
+def test_fp32_cycle_matches_oracle(hoc, shape, levels, sweeps):
+    """The fp32 preconditioner against the same cycle in NumPy, bitwise, at
+    every tile shape (two sweeps; the other numbers have one)."""
+    ny, nx = shape
+    kw = {"mg_levels": levels, "mg_sweeps": sweeps}
+    for tile in range(4 if sweeps == 2 else 1):
+        st, grid, mask, Ku, Kv, rhs = _stepper(hoc, shape, "periodic", tile, "mixed",
+                                               solver="pcg_mg", **kw)
+        if tile == 0:
+            ref = _fp32_oracle(nx, ny, grid.dx, grid.dy, st.cfg.g * 0.25 * 600.0 ** 2, Ku, Kv,
+                               mask, kind="pcg_mg", rtol=1e-12, max_iter=5000, **kw)
+            want, rep = ref.solve(rhs)
         x, iters, conv = st.helmholtz_solve(Ku, Kv, rhs)
-        assert conv
-        outs.append((x.detach().cpu().numpy(), iters))
-    for x, iters in outs[1:]:
-        assert iters == outs[0][1] and np.array_equal(x, outs[0][0])
+        got = x.detach().cpu().numpy()
+        assert conv and rep.converged and iters == rep.iterations, (tile, iters, rep.iterations)
+        assert np.array_equal(got, want), (tile, rel_l2(got, want))
