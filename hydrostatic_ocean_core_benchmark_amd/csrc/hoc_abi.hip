@@ -898,9 +898,22 @@ int pcg_iteration(hoc_stepper* h, const PcgArgs& a, hipStream_t s, int it) {
   return HOC_OK;
 }
 
+// Where the Jacobi iterations are replayed. A launch costs the host 4 to 4.4
+// us, as much as one of these kernels runs on a grid up to ITER_GRAPH_CELLS:
+// per solve launched and replayed, 64 x 64 1732 and 1509 us, 131 x 77 (195
+// iterations) 1861 and 1654, 256 x 256 1870 and 1743, 512 x 512 2828 and 2829,
+// 1024 x 1024 8309 and 8384. The graphs' own launches and the copy of the
+// solution take some of that back, so the larger grids need an iteration per
+// ITER_GRAPH_CELLS_PER_ITER cells: a step alone with 7 iterations per solve 306
+// and 333 us on 256 x 256, with 24 660 and 638, on 362 x 362 with 43 1203 and
+// 1245, with 77 2080 and 2020. The V-cycle's iterations (8 kernels and more, 10
+// to 20 of them) gain nothing: 128 x 128 438 and 427, 512 x 512 676 and 692.
+constexpr long long ITER_GRAPH_CELLS = 1 << 17, ITER_GRAPH_CELLS_PER_ITER = 2048;
+
 // Whether the Jacobi iterations on the step's own operands may be replayed on
-// stream s: after WARM_SOLVES solves with them, not while a phase is profiled
-// by name or the caller captures the stream.
+// stream s: after WARM_SOLVES solves with them, with enough iterations in the
+// last one, not while a phase is profiled by name or the caller captures the
+// stream.
 bool iteration_graphs_usable(hoc_stepper* h, hipStream_t s) {
   IterGraphs& g = h->it_graphs;
   if (h->prof_name == "k_pcg_ap" || h->prof_name == "k_pcg_update") return false;
@@ -909,7 +922,8 @@ bool iteration_graphs_usable(hoc_stepper* h, hipStream_t s) {
     if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
       return false;
   }
-  return ++g.solves > IterGraphs::WARM_SOLVES && !g.failed;
+  return ++g.solves > IterGraphs::WARM_SOLVES && !g.failed &&
+         h->last_iters >= h->d.n2 / ITER_GRAPH_CELLS_PER_ITER;
 }
 
 // The graph of 2 << q iterations from an even one on, built on first use; null
@@ -950,13 +964,7 @@ hipGraphExec_t iteration_graph(hoc_stepper* h, PcgArgs a, int q) {
 // PCG iterations it .. it + count - 1 (it is advanced). replay: runs of Jacobi
 // iterations with an even first number are replayed from graphs of 64, 32, ..,
 // 2 iterations and only the rest is launched; the replayed kernels take the
-// iteration's number from the device. A launch costs the host 4 to 4.4 us, as
-// much as one of these kernels runs on a grid up to ITER_GRAPH_CELLS: per solve
-// launched and replayed, 64 x 64 1732 and 1509 us, 131 x 77 (195 iterations)
-// 1861 and 1654, 256 x 256 1870 and 1743, 512 x 512 2828 and 2829, 1024 x 1024
-// 8309 and 8384. The V-cycle's iterations (8 kernels and more, 10 to 20 of
-// them) gain nothing: 128 x 128 438 and 427, 512 x 512 676 and 692.
-constexpr long long ITER_GRAPH_CELLS = 1 << 17;
+// iteration's number from the device.
 int pcg_iterations(hoc_stepper* h, const PcgArgs& a, bool replay, hipStream_t s, int& it,
                    int count) {
   while (count > 0) {

@@ -198,8 +198,9 @@ int32_t hoc_stepper_solver_path(hoc_stepper* h);
 
 /* PCG-Jacobi iterations the handle's solves have replayed from graphs, those
  * past a solve's convergence included (path 1, up to 131072 columns, from the
- * ninth solve on; the results are those of launches). No reference
- * counterpart: tells a replay from its fallback. */
+ * ninth solve on where the solve before took an iteration per 2048 columns;
+ * the results are those of launches). No reference counterpart: tells a replay
+ * from its fallback. */
 int hoc_stepper_replayed_iterations(hoc_stepper* h, int64_t* n);
 
 /* Time every launch of one step kernel (e.g. "k_tracers") with HIP events

@@ -101,3 +101,23 @@ def test_steps_while_another_thread_captures(hoc):
             assert torch.all(y == n + 1.0), n
         for k, w in want.items():
             assert torch.equal(got[k], w), k
+
+
+@pytest.mark.parametrize("dt,replays", [(20.0, False), (600.0, True)])
+def test_few_iterations_are_launched(hoc, dt, replays):
+    """256 x 256: 7 iterations a solve are launched, 77 replayed (from 32 on at
+    this size), with the bits of a handle whose phases are profiled by name,
+    which launches all."""
+    dom, phys, params, f = _problem(256, 256, 2, "zlevel", "up3_tvd")
+    params = dataclasses.replace(params, name="theta")
+    ends = []
+    for name in (None, "k_pcg_ap"):
+        with hoc.HipStepper(dom, phys, params, dt) as st:
+            st.profile_kernel(name)
+            a, b = st._new_state_buffers(), st._new_state_buffers()
+            for k, buf in a.items():
+                buf.copy_(torch.as_tensor(f[k]))
+            ends.append({k: x.clone() for k, x in st._step_n_into(a, b, 7).items()})
+            assert (st.replayed_iterations > 0) == (replays and name is None)
+    for k, want in ends[1].items():
+        assert torch.equal(ends[0][k], want), k
