@@ -200,7 +200,7 @@ struct hoc_stepper {
   int* host_flag = nullptr;     // pinned: done, iters
   Reducer red;
   int last_iters = 8;
-  int sync_free_budget = 0;
+  int sync_free_budget = 0;  // > 0: PCG solves launch this many iterations, no host polling
   // sync-free solves replayed as one HIP graph (captured on first use, again
   // when any operand pointer, the budget or the leg tile shape changes)
   hipGraph_t sf_graph = nullptr;
@@ -212,7 +212,7 @@ struct hoc_stepper {
   int mg_tile_shape = 0;     // fused V-cycle leg tile shape (0..MG_TILE_SHAPES-1)
                              // default by size: 16x16 up to 512x512 columns
                              // (5.50 vs 5.66 ms/step at 512x512x40), else 32x16
-                             // (26.11 vs 26.33 ms/step at 1024x1024x60)  // > 0: PCG solves launch this many iterations, no host polling
+                             // (26.11 vs 26.33 ms/step at 1024x1024x60)
   // multigrid hierarchy (level 0 = the model grid)
   static constexpr int MAXLEV = 12;
   int nlev = 1;
@@ -866,7 +866,8 @@ int precondition(hoc_stepper* h, const double* r, double* z, hipStream_t s) {
     }
     const float* ec = h->mgf_x[l0];
     for (int l = l0 - 1; l >= 0; --l) {
-      launch_mg_up_f32(S, h->mg_tile_shape, s, h->levf[l], om, h->mgf_x[l], ec, l == 0 ? r : nullptr, l == 0 ? nullptr : h->mgf_b[l],
+      launch_mg_up_f32(S, h->mg_tile_shape, s, h->levf[l], om, h->mgf_x[l], ec,
+                       l == 0 ? r : nullptr, l == 0 ? nullptr : h->mgf_b[l],
                        l == 0 ? z : nullptr, l == 0 ? nullptr : h->mgf_t[l], h->sc);
       ec = h->mgf_t[l];
     }
@@ -2108,8 +2109,8 @@ int hoc_stepper_tke_step(hoc_stepper* h, const double* e_in, const double* u, co
     launch_closure_lengths(d, h->p, h->geo, e_in, u, v, b, h->s_n2, h->s_sh, h->s_l, h->s_le, s);
   }
   { ProfScope _ps(h, "k_closure", s);
-  launch_closure(s, d, h->p, h->geo, e_in, h->Km, h->Kh, e_out, h->s_n2,
-                                         h->s_sh, h->s_l, h->s_le, h->s_c); }
+  launch_closure(s, d, h->p, h->geo, e_in, h->Km, h->Kh, e_out, h->s_n2, h->s_sh, h->s_l,
+                 h->s_le, h->s_c); }
   LAUNCH_CHECK("k_closure");
   return HOC_OK;
 }
@@ -2254,9 +2255,8 @@ static int step_impl(hoc_stepper* h, const hoc_state* in, hoc_state* out, void* 
   // phi, the transports of the state (theta, split_explicit) and, unless the
   // previous step formed it, w of the state: one column pass
   { ProfScope _ps(h, "k_prologue", s);
-  launch_prologue(s, d, p, geo, in->u, in->v, in->b, h->phi,
-                                          (theta || split) ? h->U0 : nullptr, h->V0,
-                                          w_ready ? nullptr : h->w); }
+  launch_prologue(s, d, p, geo, in->u, in->v, in->b, h->phi, (theta || split) ? h->U0 : nullptr,
+                  h->V0, w_ready ? nullptr : h->w); }
   if (tape)
     HIP_TRY(hipMemcpyAsync(tape->w_old, h->w, d.ni * sizeof(double), hipMemcpyDeviceToDevice, s));
   { ProfScope _ps(h, "k_momentum_explicit", s);
@@ -2302,8 +2302,7 @@ static int step_impl(hoc_stepper* h, const hoc_state* in, hoc_state* out, void* 
         // the last pass: back-substitution and w of the new velocity in one
         // column pass (the tracers read w next)
         ProfScope _ps(h, "k_backsub_w", s);
-        launch_backsub_w(s, d, p, geo, gu, gv, h->q, out->eta, out->u,
-                                                 out->v, h->w);
+        launch_backsub_w(s, d, p, geo, gu, gv, h->q, out->eta, out->u, out->v, h->w);
       } else {
         ProfScope _ps(h, "k_backsub", s);
         k_backsub<<<blocks(d.n3), TPB, 0, s>>>(d, p, geo, gu, gv, h->q, out->eta, out->u,
@@ -2331,9 +2330,8 @@ static int step_impl(hoc_stepper* h, const hoc_state* in, hoc_state* out, void* 
     launch_w_diag(s, d, p, geo, out->u, out->v, h->w);
   }
   { ProfScope _ps(h, "k_tracers", s);
-  launch_tracers((h->fp32_parts & HOC_FP32_TRACER_FLUX) != 0, s, d, p, geo, in->T, in->S,
-                       in->b, out->u, out->v,
-                       h->w, h->Kh, h->cst_b, out->T, out->S, out->b); }
+  launch_tracers((h->fp32_parts & HOC_FP32_TRACER_FLUX) != 0, s, d, p, geo, in->T, in->S, in->b,
+                 out->u, out->v, h->w, h->Kh, h->cst_b, out->T, out->S, out->b); }
   LAUNCH_CHECK("k_tracers");
   h->tridiagonal_solves += ts ? 2 : 1;
   if (ts) h->eos_cells += d.n3;

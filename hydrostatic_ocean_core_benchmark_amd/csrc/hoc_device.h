@@ -8,7 +8,9 @@
 //
 // Every arithmetic expression keeps the operand order of the reference's
 // NumPy code and the library is built with -ffp-contract=off, so no
-// multiply-add is fused and results are bitwise those of the oracle.
+// multiply-add is fused and results are bitwise those of the oracle, in the
+// range of Divisor's quotients: numerators of 2^-969 and above, quotients that
+// do not overflow.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -301,7 +303,8 @@ __device__ __forceinline__ F half_superbee(F r) {
 // 1990), so the quotient has the same bits: 4 instructions against 11 with a quarter-rate
 // reciprocal. Without the scaling that holds for a normal divisor of moderate exponent
 // (every spacing, thickness and pivot here) and numerators that are 0, non-finite or of
-// magnitude 2^-969 and above; below that the last bit may differ.
+// magnitude 2^-969 and above; below that the last bit may differ, and a quotient that
+// overflows is NaN instead of infinite.
 template <class F>
 struct Divisor;
 template <>

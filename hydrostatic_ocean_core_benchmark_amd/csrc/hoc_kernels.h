@@ -349,11 +349,12 @@ __global__ void k_seq_sum(const double* part, long long nchunks, double* out);
 
 namespace hoc {
 
-// PCG arguments. Full 8192-element chunks are cut into `sub` aligned
+// PCG arguments. Full 8192-element chunks are cut into PCG_SUB aligned
 // subtrees of the pairwise tree, one workgroup each; the trailing partial
-// chunk, if any, adds one workgroup per leaf of its plan. Partial sums land
-// in part_*[part]; the consumer of a sum rebuilds each chunk's top levels
-// and the in-order chunk sum.
+// chunk, if any, adds one workgroup per slot of its halving tree filled up to
+// a perfect one (tail_slots, a power of two). Partial sums land in
+// part_*[part]; the consumer of a sum rebuilds each chunk's top levels and
+// the in-order chunk sum.
 struct PcgArgs {
   Dims d;
   HelmOp op;
@@ -384,9 +385,8 @@ constexpr int PCG_MAX_CHUNKS = 1024;
 constexpr int PCG_COOP_CHUNKS = 256;  // ... of the cooperative launch
 constexpr int PCG_COOP_CS = PCG_COOP_CHUNKS + 8;
 
-// One level of the multigrid hierarchy (level 0 is the model grid).
-// One multigrid level: face coefficients, diagonal and constants in the
-// arithmetic type R (double for the solvers, float for the mixed-precision
+// One level of the multigrid hierarchy (level 0 is the model grid): face
+// coefficients, diagonal and constants in the arithmetic type R (double for the solvers, float for the mixed-precision
 // V-cycle preconditioner); the mask is shared.
 template <class R>
 struct MgLevelT {

@@ -597,7 +597,7 @@ __global__ __launch_bounds__((JacRegion<S, TW, TH>::NT)) void k_mg_up(
 // tiles) and from 6.1 and 5.7 to 5.2 and 5.1 under 512 x 512. The stationary
 // multigrid's level-0 sweeps start from x_in with one more cell of halo; in
 // legs its cycle on 400 x 400 takes 4 launches fewer per level, and a solve
-// 0.55 instead of 1.28 ms.
+// 0.49 instead of 1.28 ms.
 // One cell of a thread's pair: its coefficients towards the horizontal
 // neighbour outside the pair and to the north and south, its right-hand
 // side, 1/diag and mask, the LDS positions of those neighbours and of itself.
@@ -815,7 +815,9 @@ __global__ __launch_bounds__((RbRegion<2 * S, TW, TH>::NT)) void k_mg_up_rb(
 // buffers, because a level with an odd periodic side has same-colour
 // neighbours across the wrap, whose old values the reference reads.
 // The three levels from 32 x 32 down: 11.2 us against 14.9 with every field
-// in LDS and 1024 threads (rbgs), 10.4 against 14.7 (Jacobi).
+// in LDS and 1024 threads (rbgs), 10.4 against 14.7 (Jacobi). The 1024 x 4 form
+// (a last level of 2049 to 4096 cells) does not fit its 128 registers: 78 are
+// spilled in fp64 (304 bytes a lane), 14 in fp32 (60).
 template <class R>
 struct CycCell {
   R inv, b, ke, kw, kn, ks, m;

@@ -11,7 +11,8 @@
 //   cell kernels: one lane per (k, j, i) for the pure 3D stencils.
 //
 // Column recurrences keep their forward-sweep values (c*, d*) in LDS where the
-// column fits (COL_LDS_MAX), in global scratch for deeper ones.
+// column fits (COL_LDS_MAX; the closure's rule is narrower), in global scratch
+// for deeper ones.
 #include <type_traits>
 
 #include "hoc_device.h"
@@ -969,8 +970,8 @@ __device__ __forceinline__ double avg_u_to_v(const double* u, const uint8_t* mu,
 
 // Mean over the open ones of four faces (libs/core/operators_masked.py:46-61):
 // the weighted sum over the number of open faces, in the reference's order.
-// The quotient by 1, 2, 3 or 4 is formed like Divisor's, whose reciprocals are
-// the constants here.
+// The quotient by 1, 2, 3 or 4 is formed like Divisor's, in the same range, whose
+// reciprocals are the constants here.
 struct Avg4 {
   double w[4], den, y, own;
   bool any;

@@ -4,7 +4,8 @@
 // so every value is read from HBM about once instead of once per stencil
 // point; the column's own vertical neighbours stay in a register window.
 // Arithmetic and operand order are those of the untiled kernels (and of the
-// reference's NumPy expressions), so the results are bitwise the same.
+// reference's NumPy expressions), so the results are bitwise the same (in the
+// range stated at Divisor).
 #include <type_traits>
 
 #include "hoc_device.h"
