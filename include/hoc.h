@@ -314,7 +314,8 @@ int hoc_stepper_set_sync_free(hoc_stepper* h, int32_t budget);
 
 /* Tile shape of the fused multigrid V-cycle legs of pcg_mg (no reference
  * counterpart; a launch choice for the autotuner, the results are the same
- * bits for every shape): 0 32x16 (default), 1 64x8, 2 16x16, 3 64x16 cells. */
+ * bits for every shape): 0 32x16, 1 64x8, 2 16x16, 3 64x16 cells; by default 2
+ * up to 512 x 512 columns, else 0. Fewer or more sweeps than 2 use 0. */
 int hoc_stepper_set_mg_tile(hoc_stepper* h, int32_t shape);
 
 /* The parts of a mixed-precision step that run in fp32 (no reference
