@@ -989,9 +989,7 @@ struct Avg4 {
   }
   __device__ __forceinline__ double operator()(double a0, double a1, double a2, double a3) const {
     const double num = 0.0 + w[0] * a0 + w[1] * a1 + w[2] * a2 + w[3] * a3;
-    const double q = num * y;
-    const double r = __builtin_fma(-den, q, num);
-    const double m = __builtin_amdgcn_div_fixup(__builtin_fma(r, y, q), den, num);
+    const double m = __builtin_amdgcn_div_fixup(scaled_quotient(num, den, y), den, num);
     return (any ? m : 0.0) * own;
   }
 };
