@@ -815,9 +815,8 @@ __global__ __launch_bounds__((RbRegion<2 * S, TW, TH>::NT)) void k_mg_up_rb(
 // buffers, because a level with an odd periodic side has same-colour
 // neighbours across the wrap, whose old values the reference reads.
 // The three levels from 32 x 32 down: 11.2 us against 14.9 with every field
-// in LDS and 1024 threads (rbgs), 10.4 against 14.7 (Jacobi). The 1024 x 4 form
-// (a last level of 2049 to 4096 cells) does not fit its 128 registers: 78 are
-// spilled in fp64 (304 bytes a lane), 14 in fp32 (60).
+// in LDS and 1024 threads (rbgs), 10.4 against 14.7 (Jacobi). A last level of
+// more than 1024 cells is k_mg_last_level's.
 template <class R>
 struct CycCell {
   R inv, b, ke, kw, kn, ks, m;
@@ -946,11 +945,13 @@ __device__ __forceinline__ void cyc_residual(const MgLevelT<R>& L, const CycCell
   __syncthreads();
 }
 
-template <class R, class RB, class RO, int NT, int Q>
-__global__ __launch_bounds__(NT) void k_mg_coarse_cycle(MgCycleT<R> C, R omega, int S,
-                                                        const RB* __restrict__ b0,
-                                                        const R* x0, RO* out,
-                                                        const PcgScalars* sc) {
+constexpr int CYC_THREADS = 256, CYC_CELLS = MG_COARSE_MAX / CYC_THREADS;
+template <class R, class RB, class RO>
+__global__ __launch_bounds__(CYC_THREADS) void k_mg_coarse_cycle(MgCycleT<R> C, R omega, int S,
+                                                                 const RB* __restrict__ b0,
+                                                                 const R* x0, RO* out,
+                                                                 const PcgScalars* sc) {
+  constexpr int NT = CYC_THREADS, Q = CYC_CELLS;
   const bool done = finished(sc);  // tested once the loads are on their way
   extern __shared__ __align__(16) unsigned char cyc_raw[];
   R* cyc = reinterpret_cast<R*>(cyc_raw);
@@ -1049,6 +1050,122 @@ __global__ __launch_bounds__(NT) void k_mg_coarse_cycle(MgCycleT<R> C, R omega, 
     if (K0[q].on) out[K0[q].c] = (RO)v0[q];
 }
 
+// A last level alone of 1025 to MG_COARSE_LAST_MAX cells in one workgroup: S
+// sweeps and S reversed ones from x0 (null: zero), the same arithmetic per cell
+// as k_mg_coarse_cycle's. RBS: red-black Gauss-Seidel, else damped Jacobi. A
+// thread owns P pairs of consecutive cells, which are one red and one black on
+// any width, so a half-sweep updates one cell of each pair; coefficients,
+// right-hand sides and values are in registers, the fields neighbours read in
+// LDS (two buffers of n0 values).
+// Bound by latency, and with 16 waves by LDS reads. A solve on one level of
+// 64 x 64, rbgs and Jacobi: 1207 and 1655 us; with every field in LDS and the
+// coefficients from memory 2187 and 2587; in the form above, where cells of both
+// colours compute in every half-sweep and four cells per thread spill 78
+// registers, 2885 and 3070. On 50 x 50 1155 and 1634, 1506 and 1983, 2788 and 2988.
+template <class R>
+struct LastCell {
+  R inv, b, ke, kw, kn, ks, m;
+  int c, ce, cw, cn, cs;
+  bool on;
+};
+template <class R, class RB, class RO, int P, bool RBS>
+__global__ __launch_bounds__(1024) void k_mg_last_level(MgLevelT<R> L, R omega, int S,
+                                                        const RB* __restrict__ b0, const R* x0,
+                                                        RO* out, const PcgScalars* sc) {
+  const bool done = finished(sc);  // tested once the loads are on their way
+  extern __shared__ __align__(16) unsigned char last_raw[];
+  const int n = (int)L.n;
+  R* cur = reinterpret_cast<R*>(last_raw);
+  R* next = cur + n;
+  LastCell<R> K[P][2];  // a pair's red and black cell
+  R v[P][2];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int c0 = 2 * ((int)threadIdx.x + p * 1024);
+    const int j0 = c0 / L.nx, black = (c0 - j0 * L.nx + j0) & 1;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      LastCell<R>& k = K[p][q];
+      const int c = c0 + (q ^ black);
+      k.on = c < n;
+      k.c = k.on ? c : 0;
+      const int j = k.c / L.nx, i = k.c - j * L.nx;
+      k.ce = j * L.nx + wrap(i, 1, L.nx);
+      k.cw = j * L.nx + wrap(i, -1, L.nx);
+      k.cn = wrap(j, 1, L.ny) * L.nx + i;
+      k.cs = wrap(j, -1, L.ny) * L.nx + i;
+      k.inv = L.inv_diag[k.c];
+      k.b = (R)b0[k.c];
+      k.ke = L.Ku[k.c];
+      k.kw = L.Ku[k.cw];
+      k.kn = L.Kv[k.c];
+      k.ks = L.Kv[k.cs];
+      k.m = mkr<R>(L.mask[k.c]);
+      v[p][q] = x0 ? x0[k.c] : R(0);
+    }
+  }
+  auto put = [&] {
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        if (K[p][q].on) next[K[p][q].c] = v[p][q];
+    __syncthreads();
+    R* t = cur;
+    cur = next;
+    next = t;
+  };
+  put();  // the starting field
+  if (done) return;
+  const Divisor<R> by_dx2 = uniform_divisor<R>(L.dx2), by_dy2 = uniform_divisor<R>(L.dy2);
+  for (int s = 0; s < 2 * S; ++s) {
+    if constexpr (RBS) {
+      const bool reverse = s >= S;
+      auto half = [&](auto colour, bool last) {
+        constexpr int q = decltype(colour)::value;
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          const LastCell<R>& k = K[p][q];
+          v[p][q] = rbgs_from<R>(k.inv, k.b, L.cx, L.cy, k.ke, k.kw, k.kn, k.ks, cur[k.ce],
+                                 cur[k.cw], cur[k.cn], cur[k.cs]);
+          if (last) {
+            v[p][0] = v[p][0] * K[p][0].m;
+            v[p][1] = v[p][1] * K[p][1].m;
+          }
+        }
+        put();
+      };
+      using Red = std::integral_constant<int, 0>;
+      using Black = std::integral_constant<int, 1>;
+      if (reverse) {
+        half(Black{}, false);
+        half(Red{}, true);
+      } else {
+        half(Red{}, false);
+        half(Black{}, true);
+      }
+    } else {
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const LastCell<R>& k = K[p][q];
+          const R xc = v[p][q];
+          const R lap = by_dx2(k.ke * (cur[k.ce] - xc) - k.kw * (xc - cur[k.cw])) +
+                        by_dy2(k.kn * (cur[k.cn] - xc) - k.ks * (xc - cur[k.cs]));
+          const R ax = (xc - L.coef * lap) * k.m + xc * (R(1) - k.m);
+          v[p][q] = xc + omega * (k.inv * (k.b - ax)) * k.m;
+        }
+      put();
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      if (K[p][q].on) out[K[p][q].c] = (RO)v[p][q];
+}
+
 // LDS of a cycle: two field buffers and the residual, the lower levels'
 // right-hand sides and x_S, and their coefficients when they fit.
 template <class R>
@@ -1078,44 +1195,50 @@ template size_t mg_cycle_layout<double>(MgCycle&);
 template size_t mg_cycle_layout<float>(MgCycleF&);
 
 namespace {
-// Threads and cells per thread by the first level's cells: 256 x 4 up to 1024
-// cells (one wave per SIMD: the barriers of 16 waves cost more than their
-// parallelism gives), 1024 x 2 and 1024 x 4 beyond (a last level alone).
-template <class R, class RB, class RO>
-const void* cycle_kernel(long long n0) {
-  if (n0 <= 1024) return (const void*)k_mg_coarse_cycle<R, RB, RO, 256, 4>;
-  if (n0 <= 2048) return (const void*)k_mg_coarse_cycle<R, RB, RO, 1024, 2>;
-  return (const void*)k_mg_coarse_cycle<R, RB, RO, 1024, 4>;
+// go(kernel, threads) for the cycle's first level of n0 cells: the cycle up to
+// MG_COARSE_MAX, beyond that (a last level alone) one or two pairs of cells for
+// each of 1024 threads.
+template <class R, class RB, class RO, class Cycle, class Last>
+auto with_cycle(long long n0, bool rb, const Cycle& cycle, const Last& last) {
+  if (n0 <= MG_COARSE_MAX) return cycle(k_mg_coarse_cycle<R, RB, RO>);
+  if constexpr (std::is_same_v<R, double>) {
+    if (rb)
+      return n0 <= 2048 ? last(k_mg_last_level<R, RB, RO, 1, true>)
+                        : last(k_mg_last_level<R, RB, RO, 2, true>);
+  }
+  return n0 <= 2048 ? last(k_mg_last_level<R, RB, RO, 1, false>)
+                    : last(k_mg_last_level<R, RB, RO, 2, false>);
 }
 template <class R, class RB, class RO>
-int cycle_lds(long long n0, size_t lds) {
-  if (lds > MG_CYCLE_LDS || n0 > MG_COARSE_LAST_MAX) return -1;
-  return hipFuncSetAttribute(cycle_kernel<R, RB, RO>(n0),
-                             hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)lds) == hipSuccess
-             ? 0
-             : -2;
+int cycle_lds(const MgCycleT<R>& C, size_t lds) {
+  const long long n0 = C.lev[0].n;
+  if (lds > MG_CYCLE_LDS || n0 > MG_COARSE_LAST_MAX || (n0 > MG_COARSE_MAX && C.nl != 1))
+    return -1;
+  auto set = [&](auto kernel) {
+    return hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds) == hipSuccess
+               ? 0
+               : -2;
+  };
+  return with_cycle<R, RB, RO>(n0, C.rb != 0, set, set);
 }
 template <class R, class RB, class RO>
 void launch_cycle(const MgCycleT<R>& C, size_t lds, R omega, int S, const RB* b0, const R* x0,
                   RO* out, const PcgScalars* sc, hipStream_t s) {
-  const long long n0 = C.lev[0].n;
-  if (n0 <= 1024)
-    k_mg_coarse_cycle<R, RB, RO, 256, 4><<<1, 256, lds, s>>>(C, omega, S, b0, x0, out, sc);
-  else if (n0 <= 2048)
-    k_mg_coarse_cycle<R, RB, RO, 1024, 2><<<1, 1024, lds, s>>>(C, omega, S, b0, x0, out, sc);
-  else
-    k_mg_coarse_cycle<R, RB, RO, 1024, 4><<<1, 1024, lds, s>>>(C, omega, S, b0, x0, out, sc);
+  with_cycle<R, RB, RO>(
+      C.lev[0].n, C.rb != 0,
+      [&](auto kernel) { kernel<<<1, CYC_THREADS, lds, s>>>(C, omega, S, b0, x0, out, sc); },
+      [&](auto kernel) { kernel<<<1, 1024, lds, s>>>(C.lev[0], omega, S, b0, x0, out, sc); });
 }
 }  // namespace
 
 int mg_cycle_prepare(const MgCycle& C, size_t lds) {
-  return cycle_lds<double, double, double>(C.lev[0].n, lds);
+  return cycle_lds<double, double, double>(C, lds);
 }
 
 int mg_cycle_prepare_f32(const MgCycleF& C, size_t lds) {
-  const int rc = cycle_lds<float, double, double>(C.lev[0].n, lds);
-  return rc ? rc : cycle_lds<float, float, float>(C.lev[0].n, lds);
+  const int rc = cycle_lds<float, double, double>(C, lds);
+  return rc ? rc : cycle_lds<float, float, float>(C, lds);
 }
 
 void launch_mg_coarse_cycle(const MgCycle& C, size_t lds, double omega, int S, const double* b0,

@@ -19,10 +19,11 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 # (ny, nx), levels: a 12-wide level in a 64-wide region; 10-cell sides; 25 x 17
-# and 1023-, 1024-, 1056-, 2048- and 2080-cell last levels
+# and 1023-, 1024-, 1056-, 2048-, 2080-, 4050- and 4095-cell last levels (65 x 32,
+# 90 x 45 and 63 x 65 with odd sides)
 SHAPES = [((512, 24), 5), ((24, 512), 5), ((40, 20), 2), ((100, 50), 5), ((8, 8), 5),
           ((100, 68), 3), ((66, 62), 2), ((64, 64), 2), ((66, 64), 2), ((128, 64), 2),
-          ((130, 64), 2), ((180, 90), 2)]
+          ((130, 64), 2), ((180, 90), 2), ((63, 65), 1)]
 
 
 @pytest.fixture(scope="module")
@@ -92,7 +93,7 @@ def _fp32_oracle(*args, **kw):
 
 @pytest.mark.parametrize("sweeps", [1, 2, 3])
 @pytest.mark.parametrize("shape,levels", [((160, 232), 3), ((40, 20), 2), ((24, 512), 5),
-                                          ((130, 64), 2)])
+                                          ((130, 64), 2), ((128, 64), 2), ((63, 65), 1)])
 def test_fp32_cycle_matches_oracle(hoc, shape, levels, sweeps):
     """The fp32 preconditioner against the same cycle in NumPy, bitwise, at
     every tile shape (two sweeps; the other numbers have one)."""
