@@ -145,7 +145,7 @@ struct TracerFaceRegs {
 // memory than with the solve in the same march (67 us of traffic at 512 x 512
 // x 40), which marched 64 tiles at 128 x 128 with the recurrence in every
 // level. Both kernels per step, before -> now: 128 x 4 x 20 135 -> 24 us,
-// 128 x 128 x 30 224 -> 64, 512 x 512 x 40 689 -> 426, 1000 x 1000 x 30 1690 ->
+// 128 x 128 x 30 224 -> 64, 512 x 512 x 40 689 -> 430, 1000 x 1000 x 30 1690 ->
 // 1179; fp32 fluxes at 640 x 512 x 48 1244 -> 626.
 template <class R, bool ZC, bool TVD>
 __global__ __launch_bounds__(TILE_THREADS) void k_tracer_rhs(
@@ -927,7 +927,7 @@ __device__ __forceinline__ void momentum_component(
 // resident workgroups left a third of the second round idle, and 64 tiles of
 // 128 x 128 three quarters of the chip). Measured per launch, before -> now:
 // 128 x 4 x 20 132 -> 11 us, 128 x 128 x 30 204 -> 37, 512 x 512 x 40 600 ->
-// 373, 1000 x 1000 x 30 1487 -> 1097. At 4 waves per SIMD it spilled 30
+// 377, 1000 x 1000 x 30 1487 -> 1097. At 4 waves per SIMD it spilled 30
 // registers and took 478 us at 512 x 512 x 40 (364 at 3).
 template <class R, bool ZC, bool TVD>
 __global__ __launch_bounds__(TILE_THREADS) __attribute__((amdgpu_waves_per_eu(3))) void k_momentum_explicit_tiled(
