@@ -306,7 +306,7 @@ __device__ __forceinline__ F half_superbee(F r) {
 // 2^960 on and quotients that overflow give NaN. Without the scaling (4 instructions) the
 // remainder underflows for numerators below 2^-969, which the tails of column solves reach
 // where a wall is some 100 levels deep; it costs the momentum and tracer kernels up to 4% (512 x
-// 512 x 40 367 -> 377 and 251 -> 261 us), the others less, a step about 0.5%.
+// 512 x 40 367 -> 377 and 251 -> 261 us), the others less, a step 0.3 to 1.2%.
 __device__ __forceinline__ double scaled_quotient(double a, double d, double y) {
   const double t = a * 0x1p64;
   const double q = t * y;
